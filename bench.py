@@ -618,7 +618,7 @@ def main():
                                    "frac": round(tflops / 2500.0, 5)}
     if a.prefill_tokens > 1 and B == 1 and a.prefill_tokens <= a.ctx:
         progress("prefill")
-        # prompt prefill: positions 0..n-2 in chunks of up to 256 through the MFMA GEMMs
+        # prompt prefill: positions 0..n-2 in chunks of up to 4096 through the MFMA GEMMs
         # (prefill.h); the last prompt position is the first decode step (not part of this timing)
         n = a.prefill_tokens
         ids = [(1 + 7919 * i) % cfg.vocab_size for i in range(n)]
@@ -634,45 +634,21 @@ def main():
         layer_bytes = wbytes - cfg.vocab_size * cfg.hidden_size * wb_el / world  # this rank's layer weights
         params = layer_bytes / wb_el
         mfma = model.prefill_path() == "mfma"  # the path the engine took (sli_model_prefill_path)
-        chunks = []  # (valid rows, padded rows) per chunk (engine.hip kPfSizes)
-        for p0 in range(0, n - 1, 256):
-            nv = min(256, n - 1 - p0)
-            chunks.append((nv, next(m for m in (32, 64, 128, 256) if nv <= m)))
-        # weight passes: a GEMM workgroup reads its weight rows once per BM chunk rows (engine.hip
-        # StepRecorder::pg tilings); the workgroups of one row block share an XCD and run together, so HBM
-        # sees ~one pass per chunk and the rest are L2 hits (PMC: profiles/r3_prefill_pmc.txt)
-        D, Il, QD = cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads * cfg.head_dim
-        KVD = cfg.num_key_value_heads * cfg.head_dim
-        role_w = {"qkv": D * (QD + 2 * KVD), "gu": 2 * D * Il, "out": D * QD + D * Il}
-        tot_w = float(sum(role_w.values()))
-
-        def bm(role, M):  # chunk rows per workgroup (engine.hip StepRecorder::pg_pick)
-            if M == 32:
-                return 32
-            if role == "out":
-                return 64 if M == 256 else 32
-            if a.w_dtype == "i8":
-                if role == "gu":
-                    return 128 if M == 128 else 64
-                return 128 if M == 256 else 64
-            if M == 64 or (M == 128 and role == "qkv"):
-                return 64
-            if M == 256 and role == "gu":
-                return 64
-            return 128
-        passes = sum(role_w[r] / tot_w * (M // bm(r, M)) for _, M in chunks for r in role_w)
+        chunks = []  # (valid rows, rows of the launches) per weight pass (engine.hip pf_rows, prefill.h kPfMaxChunk)
+        for p0 in range(0, n - 1, 4096):
+            nv = min(4096, n - 1 - p0)
+            chunks.append((nv, 32 if nv <= 32 else 64 if nv <= 64 else -(-nv // 128) * 128))
         useful = 2.0 * params * (n - 1) * world  # whole-job flops of the projections (1 flop per MAC x 2)
         issued = 4.0 * params * sum(M for _, M in chunks) * world  # hi + lo MFMAs over the padded rows
         out["prefill"] = {"prompt_tokens": n, "positions_prefilled": n - 1,
                           "chunks": [{"rows": nv, "padded": M} for nv, M in chunks],
                           "seconds": round(tp, 5), "tokens_per_s": round((n - 1) / tp, 1),
                           "hbm_weight_passes": len(chunks) if mfma else n - 1,
-                          "l2_weight_passes": round(passes, 2) if mfma else n - 1,
                           "projection_tflops": round(useful / tp / 1e12, 2),
                           "mfma_issued_tflops": round(issued / tp / 1e12, 2) if mfma else None,
                           "mfma_peak_tflops": 2500.0,
                           "path": ("MFMA pgemm (v_mfma_f32_16x16x32_f16, fp16 hi + lo activations), chunks of "
-                                   "<= 256 positions, block-causal attention" if mfma
+                                   "<= 4096 positions, block-causal attention" if mfma
                                    else "decode step, teacher-forced (sli_model_prefill_path = 0: fp32 weights, an "
                                         "unsupported shard shape, or a TP rank without an RCCL communicator)"),
                           "vs_token_by_token_s": round((n - 1) * ms * 1e-3, 4)}

@@ -197,7 +197,7 @@ int sli_model_set_prompt_seq(sli_model* m, int32_t seq, const int32_t* ids, int3
 int sli_model_get_state_seq(sli_model* m, int32_t seq, int32_t* pos, int32_t* token, int32_t* last_argmax,
                             int32_t* error);
 /* Prompt prefill (batch-1 models): positions 0 .. n-2 of the prompt run through the layers in chunks of up
- * to 256 positions, every projection one MFMA GEMM over the chunk and attention block-causal over the
+ * to 4096 positions, every projection one MFMA GEMM over the chunk and attention block-causal over the
  * cache (fp16 / int8 weights, head_dim 64 / 128; otherwise through the decode step, teacher-forced; under
  * multi-process tensor parallelism every rank calls it, the chunk's residual rows all-reduced over RCCL
  * twice per layer), filling the K/V cache; the state is left at

@@ -104,14 +104,13 @@ struct sli_model {
     unsigned long long* bkeys = nullptr;  // [B] per-sequence argmax keys (all-reduced MAX under TP)
     int key_ld = 0;                       // per-sequence stride of the per-workgroup argmax keys
     // prompt prefill (sli_model_prefill, prefill.h): chunks of up to kPfMaxChunk prompt positions through
-    // every layer per weight pass; one captured graph per chunk size (kPfSizes)
+    // every layer per weight pass
     struct Prefill {
         float *x = nullptr, *xpart = nullptr, *q = nullptr;  // [chunk][D], [chunk][D] (TP partials), [chunk][hq hd]
         __half *hhi = nullptr, *hlo = nullptr;  // [chunk][max(D, hq hd)]: normed x / attention out, fp16 hi + lo
         __half *ahi = nullptr, *alo = nullptr;  // [chunk][Il]: SwiGLU out, fp16 hi + lo
-        sli::PfState* ps = nullptr;             // chunk start position + valid rows (device)
-        hipGraph_t graph[4] = {};
-        hipGraphExec_t exec[4] = {};
+        float* ws = nullptr;                    // partial sums of the tiles that a GEMM cuts over its depth (PgIn::ws)
+        unsigned* cnt = nullptr;
     } pf;
     // tensor-parallel all-reduce: SLI_ALLREDUCE_RCCL (ncclAllReduce) or SLI_ALLREDUCE_ONESHOT (oneshot.h)
     int ar_mode = SLI_ALLREDUCE_RCCL;
@@ -143,7 +142,6 @@ struct sli_model {
 // device-side reduction over the ranks' buffers in rank order (the ranks' kernels are the multi-GPU
 // ones, so the sharded engine itself is what the group tests run).
 constexpr int kMaxGroup = 8;
-constexpr int kPfSizes[4] = {32, 64, 128, 256};  // prefill chunk sizes (the last is prefill.h kPfMaxChunk)
 struct sli_tp_group {
     int n = 0;
     int device = 0;
@@ -151,8 +149,6 @@ struct sli_tp_group {
     std::vector<sli_model*> ranks;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    hipGraph_t pf_graph[4] = {};  // the ranks' prefill chunks in lockstep, per chunk size
-    hipGraphExec_t pf_exec[4] = {};
 };
 
 namespace sli {
@@ -591,6 +587,9 @@ static int tpl_launch(sli_model* m) {
     SLI_HIP(hipGetLastError());
     return SLI_OK;
 }
+
+// rows of the launches for a chunk of nv prompt positions
+static int pf_rows(int nv) { return nv <= 32 ? 32 : nv <= 64 ? 64 : (nv + 127) / 128 * 128; }
 
 template <typename WT, typename KT>
 struct StepRecorder {
@@ -1033,55 +1032,57 @@ struct StepRecorder {
     // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); the last prompt
     // position runs as an ordinary decode step. Phases as record_phase: 2l = qkv, attention, wo; 2l+1 =
     // gate/up, down; under tensor parallelism each ends with the all-reduce of the chunk's residual rows.
-    template <class Epi, class Cfg>
-    static int pg_cfg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
-                      int M) {
-        if constexpr (std::is_same<WT, float>::value) {
-            return fail(SLI_ERR_ARG, "prefill needs fp16 or int8 weights");
-        } else {
-            const PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
-            SLI_HIP((launch_pgemm<Epi, Cfg, WT>(in, e, m->pf.ps, m->stream)));
-            return SLI_OK;
-        }
-    }
-    // The GEMM tiling (prefill.h PgCfg<BM, WR, S, AT, PIPE>) per weight type, projection role and chunk size: the
-    // fastest of the tools/pgemm_lab sweeps on the 7B shapes (profiles/r3_pgemm_lab.txt; round 6: the pipelined
-    // fragment reads, 5-20 % faster at every tiling, the M = 128 choices, profiles/r6b_pg_pipe.txt, and the M = 256
-    // ones re-timed with the weights streamed from HBM as in the engine, profiles/r6b_pg_cold.txt).
-    // role 0: qkv, 1: gate/up, 2: wo / down (N = D: few row blocks, so small chunk blocks for a full grid).
-    // f(PgCfg<...>{}) is called with the chosen tiling (pg launches it, allow_pg sets its LDS limit).
+    // The GEMM tilings (prefill.h PgCfg<BM, WR, S, AT, SA>) of a chunk size, each with the time of one stage of a workgroup
+    // when every CU has one, in us (tools/pgemm_lab, one MI355X, 7B shapes): f(PgCfg<...>{}, us). The launch takes the one
+    // whose plan (prefill.h pg_plan: rounds, and the last round's tiles cut over the depth) costs least. Measured at 512
+    // rows, q/k/v | gate/up | wo | down in us: 123 | 214 | 45 | 102, against 144 | 263 | 122 | 122 of two 256-row chunks
+    // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
     template <class F>
-    static int pg_pick(int M, int role, F&& f) {
+    static void pg_each(int M, F&& f) {
         if constexpr (std::is_same<WT, int8_t>::value) {
-            if (M == 32) return f(PgCfg<32, 2, 4, 2, true>{});
-            if (role == 2) return M == 256 ? f(PgCfg<64, 2, 2, 2, true>{}) : f(PgCfg<32, 2, 4, 2, true>{});
-            if (role == 1) return M == 128 ? f(PgCfg<128, 4, 2, 2, true>{}) : f(PgCfg<64, 4, 2, 2, true>{});
-            return M == 256 ? f(PgCfg<128, 4, 2, 2, true>{}) : f(PgCfg<64, 4, 2, 2, true>{});
+            if (M % 128 == 0) f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
+            else if (M % 64 == 0) f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 2, 4>{}, 1.65f);
+            else f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
         } else {
-            if (M == 32) return f(PgCfg<32, 2, 4, 2, true>{});
-            if (role == 2) return M == 256 ? f(PgCfg<64, 2, 3, 2, true>{}) : f(PgCfg<32, 2, 4, 2, true>{});
-            if (M == 64 || (M == 128 && role == 0)) return f(PgCfg<64, 2, 3, 2, true>{});
-            // M = 256 with the weights streamed from HBM (profiles/r6b_pg_cold.txt): 8-wave workgroups
-            // (q/k/v: the weights in a 4-deep ring of their own, profiles/r6b_pg_split.txt)
-            if (M == 256) return role == 0 ? f(PgCfg<128, 4, 2, 2, true, 4>{}) : f(PgCfg<64, 4, 3, 2, true>{});
-            return f(PgCfg<128, 2, 2, 2, true>{});
+            if (M % 128 == 0) f(PgCfg<128, 4, 2, 4, 3>{}, 1.85f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.1f), f(PgCfg<64, 4, 3, 2>{}, 0.67f);
+            else if (M % 64 == 0) f(PgCfg<64, 4, 4, 2>{}, 0.72f), f(PgCfg<64, 4, 3, 4>{}, 0.97f), f(PgCfg<64, 2, 4, 2>{}, 0.52f);
+            else f(PgCfg<32, 4, 4, 2>{}, 0.6f), f(PgCfg<32, 4, 3, 4>{}, 0.77f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
         }
     }
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e, int M,
-                  int role) {
-        return pg_pick(M, role, [&](auto cfg) { return pg_cfg<Epi, decltype(cfg)>(m, W, N, K, hi, lo, e, M); });
+                  const PfState& st) {
+        if constexpr (std::is_same<WT, float>::value) {
+            return fail(SLI_ERR_ARG, "prefill needs fp16 or int8 weights");
+        } else {
+            PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
+            in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nv;
+            float best = INFINITY;
+            int pick = 0, i = 0;
+            pg_each(M, [&](auto cfg, float us) {
+                const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
+                if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
+                ++i;
+            });
+            hipError_t err = hipSuccess;
+            i = 0;
+            pg_each(M, [&](auto cfg, float) {
+                if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
+            });
+            SLI_HIP(err);
+            return SLI_OK;
+        }
     }
     template <class Epi>
     static int allow_pg(sli_model*) {
-        if constexpr (std::is_same<WT, int8_t>::value || std::is_same<WT, __half>::value) {
-            for (int M : {32, 64, 128, 256})
-                for (int role = 0; role < 3; ++role)
-                    SLI_TRY(pg_pick(M, role, [&](auto cfg) -> int {
-                        SLI_HIP((pgemm_allow_lds<Epi, decltype(cfg), WT>()));
-                        return SLI_OK;
-                    }));
-        }
+        hipError_t err = hipSuccess;
+        if constexpr (!std::is_same<WT, float>::value)
+            for (int M : {32, 64, 128})
+                pg_each(M, [&](auto cfg, float) {
+                    const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
+                    if (e != hipSuccess) err = e;
+                });
+        SLI_HIP(err);
         return SLI_OK;
     }
     static int prepare_prefill(sli_model* m) {
@@ -1090,12 +1091,12 @@ struct StepRecorder {
         SLI_TRY(allow_pg<PgEpiSwiGLU>(m));
         return SLI_OK;
     }
-    static int record_pf_phase(sli_model* m, int p, int M) {
+    static int record_pf_phase(sli_model* m, int p, int M, const PfState& ps) {
         auto& f = m->pf;
         hipStream_t s = m->stream;
         const int D = m->D, hd = m->hd, QD = m->hq * hd;
         if (p == 0) {
-            hipLaunchKernelGGL(pf_embed_kernel<WT>, dim3(M), dim3(256), 0, s, f.ps, m->prompt, (const WT*)m->emb,
+            hipLaunchKernelGGL(pf_embed_kernel<WT>, dim3(M), dim3(256), 0, s, ps, m->prompt, (const WT*)m->emb,
                                m->emb_s, f.x, D);
             SLI_HIP(hipGetLastError());
         }
@@ -1109,34 +1110,35 @@ struct StepRecorder {
         if (p % 2 == 0) {
             const size_t ls = (size_t)l * m->hkv * m->T * hd;
             PgEpiQKV<KT> eq{f.q, (KT*)m->kc + ls, (KT*)m->vc + ls, w.qkv_s, m->sin_t, m->cos_t, m->hq, m->hkv, hd, m->T};
-            SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, 0));
+            SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, ps));
             PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, f.hhi, f.hlo, m->hq, m->hkv, m->T,
                               1.0f / sqrtf((float)hd)};
             if constexpr (std::is_same<KT, __half>::value) {  // MFMA, 16 chunk rows per workgroup
                 const dim3 ag(M / 16, m->hq);
                 if (hd == 128)
-                    hipLaunchKernelGGL((pf_attn_mfma_kernel<128>), ag, dim3(256), 0, s, aa, f.ps, PfRowsArgs{});
+                    hipLaunchKernelGGL((pf_attn_mfma_kernel<128>), ag, dim3(256), 0, s, aa, ps, PfRowsArgs{});
                 else
-                    hipLaunchKernelGGL((pf_attn_mfma_kernel<64>), ag, dim3(256), 0, s, aa, f.ps, PfRowsArgs{});
+                    hipLaunchKernelGGL((pf_attn_mfma_kernel<64>), ag, dim3(256), 0, s, aa, ps, PfRowsArgs{});
             } else {  // fp32 cache: fp32 VALU, 64 chunk rows per workgroup
                 const dim3 ag((M + kPaQB - 1) / kPaQB, m->hq);
                 if (hd == 128)
-                    hipLaunchKernelGGL((pf_attn_kernel<KT, 128>), ag, dim3(256), 0, s, aa, f.ps);
+                    hipLaunchKernelGGL((pf_attn_kernel<KT, 128>), ag, dim3(256), 0, s, aa, ps);
                 else
-                    hipLaunchKernelGGL((pf_attn_kernel<KT, 64>), ag, dim3(256), 0, s, aa, f.ps);
+                    hipLaunchKernelGGL((pf_attn_kernel<KT, 64>), ag, dim3(256), 0, s, aa, ps);
             }
             SLI_HIP(hipGetLastError());
             er.rscale = w.wo_s;
-            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, M, 2);
+            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, M, ps);
         }
         PgEpiSwiGLU eg{f.ahi, f.alo, w.gu_s, m->Il, m->c.act_mode};
-        SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, M, 1));
+        SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, M, ps));
         er.rscale = w.down_s;
-        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, M, 2);
+        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, M, ps);
     }
-    static int record_prefill(sli_model* m, int M) {
+    static int record_prefill(sli_model* m, const PfState& ps) {
+        const int M = pf_rows(ps.nv);
         for (int p = 0; p < 2 * m->L; ++p) {
-            SLI_TRY(record_pf_phase(m, p, M));
+            SLI_TRY(record_pf_phase(m, p, M, ps));
             const size_t n = (size_t)M * m->D;
             if (m->collectives)
                 SLI_NCCL(ncclAllReduce(m->pf.xpart, m->pf.x, n, ncclFloat32, ncclSum, m->comm, m->stream));
@@ -1145,8 +1147,9 @@ struct StepRecorder {
         }
         return SLI_OK;
     }
-    static int record_group_prefill(sli_tp_group* g, int M) {
+    static int record_group_prefill(sli_tp_group* g, const PfState& ps) {
         sli_model* m0 = g->ranks[0];
+        const int M = pf_rows(ps.nv);
         GroupSumArgs sa{};
         sa.n_ranks = g->n;
         sa.n = M * m0->D;
@@ -1156,7 +1159,7 @@ struct StepRecorder {
         }
         const int blocks = std::min(256, (sa.n + 255) / 256);
         for (int p = 0; p < 2 * m0->L; ++p) {
-            for (int r = 0; r < g->n; ++r) SLI_TRY(record_pf_phase(g->ranks[r], p, M));
+            for (int r = 0; r < g->n; ++r) SLI_TRY(record_pf_phase(g->ranks[r], p, M, ps));
             hipLaunchKernelGGL(group_sum_kernel, dim3(blocks), dim3(256), 0, g->stream, sa);
             SLI_HIP(hipGetLastError());
         }
@@ -1415,10 +1418,6 @@ static void destroy(sli_model* m) {
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
     if (m->graph) (void)hipGraphDestroy(m->graph);
-    for (int b = 0; b < 4; ++b) {
-        if (m->pf.exec[b]) (void)hipGraphExecDestroy(m->pf.exec[b]);
-        if (m->pf.graph[b]) (void)hipGraphDestroy(m->pf.graph[b]);
-    }
     if (m->comm) ncclCommDestroy(m->comm);
     hy_destroy(m->bs);
     for (int r = 0; r < sli::kOsMaxRanks; ++r)
@@ -1903,16 +1902,10 @@ static bool pf_supported(const sli_model* m) {
            m->D <= 8192 && m->Il % 64 == 0 && (m->hq * m->hd) % 64 == 0;
 }
 
-static int pf_bucket(int nv) {
-    for (int b = 0; b < 3; ++b)
-        if (nv <= kPfSizes[b]) return b;
-    return 3;
-}
-
 static int pf_alloc(sli_model* m) {
     auto& p = m->pf;
     if (p.x) return SLI_OK;
-    const size_t M = kPfMaxChunk, D = m->D, QD = (size_t)m->hq * m->hd;
+    const size_t M = pf_rows(std::min(m->T, kPfMaxChunk)), D = m->D, QD = (size_t)m->hq * m->hd;
     int rc = SLI_OK;
     auto A = [&](void** ptr, size_t bytes) {
         if (rc == SLI_OK) rc = model_alloc(m, ptr, bytes);
@@ -1924,8 +1917,10 @@ static int pf_alloc(sli_model* m) {
     A((void**)&p.hlo, sizeof(__half) * M * std::max(D, QD));
     A((void**)&p.ahi, sizeof(__half) * M * m->Il);
     A((void**)&p.alo, sizeof(__half) * M * m->Il);
-    A((void**)&p.ps, sizeof(PfState));
+    A((void**)&p.ws, kPgWsBytes);
+    A((void**)&p.cnt, sizeof(unsigned) * kPgWsTiles);
     if (rc != SLI_OK) return rc;
+    SLI_HIP(hipMemsetAsync(p.cnt, 0, sizeof(unsigned) * kPgWsTiles, m->stream));
     return SLI_DISPATCH(m, prepare_prefill, m);
 }
 
@@ -2069,16 +2064,7 @@ extern "C" int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n) {
     SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
     if (n > 1 && pf_supported(m)) {
         SLI_TRY(pf_alloc(m));
-        const std::vector<PfState> cs = pf_chunks(n);
-        for (const PfState& c : cs) {  // capture before anything is enqueued behind the capture
-            const int b = pf_bucket(c.nv);
-            SLI_TRY(capture_graph(m->stream, m->pf.graph[b], m->pf.exec[b],
-                                  [&]() { return SLI_DISPATCH(m, record_prefill, m, kPfSizes[b]); }));
-        }
-        for (const PfState& c : cs) {  // each copy reads its own element of cs: enqueued back to back
-            SLI_HIP(hipMemcpyAsync(m->pf.ps, &c, sizeof(PfState), hipMemcpyHostToDevice, m->stream));
-            SLI_HIP(hipGraphLaunch(m->pf.exec[pf_bucket(c.nv)], m->stream));
-        }
+        for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
         SLI_TRY(wait_stream(m));
     } else {
         for (int p = 0; p < n - 1; ++p) {  // the decode step, teacher-forced (model.cpp:159-165)
@@ -2102,17 +2088,7 @@ extern "C" int sli_tp_group_prefill(sli_tp_group* g, const int32_t* ids, int32_t
     }
     if (n > 1 && pf_supported(m0)) {
         for (sli_model* m : g->ranks) SLI_TRY(pf_alloc(m));
-        const std::vector<PfState> cs = pf_chunks(n);
-        for (const PfState& c : cs) {
-            const int b = pf_bucket(c.nv);
-            SLI_TRY(capture_graph(g->stream, g->pf_graph[b], g->pf_exec[b],
-                                  [&]() { return SLI_DISPATCH(m0, record_group_prefill, g, kPfSizes[b]); }));
-        }
-        for (const PfState& c : cs) {
-            for (sli_model* m : g->ranks)
-                SLI_HIP(hipMemcpyAsync(m->pf.ps, &c, sizeof(PfState), hipMemcpyHostToDevice, g->stream));
-            SLI_HIP(hipGraphLaunch(g->pf_exec[pf_bucket(c.nv)], g->stream));
-        }
+        for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m0, record_group_prefill, g, c));
         SLI_HIP(hipStreamSynchronize(g->stream));
     } else {
         for (int p = 0; p < n - 1; ++p) {
@@ -2707,10 +2683,6 @@ int sli_tp_group_destroy(sli_tp_group* g) {
     if (g->stream) (void)hipStreamSynchronize(g->stream);
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
-    for (int b = 0; b < 4; ++b) {
-        if (g->pf_exec[b]) (void)hipGraphExecDestroy(g->pf_exec[b]);
-        if (g->pf_graph[b]) (void)hipGraphDestroy(g->pf_graph[b]);
-    }
     for (sli_model* m : g->ranks) destroy(m);
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;

@@ -268,7 +268,7 @@ struct PgPair {  // prefill.h: plain 16-row tiles, 4 consecutive rows per store
     Epi e;
     int n, u0;
     __device__ int row(int t, int i) const { return t * 16 + i; }
-    __device__ void store(int t, int i0, int m, const float* v, const PfState*) const {
+    __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
         const int u = t * 8 + (i0 >> 1);
         if (u < n) e.pair2(u0 + u, m, v, u + 1 < n);
     }

@@ -62,7 +62,7 @@ struct HyProj {
             PgIn<__half> in{w, X, nullptr, pad_to(2 * npairs, 16), K, M};
             if (X2) in.Bhi2 = X2, in.row_b2 = 2 * split;
             return pg_pick(M, in.N, [&](auto cfg) -> int {
-                SLI_HIP((launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, u0}, nullptr, st())));
+                SLI_HIP((launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, u0}, PfState{}, st())));
                 return SLI_OK;
             });
         } else {
@@ -75,12 +75,12 @@ struct HyProj {
     template <class F>
     static int pg_pick(int M, int N, F&& f) {
         const long long t128 = (long long)((N + 127) / 128) * (M / 128);
-        if (M % 256 == 0 && M != 512 && t128 >= 512) return f(PgCfg<256, 4, 2, 4, true, 0, 1>{});
-        if (M % 128 == 0 && M >= 512 && t128 >= 512) return f(PgCfg<128, 4, 2, 2, true, 0, 1>{});
-        if (M % 128 == 0 && t128 >= 256) return f(PgCfg<128, 2, 3, 4, true, 0, 1>{});
-        if (M % 64 == 0 && M >= 128) return f(PgCfg<64, 4, 4, 2, true, 0, 1>{});
-        if (M % 64 == 0) return f(PgCfg<64, 2, 4, 2, true, 0, 1>{});
-        return f(PgCfg<32, 2, 4, 2, true, 0, 1>{});
+        if (M % 256 == 0 && M != 512 && t128 >= 512) return f(PgCfg<256, 4, 2, 4, 0, 1>{});
+        if (M % 128 == 0 && M >= 512 && t128 >= 512) return f(PgCfg<128, 4, 2, 2, 0, 1>{});
+        if (M % 128 == 0 && t128 >= 256) return f(PgCfg<128, 2, 3, 4, 0, 1>{});
+        if (M % 64 == 0 && M >= 128) return f(PgCfg<64, 4, 4, 2, 0, 1>{});
+        if (M % 64 == 0) return f(PgCfg<64, 2, 4, 2, 0, 1>{});
+        return f(PgCfg<32, 2, 4, 2, 0, 1>{});
     }
     template <class Epi>
     static int allow() {
@@ -105,7 +105,7 @@ struct HyProj {
             PgIn<__half> in{(const __half*)W, (const __half*)X, nullptr, pad_to(2 * npairs, 16), K, maxtiles * bm};
             in.grp = g;
             return pg_group_pick(bm, [&](auto cfg) -> int {
-                SLI_HIP((launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, 0}, nullptr, st())));
+                SLI_HIP((launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, 0}, PfState{}, st())));
                 return SLI_OK;
             });
         } else {
@@ -115,9 +115,9 @@ struct HyProj {
     }
     template <class F>
     static int pg_group_pick(int bm, F&& f) {
-        if (bm == 128) return f(PgCfg<128, 2, 3, 4, true, 0, 1, true>{});
-        if (bm == 64) return f(PgCfg<64, 4, 4, 2, true, 0, 1, true>{});
-        return f(PgCfg<32, 2, 4, 2, true, 0, 1, true>{});
+        if (bm == 128) return f(PgCfg<128, 2, 3, 4, 0, 1, true>{});
+        if (bm == 64) return f(PgCfg<64, 4, 4, 2, 0, 1, true>{});
+        return f(PgCfg<32, 2, 4, 2, 0, 1, true>{});
     }
     template <class Epi>
     static int allow_grouped() {

@@ -11,9 +11,8 @@
 //      through an S-deep LDS ring by LDS-DMA (global_load_lds_dwordx4: one 1-KiB fragment image per
 //      wave-instruction, read back conflict-free by ds_read_b128), S - 1 stages in flight behind a counted
 //      vmcnt and a raw s_barrier (cdna_hip_programming.md §5 "Pipelining across barriers"), or the weight images
-//      in a deeper ring of their own (PgCfg::SA, round 6); the fragment reads of
-//      the next k-block are issued ahead of the current k-block's MFMAs (two register sets, across the stage
-//      barrier too: PgCfg::PIPE, round 6, 5-20 % faster per GEMM, bit-identical sums). Fused epilogues:
+//      in a deeper ring of their own (PgCfg::SA); the fragment reads of the next k-block are issued ahead of the
+//      current k-block's MFMAs. Fused epilogues:
 //      RoPE + K/V cache rows + q (model.cpp:52-67), residual add (:86-90, :124-128), SwiGLU (:111-115,
 //      written straight as the down projection's hi/lo operand);
 //   3. pf_attn_mfma_kernel (fp16 KV, the default): block-causal attention of 16 chunk rows x one head against
@@ -23,15 +22,20 @@
 //      blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches.
 // int8 weights: stages of 128 k; a depth that is 64 mod 128 (e.g. Llama-2-7B int8 down at TP 4, 2752) ends with
 // a half stage (pgemm_kernel).
-// The chunk's start position and valid count live in device memory (PfState), so one captured graph per
-// chunk size serves every chunk of every prompt.
+// The launches of a chunk go to the stream one by one (its start position and valid count are kernel arguments): each
+// runs longer than it takes to enqueue, so a captured graph would only add its capture to a model's first prompt.
 #pragma once
+#include <algorithm>
+
 #include "common.h"
 #include "step_state.h"
 
 namespace sli {
 
-constexpr int kPfMaxChunk = 256;   // prompt positions per weight pass
+// Prompt positions per weight pass. The activations of a chunk (at 4096 rows of a 7B model 0.6 GB) are small beside the
+// weights, and every chunk pays a partial last round of tiles per GEMM (pg_plan) and reads the weights once.
+constexpr int kPfMaxChunk = 4096;
+constexpr int kPgGroup = 8;        // position blocks that an XCD takes through its row blocks together
 
 struct PfState {
     int32_t p0;  // position of chunk row 0
@@ -55,12 +59,11 @@ __device__ __forceinline__ void pf_split(float v, __half& hi, __half& lo) {
 // ---------------------------------------------------------------- 1. embedding + RMSNorm / split
 // x[m] = emb[prompt[p0 + m]] (emb_kernel.cpp:4-21; padding rows repeat the last valid token)
 template <typename WT>
-__global__ void __launch_bounds__(256) pf_embed_kernel(const PfState* __restrict__ ps, const int32_t* __restrict__ prompt,
+__global__ void __launch_bounds__(256) pf_embed_kernel(PfState ps, const int32_t* __restrict__ prompt,
                                                       const WT* __restrict__ emb, const float* __restrict__ emb_s,
                                                       float* __restrict__ x, int D) {
     const int m = blockIdx.x;
-    const int nv = ps->nv;
-    const int tok = prompt[ps->p0 + min(m, nv - 1)];
+    const int tok = prompt[ps.p0 + min(m, ps.nv - 1)];
     const float s = emb_s ? emb_s[tok] : 1.0f;
     for (int i = threadIdx.x; i < D; i += 256) x[(size_t)m * D + i] = to_f32(emb[(size_t)tok * D + i]) * s;
 }
@@ -150,6 +153,12 @@ struct PgIn {
     const __half* Bhi2 = nullptr;
     int row_b2 = 0x7fffffff;
     PgGroups grp;
+    // The launch's slots, per XCD (pg_plan): the first `full` own a whole tile each, the tiles after them are cut into
+    // `splits` depth ranges (partial sums in ws [tail tile][split], arrival counters in cnt, zero between launches).
+    int full = 0x7fffffff, splits = 1;
+    float* ws = nullptr;
+    unsigned* cnt = nullptr;
+    int valid = 0x7fffffff;  // chunk rows from here on are padding: a wave that holds only such rows multiplies nothing
 };
 
 // Tiling: a workgroup of 2 WR waves owns BN = 32 WR weight rows x BM chunk rows; wave w holds the 2 x BM/32
@@ -162,21 +171,20 @@ struct PgIn {
 // Epilogue contract: row(t, i) = weight row of 16-row tile t's row i (i < 16, always valid); store(t, i0, m, v)
 // gets the fp32 sums of tile rows i0 .. i0+3 (i0 % 4 == 0) for chunk row m.
 // AT_: 16-row weight tiles per wave (2: a wave's 32 rows; 4: 64 rows, so every B fragment read from LDS feeds twice
-// the MFMAs). PIPE_: the fragment reads of k-block j + 1 issued before the MFMAs of k-block j (two register sets),
-// across the stage barrier too, and every hi MFMA of a k-block ahead of its lo MFMAs (no back-to-back MFMAs on one
-// accumulator); each tile's sums are added in the same order either way (bit-identical).
-// SA_ > 0 (PIPE only): the weight (A) images get a ring of their own, SA_ stages deep (SA_ - 1 issued ahead), and
+// the MFMAs). The fragment reads of k-block j + 1 are issued before the MFMAs of k-block j (two register sets),
+// across the stage barrier too, and every hi MFMA of a k-block goes ahead of its lo MFMAs (no back-to-back MFMAs on one
+// accumulator).
+// SA_ > 0: the weight (A) images get a ring of their own, SA_ stages deep (SA_ - 1 issued ahead), and
 // the activation (B) images a 2-stage ring (one ahead): the A bytes come from HBM (read once per chunk), the B bytes
 // from L2, so only A needs the deep prefetch, and B, the larger image, does not pay for it in LDS.
-// NB_: activation images per position: 2 (fp16 hi + lo, two MFMAs per product) or 1 (fp16 activations; PIPE only).
+// NB_: activation images per position: 2 (fp16 hi + lo, two MFMAs per product) or 1 (fp16 activations).
 // GR_: row blocks with weights of their own (PgGroups; one image).
-template <int BM_, int WR_, int S_, int AT_ = 2, bool PIPE_ = false, int SA_ = 0, int NB_ = 2, bool GR_ = false>
+template <int BM_, int WR_, int S_, int AT_ = 2, int SA_ = 0, int NB_ = 2, bool GR_ = false>
 struct PgCfg {
-    static_assert(NB_ == 2 || (NB_ == 1 && PIPE_), "activation images");
+    static_assert(NB_ == 2 || NB_ == 1, "activation images");
     static_assert(!GR_ || NB_ == 1, "grouped: one image");
     static constexpr bool GR = GR_;
     static constexpr int BM = BM_, WR = WR_, S = S_, AT = AT_, SA = SA_, NB = NB_;
-    static constexpr bool PIPE = PIPE_;
 };
 
 template <class Cfg, typename WT>
@@ -203,7 +211,7 @@ struct PgGeo {
     static_assert(S >= 2 && (S - 1) * DPW <= 63, "ring depth (vmcnt counts 63 loads)");
     // (SA > S: A(s) must be issued in an earlier iteration than B(s), the wait below counts on it; SA == S computed
     // wrong sums in tools/pgemm_lab)
-    static_assert(SA == 0 || (Cfg::PIPE && S == 2 && SA > S && (A_BYTES / 1024) % WAVES == 0 &&
+    static_assert(SA == 0 || (S == 2 && SA > S && (A_BYTES / 1024) % WAVES == 0 &&
                               (B_BYTES / 1024) % WAVES == 0 && (SA - 1) * DPA + DPB <= 63), "split rings");
     static_assert(LDS <= 160 * 1024, "LDS");
 };
@@ -244,7 +252,7 @@ __device__ __forceinline__ void pg_wait_stages(int later) {
 }
 
 template <class Epi, class Cfg, typename WT>
-__global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi epi, const PfState* __restrict__ ps) {
+__global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi epi, PfState ps) {
     using Geo = PgGeo<Cfg, WT>;
     constexpr int KBS = Geo::KBS, BM = Geo::BM, WR = Geo::WR, S = Geo::S;
     extern __shared__ __attribute__((aligned(1024))) char pg_smem[];
@@ -252,11 +260,15 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int wr = wave % WR, wp = wave / WR;  // row pair, position half
     const int PB = in.M / BM;
-    // workgroups that share a row block run on one XCD (blocks b and b + 8 share one under round-robin
-    // placement; speed only): the second read of the weight rows hits that XCD's L2
-    const int bid = blockIdx.x, xcd = bid & 7, slot = bid >> 3;
-    const int rb = (slot / PB) * 8 + xcd, pb = slot - (slot / PB) * PB;
     const int nrb = (in.N + Geo::BN - 1) / Geo::BN;
+    // Row block rb runs on XCD rb % 8 (blocks b and b + 8 share one under round-robin placement; speed only). An XCD
+    // walks its row blocks in groups of kPgGroup position blocks, so that what runs on its CUs together is a block of
+    // tiles that shares both operands in its L2.
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int nsp = slot < in.full ? 1 : in.splits;
+    const int ti = nsp == 1 ? slot : in.full + (slot - in.full) / nsp, sp = nsp == 1 ? 0 : (slot - in.full) % nsp;
+    const int nr8 = (nrb + 7) / 8, grp0 = ti / (nr8 * kPgGroup) * kPgGroup, gw = min(kPgGroup, PB - grp0);
+    const int tg = ti - grp0 * nr8, rb = tg / gw * 8 + xcd, pb = grp0 + tg % gw;
     if (rb >= nrb) return;  // (uniform) padding of the grid to a multiple of 8 row blocks
     int2 tile = make_int2(0, 0);
     if constexpr (Cfg::GR) {
@@ -267,8 +279,10 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     // stages: K is a multiple of 64, so with int8 weights (KS 128) the last stage may be a half stage. Its DMA
     // pieces past the row's end reload the stage's first half instead (in bounds; never read), and only its
     // first KBS / 2 k-blocks are multiplied.
-    const int ns = (in.K + Geo::KS - 1) / Geo::KS;
-    const bool half_tail = (in.K % Geo::KS) != 0;
+    // A split's stages are s0 .. s0 + ns - 1 (every split has one: pg_plan).
+    const int nsk = (in.K + Geo::KS - 1) / Geo::KS;
+    const int s0 = nsp == 1 ? 0 : nsk * sp / nsp, ns = (nsp == 1 ? nsk : nsk * (sp + 1) / nsp) - s0;
+    const bool half_tail = (in.K % Geo::KS) != 0 && s0 + ns == nsk;
     const int nt = in.N >> 4;       // row tiles
     const unsigned ring = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)pg_smem;
 
@@ -289,7 +303,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const int r = (off % Geo::A_IMG) / Geo::A_ROW + lane / 8;
             const int c = (lane % 8) ^ pg_swz(r, Geo::A_ROW);
             const int row = epi.row(min(t, nt - 1), r);
-            src[j] = reinterpret_cast<const char*>(in.W) + (size_t)row * in.K * sizeof(WT) + c * 16;
+            src[j] = reinterpret_cast<const char*>(in.W) + (size_t)row * in.K * sizeof(WT) + c * 16 + (size_t)s0 * Geo::A_ROW;
             adv[j] = Geo::A_ROW;
             back[j] = c >= 4 ? Geo::A_ROW / 2 : 0;
         } else {
@@ -301,7 +315,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const __half* B = Geo::NB == 2 ? ((u & 1) ? in.Blo : in.Bhi) : rb * Geo::BN >= in.row_b2 ? in.Bhi2 : in.Bhi;
             int m = pb * BM + pt * 16 + r;
             if constexpr (Cfg::GR) m = in.grp.rowmap ? in.grp.rowmap[m] : tile.y + pt * 16 + r;
-            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * 2 + c * 16;
+            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * 2 + c * 16 + (size_t)s0 * Geo::B_ROW;
             adv[j] = Geo::B_ROW;
             back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
         }
@@ -310,13 +324,8 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         const unsigned dst = ring + (unsigned)((s % S) * Geo::STAGE);
         const bool tail = half_tail && s == ns - 1;
 #pragma unroll
-        for (int j = 0; j < Geo::DPW; ++j) {
-#ifdef PG_LAB_SKIP  // tools/pgemm_lab only (bit 0: no A pieces, bit 1: no B pieces): timing bounds, wrong sums
-            const bool isa = (wave * Geo::DPW + j) * 1024 < Geo::A_BYTES;
-            if (((PG_LAB_SKIP & 1) && isa) || ((PG_LAB_SKIP & 2) && !isa)) continue;
-#endif
+        for (int j = 0; j < Geo::DPW; ++j)
             pf_dma(src[j] + (size_t)s * adv[j] - (tail ? back[j] : 0), dst + (unsigned)((wave * Geo::DPW + j) * 1024));
-        }
     };
 
     // split rings: A stage s in slot s % SA at ring, B stage s in slot s % 2 behind the A ring
@@ -387,7 +396,8 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
                 for (int a = 0; a < AT; ++a) acc[a][b] = pf_mfma(af[a], bl[b], acc[a][b]);
         }
     };
-    if constexpr (Cfg::PIPE) {
+    const bool live = Cfg::GR || pb * BM + wp * Geo::WPT * 16 < in.valid;  // (wave-uniform)
+    {
         // set X holds even k-blocks, set Y odd ones (KBS is even; an int8 half stage has KBS / 2 = 2): per stage
         // read(0) -> X, MFMA(Y: the previous stage's last k-block), read(1) -> Y, MFMA(X), ... The stage barrier
         // follows this wave's lgkmcnt(0), so the previous stage's buffer is free for the DMA issued after it while
@@ -420,61 +430,63 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const int kbs = (half_tail && s == ns - 1) ? KBS / 2 : KBS;  // wave-uniform, even
 #pragma unroll
             for (int kb = 0; kb < KBS; kb += 2) {
-                if (kb >= kbs) break;
+                if (kb >= kbs || !live) break;
                 read_frags(st, stb, kb, xa, xh, xl);
                 if (s > 0 || kb > 0) mfmas(ya, yh, yl);
                 read_frags(st, stb, kb + 1, ya, yh, yl);
                 mfmas(xa, xh, xl);
             }
         }
-        mfmas(ya, yh, yl);
-    } else {
-    for (int s = 0; s < ns; ++s) {
-        // this wave's pieces of stage s landed (stages s + 1 .. s + S - 2 may stay in flight)
-        pg_wait_stages<Geo::DPW>(min(S - 2, ns - 1 - s));
-        __builtin_amdgcn_s_barrier();  // every wave's pieces of s landed; every wave is done with s - 1
-        if (s + S - 1 < ns) issue(s + S - 1);  // into the buffer of s - 1
-        const char* st = pg_smem + (size_t)(s % S) * Geo::STAGE;
-        const int kbs = (half_tail && s == ns - 1) ? KBS / 2 : KBS;  // wave-uniform
+        if (live) mfmas(ya, yh, yl);
+    }
+    if (nsp > 1) {
+        // Partial sums go out write-through (sc1); the tile's last workgroup to arrive adds them in split order (the
+        // same sum whichever arrives last) and runs the epilogue.
+        constexpr int NV = AT * Geo::WPT, TILE = NV * Geo::THREADS;  // float4s per split
+        const unsigned tail = (unsigned)(ti - in.full) * 8 + xcd, bytes = 16u * TILE;
+        float* tw = in.ws + (size_t)tail * nsp * TILE * 4;
+        const auto own = __builtin_amdgcn_make_buffer_rsrc(tw + (size_t)sp * TILE * 4, 0, bytes, 0x00020000);
 #pragma unroll
-        for (int kb = 0; kb < KBS; ++kb) {
-            if (kb >= kbs) break;
-            u32x4 af[AT], bh[Geo::WPT], bl[Geo::WPT];
+        for (int a = 0; a < AT; ++a)
+#pragma unroll
+            for (int b = 0; b < Geo::WPT; ++b)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[a][b]), own,
+                                                       16u * ((a * Geo::WPT + b) * Geo::THREADS + threadIdx.x), 0, 16 /* sc1 */);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains before the arrival
+        __syncthreads();
+        unsigned* flag = reinterpret_cast<unsigned*>(pg_smem);
+        if (threadIdx.x == 0) {
+            const unsigned prev = __hip_atomic_fetch_add(in.cnt + tail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = prev == (unsigned)(nsp - 1);
+            if (*flag) __hip_atomic_store(in.cnt + tail, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (*flag == 0) return;  // uniform
+#pragma unroll
+        for (int a = 0; a < AT; ++a)
+#pragma unroll
+            for (int b = 0; b < Geo::WPT; ++b) acc[a][b] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int q = 0; q < nsp; ++q) {
+            const auto rs = __builtin_amdgcn_make_buffer_rsrc(tw + (size_t)q * TILE * 4, 0, bytes, 0x00020000);
 #pragma unroll
             for (int a = 0; a < AT; ++a) {
-                const char* img = st + (wr * AT + a) * Geo::A_IMG + r16 * Geo::A_ROW;
-                if constexpr (sizeof(WT) == 2) {
-                    af[a] = *reinterpret_cast<const u32x4*>(img + ((4 * kb + kg) ^ sa) * 16);
-                } else {  // k 32 kb + 8 kg .. +8: chunk 2 kb + kg / 2, half kg % 2
-                    const int off = ((2 * kb + (kg >> 1)) ^ sa) * 16 + 8 * (kg & 1);
-                    af[a] = pg_i8_to_f16(*reinterpret_cast<const uint2*>(img + off));
-                }
+#pragma unroll
+                for (int b = 0; b < Geo::WPT; ++b)
+                    acc[a][b] += __builtin_bit_cast(
+                        pf_float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                       rs, 16u * ((a * Geo::WPT + b) * Geo::THREADS + threadIdx.x), 0, 16));
+                asm volatile("" ::: "memory");  // (one tile row's loads in flight: more would spill at 256 columns)
             }
-#pragma unroll
-            for (int b = 0; b < Geo::WPT; ++b) {
-                const int pt = wp * Geo::WPT + b;
-                const char* img = st + Geo::A_BYTES + (2 * pt) * Geo::B_IMG + r16 * Geo::B_ROW + ((4 * kb + kg) ^ sb) * 16;
-                bh[b] = *reinterpret_cast<const u32x4*>(img);
-                bl[b] = *reinterpret_cast<const u32x4*>(img + Geo::B_IMG);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int a = 0; a < AT; ++a)
-#pragma unroll
-                for (int b = 0; b < Geo::WPT; ++b) {
-#if defined(PG_LAB_MFMA) && PG_LAB_MFMA == 0  // tools/pgemm_lab only: no MFMA (data movement alone)
-                    acc[a][b][0] += __uint_as_float(af[a][0] ^ bh[b][0] ^ bl[b][0]);
-#else
-                    acc[a][b] = pf_mfma(af[a], bh[b], acc[a][b]);
-#if !(defined(PG_LAB_MFMA) && PG_LAB_MFMA == 1)  // PG_LAB_MFMA 1: the hi MFMA only
-                    acc[a][b] = pf_mfma(af[a], bl[b], acc[a][b]);
-#endif
-#endif
-                }
         }
     }
-    }
-    // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15
+    if (!live) return;
+    // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15. (A copy of the sums: a large epilogue
+    // leaves this loop rolled, and the array that it indexes lives in scratch, which acc itself must not.)
+    pf_float4 out[AT][Geo::WPT];
+#pragma unroll
+    for (int a = 0; a < AT; ++a)
+#pragma unroll
+        for (int b = 0; b < Geo::WPT; ++b) out[a][b] = acc[a][b];
     const int i0 = 4 * (lane >> 4);
 #pragma unroll
     for (int a = 0; a < AT; ++a) {
@@ -483,7 +495,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
 #pragma unroll
         for (int b = 0; b < Geo::WPT; ++b) {
             const int m = pb * BM + (wp * Geo::WPT + b) * 16 + r16;
-            const float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
+            const float v[4] = {out[a][b][0], out[a][b][1], out[a][b][2], out[a][b][3]};
             epi.store(t, i0, m, v, ps);
         }
     }
@@ -506,9 +518,9 @@ struct PgEpiQKV {  // model.cpp:52-67: q (fp32 [M][hq*hd]), rotated k / v rows o
         const int uh = u / half, d = u - uh * half;
         return uh * hd + d + ((i & 2) ? half : 0);
     }
-    __device__ void store(int t, int i0, int m, const float* v, const PfState* ps) const {
+    __device__ void store(int t, int i0, int m, const float* v, const PfState& ps) const {
         // units u, u + 1 (u even): d, d + 1 of one head (hd / 2 is even), so every store is a pair
-        const int nv = ps->nv, pos = ps->p0 + m;
+        const int nv = ps.nv, pos = ps.p0 + m;
         const int half = hd >> 1;
         const int u = t * 8 + (i0 >> 2) * 2;
         const int uh = u / half, d = u - uh * half;
@@ -560,7 +572,7 @@ struct PgEpiSwiGLU {  // model.cpp:99-115: act = sigmoid(g) * u (or SiLU), store
     const float* rscale;
     int inter, silu;
     __device__ int row(int t, int i) const { return t * 8 + (i >> 2) * 2 + (i & 1) + ((i & 2) ? inter : 0); }
-    __device__ void store(int t, int i0, int m, const float* v, const PfState*) const {
+    __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
         const int u = t * 8 + (i0 >> 2) * 2;  // units u, u + 1: one 4-byte hi and lo store each
         __half hh[2], hl[2];
 #pragma unroll
@@ -585,7 +597,7 @@ struct PgEpiResid {  // y[m][row] = resid[m][row] + sum * row scale (matmul_kern
     const float* rscale;
     int nrows, ld;
     __device__ int row(int t, int i) const { return min(t * 16 + i, nrows - 1); }
-    __device__ void store(int t, int i0, int m, const float* v, const PfState*) const {
+    __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
         const int row = t * 16 + i0;  // rows row .. row + 3 (nrows % 16 == 0: the host's check)
         const size_t i = (size_t)m * ld + row;
         float4 p = make_float4(v[0], v[1], v[2], v[3]);
@@ -601,14 +613,47 @@ struct PgEpiResid {  // y[m][row] = resid[m][row] + sum * row scale (matmul_kern
     }
 };
 
+// How a GEMM's tiles fill the chip: whole rounds of one tile per resident workgroup, and the tiles of the last, partial
+// round cut into `splits` depth ranges each, so that it is short and all CUs share it.
+struct PgPlan {
+    int full = 0x7fffffff, splits = 1;  // PgIn
+    int slots = 0;                      // per XCD
+    float cost = 0.0f;                  // in stages of the tiling
+};
+constexpr size_t kPgWsBytes = 64u << 20;  // partial sums of a launch at most
+constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
+template <class Cfg, typename WT>
+PgPlan pg_plan(int N, int K, int M, int cus, bool ws) {
+    using Geo = PgGeo<Cfg, WT>;
+    const int nrb = (N + Geo::BN - 1) / Geo::BN, nx = (nrb + 7) / 8 * (M / Geo::BM);
+    const int ns = (K + Geo::KS - 1) / Geo::KS;
+    const int occ = (int)((160 * 1024) / Geo::LDS), cpx = std::max(1, cus / 8) * occ;
+    // entry and exit of a workgroup, and a split's share of the partial sums' way out and back, in stages
+    constexpr float kEdge = 5.0f;
+    const float part = 1.2f * (float)(16 * Geo::AT * Geo::WPT * Geo::THREADS) / (float)Geo::STAGE;
+    PgPlan best;
+    best.slots = nx;
+    best.cost = (float)((nx + cpx - 1) / cpx) * ((float)ns + kEdge);
+    const int full = nx / cpx * cpx, tail = nx - full;
+    for (int S : {2, 3, 4, 5, 6, 8, 10, 12, 16}) {
+        if (!ws || tail == 0 || ns < 4 * S || 8 * tail > kPgWsTiles ||
+            (size_t)8 * tail * S * 16 * Geo::AT * Geo::WPT * Geo::THREADS > kPgWsBytes)
+            break;
+        const float c = (float)(full / cpx) * ((float)ns + kEdge) +
+                        (float)((tail * S + cpx - 1) / cpx) * ((float)(ns + S - 1) / (float)S + kEdge) + part * (float)(S + 2);
+        if (c < best.cost) best = PgPlan{full, S, full + tail * S, c};
+    }
+    return best;
+}
+
 template <class Epi, class Cfg, typename WT>
-hipError_t launch_pgemm(const PgIn<WT>& in, const Epi& epi, const PfState* ps, hipStream_t s) {
+hipError_t launch_pgemm(const PgIn<WT>& in, const Epi& epi, const PfState& ps, hipStream_t s) {
     using Geo = PgGeo<Cfg, WT>;
     if (in.M % Geo::BM != 0) return hipErrorInvalidValue;  // rows past the last whole tile would be skipped
-    const int nrb = (in.N + Geo::BN - 1) / Geo::BN;
-    const int nrb8 = (nrb + 7) / 8 * 8;
-    const dim3 grid(nrb8 * (in.M / Geo::BM));
-    hipLaunchKernelGGL((pgemm_kernel<Epi, Cfg, WT>), grid, dim3(Geo::THREADS), Geo::LDS, s, in, epi, ps);
+    const int nx = ((in.N + Geo::BN - 1) / Geo::BN + 7) / 8 * (in.M / Geo::BM);
+    if (in.full < nx && (!in.ws || !in.cnt || in.splits < 2)) return hipErrorInvalidValue;
+    const int slots = in.full < nx ? in.full + (nx - in.full) * in.splits : nx;
+    hipLaunchKernelGGL((pgemm_kernel<Epi, Cfg, WT>), dim3(8 * slots), dim3(Geo::THREADS), Geo::LDS, s, in, epi, ps);
     return hipGetLastError();
 }
 
@@ -637,13 +682,13 @@ struct PfAttnArgs {
 };
 
 template <typename KT, int HD>
-__global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, const PfState* __restrict__ ps) {
+__global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState ps) {
     constexpr int QD = HD / 4;  // dims per lane
     __shared__ __attribute__((aligned(16))) KT ks[kPaKT][HD];
     __shared__ __attribute__((aligned(16))) KT vs[kPaKT][HD];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.y, G = a.hq / a.hkv, kvh = h / G;
-    const int p0 = ps->p0;
+    const int p0 = ps.p0;
     const int mi = blockIdx.x * kPaQB + wave * 16 + (lane & 15);  // this lane's query (chunk row)
     const int c = lane >> 4;
     const int pos = p0 + mi;                                      // its position
@@ -745,8 +790,7 @@ struct PfRowsArgs {
     const float* gate = nullptr;
 };
 template <int HD, int ROWS = 0>
-__global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, const PfState* __restrict__ ps,
-                                                           PfRowsArgs x) {
+__global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, PfState ps, PfRowsArgs x) {
     using G = PaGeo<HD>;
     constexpr int ND = HD / 32, NT = HD / 16;  // 32-d blocks (S), 16-d tiles (O)
     __shared__ __attribute__((aligned(1024))) char sm[4 * G::WAVE];
@@ -772,8 +816,8 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
             tile0 = kmin / 32;
         }
     } else {
-        pos = ps->p0 + mq;
-        last = min(ps->p0 + (int)blockIdx.x * 16 + 15, a.T - 1);
+        pos = ps.p0 + mq;
+        last = min(ps.p0 + (int)blockIdx.x * 16 + 15, a.T - 1);
     }
     const int kmax = ROWS ? last : a.T - 1;  // cache rows past it are read as this one (their scores are masked)
     float bias1 = 0.0f, bias2 = 0.0f;

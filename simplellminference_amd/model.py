@@ -261,7 +261,7 @@ class LlamaModel:
         return text
 
     def prefill(self, prompt_ids):
-        """Run prompt positions 0..n-2 through the layers in chunks of up to 256 (MFMA GEMM projections,
+        """Run prompt positions 0..n-2 through the layers in chunks of up to 4096 (MFMA GEMM projections,
         block-causal attention) and leave the state at the last prompt token, so the next step() yields the
         first greedy token (sli_model_prefill). Under multi-process tensor parallelism every rank calls it."""
         p = np.ascontiguousarray(prompt_ids, np.int32)

@@ -1,12 +1,12 @@
 """Prompt prefill (sli_model_prefill): the prompt's positions 0..n-2 run through the
-layers in chunks of up to 256 positions — every projection one MFMA GEMM over the chunk, attention
+layers in chunks of up to 4096 positions — every projection one MFMA GEMM over the chunk, attention
 block-causal over the cache — then decoding continues from the last prompt token. The reference
 teacher-forces the prompt one token per forward (model.cpp:157-165); the oracle's predict does the same, so
 the bar is the oracle's predict: greedy token ids bit-exact, logits of every computed position within 1e-3,
 and the K/V rows the prefill writes within the fp16 cache rounding.
 
-Chunk sizes 32 / 64 / 128 / 256 (prefill.h kPfMaxChunk): the prompt lengths below cover every chunk size,
-one and two chunks, a ragged last chunk and the padding rows of a chunk.
+The launches of a chunk run 32, 64 or a multiple of 128 rows: the prompt lengths below cover each, padding rows, and
+GEMMs whose last round of tiles is cut over the depth.
 """
 import numpy as np
 import pytest
@@ -60,7 +60,7 @@ def test_prefill_predict_matches_oracle(gpu, oracle, name, n):
 
 @pytest.mark.parametrize("n", [129, 200, 257, 300])
 def test_prefill_long_prompts(gpu, oracle, n):
-    """Prompts of 129..300 tokens: one chunk of 128 / 256 rows, two chunks (256 + 0 / 43 rows), GQA."""
+    """Prompts of 129..300 tokens: launches of 128, 256 and 384 rows, GQA."""
     cfg, om, gm = _pair(oracle, "tiny-gqa", max_length=320)
     prompt = _prompt(n, cfg.vocab_size)
     steps = n + 12
@@ -187,3 +187,26 @@ def test_prefill_tp_group(gpu, oracle, name, tp, w, over):
     om.close()
     assert all(s == states[0] for s in states), states
     _check(gtok, glog, otok, olog, 140)
+
+
+@pytest.mark.parametrize("w", ["f16", "i8"])
+@pytest.mark.parametrize("n", [34, 65, 66, 129, 130, 258, 514, 770, 1026])
+def test_prefill_splits_match_decode(gpu, w, n):
+    """Every row count's tilings with their last round cut over the depth (small outputs: the whole launch), a wave's and a
+    workgroup's worth of padding rows, and (int8) a depth that ends in a half stage (2752 = 21.5 x 128), against the
+    engine's own decode step over the same prompt. 1e-3: this file's bar; the two paths differ by where fp32 sums fall
+    around the fp16 rounding of K and V."""
+    from simplellminference_amd.model import LlamaModel, preset
+    cfg = preset("small-h128-gqa", max_length=1088, intermediate_size=2752)
+    m = LlamaModel(config=cfg, w_dtype=w, kv_dtype="f16", seed=4).init()
+    prompt = _prompt(n, cfg.vocab_size)
+    ref = m.predict(prompt, n + 3, want_logits=True)
+    k0 = m.kv(1, 0, n), m.kv(1, 1, n)
+    m.reset()
+    tok, log = m.predict_prefill(prompt, n + 3, want_logits=True)
+    k1 = m.kv(1, 0, n), m.kv(1, 1, n)
+    m.close()
+    assert np.array_equal(tok, ref[0])
+    assert np.abs(log[n - 1:] - ref[1][n - 1:]).max() <= 1e-3
+    for a, b in zip(k0, k1):  # one fp16 rounding of values up to 8
+        assert np.abs(a - b).max() <= 2 ** -7

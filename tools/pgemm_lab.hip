@@ -92,11 +92,26 @@ static void release(Bufs<WT>& b) {
     CK(hipFree(b.ps));
 }
 
+static float* g_ws;
+static unsigned* g_cnt;
+// force: splits of every tile (0: the plan)
 template <class Cfg, typename WT>
-static void run(const char* tag, Bufs<WT>& b, const Shape& sh, int M) {
+static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force = 0) {
     using Geo = PgGeo<Cfg, WT>;
+    if (M % Geo::BM) return;
+    PgPlan pl = pg_plan<Cfg, WT>(sh.N, sh.K, M, 256, true);
+    if (force) {
+        const int nx = ((sh.N + Geo::BN - 1) / Geo::BN + 7) / 8 * (M / Geo::BM), f = nx / (32 * (160 * 1024 / Geo::LDS)) * (32 * (160 * 1024 / Geo::LDS));
+        if (force == 1) pl.full = 0x7fffffff, pl.splits = 1, pl.slots = nx;
+        else pl.full = f, pl.splits = force, pl.slots = f + (nx - f) * force;
+        if ((size_t)8 * (nx - f) * force * 16 * Geo::AT * Geo::WPT * Geo::THREADS > kPgWsBytes || (sh.K + Geo::KS - 1) / Geo::KS < force) return;
+        if (force > 1 && nx == f) return;
+    }
+    char tag[96];
+    snprintf(tag, sizeof tag, "%s full %d S %d", name, pl.full > 100000 ? -1 : pl.full, pl.splits);
     CK((pgemm_allow_lds<PgEpiResid, Cfg, WT>()));
     PgIn<WT> in{b.W, b.hi, b.lo, sh.N, sh.K, M};
+    in.full = pl.full, in.splits = pl.splits, in.ws = g_ws, in.cnt = g_cnt;
     PgEpiResid e{b.y, nullptr, nullptr, sh.N, sh.N};
     CK(hipMemset(b.y, 0, sizeof(float) * (size_t)M * sh.N));
     CK((launch_pgemm<PgEpiResid, Cfg, WT>(in, e, b.ps, 0)));
@@ -146,55 +161,57 @@ static void run(const char* tag, Bufs<WT>& b, const Shape& sh, int M) {
     CK(hipEventDestroy(e1));
 }
 
-#define RUN(BM, WR, S) run<PgCfg<BM, WR, S>, WT>("BM" #BM " WR" #WR " S" #S, b, sh, M)
-#define RUNP(BM, WR, S, AT) run<PgCfg<BM, WR, S, AT, true>, WT>("BM" #BM " WR" #WR " S" #S " AT" #AT " pipe", b, sh, M)
-#define RUNA(BM, WR, AT, SA) \
-    run<PgCfg<BM, WR, 2, AT, true, SA>, WT>("BM" #BM " WR" #WR " AT" #AT " pipe SA" #SA, b, sh, M)
+#define RUN(BM, WR, S, AT, SA)                                                            \
+    for (int f : forces) run<PgCfg<BM, WR, S, AT, SA>, WT>("BM" #BM " WR" #WR " S" #S " AT" #AT " SA" #SA, b, sh, M, f)
 
 template <typename WT>
-static void sweep(const Shape& sh, int M) {
+static void sweep(const Shape& sh, int M, const std::vector<int>& forces) {
     Bufs<WT> b;
     make(b, sh.N, sh.K, M);
-    if (getenv("LAB_QUICK")) {  // the engine's fp16 tilings at M = 256 (prefill.h pg_pick)
-        if constexpr (sizeof(WT) == 2) {
-            RUNA(128, 4, 2, 4);
-            RUNP(64, 4, 3, 2);
-            RUNP(64, 2, 3, 2);
-        }
-        release(b);
-        return;
-    }
     if constexpr (sizeof(WT) == 2) {
-        RUN(128, 2, 2);
-        RUN(128, 2, 3);
-        RUN(128, 2, 4);
-        RUN(64, 2, 3);
-        RUN(64, 2, 4);
-        RUN(64, 2, 6);
-        RUN(64, 4, 3);
-        RUN(64, 4, 4);
-        RUN(128, 4, 2);
-        RUN(128, 4, 3);
-        RUN(256, 2, 2);
-        RUN(256, 4, 2);
-        RUN(32, 2, 4);
-        RUN(32, 2, 8);
+        if (M <= 32) {
+            RUN(32, 2, 4, 2, 0);
+            RUN(32, 4, 4, 2, 0);
+            RUN(32, 4, 3, 4, 0);
+        } else if (M <= 64) {
+            RUN(64, 2, 4, 2, 0);
+            RUN(64, 4, 4, 2, 0);
+            RUN(64, 4, 3, 4, 0);
+        } else {
+            RUN(64, 4, 3, 2, 0);
+            RUN(128, 4, 2, 2, 4);
+            RUN(128, 4, 2, 4, 3);
+            RUN(128, 4, 2, 4, 0);
+        }
     } else {
-        RUN(64, 2, 2);
-        RUN(64, 2, 3);
-        RUN(128, 2, 2);
-        RUN(64, 4, 2);
-        RUN(64, 4, 3);
-        RUN(128, 4, 2);
-        RUN(32, 2, 4);
+        if (M <= 32) {
+            RUN(32, 2, 4, 2, 0);
+            RUN(32, 4, 4, 2, 0);
+        } else if (M <= 64) {
+            RUN(64, 4, 2, 2, 0);
+            RUN(64, 4, 3, 2, 0);
+            RUN(64, 4, 2, 4, 0);
+        } else {
+            RUN(64, 4, 3, 2, 0);
+            RUN(128, 4, 2, 2, 0);
+        }
     }
     release(b);
 }
 
+// pgemm_lab M [splits ...]: splits 0 = the plan, 1 = none, n = the last round's tiles cut into n
 int main(int argc, char** argv) {
     const int M = argc > 1 ? atoi(argv[1]) : 256;
+    std::vector<int> forces;
+    for (int i = 2; i < argc; ++i) forces.push_back(atoi(argv[i]));
+    if (forces.empty()) forces = {0, 1};
+    CK(hipMalloc(&g_ws, kPgWsBytes));
+    CK(hipMalloc(&g_cnt, sizeof(unsigned) * kPgWsTiles));
+    CK(hipMemset(g_cnt, 0, sizeof(unsigned) * kPgWsTiles));
     const Shape shapes[] = {{"qkv", 12288, 4096}, {"gu", 22016, 4096}, {"wo", 4096, 4096}, {"down", 4096, 11008}};
-    for (const Shape& sh : shapes) sweep<__half>(sh, M);
-    for (const Shape& sh : shapes) sweep<int8_t>(sh, M);
+    if (!getenv("LAB_I8"))
+        for (const Shape& sh : shapes) sweep<__half>(sh, M, forces);
+    else
+        for (const Shape& sh : shapes) sweep<int8_t>(sh, M, forces);
     return 0;
 }
