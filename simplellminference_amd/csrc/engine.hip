@@ -1056,7 +1056,7 @@ struct StepRecorder {
             return fail(SLI_ERR_ARG, "prefill needs fp16 or int8 weights");
         } else {
             PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
-            in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nv;
+            in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
             float best = INFINITY;
             int pick = 0, i = 0;
             pg_each(M, [&](auto cfg, float us) {
@@ -1096,8 +1096,8 @@ struct StepRecorder {
         hipStream_t s = m->stream;
         const int D = m->D, hd = m->hd, QD = m->hq * hd;
         if (p == 0) {
-            hipLaunchKernelGGL(pf_embed_kernel<WT>, dim3(M), dim3(256), 0, s, ps, m->prompt, (const WT*)m->emb,
-                               m->emb_s, f.x, D);
+            hipLaunchKernelGGL(pf_embed_kernel<WT>, dim3(M), dim3(256), 0, s, ps, m->prompt, m->T + 1,
+                               (const WT*)m->emb, m->emb_s, f.x, D);
             SLI_HIP(hipGetLastError());
         }
         const int l = p / 2;
@@ -1113,12 +1113,8 @@ struct StepRecorder {
             SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, ps));
             PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, f.hhi, f.hlo, m->hq, m->hkv, m->T,
                               1.0f / sqrtf((float)hd)};
-            if constexpr (std::is_same<KT, __half>::value) {  // MFMA, 16 chunk rows per workgroup
-                const dim3 ag(M / 16, m->hq);
-                if (hd == 128)
-                    hipLaunchKernelGGL((pf_attn_mfma_kernel<128>), ag, dim3(256), 0, s, aa, ps, PfRowsArgs{});
-                else
-                    hipLaunchKernelGGL((pf_attn_mfma_kernel<64>), ag, dim3(256), 0, s, aa, ps, PfRowsArgs{});
+            if constexpr (std::is_same<KT, __half>::value) {
+                SLI_HIP(hd == 128 ? launch_pf_flash<128>(aa, ps, device_cus(), s) : launch_pf_flash<64>(aa, ps, device_cus(), s));
             } else {  // fp32 cache: fp32 VALU, 64 chunk rows per workgroup
                 const dim3 ag((M + kPaQB - 1) / kPaQB, m->hq);
                 if (hd == 128)
@@ -1927,7 +1923,10 @@ static int pf_alloc(sli_model* m) {
 // chunk c of the prompt's n - 1 prefilled positions
 static std::vector<PfState> pf_chunks(int n) {
     std::vector<PfState> cs;
-    for (int p0 = 0; p0 < n - 1; p0 += kPfMaxChunk) cs.push_back(PfState{p0, std::min(kPfMaxChunk, n - 1 - p0)});
+    for (int p0 = 0; p0 < n - 1; p0 += kPfMaxChunk) {
+        const int nv = std::min(kPfMaxChunk, n - 1 - p0);
+        cs.push_back(PfState{p0, nv, pf_rows(nv), 1});
+    }
     return cs;
 }
 

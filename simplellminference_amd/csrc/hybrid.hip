@@ -619,9 +619,9 @@ struct HyRec : HyProj<WT> {
                     const PfRowsArgs px{s->rows, l.r1, l.r2, l.sink, l.Kp, d.vdim};
                     const dim3 gr(M / 16, d.heads);
                     if (l.hd == 64)
-                        hipLaunchKernelGGL((pf_attn_mfma_kernel<64, 1>), gr, dim3(256), 0, st(), pa, PfState{}, px);
+                        hipLaunchKernelGGL((pf_attn_mfma_kernel<64, 1>), gr, dim3(256), 0, st(), pa, px);
                     else
-                        hipLaunchKernelGGL((pf_attn_mfma_kernel<128, 1>), gr, dim3(256), 0, st(), pa, PfState{}, px);
+                        hipLaunchKernelGGL((pf_attn_mfma_kernel<128, 1>), gr, dim3(256), 0, st(), pa, px);
                     SLI_HIP(hipGetLastError());
                     return SLI_OK;
                 }

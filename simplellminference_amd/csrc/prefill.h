@@ -15,11 +15,10 @@
 //      current k-block's MFMAs. Fused epilogues:
 //      RoPE + K/V cache rows + q (model.cpp:52-67), residual add (:86-90, :124-128), SwiGLU (:111-115,
 //      written straight as the down projection's hi/lo operand);
-//   3. pf_attn_mfma_kernel (fp16 KV, the default): block-causal attention of 16 chunk rows x one head against
-//      the cache rows 0 .. position (mha_kernel.cpp:36-77 per query: s_t = q.k_t * scale, softmax, sum p_t v_t):
-//      S = K q^T on MFMA with q split hi/lo, online softmax in fp32, P V on MFMA with V read transposed
-//      (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the VALU form (fp32, 64-position query
-//      blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches.
+//   3. pf_flash_kernel (fp16 KV): block-causal attention against the cache rows 0 .. position (mha_kernel.cpp:36-77
+//      per query: s_t = q.k_t * scale, softmax, sum p_t v_t): S = K q^T on MFMA with q split hi/lo, online softmax in
+//      fp32, P V on MFMA with V read transposed (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the
+//      VALU form (fp32, 64-position query blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches.
 // int8 weights: stages of 128 k; a depth that is 64 mod 128 (e.g. Llama-2-7B int8 down at TP 4, 2752) ends with
 // a half stage (pgemm_kernel).
 // The launches of a chunk go to the stream one by one (its start position and valid count are kernel arguments): each
@@ -37,9 +36,12 @@ namespace sli {
 constexpr int kPfMaxChunk = 4096;
 constexpr int kPgGroup = 8;        // position blocks that an XCD takes through its row blocks together
 
+// nseq sequences (cache slots in order) of rps chunk rows each, rps a multiple of 16 (fp32 cache: 64): row i of a sequence
+// is its position p0 + i.
 struct PfState {
-    int32_t p0;  // position of chunk row 0
-    int32_t nv;  // valid chunk rows (the rest is padding: computed, never written to the cache)
+    int32_t p0 = 0;
+    int32_t nv = 0;  // valid rows of a sequence (the rest is padding: computed, never written to the cache)
+    int32_t rps = 1, nseq = 1;
 };
 
 typedef _Float16 pf_half8 __attribute__((ext_vector_type(8)));
@@ -57,13 +59,14 @@ __device__ __forceinline__ void pf_split(float v, __half& hi, __half& lo) {
 }
 
 // ---------------------------------------------------------------- 1. embedding + RMSNorm / split
-// x[m] = emb[prompt[p0 + m]] (emb_kernel.cpp:4-21; padding rows repeat the last valid token)
+// x[m] = emb[prompt[p0 + i]] of the row's sequence (emb_kernel.cpp:4-21; padding rows repeat the last valid token)
 template <typename WT>
 __global__ void __launch_bounds__(256) pf_embed_kernel(PfState ps, const int32_t* __restrict__ prompt,
-                                                      const WT* __restrict__ emb, const float* __restrict__ emb_s,
-                                                      float* __restrict__ x, int D) {
+                                                      int prompt_ld, const WT* __restrict__ emb,
+                                                      const float* __restrict__ emb_s, float* __restrict__ x, int D) {
     const int m = blockIdx.x;
-    const int tok = prompt[ps.p0 + min(m, ps.nv - 1)];
+    const int b = min(m / ps.rps, ps.nseq - 1);
+    const int tok = prompt[(size_t)b * prompt_ld + ps.p0 + min(m - b * ps.rps, ps.nv - 1)];
     const float s = emb_s ? emb_s[tok] : 1.0f;
     for (int i = threadIdx.x; i < D; i += 256) x[(size_t)m * D + i] = to_f32(emb[(size_t)tok * D + i]) * s;
 }
@@ -506,7 +509,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
 template <typename KT>
 struct PgEpiQKV {  // model.cpp:52-67: q (fp32 [M][hq*hd]), rotated k / v rows of the cache at p0 + m
     float* q;
-    KT* kc;  // this layer's cache base [hkv][T][hd]
+    KT* kc;  // this layer's cache base [sequence][hkv][T][hd]
     KT* vc;
     const float* rscale;  // int8 row scales (nullable)
     const float* sin_t;
@@ -520,7 +523,8 @@ struct PgEpiQKV {  // model.cpp:52-67: q (fp32 [M][hq*hd]), rotated k / v rows o
     }
     __device__ void store(int t, int i0, int m, const float* v, const PfState& ps) const {
         // units u, u + 1 (u even): d, d + 1 of one head (hd / 2 is even), so every store is a pair
-        const int nv = ps.nv, pos = ps.p0 + m;
+        const int b = ps.nseq == 1 ? 0 : m / ps.rps, i = m - b * ps.rps, pos = ps.p0 + i;
+        const bool keep = i < ps.nv && b < ps.nseq && pos < T;
         const int half = hd >> 1;
         const int u = t * 8 + (i0 >> 2) * 2;
         const int uh = u / half, d = u - uh * half;
@@ -545,13 +549,13 @@ struct PgEpiQKV {  // model.cpp:52-67: q (fp32 [M][hq*hd]), rotated k / v rows o
                 float* qr = q + (size_t)m * hq * hd + (size_t)uh * hd;
                 *reinterpret_cast<float2*>(qr + d) = make_float2(r0[0], r0[1]);
                 *reinterpret_cast<float2*>(qr + d + half) = make_float2(r1[0], r1[1]);
-            } else if (m < nv && pos < T) {
-                KT* kr = kc + ((size_t)(uh - hq) * T + pos) * hd;
+            } else if (keep) {
+                KT* kr = kc + (((size_t)b * hkv + uh - hq) * T + pos) * hd;
                 store2(kr + d, r0);
                 store2(kr + d + half, r1);
             }
-        } else if (m < nv && pos < T) {
-            KT* vr = vc + ((size_t)(uh - hq - hkv) * T + pos) * hd;
+        } else if (keep) {
+            KT* vr = vc + (((size_t)b * hkv + uh - hq - hkv) * T + pos) * hd;
             store2(vr + d, a0);
             store2(vr + d + half, a1);
         }
@@ -664,7 +668,7 @@ hipError_t pgemm_allow_lds() {
 }
 
 // ---------------------------------------------------------------- 3. block-causal attention
-// grid (M / 64, hq); 4 waves x 16 queries; lane l: query l & 15 of the wave, dims [c * HD/4, (c+1) * HD/4) with
+// grid (rows / 64, hq); 4 waves x 16 queries; lane l: query l & 15 of the wave, dims [c * HD/4, (c+1) * HD/4) with
 // c = l >> 4. Scores: the 4 lanes of a query add their quarter dot products (xor 16 / 32 exchanges); every lane
 // of a query keeps the same online-softmax state (m, l) and its quarter of o. Output attn / l as hi / lo.
 constexpr int kPaQB = 64;  // queries per workgroup
@@ -673,7 +677,7 @@ constexpr int kPaKT = 64;  // keys per LDS tile
 template <typename KT>
 struct PfAttnArgs {
     const float* q;    // [M][hq*hd]
-    const KT* kc;      // layer base [hkv][T][hd]
+    const KT* kc;      // layer base [sequence][hkv][T][hd]
     const KT* vc;
     __half* ohi;       // [M][hq*hd]
     __half* olo;
@@ -688,7 +692,8 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
     __shared__ __attribute__((aligned(16))) KT vs[kPaKT][HD];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.y, G = a.hq / a.hkv, kvh = h / G;
-    const int p0 = ps.p0;
+    const int seq = blockIdx.x * kPaQB / ps.rps, row0 = seq * ps.rps, p0 = ps.p0 - row0;
+    if (seq >= ps.nseq) return;                                   // (uniform)
     const int mi = blockIdx.x * kPaQB + wave * 16 + (lane & 15);  // this lane's query (chunk row)
     const int c = lane >> 4;
     const int pos = p0 + mi;                                      // its position
@@ -701,8 +706,8 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
         o[e] = 0.0f;
     }
     float mx = -INFINITY, l = 0.0f;
-    const KT* kb = a.kc + (size_t)kvh * a.T * HD;
-    const KT* vb = a.vc + (size_t)kvh * a.T * HD;
+    const KT* kb = a.kc + ((size_t)seq * a.hkv + kvh) * a.T * HD;
+    const KT* vb = a.vc + ((size_t)seq * a.hkv + kvh) * a.T * HD;
     constexpr int V16 = 16 / (int)sizeof(KT);  // elements per 16-byte vector
     for (int tt = 0; tt < nt; ++tt) {
         const int t0 = tt * kPaKT;
@@ -747,17 +752,9 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
     }
 }
 
-// ---- 3b. block-causal attention on MFMA (fp16 cache). A workgroup = 16 chunk rows (queries) of one head;
-// its 4 waves split the key range into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their
-// (max, sum, o) through LDS at the end. Per tile a wave:
-//   - LDS-DMAs K and V rows t0 .. t0+31 (16 x 1 KiB pieces) into its own images, 16-B chunks XOR-swizzled;
-//   - Sᵀ = K Qᵀ: C[key][query] on v_mfma_f32_16x16x32_f16, A = K rows (exact fp16), B = Qᵀ as hi + lo fp16
-//     (two MFMAs into one accumulator);
-//   - online softmax per query (a lane's 8 keys, then the 4 lane groups of a query by xor 16 / 32);
-//   - Oᵀ += Vᵀ Pᵀ: B = Pᵀ straight from the Sᵀ accumulators (lane l holds query l & 15, keys
-//     {4g .. 4g+3, 16+4g .. 16+4g+3}, g = l >> 4 — the k order of the B operand), P as hi + lo; A = Vᵀ by
-//     two ds_read_b64_tr_b16 per 16-d tile, whose 4-row blocks are exactly those keys.
-// mha_kernel.cpp:36-77 per query: s_t = (q . k_t) * scale, softmax over t <= position, o = sum p_t v_t.
+// ---- 3b. the packed rows of block-stack models, on MFMA (fp16 cache). A workgroup = 16 rows (queries) of one head;
+// its 4 waves split the key range into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o)
+// through LDS at the end; per tile as pf_flash_kernel, with K and V in the wave's own images.
 template <int HD>
 struct PaGeo {
     static constexpr int ROWB = HD * 2;          // bytes per image row
@@ -775,7 +772,228 @@ __device__ __forceinline__ uint2 pa_tr_read(unsigned lds_addr) {
     return v;
 }
 
-//
+// the transposed reads landed: their registers are named in the wait, so the MFMAs that use them stay below it (as in
+// attn_mfma.h; an asm load's outputs count as written at its end)
+__device__ __forceinline__ void pa_tr_wait(uint2 (&x1)[8], uint2 (&x2)[8]) {
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(x1[0]), "+v"(x1[1]), "+v"(x1[2]), "+v"(x1[3]), "+v"(x1[4]), "+v"(x1[5]), "+v"(x1[6]),
+                   "+v"(x1[7]), "+v"(x2[0]), "+v"(x2[1]), "+v"(x2[2]), "+v"(x2[3]), "+v"(x2[4]), "+v"(x2[5]),
+                   "+v"(x2[6]), "+v"(x2[7])
+                 :
+                 : "memory");
+}
+__device__ __forceinline__ void pa_tr_wait(uint2 (&x1)[4], uint2 (&x2)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(x1[0]), "+v"(x1[1]), "+v"(x1[2]), "+v"(x1[3]), "+v"(x2[0]), "+v"(x2[1]), "+v"(x2[2]),
+                   "+v"(x2[3])
+                 :
+                 : "memory");
+}
+
+// ---- 3a. the same over an fp16 cache, on MFMA. A workgroup = 4 waves over one kv head: GW of its query heads x 4 / GW
+// blocks of 16 QT query positions, a wave each (GQA: 4 heads read one tile; MHA: 4 position blocks do). K and V tiles of
+// 64 keys reach LDS by DMA, double-buffered, one barrier per tile: every key row is fetched once per 64 QT query rows.
+// Per tile a wave computes
+//   - Sᵀ = K Qᵀ: C[key][query] on v_mfma_f32_16x16x32_f16, A = K rows (exact fp16), B = Qᵀ as hi + lo fp16;
+//   - online softmax in base 2 (p = 2^(s c - m), one fma and one v_exp per score, its rounding that of the exponent);
+//     the row maximum over the 4 lane groups of a query, the row sum only at the end. p carries a factor 2^8, which
+//     divides out with the row sum: the lo halves of p >= 2^-21 stay normal fp16 numbers;
+//   - Oᵀ += Vᵀ Pᵀ: B = Pᵀ straight from the Sᵀ accumulators (lane l holds query l & 15, keys {4g .. 4g+3, 16+4g ..
+//     16+4g+3}, g = l >> 4 — the k order of the B operand), P as hi + lo; A = Vᵀ by ds_read_b64_tr_b16, whose 4-row
+//     blocks are exactly those keys.
+// The latest (longest) position blocks are dispatched first. mha_kernel.cpp:36-77 per query. Bound by the matrix cores and
+// the softmax between them: Llama-3-8B, 3776 rows, 299 us a layer (785 TFLOP/s with hi + lo), where a workgroup per 16 rows
+// and head, each key tile waited for as it was issued, took 651; Llama-2-7B, 511 rows, 18.7 us against 28.
+template <int HD>
+struct PfFlash {
+    static constexpr int KT = 64, ROWB = HD * 2, IMG = KT * ROWB, CPR = ROWB / 16, PIECES = IMG / 1024;
+};
+template <int HD, int QT>
+__global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, PfState ps, int GW) {
+    using F = PfFlash<HD>;
+    constexpr int ND = HD / 32, NT = HD / 16, NK = F::KT / 16, PPW = 2 * F::PIECES / 4;
+    __shared__ __attribute__((aligned(1024))) char sm[2 * 2 * F::IMG];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int g = lane >> 4, i16 = lane & 15;
+    const int G = a.hq / a.hkv, ng = G / GW, kvh = blockIdx.y / ng;
+    const int h = kvh * G + (blockIdx.y - kvh * ng) * GW + wave % GW;
+    const int RB = (4 / GW) * 16 * QT;  // query positions per workgroup
+    const int bx = gridDim.x - 1 - blockIdx.x, blk = bx / ps.nseq, seq = bx - blk * ps.nseq;
+    if (blk * RB >= ps.nv) return;  // (uniform) only padding rows
+    const int i0 = blk * RB + (wave / GW) * 16 * QT;
+    const int last = min(ps.p0 + min(blk * RB + RB, ps.nv) - 1, a.T - 1);                   // the workgroup's
+    const int wlast = i0 < ps.nv ? min(ps.p0 + min(i0 + 16 * QT, ps.nv) - 1, a.T - 1) : -1;  // the wave's
+    const size_t qs = (size_t)a.hq * HD;
+    u32x4 qh[QT][ND], ql[QT][ND];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        const int row = seq * ps.rps + min(i0 + t * 16 + i16, ps.rps - 1);
+#pragma unroll
+        for (int db = 0; db < ND; ++db) {
+            const float4* qp = reinterpret_cast<const float4*>(a.q + (size_t)row * qs + (size_t)h * HD + db * 32 + g * 8);
+            const float4 v0 = qp[0], v1 = qp[1];
+            const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+            __half hh[8], hl[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pf_split(f[e], hh[e], hl[e]);
+            qh[t][db] = *reinterpret_cast<const u32x4*>(hh);
+            ql[t][db] = *reinterpret_cast<const u32x4*>(hl);
+        }
+    }
+    pf_float4 o[QT][NT];
+    float mx[QT], l[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        mx[t] = -INFINITY, l[t] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < NT; ++d) o[t][d] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const unsigned base = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)sm;
+    const size_t head = ((size_t)seq * a.hkv + kvh) * a.T * HD;
+    // this wave's DMA pieces of a tile: piece p < PIECES of K, then of V; lane i of a piece: row (piece rows) + i / CPR,
+    // physical chunk i % CPR <- logical chunk (i % CPR) ^ swizzle(row)
+    auto issue = [&](int tt) {
+#pragma unroll
+        for (int j = 0; j < PPW; ++j) {
+            const int p = wave * PPW + j;
+            const bool isv = p >= F::PIECES;
+            const int r = (isv ? p - F::PIECES : p) * (1024 / F::ROWB) + lane / F::CPR;
+            const int c = (lane % F::CPR) ^ (isv ? pa_swz_v(r, F::ROWB) : pa_swz_k(r, F::ROWB));
+            pf_dma((isv ? a.vc : a.kc) + head + (size_t)min(tt * F::KT + r, last) * HD + c * 8,
+                   base + (unsigned)((tt & 1) * 2 * F::IMG + p * 1024));
+        }
+    };
+    const float c2 = a.scale * 1.44269504088896340736f;
+    const int nt = last / F::KT + 1;
+    issue(0);
+    for (int tt = 0; tt < nt; ++tt) {
+        pf_wait_vm<0>();
+        __builtin_amdgcn_s_barrier();  // every wave's pieces of tile tt landed; every wave is done with tile tt - 1
+        if (tt + 1 < nt) issue(tt + 1);
+        const int t0 = tt * F::KT;
+        if (t0 > wlast) continue;  // (wave-uniform) nothing of this tile is seen
+        const char* kimg = sm + (tt & 1) * 2 * F::IMG;
+        const unsigned vbase = base + (unsigned)((tt & 1) * 2 * F::IMG + F::IMG);
+        // Sᵀ[key][query] for keys t0 + 16 kt + (0..15)
+        pf_float4 s[NK][QT];
+#pragma unroll
+        for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+            for (int t = 0; t < QT; ++t) s[kt][t] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int db = 0; db < ND; ++db) {
+            u32x4 kf[NK];
+#pragma unroll
+            for (int kt = 0; kt < NK; ++kt) {
+                const int r = kt * 16 + i16;
+                kf[kt] = *reinterpret_cast<const u32x4*>(kimg + r * F::ROWB + ((4 * db + g) ^ pa_swz_k(r, F::ROWB)) * 16);
+            }
+#pragma unroll
+            for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+                for (int t = 0; t < QT; ++t) s[kt][t] = pf_mfma(kf[kt], qh[t][db], s[kt][t]);
+#pragma unroll
+            for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+                for (int t = 0; t < QT; ++t) s[kt][t] = pf_mfma(kf[kt], ql[t][db], s[kt][t]);
+        }
+        // lane holds keys t0 + 16 kt + 4 g + r of query i0 + 16 t + i16
+        u32x4 ph[QT][NK / 2], pl[QT][NK / 2];
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const int pos = ps.p0 + i0 + t * 16 + i16;
+            if (t0 + F::KT - 1 > ps.p0 + i0 + t * 16) {  // (wave-uniform) the diagonal
+#pragma unroll
+                for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (t0 + kt * 16 + 4 * g + r > pos) s[kt][t][r] = -INFINITY;
+            }
+            float cmax = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < NK; ++kt)
+                cmax = fmaxf(cmax, fmaxf(fmaxf(s[kt][t][0], s[kt][t][1]), fmaxf(s[kt][t][2], s[kt][t][3])));
+            cmax = max_xor32(max_xor16(cmax)) * c2;
+            const float mn = fmaxf(mx[t], cmax);
+            if (__any(mn > mx[t])) {  // (key 0 is seen by every row: the maximum is finite from the first tile on)
+                const float corr = __builtin_amdgcn_exp2f(mx[t] - mn);
+                l[t] *= corr;
+#pragma unroll
+                for (int d = 0; d < NT; ++d) o[t][d] *= corr;
+                mx[t] = mn;
+            }
+            const float off = 8.0f - mx[t];
+#pragma unroll
+            for (int kb = 0; kb < NK / 2; ++kb) {
+                __half hh[8], hl[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float p = __builtin_amdgcn_exp2f(fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, off));
+                    l[t] += p;
+                    pf_split(p, hh[e], hl[e]);
+                }
+                ph[t][kb] = *reinterpret_cast<const u32x4*>(hh);
+                pl[t][kb] = *reinterpret_cast<const u32x4*>(hl);
+            }
+        }
+        // Vᵀ 16-d tile d: lane 16 g + 4 q + p addresses row (4 g + q) [+16] of the 32-key block, d 16 d + 4 p .. +3
+        const int q4 = (lane & 15) >> 2, p4 = lane & 3;
+#pragma unroll
+        for (int kb = 0; kb < NK / 2; ++kb) {
+            const int r1 = kb * 32 + 4 * g + q4, r2 = r1 + 16;
+            const unsigned a1 = vbase + r1 * F::ROWB + 8 * (p4 & 1), a2 = vbase + r2 * F::ROWB + 8 * (p4 & 1);
+            const int s1 = pa_swz_v(r1, F::ROWB), s2 = pa_swz_v(r2, F::ROWB);
+            uint2 x1[NT], x2[NT];
+#pragma unroll
+            for (int d = 0; d < NT; ++d) {
+                const int c = 2 * d + (p4 >> 1);
+                x1[d] = pa_tr_read(a1 + ((c ^ s1) * 16));
+                x2[d] = pa_tr_read(a2 + ((c ^ s2) * 16));
+            }
+            pa_tr_wait(x1, x2);
+#pragma unroll
+            for (int d = 0; d < NT; ++d)
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+                    o[t][d] = pf_mfma(u32x4{x1[d].x, x1[d].y, x2[d].x, x2[d].y}, ph[t][kb], o[t][d]);
+#pragma unroll
+            for (int d = 0; d < NT; ++d)
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+                    o[t][d] = pf_mfma(u32x4{x1[d].x, x1[d].y, x2[d].x, x2[d].y}, pl[t][kb], o[t][d]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        const int i = i0 + t * 16 + i16;
+        const float inv = 1.0f / sum_xor32(sum_xor16(l[t]));
+        if (i >= ps.nv) continue;
+#pragma unroll
+        for (int d = 0; d < NT; ++d) {  // lane holds d = 16 d + 4 g + r of query i
+            const size_t idx = (size_t)(seq * ps.rps + i) * qs + (size_t)h * HD + d * 16 + 4 * g;
+            __half hh[4], hl[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pf_split(o[t][d][r] * inv, hh[r], hl[r]);
+            *reinterpret_cast<uint2*>(a.ohi + idx) = *reinterpret_cast<const uint2*>(hh);
+            *reinterpret_cast<uint2*>(a.olo + idx) = *reinterpret_cast<const uint2*>(hl);
+        }
+    }
+}
+
+// Heads and positions per workgroup and wave: 32 query positions per wave where that still gives every CU two workgroups,
+// 16 (twice as many workgroups, each key row read twice as often) below (511 rows of 32 heads: 256 workgroups, not 128).
+template <int HD>
+hipError_t launch_pf_flash(const PfAttnArgs<__half>& a, const PfState& ps, int cus, hipStream_t s) {
+    const int G = a.hq / a.hkv, GW = G < 4 ? G : 4;
+    const int ny = a.hkv * (G / GW);
+    auto blocks = [&](int qt) { return (ps.nv + (4 / GW) * 16 * qt - 1) / ((4 / GW) * 16 * qt) * ps.nseq; };
+    if (blocks(2) * ny >= 2 * cus)
+        hipLaunchKernelGGL((pf_flash_kernel<HD, 2>), dim3(blocks(2), ny), dim3(256), 0, s, a, ps, GW);
+    else
+        hipLaunchKernelGGL((pf_flash_kernel<HD, 1>), dim3(blocks(1), ny), dim3(256), 0, s, a, ps, GW);
+    return hipGetLastError();
+}
+
 // ROWS: the rows are packed portions of several sequences (step_state.h RowRef; a 16-row group belongs to one portion,
 // its valid rows first), with a distance bias and a sink per head (attn_rows.h) and one fp16 output [M][ldo] of vdim
 // dims per head; the caches hold one [hkv][T][HD] block per sequence slot.
@@ -789,8 +1007,8 @@ struct PfRowsArgs {
     const int32_t* koff = nullptr;
     const float* gate = nullptr;
 };
-template <int HD, int ROWS = 0>
-__global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, PfState ps, PfRowsArgs x) {
+template <int HD, int ROWS>
+__global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, PfRowsArgs x) {
     using G = PaGeo<HD>;
     constexpr int ND = HD / 32, NT = HD / 16;  // 32-d blocks (S), 16-d tiles (O)
     __shared__ __attribute__((aligned(1024))) char sm[4 * G::WAVE];
@@ -802,24 +1020,19 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
     int pos, last, slot = 0;  // last: the group's last query position
     int kmin = 0, koff = 0, tile0 = 0;
     bool live = true;
-    if constexpr (ROWS) {
-        const RowRef r0 = x.rows[blockIdx.x * 16];
-        if (r0.slot < 0) return;  // (uniform) a group of padding rows
-        slot = r0.slot;
-        live = x.rows[mq].slot >= 0;
-        pos = r0.pos + i16;
-        last = r0.pos + (int)__popcll(__ballot(live)) / 4 - 1;  // (a row is the query of 4 lanes)
-        if constexpr (ROWS == 2) {
-            slot = 0;
-            kmin = max(0, r0.pos - x.window + 1);  // the first key any row of the group sees
-            koff = x.koff[blockIdx.x >> 1];
-            tile0 = kmin / 32;
-        }
-    } else {
-        pos = ps.p0 + mq;
-        last = min(ps.p0 + (int)blockIdx.x * 16 + 15, a.T - 1);
+    const RowRef r0 = x.rows[blockIdx.x * 16];
+    if (r0.slot < 0) return;  // (uniform) a group of padding rows
+    slot = r0.slot;
+    live = x.rows[mq].slot >= 0;
+    pos = r0.pos + i16;
+    last = r0.pos + (int)__popcll(__ballot(live)) / 4 - 1;  // (a row is the query of 4 lanes)
+    if constexpr (ROWS == 2) {
+        slot = 0;
+        kmin = max(0, r0.pos - x.window + 1);  // the first key any row of the group sees
+        koff = x.koff[blockIdx.x >> 1];
+        tile0 = kmin / 32;
     }
-    const int kmax = ROWS ? last : a.T - 1;  // cache rows past it are read as this one (their scores are masked)
+    const int kmax = last;  // cache rows past it are read as this one (their scores are masked)
     float bias1 = 0.0f, bias2 = 0.0f;
     if constexpr (ROWS == 1) {
         bias1 = x.r1[h];
@@ -924,21 +1137,7 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
             x1[t] = pa_tr_read(a1 + ((c ^ s1) * 16));
             x2[t] = pa_tr_read(a2 + ((c ^ s2) * 16));
         }
-        // the transposed reads landed: their registers are named in the wait, so the MFMAs that use them stay below it
-        // (as in attn_mfma.h; an asm load's outputs count as written at its end)
-        if constexpr (NT == 8)
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+v"(x1[0]), "+v"(x1[1]), "+v"(x1[2]), "+v"(x1[3]), "+v"(x1[4]), "+v"(x1[5]), "+v"(x1[6]),
-                           "+v"(x1[7]), "+v"(x2[0]), "+v"(x2[1]), "+v"(x2[2]), "+v"(x2[3]), "+v"(x2[4]), "+v"(x2[5]),
-                           "+v"(x2[6]), "+v"(x2[7])
-                         :
-                         : "memory");
-        else
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+v"(x1[0]), "+v"(x1[1]), "+v"(x1[2]), "+v"(x1[3]), "+v"(x2[0]), "+v"(x2[1]), "+v"(x2[2]),
-                           "+v"(x2[3])
-                         :
-                         : "memory");
+        pa_tr_wait(x1, x2);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             o[t] *= corr;
@@ -980,33 +1179,24 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
 #pragma unroll
         for (int w = 0; w < 4; ++w) acc += *reinterpret_cast<const pf_float4*>(fo + ((w * NT + t) * 64 + lane) * 4) * w4[w];
         // lane holds d = 16 t + 4 g + r of query mq
-        if constexpr (ROWS) {
-            const int d0 = t * 16 + 4 * g;
-            __half* dst = a.ohi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
-            if (!live) continue;
-            if constexpr (ROWS == 2) {
-                const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
+        const int d0 = t * 16 + 4 * g;
+        __half* dst = a.ohi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
+        if (!live) continue;
+        if constexpr (ROWS == 2) {
+            const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (d0 + r < x.vdim) acc[r] *= gt[r];
-            }
-            if (x.vdim % 4 == 0 && d0 < x.vdim) {
-                const __half hv[4] = {__float2half_rn(acc[0] * inv), __float2half_rn(acc[1] * inv),
-                                      __float2half_rn(acc[2] * inv), __float2half_rn(acc[3] * inv)};
-                *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(hv);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (d0 + r < x.vdim) dst[r] = __float2half_rn(acc[r] * inv);
-            }
-            continue;
+            for (int r = 0; r < 4; ++r)
+                if (d0 + r < x.vdim) acc[r] *= gt[r];
         }
-        const size_t idx = (size_t)mq * qs + (size_t)h * HD + t * 16 + 4 * g;
-        __half hh[4], hl[4];
+        if (x.vdim % 4 == 0 && d0 < x.vdim) {
+            const __half hv[4] = {__float2half_rn(acc[0] * inv), __float2half_rn(acc[1] * inv),
+                                  __float2half_rn(acc[2] * inv), __float2half_rn(acc[3] * inv)};
+            *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(hv);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pf_split(acc[r] * inv, hh[r], hl[r]);
-        *reinterpret_cast<uint2*>(a.ohi + idx) = *reinterpret_cast<const uint2*>(hh);
-        *reinterpret_cast<uint2*>(a.olo + idx) = *reinterpret_cast<const uint2*>(hl);
+            for (int r = 0; r < 4; ++r)
+                if (d0 + r < x.vdim) dst[r] = __float2half_rn(acc[r] * inv);
+        }
     }
 }
 

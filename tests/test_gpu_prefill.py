@@ -210,3 +210,25 @@ def test_prefill_splits_match_decode(gpu, w, n):
     assert np.abs(log[n - 1:] - ref[1][n - 1:]).max() <= 1e-3
     for a, b in zip(k0, k1):  # one fp16 rounding of values up to 8
         assert np.abs(a - b).max() <= 2 ** -7
+
+
+@pytest.mark.parametrize("hd,heads,kvh,n", [(128, 8, 1, 65), (128, 8, 2, 130), (64, 8, 4, 17), (64, 8, 8, 300), (128, 8, 2, 64),
+                                            (64, 32, 32, 2050), (128, 16, 4, 2100)])
+def test_prefill_attention_groups(gpu, hd, heads, kvh, n):
+    """The prompt attention's heads per workgroup (1, 2, 4 of a kv head, 8 as two workgroups), 16 and (the long prompts)
+    32 positions per wave, last tiles and position blocks of 1, 16 and 64 rows, against the engine's decode step. 1e-3 as
+    above."""
+    from simplellminference_amd.model import LlamaModel, LlamaModelConfig
+    cfg = LlamaModelConfig(vocab_size=600, head_dim=hd, hidden_size=hd * heads, kv_hidden_size=hd * kvh,
+                           intermediate_size=512, max_length=n + 8, num_hidden_layers=1, num_attention_heads=heads,
+                           num_key_value_heads=kvh, rms_norm_eps=1e-5, rope_theta=1e4)
+    m = LlamaModel(config=cfg, w_dtype="f16", kv_dtype="f16", seed=2).init()
+    prompt = _prompt(n, cfg.vocab_size)
+    ref = m.predict(prompt, n + 2)
+    lref = m.logits()[0]
+    m.reset()
+    tok = m.predict_prefill(prompt, n + 2)
+    log = m.logits()[0]
+    m.close()
+    assert np.array_equal(tok, ref)
+    assert np.abs(log - lref).max() <= 1e-3
