@@ -1060,6 +1060,9 @@ struct StepRecorder {
             float best = INFINITY;
             int pick = 0, i = 0;
             pg_each(M, [&](auto cfg, float us) {
+                // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
+                // in 16 ranges and more
+                if (st.nseq > 1 && PgGeo<decltype(cfg), WT>::FOLD == 0) us = INFINITY;
                 const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
                 if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
                 ++i;
@@ -1108,7 +1111,7 @@ struct StepRecorder {
                            D, m->c.eps);
         SLI_HIP(hipGetLastError());
         if (p % 2 == 0) {
-            const size_t ls = (size_t)l * m->hkv * m->T * hd;
+            const size_t ls = (size_t)l * m->B * m->hkv * m->T * hd;
             PgEpiQKV<KT> eq{f.q, (KT*)m->kc + ls, (KT*)m->vc + ls, w.qkv_s, m->sin_t, m->cos_t, m->hq, m->hkv, hd, m->T};
             SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, ps));
             PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, f.hhi, f.hlo, m->hq, m->hkv, m->T,
@@ -1132,7 +1135,7 @@ struct StepRecorder {
         return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, M, ps);
     }
     static int record_prefill(sli_model* m, const PfState& ps) {
-        const int M = pf_rows(ps.nv);
+        const int M = pf_rows(ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps);
         for (int p = 0; p < 2 * m->L; ++p) {
             SLI_TRY(record_pf_phase(m, p, M, ps));
             const size_t n = (size_t)M * m->D;
@@ -1894,14 +1897,20 @@ static int get_state(sli_model* m, int seq, int32_t* pos, int32_t* token, int32_
 // whose exchange it does have; an in-process group sums the chunk rows itself (record_group_prefill).
 static bool pf_supported(const sli_model* m) {
     if (m->partial && !m->collectives && !m->group) return false;
-    return m->c.w_dtype != SLI_DT_F32 && m->B == 1 && (m->hd == 64 || m->hd == 128) && m->D % 64 == 0 &&
-           m->D <= 8192 && m->Il % 64 == 0 && (m->hq * m->hd) % 64 == 0;
+    return m->c.w_dtype != SLI_DT_F32 && (m->hd == 64 || m->hd == 128) && m->D % 64 == 0 && m->D <= 8192 && m->Il % 64 == 0 && (m->hq * m->hd) % 64 == 0;
+}
+
+// rows of a sequence of n positions among a batch's rows: whole attention workgroups
+static int pad_rows(const sli_model* m, int n) {
+    const int q = m->c.kv_dtype == SLI_DT_F32 ? kPaQB : 16;
+    return (n + q - 1) / q * q;
 }
 
 static int pf_alloc(sli_model* m) {
     auto& p = m->pf;
     if (p.x) return SLI_OK;
-    const size_t M = pf_rows(std::min(m->T, kPfMaxChunk)), D = m->D, QD = (size_t)m->hq * m->hd;
+    // (64: a workgroup of the fp32 cache's attention)
+    const size_t M = std::max(64, pf_rows(std::min(m->B * pad_rows(m, m->T), kPfMaxChunk))), D = m->D, QD = (size_t)m->hq * m->hd;
     int rc = SLI_OK;
     auto A = [&](void** ptr, size_t bytes) {
         if (rc == SLI_OK) rc = model_alloc(m, ptr, bytes);
@@ -1918,6 +1927,27 @@ static int pf_alloc(sli_model* m) {
     if (rc != SLI_OK) return rc;
     SLI_HIP(hipMemsetAsync(p.cnt, 0, sizeof(unsigned) * kPgWsTiles, m->stream));
     return SLI_DISPATCH(m, prepare_prefill, m);
+}
+
+// chunks of n positions of every sequence of a batch
+static std::vector<PfState> pf_batch_chunks(const sli_model* m, int n) {
+    std::vector<PfState> cs;
+    const int most = pad_rows(m, kPfMaxChunk / m->B - 63);
+    for (int p0 = 0; p0 < n; p0 += most) {
+        const int nv = std::min(most, n - p0);
+        cs.push_back(PfState{p0, nv, pad_rows(m, nv), m->B});
+    }
+    return cs;
+}
+
+// Positions of a batch's prompts that sli_model_predict_batch runs as chunks before its steps (0: all of them as steps):
+// what every prompt has and the steps need not produce. A chunk costs about two steps (Llama-3-8B batch 8, 9 ms for 64
+// rows against 3.3 a step) whatever it holds, so short prompts stay with the steps; so do single sequences with fp16 or
+// int8 weights, whose step keeps activations in fp32 where a chunk splits them in two fp16 terms.
+static int pf_predict_positions(const sli_model* m, const int32_t* lens, int max_length) {
+    if (m->partial || m->B == 1 || !pf_supported(m)) return 0;
+    const int n = std::min(*std::min_element(lens, lens + m->B), max_length) - 1;
+    return n >= 8 ? n : 0;
 }
 
 // chunk c of the prompt's n - 1 prefilled positions
@@ -2208,10 +2238,21 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     for (int b = 0; b < m->B; ++b) {
         SLI_CHECK(lens[b] >= 1 && lens[b] <= ld, SLI_ERR_RANGE, "prompt length out of range");
         SLI_TRY(set_prompt(m, b, prompts + (size_t)b * ld, lens[b]));
-        SLI_TRY(set_state(m, b, prompts[(size_t)b * ld], 0, 1));
+    }
+    // (the prompt positions' logits come from the steps)
+    const int n0 = logits_out || m->bs ? 0 : pf_predict_positions(m, lens, max_length);
+    if (n0 > 0) {
+        SLI_TRY(pf_alloc(m));
+        for (const PfState& c : pf_batch_chunks(m, n0)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
+    }
+    for (int b = 0; b < m->B; ++b) {
+        const int32_t* p = prompts + (size_t)b * ld;
+        if (n0 > 0)
+            SLI_HIP(hipMemcpyAsync(m->hist + (size_t)b * (m->T + 1), p, sizeof(int32_t) * n0, hipMemcpyHostToDevice, m->stream));
+        SLI_TRY(set_state(m, b, p[n0], n0, 1));
     }
     const size_t per_step = (size_t)m->B * m->v_n;
-    for (int t = 0; t < max_length; ++t) {  // model.cpp:157
+    for (int t = n0; t < max_length; ++t) {  // model.cpp:157
         SLI_TRY(sli_model_step(m));
         if (logits_out) SLI_TRY(sli_model_get_logits(m, logits_out + (size_t)t * per_step, (int32_t)per_step, nullptr));
     }

@@ -205,6 +205,11 @@ struct PgGeo {
     static constexpr int A_BYTES = NA * A_IMG;
     static constexpr int STAGE = A_BYTES + NB * PT * B_IMG;
     static constexpr int NDMA = STAGE / 1024;  // wave-instructions per stage
+    // depth after which a wave's sums go into a second set of accumulators (0: one chain over the whole depth). hi + lo
+    // activations keep 2^-23 of a value, one fp32 chain over 4096 k loses more: with it the logits after 100 tokens of
+    // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave: the
+    // second set of a 64 x 64 wave tile would spill (14 % of a 3776-row prompt).
+    static constexpr int FOLD = NB == 2 && AT * WPT <= 8 ? 256 : 0;
     static constexpr int DPW = NDMA / WAVES;   // per wave
     static constexpr int SA = Cfg::SA;         // split rings (PgCfg): A pieces per wave DPA, B pieces DPB
     static constexpr int B_BYTES = STAGE - A_BYTES;
@@ -399,6 +404,17 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
                 for (int a = 0; a < AT; ++a) acc[a][b] = pf_mfma(af[a], bl[b], acc[a][b]);
         }
     };
+    constexpr bool TWO = Geo::FOLD > 0;
+    pf_float4 tot[TWO ? AT : 1][TWO ? Geo::WPT : 1] = {};
+    auto fold = [&] {
+#pragma unroll
+        for (int a = 0; a < AT; ++a)
+#pragma unroll
+            for (int b = 0; b < Geo::WPT; ++b) {
+                tot[a][b] += acc[a][b];
+                acc[a][b] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
     const bool live = Cfg::GR || pb * BM + wp * Geo::WPT * 16 < in.valid;  // (wave-uniform)
     {
         // set X holds even k-blocks, set Y odd ones (KBS is even; an int8 half stage has KBS / 2 = 2): per stage
@@ -439,8 +455,16 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
                 read_frags(st, stb, kb + 1, ya, yh, yl);
                 mfmas(xa, xh, xl);
             }
+            if constexpr (TWO)
+                if (s % (Geo::FOLD / Geo::KS) == Geo::FOLD / Geo::KS - 1) fold();
         }
         if (live) mfmas(ya, yh, yl);
+        if constexpr (TWO) {
+#pragma unroll
+            for (int a = 0; a < AT; ++a)
+#pragma unroll
+                for (int b = 0; b < Geo::WPT; ++b) acc[a][b] += tot[a][b];
+        }
     }
     if (nsp > 1) {
         // Partial sums go out write-through (sc1); the tile's last workgroup to arrive adds them in split order (the
@@ -922,13 +946,12 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
                 for (int d = 0; d < NT; ++d) o[t][d] *= corr;
                 mx[t] = mn;
             }
-            const float off = 8.0f - mx[t];
 #pragma unroll
             for (int kb = 0; kb < NK / 2; ++kb) {
                 __half hh[8], hl[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, off));
+                    const float p = __builtin_amdgcn_exp2f(fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, -mx[t])) * 256.0f;
                     l[t] += p;
                     pf_split(p, hh[e], hl[e]);
                 }

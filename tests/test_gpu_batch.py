@@ -253,3 +253,30 @@ def test_batch_tp_shard_step_nocomm(gpu, monkeypatch, world):
     b = m.forward_batch([5 + b for b in range(8)], [4095, 17, 4000, 1, 2048, 3000, 4095, 9])
     assert a.shape == (8, m.local_vocab) and np.isfinite(a).all() and np.array_equal(a, b)
     m.close()
+
+
+@pytest.mark.parametrize("kv", ["f16", "f32"])
+@pytest.mark.parametrize("name,batch,short,long,length", [
+    ("tiny-gqa", 2, 9, 9, 30), ("tiny", 3, 8, 12, 20), ("tiny-gqa", 8, 10, 17, 17), ("small-h128-gqa", 8, 40, 49, 60),
+    ("small-h128", 5, 200, 210, 214), ("small-h128-gqa", 8, 500, 508, 511)])
+def test_predict_batch_prompt_chunks_match_steps(gpu, kv, name, batch, short, long, length):
+    """Without wanted logits predict_batch runs what every prompt has as packed chunks (9 shared positions and more; 8:
+    steps; 8 sequences of 499: two chunks), with them as steps: the same tokens, states, last logits (1e-3, the bar of these
+    files) and K/V rows (one fp16 rounding of values up to 8)."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset(name), w_dtype="f16", kv_dtype=kv, seed=6, batch=batch).init()
+    r = np.random.default_rng(batch)
+    lens = [short + (long - short) * b // (batch - 1) for b in range(batch)]
+    prompts = [r.integers(0, m.config.vocab_size, n).tolist() for n in lens]
+    want, wl = m.predict_batch(prompts, length, want_logits=True)
+    states = [m.state(b) for b in range(batch)]
+    kv0 = [m.kv(1, w, length, seq=b) for w in (0, 1) for b in range(batch)]
+    m.reset()
+    got = m.predict_batch(prompts, length)
+    lg = m.logits()[0]
+    assert np.array_equal(got, want)
+    assert [m.state(b) for b in range(batch)] == states
+    assert np.abs(lg - wl[:, -1]).max() <= 1e-3
+    for a, b in zip(kv0, [m.kv(1, w, length, seq=b) for w in (0, 1) for b in range(batch)]):
+        assert np.abs(a - b).max() <= 2 ** -7
+    m.close()
