@@ -107,8 +107,9 @@ struct sli_model {
     // every layer per weight pass
     struct Prefill {
         float *x = nullptr, *xpart = nullptr, *q = nullptr;  // [chunk][D], [chunk][D] (TP partials), [chunk][hq hd]
-        __half *hhi = nullptr, *hlo = nullptr;  // [chunk][max(D, hq hd)]: normed x / attention out, fp16 hi + lo
-        __half *ahi = nullptr, *alo = nullptr;  // [chunk][Il]: SwiGLU out, fp16 hi + lo
+        // [chunk][max(D, hq hd)]: normed x / attention out; [chunk][Il]: SwiGLU out: fp16 hi + lo (fp32 weights: fp32, in
+        // the first)
+        __half *hhi = nullptr, *hlo = nullptr, *ahi = nullptr, *alo = nullptr;
         float* ws = nullptr;                    // partial sums of the tiles that a GEMM cuts over its depth (PgIn::ws)
         unsigned* cnt = nullptr;
     } pf;
@@ -1037,9 +1038,14 @@ struct StepRecorder {
     // whose plan (prefill.h pg_plan: rounds, and the last round's tiles cut over the depth) costs least. Measured at 512
     // rows, q/k/v | gate/up | wo | down in us: 123 | 214 | 45 | 102, against 144 | 263 | 122 | 122 of two 256-row chunks
     // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
+    // fp32, 74 rows: 137 | 229 | 54 | 110 (the matrix cores' fp32 rate: 75 TFLOP/s of 151 in padded rows).
     template <class F>
     static void pg_each(int M, F&& f) {
-        if constexpr (std::is_same<WT, int8_t>::value) {
+        if constexpr (std::is_same<WT, float>::value) {
+            if (M % 128 == 0) f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.6f);
+            if (M % 64 == 0) f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.35f);
+            f(PgCfg<32, 2, 6, 2, 0, 1>{}, 0.5f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.95f);
+        } else if constexpr (std::is_same<WT, int8_t>::value) {
             if (M % 128 == 0) f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
             else if (M % 64 == 0) f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 2, 4>{}, 1.65f);
             else f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
@@ -1052,39 +1058,34 @@ struct StepRecorder {
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e, int M,
                   const PfState& st) {
-        if constexpr (std::is_same<WT, float>::value) {
-            return fail(SLI_ERR_ARG, "prefill needs fp16 or int8 weights");
-        } else {
-            PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
-            in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
-            float best = INFINITY;
-            int pick = 0, i = 0;
-            pg_each(M, [&](auto cfg, float us) {
-                // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
-                // in 16 ranges and more
-                if (st.nseq > 1 && PgGeo<decltype(cfg), WT>::FOLD == 0) us = INFINITY;
-                const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
-                if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
-                ++i;
-            });
-            hipError_t err = hipSuccess;
-            i = 0;
-            pg_each(M, [&](auto cfg, float) {
-                if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
-            });
-            SLI_HIP(err);
-            return SLI_OK;
-        }
+        PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
+        in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
+        float best = INFINITY;
+        int pick = 0, i = 0;
+        pg_each(M, [&](auto cfg, float us) {
+            // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
+            // in 16 ranges and more
+            if (st.nseq > 1 && PgGeo<decltype(cfg), WT>::FOLD == 0) us = INFINITY;
+            const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
+            if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
+            ++i;
+        });
+        hipError_t err = hipSuccess;
+        i = 0;
+        pg_each(M, [&](auto cfg, float) {
+            if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
+        });
+        SLI_HIP(err);
+        return SLI_OK;
     }
     template <class Epi>
     static int allow_pg(sli_model*) {
         hipError_t err = hipSuccess;
-        if constexpr (!std::is_same<WT, float>::value)
-            for (int M : {32, 64, 128})
-                pg_each(M, [&](auto cfg, float) {
-                    const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
-                    if (e != hipSuccess) err = e;
-                });
+        for (int M : {32, 64, 128})
+            pg_each(M, [&](auto cfg, float) {
+                const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
+                if (e != hipSuccess) err = e;
+            });
         SLI_HIP(err);
         return SLI_OK;
     }
@@ -1107,14 +1108,15 @@ struct StepRecorder {
         const LayerW& w = m->layers[l];
         const bool tp = m->partial;
         PgEpiResid er{tp ? f.xpart : f.x, (!tp || m->c.tp_rank == 0) ? f.x : nullptr, nullptr, D, D};
-        hipLaunchKernelGGL(pf_norm_split_kernel, dim3(M), dim3(256), 0, s, f.x, m->norms + (size_t)p * D, f.hhi, f.hlo,
-                           D, m->c.eps);
+        constexpr bool F32 = std::is_same<WT, float>::value;
+        const PfOut h = F32 ? PfOut{nullptr, nullptr, (float*)f.hhi} : PfOut{f.hhi, f.hlo};
+        hipLaunchKernelGGL(pf_norm_split_kernel, dim3(M), dim3(256), 0, s, f.x, m->norms + (size_t)p * D, h, D, m->c.eps);
         SLI_HIP(hipGetLastError());
         if (p % 2 == 0) {
             const size_t ls = (size_t)l * m->B * m->hkv * m->T * hd;
             PgEpiQKV<KT> eq{f.q, (KT*)m->kc + ls, (KT*)m->vc + ls, w.qkv_s, m->sin_t, m->cos_t, m->hq, m->hkv, hd, m->T};
             SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, ps));
-            PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, f.hhi, f.hlo, m->hq, m->hkv, m->T,
+            PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, h, m->hq, m->hkv, m->T,
                               1.0f / sqrtf((float)hd)};
             if constexpr (std::is_same<KT, __half>::value) {
                 SLI_HIP(hd == 128 ? launch_pf_flash<128>(aa, ps, device_cus(), s) : launch_pf_flash<64>(aa, ps, device_cus(), s));
@@ -1129,13 +1131,15 @@ struct StepRecorder {
             er.rscale = w.wo_s;
             return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, M, ps);
         }
-        PgEpiSwiGLU eg{f.ahi, f.alo, w.gu_s, m->Il, m->c.act_mode};
+        PgEpiSwiGLU eg{F32 ? PfOut{nullptr, nullptr, (float*)f.ahi} : PfOut{f.ahi, f.alo}, w.gu_s, m->Il, m->c.act_mode};
         SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, M, ps));
         er.rscale = w.down_s;
         return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, M, ps);
     }
     static int record_prefill(sli_model* m, const PfState& ps) {
-        const int M = pf_rows(ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps);
+        const int n = ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps;
+        // (fp32 matrix instructions run at a sixteenth of the rate of fp16: padding rows cost more than tiles of 32)
+        const int M = std::is_same<WT, float>::value && n < 512 ? (n + 31) / 32 * 32 : pf_rows(n);
         for (int p = 0; p < 2 * m->L; ++p) {
             SLI_TRY(record_pf_phase(m, p, M, ps));
             const size_t n = (size_t)M * m->D;
@@ -1888,16 +1892,16 @@ static int get_state(sli_model* m, int seq, int32_t* pos, int32_t* token, int32_
 }  // extern "C" (reopened below)
 
 // ---------------------------------------------------------------- prompt prefill
-// The GEMM prefill (prefill.h) needs fp16 or int8 weights, batch 1, head_dim 64 or 128 and 64-multiple
-// projection depths; otherwise the prompt runs through the decode step itself (teacher forcing), which gives
-// the same tokens.
+// sli_model_prefill takes the chunks (prefill.h) with fp16 or int8 weights at batch 1, head_dim 64 or 128 and 64-multiple
+// projection depths; otherwise the prompt runs through the decode step itself (teacher forcing), which gives the same
+// tokens. Fp32 weights and batches take them in sli_model_predict_batch (pf_predict_positions).
 // The chunked MFMA prefill (prefill.h) takes GEMM depths that are multiples of 64 (int8: 128-deep stages with a
 // half last stage). A multi-process TP rank without an RCCL communicator (SLI_DEBUG_NOCOMM, with or without the
 // one-shot exchange) has no all-reduce for a chunk's M x D residual rows, so it prefills through the decode step,
 // whose exchange it does have; an in-process group sums the chunk rows itself (record_group_prefill).
 static bool pf_supported(const sli_model* m) {
     if (m->partial && !m->collectives && !m->group) return false;
-    return m->c.w_dtype != SLI_DT_F32 && (m->hd == 64 || m->hd == 128) && m->D % 64 == 0 && m->D <= 8192 && m->Il % 64 == 0 && (m->hq * m->hd) % 64 == 0;
+    return (m->hd == 64 || m->hd == 128) && m->D % 64 == 0 && m->D <= 8192 && m->Il % 64 == 0 && (m->hq * m->hd) % 64 == 0;
 }
 
 // rows of a sequence of n positions among a batch's rows: whole attention workgroups
@@ -1910,7 +1914,7 @@ static int pf_alloc(sli_model* m) {
     auto& p = m->pf;
     if (p.x) return SLI_OK;
     // (64: a workgroup of the fp32 cache's attention)
-    const size_t M = std::max(64, pf_rows(std::min(m->B * pad_rows(m, m->T), kPfMaxChunk))), D = m->D, QD = (size_t)m->hq * m->hd;
+    const size_t M = pf_rows(std::max(64, std::min(m->B * pad_rows(m, m->T), kPfMaxChunk))), D = m->D, QD = (size_t)m->hq * m->hd;
     int rc = SLI_OK;
     auto A = [&](void** ptr, size_t bytes) {
         if (rc == SLI_OK) rc = model_alloc(m, ptr, bytes);
@@ -1918,10 +1922,11 @@ static int pf_alloc(sli_model* m) {
     A((void**)&p.x, sizeof(float) * M * D);
     if (m->partial) A((void**)&p.xpart, sizeof(float) * M * D);
     A((void**)&p.q, sizeof(float) * M * QD);
-    A((void**)&p.hhi, sizeof(__half) * M * std::max(D, QD));
-    A((void**)&p.hlo, sizeof(__half) * M * std::max(D, QD));
-    A((void**)&p.ahi, sizeof(__half) * M * m->Il);
-    A((void**)&p.alo, sizeof(__half) * M * m->Il);
+    const bool f32 = m->c.w_dtype == SLI_DT_F32;
+    A((void**)&p.hhi, (f32 ? sizeof(float) : sizeof(__half)) * M * std::max(D, QD));
+    A((void**)&p.ahi, (f32 ? sizeof(float) : sizeof(__half)) * M * m->Il);
+    if (!f32) A((void**)&p.hlo, sizeof(__half) * M * std::max(D, QD));
+    if (!f32) A((void**)&p.alo, sizeof(__half) * M * m->Il);
     A((void**)&p.ws, kPgWsBytes);
     A((void**)&p.cnt, sizeof(unsigned) * kPgWsTiles);
     if (rc != SLI_OK) return rc;
@@ -1941,11 +1946,11 @@ static std::vector<PfState> pf_batch_chunks(const sli_model* m, int n) {
 }
 
 // Positions of a batch's prompts that sli_model_predict_batch runs as chunks before its steps (0: all of them as steps):
-// what every prompt has and the steps need not produce. A chunk costs about two steps (Llama-3-8B batch 8, 9 ms for 64
-// rows against 3.3 a step) whatever it holds, so short prompts stay with the steps; so do single sequences with fp16 or
-// int8 weights, whose step keeps activations in fp32 where a chunk splits them in two fp16 terms.
+// what every prompt has and the steps need not produce. A chunk costs two or three steps whatever it holds, so short
+// prompts stay with the steps; so do single sequences with fp16 or int8 weights, whose step keeps activations in fp32
+// where a chunk splits them in two fp16 terms (fp32 weights multiply fp32 activations in both).
 static int pf_predict_positions(const sli_model* m, const int32_t* lens, int max_length) {
-    if (m->partial || m->B == 1 || !pf_supported(m)) return 0;
+    if (m->partial || (m->B == 1 && m->c.w_dtype != SLI_DT_F32) || !pf_supported(m)) return 0;
     const int n = std::min(*std::min_element(lens, lens + m->B), max_length) - 1;
     return n >= 8 ? n : 0;
 }
@@ -1960,7 +1965,7 @@ static std::vector<PfState> pf_chunks(int n) {
     return cs;
 }
 
-extern "C" int sli_model_prefill_path(const sli_model* m) { return m && m->bs ? 1 : m && m->B == 1 && pf_supported(m) ? 1 : 0; }
+extern "C" int sli_model_prefill_path(const sli_model* m) { return m && m->bs ? 1 : m && m->B == 1 && m->c.w_dtype != SLI_DT_F32 && pf_supported(m) ? 1 : 0; }
 
 extern "C" int sli_model_fused_qkv_attn(sli_model* m) {
     if (!m || m->B != 1 || m->bs) return 0;
@@ -2091,7 +2096,7 @@ extern "C" int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n) {
     SLI_HIP(hipSetDevice(m->c.device));
     SLI_TRY(set_prompt(m, 0, ids, n));
     SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
-    if (n > 1 && pf_supported(m)) {
+    if (n > 1 && sli_model_prefill_path(m)) {
         SLI_TRY(pf_alloc(m));
         for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
         SLI_TRY(wait_stream(m));
@@ -2115,7 +2120,7 @@ extern "C" int sli_tp_group_prefill(sli_tp_group* g, const int32_t* ids, int32_t
         SLI_TRY(set_prompt(m, 0, ids, n));
         SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
     }
-    if (n > 1 && pf_supported(m0)) {
+    if (n > 1 && sli_model_prefill_path(m0)) {
         for (sli_model* m : g->ranks) SLI_TRY(pf_alloc(m));
         for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m0, record_group_prefill, g, c));
         SLI_HIP(hipStreamSynchronize(g->stream));

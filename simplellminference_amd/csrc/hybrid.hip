@@ -614,7 +614,7 @@ struct HyRec : HyProj<WT> {
             }
             if constexpr (!std::is_same<OT, float>::value) {
                 if (!one && l.hd <= 128) {
-                    const PfAttnArgs<__half> pa{l.q, (const __half*)r.kc, (const __half*)r.vc, cat<OT>(l), nullptr,
+                    const PfAttnArgs<__half> pa{l.q, (const __half*)r.kc, (const __half*)r.vc, {cat<OT>(l), nullptr},
                                                 d.heads, d.kv_heads, s->T, d.scale};
                     const PfRowsArgs px{s->rows, l.r1, l.r2, l.sink, l.Kp, d.vdim};
                     const dim3 gr(M / 16, d.heads);

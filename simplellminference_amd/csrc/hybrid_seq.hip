@@ -461,7 +461,7 @@ struct SeqRec : HyProj<WT> {
             g.tiles = w.tiles, g.ntiles = w.ntiles;
             const LatExpand e{q().ks, q().vs, l.Hq, (int)d.dim, l.Hv, (int)d.vdim, l.v0, cap, l.hd};
             HY_TRY(grouped(l.ukv, r.kc, l.Rp, (l.v0 + l.Hv + 1) / 2, g, kLatTile, key_tiles, e));
-            const PfAttnArgs<__half> pa{l.q, q().ks, q().vs, cat, nullptr, (int)d.heads, (int)d.heads, cap, d.scale};
+            const PfAttnArgs<__half> pa{l.q, q().ks, q().vs, {cat, nullptr}, (int)d.heads, (int)d.heads, cap, d.scale};
             PfRowsArgs px{};
             px.rows = s->rows, px.ldo = l.KA, px.vdim = d.vdim, px.window = l.window, px.koff = w.koff, px.gate = q().gate;
             const dim3 gr(M / 16, d.heads);

@@ -19,12 +19,14 @@
 //      per query: s_t = q.k_t * scale, softmax, sum p_t v_t): S = K q^T on MFMA with q split hi/lo, online softmax in
 //      fp32, P V on MFMA with V read transposed (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the
 //      VALU form (fp32, 64-position query blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches.
+// fp32 weights: the same GEMM on v_mfma_f32_16x16x4_f32 with fp32 activations (one image, stages of 32 k).
 // int8 weights: stages of 128 k; a depth that is 64 mod 128 (e.g. Llama-2-7B int8 down at TP 4, 2752) ends with
 // a half stage (pgemm_kernel).
 // The launches of a chunk go to the stream one by one (its start position and valid count are kernel arguments): each
 // runs longer than it takes to enqueue, so a captured graph would only add its capture to a model's first prompt.
 #pragma once
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "step_state.h"
@@ -58,6 +60,28 @@ __device__ __forceinline__ void pf_split(float v, __half& hi, __half& lo) {
     lo = __float2half_rn(v - __half2float(hi));
 }
 
+// What a GEMM reads: fp16 hi + lo, or fp32 (beside fp32 weights)
+struct PfOut {
+    __half *hi = nullptr, *lo = nullptr;
+    float* f = nullptr;
+    template <int N>
+    __device__ __forceinline__ void store(size_t i, const float* v) const {  // N = 2 or 4 values, i a multiple of N
+        if (f) {
+            if constexpr (N == 4)
+                *reinterpret_cast<float4*>(f + i) = make_float4(v[0], v[1], v[2], v[3]);
+            else
+                *reinterpret_cast<float2*>(f + i) = make_float2(v[0], v[1]);
+            return;
+        }
+        __half hh[N], hl[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) pf_split(v[e], hh[e], hl[e]);
+        typedef typename std::conditional<N == 4, uint2, unsigned>::type T;
+        *reinterpret_cast<T*>(hi + i) = *reinterpret_cast<const T*>(hh);
+        *reinterpret_cast<T*>(lo + i) = *reinterpret_cast<const T*>(hl);
+    }
+};
+
 // ---------------------------------------------------------------- 1. embedding + RMSNorm / split
 // x[m] = emb[prompt[p0 + i]] of the row's sequence (emb_kernel.cpp:4-21; padding rows repeat the last valid token)
 template <typename WT>
@@ -75,8 +99,7 @@ __global__ void __launch_bounds__(256) pf_embed_kernel(PfState ps, const int32_t
 // The row is held in registers (a float4 per thread and pass; D % 4 == 0, D <= 8192): one read of x, 8-byte
 // hi / lo stores.
 static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                           __half* __restrict__ hi, __half* __restrict__ lo, int D,
-                                                           float eps) {
+                                                           PfOut out, int D, float eps) {
     constexpr int MAXV = 8;  // float4 per thread: D <= 8192
     const int m = blockIdx.x;
     const float* xr = x + (size_t)m * D;
@@ -108,11 +131,10 @@ static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* 
         if (j * 256 + (int)threadIdx.x < n4) {
             const int i = (j * 256 + threadIdx.x) * 4;
             const float f[4] = {v[j].x, v[j].y, v[j].z, v[j].w}, g[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
-            __half hh[4], hl[4];
+            float y[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) pf_split(w ? (f[e] * inv) * g[e] : f[e], hh[e], hl[e]);  // :20-22
-            *reinterpret_cast<uint2*>(hi + (size_t)m * D + i) = *reinterpret_cast<const uint2*>(hh);
-            *reinterpret_cast<uint2*>(lo + (size_t)m * D + i) = *reinterpret_cast<const uint2*>(hl);
+            for (int e = 0; e < 4; ++e) y[e] = w ? (f[e] * inv) * g[e] : f[e];  // :20-22
+            out.store<4>((size_t)m * D + i, y);
         }
 }
 
@@ -148,8 +170,8 @@ struct PgGroups {
 
 template <typename WT>
 struct PgIn {
-    const WT* W;        // [N][K] fp16 or int8 (row-major, PyTorch [out][in]; int8 row scales in the epilogue)
-    const __half* Bhi;  // [M][K] activations, fp16 hi
+    const WT* W;        // [N][K] fp32, fp16 or int8 (row-major, PyTorch [out][in]; int8 row scales in the epilogue)
+    const __half* Bhi;  // [M][K] activations, fp16 hi (fp32 weights: fp32)
     const __half* Blo;  // [M][K] fp16 lo
     int N, K, M;        // rows, depth, chunk rows (a multiple of BM)
     // weight rows from row_b2 on (a multiple of the tiling's BN) read their activations from Bhi2 (one image only)
@@ -194,10 +216,11 @@ template <class Cfg, typename WT>
 struct PgGeo {
     static constexpr int BM = Cfg::BM, WR = Cfg::WR, S = Cfg::S, AT = Cfg::AT, NB = Cfg::NB;
     static constexpr int WAVES = 2 * WR, THREADS = 64 * WAVES, BN = 16 * AT * WR;
-    static constexpr int KS = sizeof(WT) == 1 ? 128 : 64;  // depth per stage
-    static constexpr int KBS = KS / 32;                    // MFMA k-blocks per stage
+    static constexpr bool F32 = sizeof(WT) == 4;
+    static constexpr int KS = sizeof(WT) == 1 ? 128 : F32 ? 32 : 64;  // depth per stage
+    static constexpr int KBS = KS / (F32 ? 16 : 32);       // k-blocks per stage: an MFMA per tile, fp32 four
     static constexpr int A_ROW = KS * (int)sizeof(WT);     // 128 B
-    static constexpr int B_ROW = KS * 2;                   // 128 or 256 B
+    static constexpr int B_ROW = KS * (F32 ? 4 : 2);       // 128 or 256 B
     static constexpr int A_IMG = 16 * A_ROW, B_IMG = 16 * B_ROW;
     static constexpr int PT = BM / 16;  // position tiles per workgroup
     static constexpr int WPT = PT / 2;  // per wave
@@ -209,7 +232,9 @@ struct PgGeo {
     // activations keep 2^-23 of a value, one fp32 chain over 4096 k loses more: with it the logits after 100 tokens of
     // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave: the
     // second set of a 64 x 64 wave tile would spill (14 % of a 3776-row prompt).
-    static constexpr int FOLD = NB == 2 && AT * WPT <= 8 ? 256 : 0;
+    // fp32: chains of 32 k, and those sums in turn every 512: no longer than the chains of the decode step's lanes.
+    static constexpr int FOLD = F32 ? 32 : NB == 2 && AT * WPT <= 8 ? 256 : 0;
+    static_assert(!F32 || NB == 1, "fp32: one image");
     static constexpr int DPW = NDMA / WAVES;   // per wave
     static constexpr int SA = Cfg::SA;         // split rings (PgCfg): A pieces per wave DPA, B pieces DPB
     static constexpr int B_BYTES = STAGE - A_BYTES;
@@ -323,7 +348,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const __half* B = Geo::NB == 2 ? ((u & 1) ? in.Blo : in.Bhi) : rb * Geo::BN >= in.row_b2 ? in.Bhi2 : in.Bhi;
             int m = pb * BM + pt * 16 + r;
             if constexpr (Cfg::GR) m = in.grp.rowmap ? in.grp.rowmap[m] : tile.y + pt * 16 + r;
-            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * 2 + c * 16 + (size_t)s0 * Geo::B_ROW;
+            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * (Geo::F32 ? 4 : 2) + c * 16 + (size_t)s0 * Geo::B_ROW;
             adv[j] = Geo::B_ROW;
             back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
         }
@@ -377,7 +402,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
 #pragma unroll
         for (int a = 0; a < AT; ++a) {
             const char* img = st + (wr * AT + a) * Geo::A_IMG + r16 * Geo::A_ROW;
-            if constexpr (sizeof(WT) == 2) {
+            if constexpr (sizeof(WT) != 1) {
                 af[a] = *reinterpret_cast<const u32x4*>(img + ((4 * kb + kg) ^ sa) * 16);
             } else {
                 const int off = ((2 * kb + (kg >> 1)) ^ sa) * 16 + 8 * (kg & 1);
@@ -393,6 +418,17 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         }
     };
     auto mfmas = [&](const u32x4(&af)[AT], const u32x4(&bh)[Geo::WPT], const u32x4(&bl)[Geo::WPT]) {
+        if constexpr (Geo::F32) {  // lane group kg holds k 4 kg .. +3 of the 16-k block: MFMA e takes k 4 kg + e of each
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int b = 0; b < Geo::WPT; ++b)
+#pragma unroll
+                    for (int a = 0; a < AT; ++a)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[a][e]), __uint_as_float(bh[b][e]),
+                                                                         acc[a][b], 0, 0, 0);
+            return;
+        }
 #pragma unroll
         for (int b = 0; b < Geo::WPT; ++b)
 #pragma unroll
@@ -406,13 +442,14 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     };
     constexpr bool TWO = Geo::FOLD > 0;
     pf_float4 tot[TWO ? AT : 1][TWO ? Geo::WPT : 1] = {};
-    auto fold = [&] {
+    pf_float4 top[Geo::F32 ? AT : 1][Geo::F32 ? Geo::WPT : 1] = {};
+    auto fold = [&](auto& to, auto& from) {
 #pragma unroll
         for (int a = 0; a < AT; ++a)
 #pragma unroll
             for (int b = 0; b < Geo::WPT; ++b) {
-                tot[a][b] += acc[a][b];
-                acc[a][b] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
+                to[a][b] += from[a][b];
+                from[a][b] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
             }
     };
     const bool live = Cfg::GR || pb * BM + wp * Geo::WPT * 16 < in.valid;  // (wave-uniform)
@@ -456,15 +493,13 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
                 mfmas(xa, xh, xl);
             }
             if constexpr (TWO)
-                if (s % (Geo::FOLD / Geo::KS) == Geo::FOLD / Geo::KS - 1) fold();
+                if (s % (Geo::FOLD / Geo::KS) == Geo::FOLD / Geo::KS - 1) fold(tot, acc);
+            if constexpr (Geo::F32)
+                if (s % 16 == 15) fold(top, tot);
         }
         if (live) mfmas(ya, yh, yl);
-        if constexpr (TWO) {
-#pragma unroll
-            for (int a = 0; a < AT; ++a)
-#pragma unroll
-                for (int b = 0; b < Geo::WPT; ++b) acc[a][b] += tot[a][b];
-        }
+        if constexpr (TWO) fold(acc, tot);
+        if constexpr (Geo::F32) fold(acc, top);
     }
     if (nsp > 1) {
         // Partial sums go out write-through (sc1); the tile's last workgroup to arrive adds them in split order (the
@@ -594,15 +629,14 @@ struct PgEpiQKV {  // model.cpp:52-67: q (fp32 [M][hq*hd]), rotated k / v rows o
     }
 };
 
-struct PgEpiSwiGLU {  // model.cpp:99-115: act = sigmoid(g) * u (or SiLU), stored as the down GEMM's hi / lo
-    __half* ahi;
-    __half* alo;
+struct PgEpiSwiGLU {  // model.cpp:99-115: act = sigmoid(g) * u (or SiLU), stored as the down GEMM's input
+    PfOut out;
     const float* rscale;
     int inter, silu;
     __device__ int row(int t, int i) const { return t * 8 + (i >> 2) * 2 + (i & 1) + ((i & 2) ? inter : 0); }
     __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
-        const int u = t * 8 + (i0 >> 2) * 2;  // units u, u + 1: one 4-byte hi and lo store each
-        __half hh[2], hl[2];
+        const int u = t * 8 + (i0 >> 2) * 2;  // units u, u + 1: stored together
+        float y[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             float g = v[e], up = v[2 + e];
@@ -612,10 +646,9 @@ struct PgEpiSwiGLU {  // model.cpp:99-115: act = sigmoid(g) * u (or SiLU), store
             }
             float sg = 1.0f / (1.0f + expf(-g));  // swiglu_kernel.cpp:12
             if (silu) sg = g * sg;
-            pf_split(sg * up, hh[e], hl[e]);  // :13
+            y[e] = sg * up;  // :13
         }
-        *reinterpret_cast<unsigned*>(ahi + (size_t)m * inter + u) = *reinterpret_cast<const unsigned*>(hh);
-        *reinterpret_cast<unsigned*>(alo + (size_t)m * inter + u) = *reinterpret_cast<const unsigned*>(hl);
+        out.store<2>((size_t)m * inter + u, y);
     }
 };
 
@@ -703,8 +736,7 @@ struct PfAttnArgs {
     const float* q;    // [M][hq*hd]
     const KT* kc;      // layer base [sequence][hkv][T][hd]
     const KT* vc;
-    __half* ohi;       // [M][hq*hd]
-    __half* olo;
+    PfOut out;         // [M][hq*hd]
     int hq, hkv, T;
     float scale;       // 1/sqrt(hd) (mha_kernel.cpp:41)
 };
@@ -770,9 +802,9 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
         }
     }
 #pragma unroll
-    for (int e = 0; e < QD; ++e) {
-        const size_t idx = (size_t)mi * a.hq * HD + (size_t)h * HD + c * QD + e;
-        pf_split(o[e] / l, a.ohi[idx], a.olo[idx]);
+    for (int e = 0; e < QD; e += 4) {
+        const float y[4] = {o[e] / l, o[e + 1] / l, o[e + 2] / l, o[e + 3] / l};
+        a.out.template store<4>((size_t)mi * a.hq * HD + (size_t)h * HD + c * QD + e, y);
     }
 }
 
@@ -994,11 +1026,8 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
 #pragma unroll
         for (int d = 0; d < NT; ++d) {  // lane holds d = 16 d + 4 g + r of query i
             const size_t idx = (size_t)(seq * ps.rps + i) * qs + (size_t)h * HD + d * 16 + 4 * g;
-            __half hh[4], hl[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) pf_split(o[t][d][r] * inv, hh[r], hl[r]);
-            *reinterpret_cast<uint2*>(a.ohi + idx) = *reinterpret_cast<const uint2*>(hh);
-            *reinterpret_cast<uint2*>(a.olo + idx) = *reinterpret_cast<const uint2*>(hl);
+            const float y[4] = {o[t][d][0] * inv, o[t][d][1] * inv, o[t][d][2] * inv, o[t][d][3] * inv};
+            a.out.template store<4>(idx, y);
         }
     }
 }
@@ -1203,7 +1232,7 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
         for (int w = 0; w < 4; ++w) acc += *reinterpret_cast<const pf_float4*>(fo + ((w * NT + t) * 64 + lane) * 4) * w4[w];
         // lane holds d = 16 t + 4 g + r of query mq
         const int d0 = t * 16 + 4 * g;
-        __half* dst = a.ohi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
+        __half* dst = a.out.hi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
         if (!live) continue;
         if constexpr (ROWS == 2) {
             const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;

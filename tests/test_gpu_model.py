@@ -184,3 +184,22 @@ def test_predict_matches_reference_build_vectors(gpu, name):
     assert np.array_equal(toks, g["tokens"]), (toks, g["tokens"])
     err = float(np.abs(logits - g["logits"]).max())
     assert err <= 1e-4, err
+
+
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+@pytest.mark.parametrize("name,n,length", [("tiny-gqa", 9, 20), ("tiny", 33, 40), ("small-h128-gqa", 10, 16),
+                                           ("small-h128", 76, 90), ("small-h128-gqa", 130, 140), ("small-h128", 500, 512)])
+def test_predict_f32_prompt_chunk_matches_steps(gpu, name, kv, n, length):
+    """fp32 weights: without wanted logits predict runs the prompt as one chunk (rows of 32, 64 and 128 per tile, cut over
+    the depth), with them as steps: the same tokens and state, logits within this file's fp32 bar (1e-4; an fp16 cache's
+    roundings 1e-3)."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset(name), w_dtype="f32", kv_dtype=kv, seed=8).init()
+    prompt = np.random.default_rng(n).integers(0, m.config.vocab_size, n)
+    want, wl = m.predict(prompt, length, want_logits=True)
+    state = m.state()
+    m.reset()
+    got = m.predict(prompt, length)
+    assert np.array_equal(got, want) and m.state() == state
+    assert np.abs(m.logits()[0] - wl[-1]).max() <= (1e-4 if kv == "f32" else 1e-3)
+    m.close()
