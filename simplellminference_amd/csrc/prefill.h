@@ -232,8 +232,9 @@ struct PgGeo {
     // activations keep 2^-23 of a value, one fp32 chain over 4096 k loses more: with it the logits after 100 tokens of
     // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave: the
     // second set of a 64 x 64 wave tile would spill (14 % of a 3776-row prompt).
-    // fp32: chains of 32 k, and those sums in turn every 512: no longer than the chains of the decode step's lanes.
-    static constexpr int FOLD = F32 ? 32 : NB == 2 && AT * WPT <= 8 ? 256 : 0;
+    // fp32: every 4 k are a sum of their own (mfmas), chained up to 512 k: no longer than the chains of the decode step's
+    // lanes.
+    static constexpr int FOLD = F32 ? 512 : NB == 2 && AT * WPT <= 8 ? 256 : 0;
     static_assert(!F32 || NB == 1, "fp32: one image");
     static constexpr int DPW = NDMA / WAVES;   // per wave
     static constexpr int SA = Cfg::SA;         // split rings (PgCfg): A pieces per wave DPA, B pieces DPB
@@ -420,13 +421,16 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     auto mfmas = [&](const u32x4(&af)[AT], const u32x4(&bh)[Geo::WPT], const u32x4(&bl)[Geo::WPT]) {
         if constexpr (Geo::F32) {  // lane group kg holds k 4 kg .. +3 of the 16-k block: MFMA e takes k 4 kg + e of each
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int b = 0; b < Geo::WPT; ++b)
 #pragma unroll
-                for (int b = 0; b < Geo::WPT; ++b)
+                for (int a = 0; a < AT; ++a) {
+                    pf_float4 p[4];
 #pragma unroll
-                    for (int a = 0; a < AT; ++a)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[a][e]), __uint_as_float(bh[b][e]),
-                                                                         acc[a][b], 0, 0, 0);
+                    for (int e = 0; e < 4; ++e)
+                        p[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[a][e]), __uint_as_float(bh[b][e]),
+                                                                    pf_float4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                    acc[a][b] += (p[0] + p[1]) + (p[2] + p[3]);
+                }
             return;
         }
 #pragma unroll
@@ -442,7 +446,6 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     };
     constexpr bool TWO = Geo::FOLD > 0;
     pf_float4 tot[TWO ? AT : 1][TWO ? Geo::WPT : 1] = {};
-    pf_float4 top[Geo::F32 ? AT : 1][Geo::F32 ? Geo::WPT : 1] = {};
     auto fold = [&](auto& to, auto& from) {
 #pragma unroll
         for (int a = 0; a < AT; ++a)
@@ -494,12 +497,9 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             }
             if constexpr (TWO)
                 if (s % (Geo::FOLD / Geo::KS) == Geo::FOLD / Geo::KS - 1) fold(tot, acc);
-            if constexpr (Geo::F32)
-                if (s % 16 == 15) fold(top, tot);
         }
         if (live) mfmas(ya, yh, yl);
         if constexpr (TWO) fold(acc, tot);
-        if constexpr (Geo::F32) fold(acc, top);
     }
     if (nsp > 1) {
         // Partial sums go out write-through (sc1); the tile's last workgroup to arrive adds them in split order (the

@@ -39,7 +39,6 @@ struct Bufs {
                           // the engine, where a layer's weights are read once per chunk)
     __half *hi, *lo;
     float* y;
-    PfState* ps;
     std::vector<WT> hW;
     std::vector<__half> hhi, hlo;
 };
@@ -67,7 +66,6 @@ static void make(Bufs<WT>& b, int N, int K, int M) {
     CK(hipMalloc(&b.hi, 2 * b.hhi.size()));
     CK(hipMalloc(&b.lo, 2 * b.hlo.size()));
     CK(hipMalloc(&b.y, sizeof(float) * (size_t)M * N));
-    CK(hipMalloc(&b.ps, sizeof(PfState)));
     CK(hipMemcpy(b.W, b.hW.data(), sizeof(WT) * b.hW.size(), hipMemcpyHostToDevice));
     const int ncopy = getenv("LAB_HOT") ? 1 : 4;
     b.Wc.assign(1, b.W);
@@ -79,8 +77,6 @@ static void make(Bufs<WT>& b, int N, int K, int M) {
     }
     CK(hipMemcpy(b.hi, b.hhi.data(), 2 * b.hhi.size(), hipMemcpyHostToDevice));
     CK(hipMemcpy(b.lo, b.hlo.data(), 2 * b.hlo.size(), hipMemcpyHostToDevice));
-    PfState p{0, M};
-    CK(hipMemcpy(b.ps, &p, sizeof p, hipMemcpyHostToDevice));
 }
 
 template <typename WT>
@@ -89,7 +85,6 @@ static void release(Bufs<WT>& b) {
     CK(hipFree(b.hi));
     CK(hipFree(b.lo));
     CK(hipFree(b.y));
-    CK(hipFree(b.ps));
 }
 
 static float* g_ws;
@@ -114,7 +109,7 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
     in.full = pl.full, in.splits = pl.splits, in.ws = g_ws, in.cnt = g_cnt;
     PgEpiResid e{b.y, nullptr, nullptr, sh.N, sh.N};
     CK(hipMemset(b.y, 0, sizeof(float) * (size_t)M * sh.N));
-    CK((launch_pgemm<PgEpiResid, Cfg, WT>(in, e, b.ps, 0)));
+    CK((launch_pgemm<PgEpiResid, Cfg, WT>(in, e, PfState{0, M, M, 1}, 0)));
     CK(hipDeviceSynchronize());
     // spot check (y[m][row] = sum_k W[row][k] (hi + lo)[m][k])
     std::vector<float> y((size_t)M * sh.N);
@@ -130,7 +125,7 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
                 w = (double)b.hW[(size_t)row * sh.K + k];
             else
                 w = (double)h2f(b.hW[(size_t)row * sh.K + k]);
-            const double x = (double)h2f(b.hhi[(size_t)m * sh.K + k]) + (double)h2f(b.hlo[(size_t)m * sh.K + k]);
+            const double x = (double)h2f(b.hhi[(size_t)m * sh.K + k]) + (Cfg::NB == 2 ? (double)h2f(b.hlo[(size_t)m * sh.K + k]) : 0.0);
             ref += w * x;
             mag += fabs(w * x);
         }
@@ -144,14 +139,14 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
     for (int i = 0; i < iters; ++i) {
         PgIn<WT> ic = in;
         ic.W = b.Wc[i % b.Wc.size()];
-        CK((launch_pgemm<PgEpiResid, Cfg, WT>(ic, e, b.ps, 0)));
+        CK((launch_pgemm<PgEpiResid, Cfg, WT>(ic, e, PfState{0, M, M, 1}, 0)));
     }
     CK(hipEventRecord(e1, 0));
     CK(hipEventSynchronize(e1));
     float ms = 0.0f;
     CK(hipEventElapsedTime(&ms, e0, e1));
     const double us = 1000.0 * ms / iters;
-    const double tf = 4.0 * sh.N * sh.K * (double)M / (us * 1e-6) / 1e12;
+    const double tf = 2.0 * Cfg::NB * sh.N * sh.K * (double)M / (us * 1e-6) / 1e12;
     const double wgbs = (double)sh.N * sh.K * sizeof(WT) / (us * 1e-6) / 1e9;
     const int nrb = (sh.N + Geo::BN - 1) / Geo::BN;
     printf("%-5s %-6s %-22s grid %5d lds %6zu  %8.1f us  %6.1f TF issued  W %6.0f GB/s  relerr %.1e\n", sh.name,
@@ -164,10 +159,30 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
 #define RUN(BM, WR, S, AT, SA)                                                            \
     for (int f : forces) run<PgCfg<BM, WR, S, AT, SA>, WT>("BM" #BM " WR" #WR " S" #S " AT" #AT " SA" #SA, b, sh, M, f)
 
+// LAB_ONE: one fp16 image (block-stack models)
+#define RUN1(BM, WR, S, AT)                                                               \
+    for (int f : forces) run<PgCfg<BM, WR, S, AT, 0, 1>, WT>("BM" #BM " WR" #WR " S" #S " AT" #AT " NB1", b, sh, M, f)
+
 template <typename WT>
 static void sweep(const Shape& sh, int M, const std::vector<int>& forces) {
     Bufs<WT> b;
     make(b, sh.N, sh.K, M);
+    if (getenv("LAB_ONE")) {
+        if constexpr (sizeof(WT) == 2) {
+            RUN1(256, 4, 2, 4);
+            RUN1(128, 4, 2, 4);
+            RUN1(128, 4, 3, 4);
+            RUN1(128, 4, 2, 2);
+            RUN1(128, 2, 3, 4);
+            RUN1(64, 4, 3, 4);
+            RUN1(64, 4, 4, 2);
+            RUN1(64, 2, 4, 2);
+            RUN1(32, 2, 4, 2);
+            RUN1(32, 2, 4, 4);
+        }
+        release(b);
+        return;
+    }
     if constexpr (sizeof(WT) == 2) {
         if (M <= 32) {
             RUN(32, 2, 4, 2, 0);
@@ -208,7 +223,8 @@ int main(int argc, char** argv) {
     CK(hipMalloc(&g_ws, kPgWsBytes));
     CK(hipMalloc(&g_cnt, sizeof(unsigned) * kPgWsTiles));
     CK(hipMemset(g_cnt, 0, sizeof(unsigned) * kPgWsTiles));
-    const Shape shapes[] = {{"qkv", 12288, 4096}, {"gu", 22016, 4096}, {"wo", 4096, 4096}, {"down", 4096, 11008}};
+    std::vector<Shape> shapes = {{"qkv", 12288, 4096}, {"gu", 22016, 4096}, {"wo", 4096, 4096}, {"down", 4096, 11008}};
+    if (getenv("LAB_ONE")) shapes = {{"in7b", 34304, 4096}, {"out7b", 4096, 15104}, {"in1b", 22528, 2048}, {"out1b", 2048, 10240}};
     if (!getenv("LAB_I8"))
         for (const Shape& sh : shapes) sweep<__half>(sh, M, forces);
     else
