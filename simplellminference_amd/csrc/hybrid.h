@@ -16,7 +16,9 @@
 
 namespace sli {
 
-constexpr int kHyMaxRows = 1024;  // rows of one pass
+// Rows of one pass: a prompt past it starts another one, which reads the weights again (1025 tokens of a 7B stack with
+// passes of 1024: 4.4 of 33 ms for the last row).
+constexpr int kHyMaxRows = 2048;
 constexpr int kHyTile = 32;      // a portion's rows start at a multiple of this (one sequence per row tile)
 
 struct BlockStack;

@@ -265,6 +265,10 @@ int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out)
     HY_TRY(s->seq ? seq_create(s) : par_create(s));
     HY_TRY(hy_alloc(s, (void**)&s->bg_ws, s->bg_ws_bytes + 256));
     HY_TRY(hy_new(s, &s->bg_cnt, s->bg_groups));
+    if (s->f16) {
+        HY_TRY(hy_alloc(s, (void**)&s->pg_ws, kPgWsBytes, false));
+        HY_TRY(hy_new(s, &s->pg_cnt, kPgWsTiles));
+    }
     return hy_allow_lds();
 }
 
@@ -793,19 +797,14 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
             const std::vector<int32_t>& want, float* logits_host, float* hidden_host) {
     const int n = (int)rows_in.size();
     SLI_CHECK(n >= 1 && n <= s->M && !segs.empty() && (int)segs.size() <= s->M, SLI_ERR_SHAPE, "pass: too many rows");
-    // a decode step runs its rows as they are; a prompt pass is padded to a row count with a captured graph
+    // a decode step runs its rows as they are, from a captured graph; a prompt pass is padded to the GEMM's row tiles and
+    // launched directly (its launches run longer than they take to enqueue, and every row count would be a graph)
     int M = s->f16 ? HyRec<__half>::rows_for(n) : n, kt = 0;
     SLI_CHECK(!one || n <= s->B, SLI_ERR_SHAPE, "pass: more sequences than slots");
     if (!one) {
-        M = kHyTile;
-        while (M < n) M *= 2;
+        M = n <= 64 ? pad_to(n, kHyTile) : std::min(pad_to(n, 128), s->M);
         for (const SegRef& g : segs) kt += seq_key_tiles(s, g.pos0, g.n);
         SLI_CHECK(kt <= hy_key_tiles_max(s), SLI_ERR_SHAPE, "pass: too many expanded rows");
-        if (kt > 0) {  // (the grid of the expansion: a power of two, so that few graphs are captured)
-            int p = M / kLatTile + 1;
-            while (p < kt) p *= 2;
-            kt = std::min(p, hy_key_tiles_max(s));
-        }
     }
     std::vector<RowRef> rows(rows_in);
     rows.resize(M, RowRef{-1, 0, 0, 0});
@@ -821,8 +820,10 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
             SLI_HIP(hipMemcpy2DAsync(hidden_host + r * (size_t)n * s->D, sizeof(float) * s->D, s->x, sizeof(float) * s->Dp,
                                      sizeof(float) * s->D, n, hipMemcpyDeviceToHost, s->stream));
         }
+    } else if (!one) {
+        HY_TRY(HY_DISPATCH(s, M, one, msegs, kt, pass()));
     } else {
-        auto& g = s->graphs[{one ? 0 : 1 + kt, M}];
+        auto& g = s->graphs[M];
         SLI_HIP(hipStreamSynchronize(s->stream));
         HY_TRY(hy_capture(s, g, M, one, msegs, kt));
         SLI_HIP(hipGraphLaunch(g.second, s->stream));

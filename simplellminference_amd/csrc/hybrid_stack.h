@@ -121,7 +121,9 @@ struct BlockStack {
     size_t bg_ws_bytes = 0, bg_groups = 1;  // the most any projection needs (hy_bg_need)
     std::vector<void*> allocs;
     // captured passes: {0, rows} of a decode step, {1 + key tile bucket, rows} of a prompt pass
-    std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+    std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // decode passes of `feed`, by row count
+    float* pg_ws = nullptr;  // partial sums and arrival counters of the prompt GEMM (prefill.h PgIn)
+    unsigned* pg_cnt = nullptr;
 };
 
 // device memory of the stack (zeroed), freed with it

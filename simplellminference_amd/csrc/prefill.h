@@ -285,6 +285,12 @@ __device__ __forceinline__ void pg_wait_stages(int later) {
     }
 }
 
+// Epilogues with a member kRolled = true are looped over a wave's tiles instead of unrolled
+template <class Epi, class = void>
+struct PgRolled : std::false_type {};
+template <class Epi>
+struct PgRolled<Epi, std::enable_if_t<Epi::kRolled>> : std::true_type {};
+
 template <class Epi, class Cfg, typename WT>
 __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi epi, PfState ps) {
     using Geo = PgGeo<Cfg, WT>;
@@ -541,15 +547,30 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             }
         }
     }
-    if (!live) return;
-    // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15. (A copy of the sums: a large epilogue
-    // leaves this loop rolled, and the array that it indexes lives in scratch, which acc itself must not.)
-    pf_float4 out[AT][Geo::WPT];
-#pragma unroll
-    for (int a = 0; a < AT; ++a)
-#pragma unroll
-        for (int b = 0; b < Geo::WPT; ++b) out[a][b] = acc[a][b];
+    // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15
     const int i0 = 4 * (lane >> 4);
+    if constexpr (PgRolled<Epi>::value) {
+        // an epilogue too large to be unrolled over the tiles: a loop over them, the sums indexed in the ring's LDS
+        // (indexed registers would live in scratch)
+        constexpr int NV = AT * Geo::WPT, H = NV * 16 * Geo::THREADS <= Geo::LDS ? NV : NV / 2;
+        static_assert(H * 16 * Geo::THREADS <= Geo::LDS && NV % H == 0, "sums in the ring");
+        __syncthreads();  // every wave is done with its fragments
+        pf_float4* mine = reinterpret_cast<pf_float4*>(pg_smem) + threadIdx.x;
+#pragma unroll
+        for (int h = 0; h < NV; h += H) {
+#pragma unroll
+            for (int j = 0; j < H; ++j) mine[j * Geo::THREADS] = acc[(h + j) / Geo::WPT][(h + j) % Geo::WPT];
+#pragma unroll 1
+            for (int j = 0; j < H; ++j) {
+                const int t = rb * Geo::NA + wr * AT + (h + j) / Geo::WPT;
+                const pf_float4 o = mine[j * Geo::THREADS];
+                const float v[4] = {o[0], o[1], o[2], o[3]};
+                if (t < nt && live) epi.store(t, i0, pb * BM + (wp * Geo::WPT + (h + j) % Geo::WPT) * 16 + r16, v, ps);
+            }
+        }
+        return;
+    }
+    if (!live) return;
 #pragma unroll
     for (int a = 0; a < AT; ++a) {
         const int t = rb * Geo::NA + wr * AT + a;
@@ -557,7 +578,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
 #pragma unroll
         for (int b = 0; b < Geo::WPT; ++b) {
             const int m = pb * BM + (wp * Geo::WPT + b) * 16 + r16;
-            const float v[4] = {out[a][b][0], out[a][b][1], out[a][b][2], out[a][b][3]};
+            const float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
             epi.store(t, i0, m, v, ps);
         }
     }

@@ -493,3 +493,24 @@ def test_errors_come_from_the_host(gpu):
         StackModel(StackSpec(8, 8, (BlockSpec("attention", 1, 4, 4, kv_heads=1),))).init().feed([0], [0], [[1]])
     with pytest.raises(SliError):
         StackModel(StackSpec(8, 8, (BlockSpec("attention", 3, 4, 4, kv_heads=2),))).init()
+
+
+@pytest.mark.parametrize("n", [33, 65, 129, 257, 300, 700, 1025, 2048, 2049])
+def test_row_counts_of_a_pass(gpu, n):
+    """Prompt passes of every tile height with padding rows, a launch's last tiles cut over the depth (narrow outputs: all of
+    them) and, past 2048 rows, two passes: the last positions' logits as when the tokens before them come in portions of
+    other row counts (fp16 rows: the tolerance of this file)."""
+    c = stack(att(heads=4, kv_heads=2, dim=64, vdim=64, ff=300), ret(heads=3, dim=64, vdim=64, ff=520), vocab=203, width=384)
+    m = make(c, R.random_tensors(c, 21), "bfloat16", max_length=2112)
+    ids = tokens(n, vocab=203, seed=n)
+    want = list(range(max(0, n - 40), n))
+    whole = m.feed([0], [0], [ids], [want])
+    cut = n - len(want)
+    p = 0
+    while p < cut:  # portions of at most 480 rows
+        e = min(cut, p + 480)
+        m.feed([0], [p], [ids[p:e]])
+        p = e
+    rest = m.feed([0], [cut], [ids[cut:]], [list(range(n - cut))])
+    close(whole, rest, "bfloat16")
+    m.close()
