@@ -327,6 +327,24 @@ __global__ void finalize_kernel(DevState* st, const int32_t* __restrict__ prompt
     finalize_state(st, prompt, hist, T);
 }
 
+// Host writes of the decode state, in stream order (no copy down, no wait): thread b is sequence b. A new position
+// (token, pos, advance) where n_forced < 0, else the prompt's length alone.
+__global__ void set_state_kernel(DevState* st, int32_t* hist, int seq, int B, int T, int token, int pos, int advance,
+                                 int n_forced) {
+    const int b = threadIdx.x;
+    if (b >= B || (seq >= 0 && b != seq)) return;
+    if (n_forced >= 0) {
+        st[b].n_forced = n_forced;
+        return;
+    }
+    st[b].token = token;
+    st[b].pos = pos;
+    st[b].advance = advance;
+    st[b].key = 0;
+    st[b].error = 0;
+    hist[(size_t)b * (T + 1) + pos] = token;
+}
+
 // ---- batch > 1: one sequence per block / thread
 // emb_kernel.cpp:4-21 per sequence, token read on device (graph-capturable)
 template <typename T>
@@ -1838,25 +1856,31 @@ int sli_model_fill_kv_synthetic(sli_model* m, uint32_t seed, int32_t upto) {
     return SLI_OK;
 }
 
-// seq < 0: every sequence
+// the model's device for a launch, the caller's again after it
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(int d) {
+        int c = d;
+        if (hipGetDevice(&c) == hipSuccess && c != d && hipSetDevice(d) == hipSuccess) was = c;
+    }
+    ~OnDevice() {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
+
+// seq < 0: every sequence (at most 64: a block-stack batch)
 static int set_state(sli_model* m, int seq, int32_t token, int32_t pos, int32_t advance) {
     SLI_CHECK(m, SLI_ERR_ARG, "null model");
     SLI_CHECK(seq < m->B, SLI_ERR_RANGE, "sequence index out of range");
     SLI_CHECK(token >= 0 && token < m->V, SLI_ERR_RANGE, "Token index is greater than vocab size.");
     SLI_CHECK(pos >= 0 && pos < m->T, SLI_ERR_RANGE, "position out of range");
-    std::vector<DevState> h;
-    SLI_TRY(download_states(m, h));
-    for (int b = 0; b < m->B; ++b) {
-        if (seq >= 0 && b != seq) continue;
-        h[b].token = token;
-        h[b].pos = pos;
-        h[b].advance = advance ? 1 : 0;
-        h[b].key = 0;
-        h[b].error = 0;
-        SLI_HIP(hipMemcpyAsync(m->hist + (size_t)b * (m->T + 1) + pos, &token, sizeof(int32_t), hipMemcpyHostToDevice,
-                               m->stream));
-    }
-    return upload_states(m, h);
+    SLI_CHECK(!m->comm_dead, SLI_ERR_COMM, "the RCCL communicator was aborted by an earlier bounded wait");
+    const OnDevice dev(m->c.device);
+    // a launch instead of copying the states down, changing and uploading them, each with a wait: a batch of 8 set its
+    // positions in 0.4 of a step's 4.2 ms
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, m->stream, m->st, m->hist, seq, m->B, m->T, token, pos, advance ? 1 : 0, -1);
+    SLI_HIP(hipGetLastError());
+    return SLI_OK;
 }
 
 static int set_prompt(sli_model* m, int seq, const int32_t* ids, int32_t n) {
@@ -1866,15 +1890,15 @@ static int set_prompt(sli_model* m, int seq, const int32_t* ids, int32_t n) {
     SLI_CHECK(!m->comm_dead, SLI_ERR_COMM, "the RCCL communicator was aborted by an earlier bounded wait");
     for (int i = 0; i < n; ++i)
         SLI_CHECK(ids[i] >= 0 && ids[i] < m->V, SLI_ERR_RANGE, "Token index is greater than vocab size.");
-    std::vector<DevState> h;
-    SLI_TRY(download_states(m, h));
+    const OnDevice dev(m->c.device);
     for (int b = 0; b < m->B; ++b) {
         if (seq >= 0 && b != seq) continue;
         SLI_HIP(hipMemcpyAsync(m->prompt + (size_t)b * (m->T + 1), ids, sizeof(int32_t) * n, hipMemcpyHostToDevice,
                                m->stream));
-        h[b].n_forced = n;
     }
-    return upload_states(m, h);
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, m->stream, m->st, m->hist, seq, m->B, m->T, 0, 0, 0, n);
+    SLI_HIP(hipGetLastError());
+    return wait_stream(m);  // (the caller's ids are read)
 }
 
 static int get_state(sli_model* m, int seq, int32_t* pos, int32_t* token, int32_t* last_argmax, int32_t* error) {
