@@ -1054,7 +1054,7 @@ struct StepRecorder {
     // The GEMM tilings (prefill.h PgCfg<BM, WR, S, AT, SA>) of a chunk size, each with the time of one stage of a workgroup
     // when every CU has one, in us (tools/pgemm_lab, one MI355X, 7B shapes): f(PgCfg<...>{}, us). The launch takes the one
     // whose plan (prefill.h pg_plan: rounds, and the last round's tiles cut over the depth) costs least. Measured at 512
-    // rows, q/k/v | gate/up | wo | down in us: 123 | 214 | 45 | 102, against 144 | 263 | 122 | 122 of two 256-row chunks
+    // rows, q/k/v | gate/up | wo | down in us: 112 | 202 | 44 | 96, against 144 | 263 | 122 | 122 of two 256-row chunks
     // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
     // fp32, 74 rows: 137 | 229 | 54 | 110 (the matrix cores' fp32 rate: 75 TFLOP/s of 151 in padded rows).
     template <class F>
@@ -1068,7 +1068,7 @@ struct StepRecorder {
             else if (M % 64 == 0) f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 2, 4>{}, 1.65f);
             else f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
         } else {
-            if (M % 128 == 0) f(PgCfg<128, 4, 2, 4, 3>{}, 1.85f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.1f), f(PgCfg<64, 4, 3, 2>{}, 0.67f);
+            if (M % 128 == 0) f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f), f(PgCfg<64, 4, 3, 2>{}, 0.65f);
             else if (M % 64 == 0) f(PgCfg<64, 4, 4, 2>{}, 0.72f), f(PgCfg<64, 4, 3, 4>{}, 0.97f), f(PgCfg<64, 2, 4, 2>{}, 0.52f);
             else f(PgCfg<32, 4, 4, 2>{}, 0.6f), f(PgCfg<32, 4, 3, 4>{}, 0.77f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
         }

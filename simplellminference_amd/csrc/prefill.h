@@ -204,11 +204,12 @@ struct PgIn {
 // from L2, so only A needs the deep prefetch, and B, the larger image, does not pay for it in LDS.
 // NB_: activation images per position: 2 (fp16 hi + lo, two MFMAs per product) or 1 (fp16 activations).
 // GR_: row blocks with weights of their own (PgGroups; one image).
-template <int BM_, int WR_, int S_, int AT_ = 2, int SA_ = 0, int NB_ = 2, bool GR_ = false>
+// FO_: short chains (PgGeo::FOLD) for a 64 x 64 wave tile too.
+template <int BM_, int WR_, int S_, int AT_ = 2, int SA_ = 0, int NB_ = 2, bool GR_ = false, bool FO_ = false>
 struct PgCfg {
     static_assert(NB_ == 2 || NB_ == 1, "activation images");
     static_assert(!GR_ || NB_ == 1, "grouped: one image");
-    static constexpr bool GR = GR_;
+    static constexpr bool GR = GR_, FO = FO_;
     static constexpr int BM = BM_, WR = WR_, S = S_, AT = AT_, SA = SA_, NB = NB_;
 };
 
@@ -230,11 +231,11 @@ struct PgGeo {
     static constexpr int NDMA = STAGE / 1024;  // wave-instructions per stage
     // depth after which a wave's sums go into a second set of accumulators (0: one chain over the whole depth). hi + lo
     // activations keep 2^-23 of a value, one fp32 chain over 4096 k loses more: with it the logits after 100 tokens of
-    // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave: the
-    // second set of a 64 x 64 wave tile would spill (14 % of a 3776-row prompt).
+    // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave it
+    // costs nothing; a 64 x 64 wave tile (16) 3 to 8 % of a GEMM, so there only where the caller's other route has them.
     // fp32: every 4 k are a sum of their own (mfmas), chained up to 512 k: no longer than the chains of the decode step's
     // lanes.
-    static constexpr int FOLD = F32 ? 512 : NB == 2 && AT * WPT <= 8 ? 256 : 0;
+    static constexpr int FOLD = F32 ? 512 : NB == 2 && (AT * WPT <= 8 || Cfg::FO) ? 256 : 0;
     static_assert(!F32 || NB == 1, "fp32: one image");
     static constexpr int DPW = NDMA / WAVES;   // per wave
     static constexpr int SA = Cfg::SA;         // split rings (PgCfg): A pieces per wave DPA, B pieces DPB
@@ -322,16 +323,19 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     // A split's stages are s0 .. s0 + ns - 1 (every split has one: pg_plan).
     const int nsk = (in.K + Geo::KS - 1) / Geo::KS;
     const int s0 = nsp == 1 ? 0 : nsk * sp / nsp, ns = (nsp == 1 ? nsk : nsk * (sp + 1) / nsp) - s0;
-    const bool half_tail = (in.K % Geo::KS) != 0 && s0 + ns == nsk;
+    constexpr bool HALF = sizeof(WT) == 1;
+    const bool half_tail = HALF && (in.K % Geo::KS) != 0 && s0 + ns == nsk;
     const int nt = in.N >> 4;       // row tiles
     const unsigned ring = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)pg_smem;
 
     // this wave's DMA instructions d in [wave*DPW, (wave+1)*DPW): stage bytes [1024 d, 1024 (d + 1)). Lane i
     // lands at byte 16 i of it: image row i / cpr, physical chunk i % cpr (cpr = 16-B chunks per image row),
     // so it loads the row's logical chunk (i % cpr) ^ swizzle(row).
+    // (src walks on with every issue; adv, back: int8 only, elsewhere both operands advance 128 bytes and every stage is whole)
     const char* src[Geo::DPW];
-    int adv[Geo::DPW];   // bytes per stage
-    int back[Geo::DPW];  // bytes to step back in a half last stage (logical chunk in the stage's second half)
+    [[maybe_unused]] int adv[HALF ? Geo::DPW : 1];   // bytes per stage
+    [[maybe_unused]] int back[HALF ? Geo::DPW : 1];  // bytes to step back in a half last stage (logical chunk in the stage's second half)
+    static_assert(HALF || Geo::A_ROW == Geo::B_ROW, "one advance");
 #pragma unroll
     for (int j = 0; j < Geo::DPW; ++j) {
         // split rings: the wave's DPA pieces of the A images, then its DPB pieces of the B images
@@ -344,8 +348,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const int c = (lane % 8) ^ pg_swz(r, Geo::A_ROW);
             const int row = epi.row(min(t, nt - 1), r);
             src[j] = reinterpret_cast<const char*>(in.W) + (size_t)row * in.K * sizeof(WT) + c * 16 + (size_t)s0 * Geo::A_ROW;
-            adv[j] = Geo::A_ROW;
-            back[j] = c >= 4 ? Geo::A_ROW / 2 : 0;
+            if constexpr (HALF) adv[j] = Geo::A_ROW, back[j] = c >= 4 ? Geo::A_ROW / 2 : 0;
         } else {
             constexpr int cpr = Geo::B_ROW / 16;
             const int o2 = off - Geo::A_BYTES;
@@ -356,34 +359,38 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             int m = pb * BM + pt * 16 + r;
             if constexpr (Cfg::GR) m = in.grp.rowmap ? in.grp.rowmap[m] : tile.y + pt * 16 + r;
             src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * (Geo::F32 ? 4 : 2) + c * 16 + (size_t)s0 * Geo::B_ROW;
-            adv[j] = Geo::B_ROW;
-            back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
+            if constexpr (HALF) adv[j] = Geo::B_ROW, back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
         }
     }
+    auto piece = [&](int j, unsigned dst, bool tail) {
+        if constexpr (HALF) {
+            pf_dma(src[j] - (tail ? back[j] : 0), dst);
+            src[j] += adv[j];
+        } else {
+            pf_dma(src[j], dst);
+            src[j] += Geo::A_ROW;
+        }
+    };
     auto issue = [&](int s) {
         const unsigned dst = ring + (unsigned)((s % S) * Geo::STAGE);
         const bool tail = half_tail && s == ns - 1;
 #pragma unroll
-        for (int j = 0; j < Geo::DPW; ++j)
-            pf_dma(src[j] + (size_t)s * adv[j] - (tail ? back[j] : 0), dst + (unsigned)((wave * Geo::DPW + j) * 1024));
+        for (int j = 0; j < Geo::DPW; ++j) piece(j, dst + (unsigned)((wave * Geo::DPW + j) * 1024), tail);
     };
 
     // split rings: A stage s in slot s % SA at ring, B stage s in slot s % 2 behind the A ring
     const unsigned ring_b = ring + (unsigned)(Geo::SA * Geo::A_BYTES);
     auto issue_a = [&](int s) {
-        const unsigned dst = ring + (unsigned)((s % Geo::SA) * Geo::A_BYTES);
+        const unsigned dst = ring + (unsigned)((s % (Geo::SA ? Geo::SA : 1)) * Geo::A_BYTES);
         const bool tail = half_tail && s == ns - 1;
 #pragma unroll
-        for (int j = 0; j < Geo::DPA; ++j)
-            pf_dma(src[j] + (size_t)s * adv[j] - (tail ? back[j] : 0), dst + (unsigned)((wave * Geo::DPA + j) * 1024));
+        for (int j = 0; j < Geo::DPA; ++j) piece(j, dst + (unsigned)((wave * Geo::DPA + j) * 1024), tail);
     };
     auto issue_b = [&](int s) {
         const unsigned dst = ring_b + (unsigned)((s & 1) * Geo::B_BYTES);
         const bool tail = half_tail && s == ns - 1;
 #pragma unroll
-        for (int j = 0; j < Geo::DPB; ++j)
-            pf_dma(src[Geo::DPA + j] + (size_t)s * adv[Geo::DPA + j] - (tail ? back[Geo::DPA + j] : 0),
-                   dst + (unsigned)((wave * Geo::DPB + j) * 1024));
+        for (int j = 0; j < Geo::DPB; ++j) piece(Geo::DPA + j, dst + (unsigned)((wave * Geo::DPB + j) * 1024), tail);
     };
     constexpr int AT = Geo::AT;
     pf_float4 acc[AT][Geo::WPT];
