@@ -637,7 +637,7 @@ def main():
         chunks = []  # (valid rows, rows of the launches) per weight pass (engine.hip pf_rows, prefill.h kPfMaxChunk)
         for p0 in range(0, n - 1, 4096):
             nv = min(4096, n - 1 - p0)
-            chunks.append((nv, 32 if nv <= 32 else 64 if nv <= 64 else -(-nv // 128) * 128))
+            chunks.append((nv, -(-nv // 32) * 32))
         useful = 2.0 * params * (n - 1) * world  # whole-job flops of the projections (1 flop per MAC x 2)
         issued = 4.0 * params * sum(M for _, M in chunks) * world  # hi + lo MFMAs over the padded rows
         out["prefill"] = {"prompt_tokens": n, "positions_prefilled": n - 1,

@@ -607,8 +607,9 @@ static int tpl_launch(sli_model* m) {
     return SLI_OK;
 }
 
-// rows of the launches for a chunk of nv prompt positions
-static int pf_rows(int nv) { return nv <= 32 ? 32 : nv <= 64 ? 64 : (nv + 127) / 128 * 128; }
+// rows of the row-wise launches for a chunk of n rows. A GEMM pads them to its own tiles: the buffers have kPfPad more.
+static int pf_rows(int n) { return (n + 31) / 32 * 32; }
+constexpr int kPfPad = 128;
 
 template <typename WT, typename KT>
 struct StepRecorder {
@@ -1051,46 +1052,51 @@ struct StepRecorder {
     // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); the last prompt
     // position runs as an ordinary decode step. Phases as record_phase: 2l = qkv, attention, wo; 2l+1 =
     // gate/up, down; under tensor parallelism each ends with the all-reduce of the chunk's residual rows.
-    // The GEMM tilings (prefill.h PgCfg<BM, WR, S, AT, SA>) of a chunk size, each with the time of one stage of a workgroup
-    // when every CU has one, in us (tools/pgemm_lab, one MI355X, 7B shapes): f(PgCfg<...>{}, us). The launch takes the one
-    // whose plan (prefill.h pg_plan: rounds, and the last round's tiles cut over the depth) costs least. Measured at 512
+    // The GEMM tilings (prefill.h PgCfg<BM, WR, S, AT, SA>), each with the time of one stage of a workgroup when every CU
+    // has one, in us (tools/pgemm_lab, one MI355X, 7B shapes): f(PgCfg<...>{}, us). The launch takes the one whose plan
+    // (prefill.h pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth) costs
+    // least. 192-row tiles of 96 chunk rows: q/k/v 33 and gate/up 51 us at 96 rows, where 128 rows take 43 and 72; of 64
+    // rows 27 and 47 (int8 25 and 41) against 30 and 51 (28 and 48) of 128- and 256-row tiles. Measured at 512
     // rows, q/k/v | gate/up | wo | down in us: 112 | 202 | 44 | 96, against 144 | 263 | 122 | 122 of two 256-row chunks
     // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
     // fp32, 74 rows: 137 | 229 | 54 | 110 (the matrix cores' fp32 rate: 75 TFLOP/s of 151 in padded rows).
     template <class F>
-    static void pg_each(int M, F&& f) {
+    static void pg_each(F&& f) {
         if constexpr (std::is_same<WT, float>::value) {
-            if (M % 128 == 0) f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.6f);
-            if (M % 64 == 0) f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.35f);
-            f(PgCfg<32, 2, 6, 2, 0, 1>{}, 0.5f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.95f);
+            f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.3f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 1.3f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.2f);
+            f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
         } else if constexpr (std::is_same<WT, int8_t>::value) {
-            if (M % 128 == 0) f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
-            else if (M % 64 == 0) f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 2, 4>{}, 1.65f);
-            else f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
+            f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.15f), f(PgCfg<96, 4, 2, 2>{}, 1.6f);
+            f(PgCfg<64, 4, 2, 3>{}, 1.5f), f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
+            f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
         } else {
-            if (M % 128 == 0) f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f), f(PgCfg<64, 4, 3, 2>{}, 0.65f);
-            else if (M % 64 == 0) f(PgCfg<64, 4, 4, 2>{}, 0.72f), f(PgCfg<64, 4, 3, 4>{}, 0.97f), f(PgCfg<64, 2, 4, 2>{}, 0.52f);
-            else f(PgCfg<32, 4, 4, 2>{}, 0.6f), f(PgCfg<32, 4, 3, 4>{}, 0.77f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
+            f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
+            f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);
+            f(PgCfg<96, 4, 2, 3, 4>{}, 1.05f), f(PgCfg<96, 4, 2, 2, 4>{}, 0.85f);
+            f(PgCfg<64, 4, 3, 3>{}, 0.85f), f(PgCfg<64, 4, 3, 2>{}, 0.65f), f(PgCfg<64, 4, 4, 2>{}, 0.72f), f(PgCfg<64, 2, 4, 2>{}, 0.52f);
+            f(PgCfg<32, 4, 4, 3>{}, 0.66f), f(PgCfg<32, 4, 4, 2>{}, 0.6f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
         }
     }
     template <class Epi>
-    static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e, int M,
+    static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
                   const PfState& st) {
-        PgIn<WT> in{(const WT*)W, hi, lo, N, K, M};
+        PgIn<WT> in{(const WT*)W, hi, lo, N, K, 0};
         in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
         float best = INFINITY;
         int pick = 0, i = 0;
-        pg_each(M, [&](auto cfg, float us) {
+        pg_each([&](auto cfg, float us) {
+            using Geo = PgGeo<decltype(cfg), WT>;
+            const int M = (in.valid + Geo::BM - 1) / Geo::BM * Geo::BM;
             // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
             // in 16 ranges and more
-            if (st.nseq > 1 && PgGeo<decltype(cfg), WT>::FOLD == 0) us = INFINITY;
+            if (st.nseq > 1 && Geo::FOLD == 0) us = INFINITY;
             const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
-            if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
+            if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
             ++i;
         });
         hipError_t err = hipSuccess;
         i = 0;
-        pg_each(M, [&](auto cfg, float) {
+        pg_each([&](auto cfg, float) {
             if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
         });
         SLI_HIP(err);
@@ -1099,11 +1105,10 @@ struct StepRecorder {
     template <class Epi>
     static int allow_pg(sli_model*) {
         hipError_t err = hipSuccess;
-        for (int M : {32, 64, 128})
-            pg_each(M, [&](auto cfg, float) {
-                const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
-                if (e != hipSuccess) err = e;
-            });
+        pg_each([&](auto cfg, float) {
+            const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
+            if (e != hipSuccess) err = e;
+        });
         SLI_HIP(err);
         return SLI_OK;
     }
@@ -1133,7 +1138,7 @@ struct StepRecorder {
         if (p % 2 == 0) {
             const size_t ls = (size_t)l * m->B * m->hkv * m->T * hd;
             PgEpiQKV<KT> eq{f.q, (KT*)m->kc + ls, (KT*)m->vc + ls, w.qkv_s, m->sin_t, m->cos_t, m->hq, m->hkv, hd, m->T};
-            SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, M, ps));
+            SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, ps));
             PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, h, m->hq, m->hkv, m->T,
                               1.0f / sqrtf((float)hd)};
             if constexpr (std::is_same<KT, __half>::value) {
@@ -1147,17 +1152,15 @@ struct StepRecorder {
             }
             SLI_HIP(hipGetLastError());
             er.rscale = w.wo_s;
-            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, M, ps);
+            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, ps);
         }
         PgEpiSwiGLU eg{F32 ? PfOut{nullptr, nullptr, (float*)f.ahi} : PfOut{f.ahi, f.alo}, w.gu_s, m->Il, m->c.act_mode};
-        SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, M, ps));
+        SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, ps));
         er.rscale = w.down_s;
-        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, M, ps);
+        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, ps);
     }
     static int record_prefill(sli_model* m, const PfState& ps) {
-        const int n = ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps;
-        // (fp32 matrix instructions run at a sixteenth of the rate of fp16: padding rows cost more than tiles of 32)
-        const int M = std::is_same<WT, float>::value && n < 512 ? (n + 31) / 32 * 32 : pf_rows(n);
+        const int M = pf_rows(ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps);
         for (int p = 0; p < 2 * m->L; ++p) {
             SLI_TRY(record_pf_phase(m, p, M, ps));
             const size_t n = (size_t)M * m->D;
@@ -1937,8 +1940,7 @@ static int pad_rows(const sli_model* m, int n) {
 static int pf_alloc(sli_model* m) {
     auto& p = m->pf;
     if (p.x) return SLI_OK;
-    // (64: a workgroup of the fp32 cache's attention)
-    const size_t M = pf_rows(std::max(64, std::min(m->B * pad_rows(m, m->T), kPfMaxChunk))), D = m->D, QD = (size_t)m->hq * m->hd;
+    const size_t M = pf_rows(std::min(m->B * pad_rows(m, m->T), kPfMaxChunk)) + kPfPad, D = m->D, QD = (size_t)m->hq * m->hd;
     int rc = SLI_OK;
     auto A = [&](void** ptr, size_t bytes) {
         if (rc == SLI_OK) rc = model_alloc(m, ptr, bytes);

@@ -231,11 +231,11 @@ struct PgGeo {
     static constexpr int NDMA = STAGE / 1024;  // wave-instructions per stage
     // depth after which a wave's sums go into a second set of accumulators (0: one chain over the whole depth). hi + lo
     // activations keep 2^-23 of a value, one fp32 chain over 4096 k loses more: with it the logits after 100 tokens of
-    // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 8 tiles a wave it
+    // Llama-3-8B are 1.2e-4 from float64, with chains of 256 9.0e-5 (the decode step's: 8.9e-5). Up to 12 tiles a wave it
     // costs nothing; a 64 x 64 wave tile (16) 3 to 8 % of a GEMM, so there only where the caller's other route has them.
     // fp32: every 4 k are a sum of their own (mfmas), chained up to 512 k: no longer than the chains of the decode step's
     // lanes.
-    static constexpr int FOLD = F32 ? 512 : NB == 2 && (AT * WPT <= 8 || Cfg::FO) ? 256 : 0;
+    static constexpr int FOLD = F32 ? 512 : NB == 2 && (AT * WPT <= 12 || Cfg::FO) ? 256 : 0;
     static_assert(!F32 || NB == 1, "fp32: one image");
     static constexpr int DPW = NDMA / WAVES;   // per wave
     static constexpr int SA = Cfg::SA;         // split rings (PgCfg): A pieces per wave DPA, B pieces DPB

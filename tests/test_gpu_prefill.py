@@ -212,6 +212,27 @@ def test_prefill_splits_match_decode(gpu, w, n):
         assert np.abs(a - b).max() <= 2 ** -7
 
 
+@pytest.mark.parametrize("n", [97, 98, 161, 193, 194, 290])
+def test_prefill_rows_of_each_tiling(gpu, n):
+    """Row counts around multiples of 96: every GEMM of a chunk pads to its own tile (96 rows where that is cheaper than 64
+    or 128), so the rows that one writes and the next reads differ. A wide MLP, so that its two GEMMs take other tiles
+    than the attention's; the same bounds as above."""
+    from simplellminference_amd.model import LlamaModel, preset
+    cfg = preset("small-h128-gqa", max_length=320, intermediate_size=14336)
+    m = LlamaModel(config=cfg, w_dtype="f16", kv_dtype="f16", seed=5).init()
+    prompt = _prompt(n, cfg.vocab_size)
+    ref = m.predict(prompt, n + 3, want_logits=True)
+    k0 = m.kv(1, 0, n), m.kv(1, 1, n)
+    m.reset()
+    tok, log = m.predict_prefill(prompt, n + 3, want_logits=True)
+    k1 = m.kv(1, 0, n), m.kv(1, 1, n)
+    m.close()
+    assert np.array_equal(tok, ref[0])
+    assert np.abs(log[n - 1:] - ref[1][n - 1:]).max() <= 1e-3
+    for a, b in zip(k0, k1):  # one fp16 rounding of values up to 8
+        assert np.abs(a - b).max() <= 2 ** -7
+
+
 @pytest.mark.parametrize("hd,heads,kvh,n", [(128, 8, 1, 65), (128, 8, 2, 130), (64, 8, 4, 17), (64, 8, 8, 300), (128, 8, 2, 64),
                                             (64, 32, 32, 2050), (128, 16, 4, 2100)])
 def test_prefill_attention_groups(gpu, hd, heads, kvh, n):

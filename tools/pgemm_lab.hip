@@ -188,10 +188,21 @@ static void sweep(const Shape& sh, int M, const std::vector<int>& forces) {
             RUN(32, 2, 4, 2, 0);
             RUN(32, 4, 4, 2, 0);
             RUN(32, 4, 3, 4, 0);
+            RUN(32, 2, 3, 2, 0);
+            RUN(32, 4, 4, 3, 0);
         } else if (M <= 64) {
             RUN(64, 2, 4, 2, 0);
             RUN(64, 4, 4, 2, 0);
             RUN(64, 4, 3, 4, 0);
+            RUN(64, 2, 3, 2, 0);
+            RUN(64, 4, 3, 3, 0);
+            RUN(64, 4, 2, 2, 0);
+        } else if (M <= 96) {
+            RUN(96, 4, 2, 2, 4);
+            RUN(96, 4, 2, 4, 3);
+            RUN(96, 4, 2, 3, 4);
+            RUN(96, 4, 3, 2, 0);
+            RUN(32, 4, 4, 2, 0);
         } else {
             RUN(64, 4, 3, 2, 0);
             RUN(128, 4, 2, 2, 4);
@@ -202,10 +213,18 @@ static void sweep(const Shape& sh, int M, const std::vector<int>& forces) {
         if (M <= 32) {
             RUN(32, 2, 4, 2, 0);
             RUN(32, 4, 4, 2, 0);
+            RUN(32, 2, 3, 2, 0);
+            RUN(32, 4, 3, 4, 0);
         } else if (M <= 64) {
             RUN(64, 4, 2, 2, 0);
             RUN(64, 4, 3, 2, 0);
             RUN(64, 4, 2, 4, 0);
+            RUN(64, 4, 2, 3, 0);
+            RUN(64, 2, 2, 2, 0);
+        } else if (M <= 96) {
+            RUN(96, 4, 2, 2, 0);
+            RUN(96, 2, 2, 2, 0);
+            RUN(32, 4, 4, 2, 0);
         } else {
             RUN(64, 4, 3, 2, 0);
             RUN(128, 4, 2, 2, 0);
