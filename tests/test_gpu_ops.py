@@ -84,6 +84,29 @@ def test_rmsnorm(gpu, oracle, dim):
     _close(got, want, rtol=2e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("dim", [1, 1023, 1025, 8191, 8192, 8193, 20000])
+def test_rmsnorm_argmax_around_the_held_part(gpu, oracle, dim):
+    """The norm holds 8192 elements in registers and loops over the rest, the arg-max takes 16384 a turn: lengths at the
+    edges (in place too), the maximum at the first and last place, beside one NaN and as a tie. The norm against float64:
+    a relative error of (20 adds of a lane + 6 of the wave + 16 of the waves + 5 single operations) x 2^-24 = 2.9e-6."""
+    torch = gpu
+    from simplellminference_amd import ops
+    r = _rng(dim)
+    x = r.standard_normal(dim).astype(np.float32)
+    w = (1 + 0.1 * r.standard_normal(dim)).astype(np.float32)
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 * x64).mean() + np.float32(1e-5)) * w
+    got = ops.rmsnorm(_t(torch, x), _t(torch, w), 1e-5).cpu().numpy()
+    _close(got, want, rtol=2.9e-6, atol=0)
+    t = _t(torch, x)
+    assert np.array_equal(ops.rmsnorm(t, _t(torch, w), 1e-5, y=t).cpu().numpy(), got)
+    for places in ([0], [dim - 1], [dim // 2, dim - 1], [16383 % dim, 16384 % dim]):
+        y = x.copy()
+        y[dim // 3 + 1 - (dim < 3)] = np.nan
+        y[places] = 9.0
+        assert int(ops.argmax(_t(torch, y)).item()) == oracle.argmax(y)
+
+
 @pytest.mark.parametrize("theta", [10000.0, 100000.0, 500000.0])
 def test_rope_cache_bit_exact(gpu, oracle, theta):
     from simplellminference_amd import ops
