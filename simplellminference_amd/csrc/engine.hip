@@ -1067,7 +1067,7 @@ struct StepRecorder {
             f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
         } else if constexpr (std::is_same<WT, int8_t>::value) {
             f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.15f), f(PgCfg<96, 4, 2, 2>{}, 1.6f);
-            f(PgCfg<64, 4, 2, 3>{}, 1.5f), f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
+            f(PgCfg<64, 4, 2, 3>{}, 1.4f), f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
             f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
         } else {
             f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
