@@ -1059,7 +1059,7 @@ struct StepRecorder {
     // rows 27 and 47 (int8 25 and 41) against 30 and 51 (28 and 48) of 128- and 256-row tiles. Measured at 512
     // rows, q/k/v | gate/up | wo | down in us: 112 | 202 | 44 | 96, against 144 | 263 | 122 | 122 of two 256-row chunks
     // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
-    // fp32, 74 rows: 137 | 229 | 54 | 110 (the matrix cores' fp32 rate: 75 TFLOP/s of 151 in padded rows).
+    // fp32, 74 rows, in the engine: 158 | 276 | 54 | 132 (gate/up: 63 TFLOP/s in padded rows of the matrix cores' 151).
     template <class F>
     static void pg_each(F&& f) {
         if constexpr (std::is_same<WT, float>::value) {

@@ -1,4 +1,4 @@
-// prefill.h — prompt prefill as real GEMMs over the prompt (SURVEY.md §8(f)2; the reference teacher-forces the
+// prefill.h — prompt prefill as real GEMMs over the prompt (the reference teacher-forces the
 // prompt one token per forward, source/model/model.cpp:157-165, so every weight is streamed once per prompt
 // token). Here a chunk of up to kPfMaxChunk prompt positions runs through each layer together:
 //
@@ -106,7 +106,7 @@ static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* 
     const int n4 = D / 4;
     float4 v[MAXV], wv[MAXV];
     float ss = 0.0f;
-    // the norm weights are loaded with x (round 6: not after the reduction, one memory round trip fewer)
+    // the norm weights are loaded with x, not after the reduction: one memory round trip fewer
     const float4* w4 = reinterpret_cast<const float4*>(w ? w : xr);
 #pragma unroll
     for (int j = 0; j < MAXV; ++j)
