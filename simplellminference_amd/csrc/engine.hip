@@ -2242,6 +2242,7 @@ int sli_model_get_exec(sli_model* m, int32_t* mode) {
 int sli_model_step(sli_model* m) {
     SLI_CHECK(m, SLI_ERR_ARG, "null model");
     SLI_CHECK(!m->group, SLI_ERR_STATE, "a rank of an in-process tp group steps with its group (sli_tp_group_step)");
+    const OnDevice dev(m->c.device);  // (a first step records its launches)
     SLI_TRY(capture(m));
     SLI_HIP(hipGraphLaunch(m->graph_exec, m->stream));
     return SLI_OK;
@@ -2266,6 +2267,7 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
                             int32_t* tokens_out, float* logits_out) {
     SLI_CHECK(m && prompts && lens && tokens_out, SLI_ERR_ARG, "null argument");
     SLI_CHECK(max_length >= 1 && max_length <= m->T, SLI_ERR_RANGE, "max_length must be in [1, max_len]");
+    const OnDevice dev(m->c.device);  // (scratch and launches of the prompt's chunks)
     for (int b = 0; b < m->B; ++b) {
         SLI_CHECK(lens[b] >= 1 && lens[b] <= ld, SLI_ERR_RANGE, "prompt length out of range");
         SLI_TRY(set_prompt(m, b, prompts + (size_t)b * ld, lens[b]));
