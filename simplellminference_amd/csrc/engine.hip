@@ -112,6 +112,7 @@ struct sli_model {
         __half *hhi = nullptr, *hlo = nullptr, *ahi = nullptr, *alo = nullptr;
         float* ws = nullptr;                    // partial sums of the tiles that a GEMM cuts over its depth (PgIn::ws)
         unsigned* cnt = nullptr;
+        int cap = 0;                            // positions of a chunk at most (0: none of this is allocated)
     } pf;
     // tensor-parallel all-reduce: SLI_ALLREDUCE_RCCL (ncclAllReduce) or SLI_ALLREDUCE_ONESHOT (oneshot.h)
     int ar_mode = SLI_ALLREDUCE_RCCL;
@@ -1937,10 +1938,11 @@ static int pad_rows(const sli_model* m, int n) {
     return (n + q - 1) / q * q;
 }
 
-static int pf_alloc(sli_model* m) {
+// The scratch of chunks of up to `cap` positions: all of it, or nothing is left behind.
+static int pf_alloc(sli_model* m, int cap) {
     auto& p = m->pf;
-    if (p.x) return SLI_OK;
-    const size_t M = pf_rows(std::min(m->B * pad_rows(m, m->T), kPfMaxChunk)) + kPfPad, D = m->D, QD = (size_t)m->hq * m->hd;
+    const size_t M = pf_rows(std::min(m->B * pad_rows(m, m->T), cap)) + kPfPad, D = m->D, QD = (size_t)m->hq * m->hd;
+    const size_t before = m->allocs.size();
     int rc = SLI_OK;
     auto A = [&](void** ptr, size_t bytes) {
         if (rc == SLI_OK) rc = model_alloc(m, ptr, bytes);
@@ -1955,15 +1957,39 @@ static int pf_alloc(sli_model* m) {
     if (!f32) A((void**)&p.alo, sizeof(__half) * M * m->Il);
     A((void**)&p.ws, kPgWsBytes);
     A((void**)&p.cnt, sizeof(unsigned) * kPgWsTiles);
-    if (rc != SLI_OK) return rc;
-    SLI_HIP(hipMemsetAsync(p.cnt, 0, sizeof(unsigned) * kPgWsTiles, m->stream));
-    return SLI_DISPATCH(m, prepare_prefill, m);
+    if (rc == SLI_OK) {
+        const hipError_t e = hipMemsetAsync(p.cnt, 0, sizeof(unsigned) * kPgWsTiles, m->stream);
+        rc = e == hipSuccess ? SLI_DISPATCH(m, prepare_prefill, m) : hip_fail(e, "hipMemsetAsync");
+    }
+    if (rc != SLI_OK) {
+        for (size_t i = before; i < m->allocs.size(); ++i) (void)hipFree(m->allocs[i]);
+        m->allocs.resize(before);
+        p = {};
+        (void)hipGetLastError();  // (else the next launch's check finds it)
+        return rc;
+    }
+    p.cap = cap;
+    return SLI_OK;
+}
+
+// The scratch is there (pf.cap positions a chunk), or pf.cap stays 0: it does not fit beside the model and the prompt takes
+// the steps, which need none. Chunks of kPfMaxChunk positions, or of a quarter (one sequence: a sixteenth) where memory
+// holds no more. Ranks of separate processes fail instead: their collectives have to agree on the chunks.
+static int pf_ready(sli_model* m) {
+    if (m->pf.cap) return SLI_OK;
+    const int need = m->B * pad_rows(m, m->T), least = kPfMaxChunk / (m->B == 1 ? 16 : 4);
+    for (int cap = kPfMaxChunk; cap >= least; cap /= 4) {
+        if (cap < kPfMaxChunk && cap >= need) continue;  // (as much as what failed)
+        const int rc = pf_alloc(m, cap);
+        if (rc != SLI_ERR_NOMEM || m->collectives) return rc;
+    }
+    return SLI_OK;
 }
 
 // chunks of n positions of every sequence of a batch
 static std::vector<PfState> pf_batch_chunks(const sli_model* m, int n) {
     std::vector<PfState> cs;
-    const int most = pad_rows(m, kPfMaxChunk / m->B - 63);
+    const int most = pad_rows(m, m->pf.cap / m->B - 63);
     for (int p0 = 0; p0 < n; p0 += most) {
         const int nv = std::min(most, n - p0);
         cs.push_back(PfState{p0, nv, pad_rows(m, nv), m->B});
@@ -1981,11 +2007,11 @@ static int pf_predict_positions(const sli_model* m, const int32_t* lens, int max
     return n >= 8 ? n : 0;
 }
 
-// chunk c of the prompt's n - 1 prefilled positions
-static std::vector<PfState> pf_chunks(int n) {
+// chunks of the prompt's n - 1 prefilled positions
+static std::vector<PfState> pf_chunks(int n, int cap) {
     std::vector<PfState> cs;
-    for (int p0 = 0; p0 < n - 1; p0 += kPfMaxChunk) {
-        const int nv = std::min(kPfMaxChunk, n - 1 - p0);
+    for (int p0 = 0; p0 < n - 1; p0 += cap) {
+        const int nv = std::min(cap, n - 1 - p0);
         cs.push_back(PfState{p0, nv, pf_rows(nv), 1});
     }
     return cs;
@@ -2122,9 +2148,10 @@ extern "C" int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n) {
     SLI_HIP(hipSetDevice(m->c.device));
     SLI_TRY(set_prompt(m, 0, ids, n));
     SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
-    if (n > 1 && sli_model_prefill_path(m)) {
-        SLI_TRY(pf_alloc(m));
-        for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
+    const bool chunks = n > 1 && sli_model_prefill_path(m);
+    if (chunks) SLI_TRY(pf_ready(m));
+    if (chunks && m->pf.cap) {
+        for (const PfState& c : pf_chunks(n, m->pf.cap)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
         SLI_TRY(wait_stream(m));
     } else {
         for (int p = 0; p < n - 1; ++p) {  // the decode step, teacher-forced (model.cpp:159-165)
@@ -2146,9 +2173,13 @@ extern "C" int sli_tp_group_prefill(sli_tp_group* g, const int32_t* ids, int32_t
         SLI_TRY(set_prompt(m, 0, ids, n));
         SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
     }
-    if (n > 1 && sli_model_prefill_path(m0)) {
-        for (sli_model* m : g->ranks) SLI_TRY(pf_alloc(m));
-        for (const PfState& c : pf_chunks(n)) SLI_TRY(SLI_DISPATCH(m0, record_group_prefill, g, c));
+    int cap = n > 1 && sli_model_prefill_path(m0) ? kPfMaxChunk : 0;  // the smallest of the ranks'
+    for (sli_model* m : g->ranks) {
+        if (cap) SLI_TRY(pf_ready(m));
+        cap = std::min(cap, m->pf.cap);
+    }
+    if (cap) {
+        for (const PfState& c : pf_chunks(n, cap)) SLI_TRY(SLI_DISPATCH(m0, record_group_prefill, g, c));
         SLI_HIP(hipStreamSynchronize(g->stream));
     } else {
         for (int p = 0; p < n - 1; ++p) {
@@ -2273,9 +2304,10 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
         SLI_TRY(set_prompt(m, b, prompts + (size_t)b * ld, lens[b]));
     }
     // (the prompt positions' logits come from the steps)
-    const int n0 = logits_out || m->bs ? 0 : pf_predict_positions(m, lens, max_length);
+    int n0 = logits_out || m->bs ? 0 : pf_predict_positions(m, lens, max_length);
+    if (n0 > 0) SLI_TRY(pf_ready(m));
+    if (m->pf.cap == 0) n0 = 0;
     if (n0 > 0) {
-        SLI_TRY(pf_alloc(m));
         for (const PfState& c : pf_batch_chunks(m, n0)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
     }
     for (int b = 0; b < m->B; ++b) {

@@ -30,9 +30,9 @@ thread_local struct {
     void* s;
 } config;
 int wrong_device = 0, launches = 0, graph_launches = 0, mallocs = 0, fail_at = -1;
-size_t fail_size = 0;
+size_t room = (size_t)-1, used = 0;
 std::map<int, int> mallocs_on, attributes_on;
-std::set<void*> live;
+std::map<void*, size_t> live;
 std::set<Stream*> streams;
 
 int done(int e) {
@@ -67,7 +67,7 @@ int hh_mallocs_on(int d) { return mallocs_on[d]; }
 int hh_attributes_on(int d) { return attributes_on[d]; }
 int hh_live() { return (int)live.size(); }
 void hh_fail_at(int k) { fail_at = k < 0 ? -1 : mallocs + k; }  // the k-th allocation from now (0: the next) fails
-void hh_fail_size(size_t n) { fail_size = n; }                  // allocations of n bytes and more fail (0: none)
+void hh_room(size_t n) { room = n ? used + n : (size_t)-1; }    // bytes left to allocate (0: no limit)
 int hh_pending_host_reads() {
     int n = 0;
     for (Stream* s : streams) n += s->host_reads;
@@ -88,16 +88,20 @@ int hipGetLastError() {
 int hipMalloc(void** p, size_t n) {
     const int i = mallocs++;
     *p = nullptr;
-    if (i == fail_at || (fail_size && n >= fail_size)) return done(kOom);
+    if (i == fail_at || used + n > room) return done(kOom);
     ++mallocs_on[current];
-    live.insert(*p = calloc(1, n ? n : 1));
+    live[*p = calloc(1, n ? n : 1)] = n;
+    used += n;
     return kOk;
 }
 int hipExtMallocWithFlags(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
 int hipFree(void* p) {
     if (!p) return kOk;
     for (Stream* s : streams) drain(s);
-    if (!live.erase(p)) return done(kInvalid);
+    const auto it = live.find(p);
+    if (it == live.end()) return done(kInvalid);
+    used -= it->second;
+    live.erase(it);
     free(p);
     return kOk;
 }

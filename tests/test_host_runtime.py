@@ -45,8 +45,68 @@ def device_of_predict(H):
     assert H.hh_wrong_device() == 0, "launches on a stream of another device"
 
 
+CHUNK_CALLS = [(dict(w_dtype="f32", kv_dtype="f32"), lambda m: m.predict_batch(_prompts(m, 20), 24)),
+               (dict(w_dtype="f16", batch=2), lambda m: m.predict_batch(_prompts(m, 20), 24)),
+               (dict(w_dtype="f16"), lambda m: m.prefill(_prompts(m, 20)[0])),
+               (dict(w_dtype="i8"), lambda m: m.predict_prefill(_prompts(m, 20)[0], 24))]
+
+
+def scratch_that_does_not_fit(H):
+    """Every allocation of the chunks' scratch in turn fails: the call runs (through the steps, which need none), nothing of
+    the scratch is left, and the next call allocates all of it."""
+    for kw, call in CHUNK_CALLS:
+        m = _llama(**kw)
+        had = H.hh_mallocs()
+        call(m)
+        n = H.hh_mallocs() - had
+        assert n >= 5
+        m.close()
+        for k in range(n):
+            m = _llama(**kw)
+            live = H.hh_live()
+            H.hh_fail_at(k)
+            steps = H.hh_graph_launches()
+            call(m)
+            assert H.hh_live() == live and H.hh_graph_launches() - steps >= 19
+            had = H.hh_mallocs()
+            call(m)
+            assert (H.hh_mallocs() - had, H.hh_live() - live) == (n, n)
+            m.close()
+    assert H.hh_live() == 0
+
+
+def scratch_of_smaller_chunks(H):
+    """Scratch for 4096 positions does not fit, for 1024 it does: chunks of 1024. Ranks in one process agree on the chunks."""
+    from simplellminference_amd.model import TPGroup, preset
+    over = dict(max_length=4500)
+    for kw, call in CHUNK_CALLS:
+        launches = []
+        for room in (0, 80 << 20):  # (64 MB of it for the partial sums)
+            m = _llama(over=over, **kw)
+            H.hh_room(room)
+            ids = _prompts(m, 4200)
+            had, steps = H.hh_launches(), H.hh_graph_launches()
+            if "f32" in kw.values() or m.batch > 1:
+                m.predict_batch(ids, 4201)
+            else:
+                m.prefill(ids[0])
+            launches.append(H.hh_launches() - had)
+            assert H.hh_graph_launches() - steps <= 2, "the prompt ran as steps"
+            H.hh_room(0)
+            m.close()
+        assert launches[1] > 2 * launches[0], launches
+    g = TPGroup(preset("tiny-gqa", **over), 2, w_dtype="f16", seed=1).init()
+    had, steps = H.hh_launches(), H.hh_graph_launches()
+    H.hh_room(160 << 20)  # the second rank's are the smaller ones
+    g.prefill([1] * 4200)
+    H.hh_room(0)
+    assert H.hh_graph_launches() == steps and H.hh_launches() - had > 4 * 2 * 2 * 2 * 5, "five chunks of both ranks"
+    g.close()
+    assert H.hh_live() == 0
+
+
 # ---------------------------------------------------------------- the tests
-CASES = ["device_of_predict"]
+CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks"]
 
 
 @pytest.fixture(scope="module")
@@ -70,6 +130,6 @@ def test_host(host_hip, case):
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     H = ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)  # before libsli.so: its references to HIP end here
-    H.hh_fail_size.argtypes = [ctypes.c_size_t]
+    H.hh_room.argtypes = [ctypes.c_size_t]
     globals()[sys.argv[1]](H)
     print("ok", sys.argv[1])
