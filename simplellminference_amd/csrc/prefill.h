@@ -781,8 +781,12 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
     const int mi = blockIdx.x * kPaQB + wave * 16 + (lane & 15);  // this lane's query (chunk row)
     const int c = lane >> 4;
     const int pos = p0 + mi;                                      // its position
-    const int pos_max = p0 + blockIdx.x * kPaQB + kPaQB - 1;      // the block's last query position
-    const int nt = min(pos_max, a.T - 1) / kPaKT + 1;             // key tiles
+    const int end = min((int)blockIdx.x * kPaQB + kPaQB, row0 + ps.nv);
+    if (end <= (int)blockIdx.x * kPaQB) return;                   // (uniform) only padding rows
+    // The block's last valid position. Rows past it are loaded as this one: their p is 0, but what the cache still holds
+    // there may be no number.
+    const int last = min(p0 + end - 1, a.T - 1);
+    const int nt = last / kPaKT + 1;                              // key tiles
     float qv[QD], o[QD];
 #pragma unroll
     for (int e = 0; e < QD; ++e) {
@@ -798,7 +802,7 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
         __syncthreads();
         for (int i = threadIdx.x; i < kPaKT * HD / V16; i += 256) {  // the tile's K and V rows
             const int r = i / (HD / V16), cc = i - r * (HD / V16);
-            const int t = min(t0 + r, a.T - 1);
+            const int t = min(t0 + r, last);
             reinterpret_cast<u32x4*>(&ks[r][0])[cc] = reinterpret_cast<const u32x4*>(kb + (size_t)t * HD)[cc];
             reinterpret_cast<u32x4*>(&vs[r][0])[cc] = reinterpret_cast<const u32x4*>(vb + (size_t)t * HD)[cc];
         }

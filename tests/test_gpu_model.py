@@ -203,3 +203,25 @@ def test_predict_f32_prompt_chunk_matches_steps(gpu, name, kv, n, length):
     assert np.array_equal(got, want) and m.state() == state
     assert np.abs(m.logits()[0] - wl[-1]).max() <= (1e-4 if kv == "f32" else 1e-3)
     m.close()
+
+
+def test_predict_f32_reads_no_stale_cache_rows(gpu):
+    """A prompt that left no numbers in the cache (a NaN embedding row) changes nothing for a shorter one after it: its chunk
+    masks the rows past the prompt, and does not multiply them by 0 either."""
+    from simplellminference_amd.model import LlamaModel, preset
+    from simplellminference_amd.tp import KINDS
+    cfg = preset("tiny-gqa")
+    prompt = np.arange(1, 13)
+    m = LlamaModel(config=cfg, w_dtype="f32", kv_dtype="f32", seed=3).init()
+    want = m.predict(prompt, 20)
+    emb = m.weight_shard(KINDS["emb"])
+    bad = emb.copy()
+    bad[cfg.vocab_size - 1] = np.nan
+    m.set_weight(KINDS["emb"], 0, bad)
+    m.predict(np.concatenate([prompt, np.full(30, cfg.vocab_size - 1)]), 50)
+    assert np.isnan(m.kv(0, 1, 42)[20:42]).any()
+    m.set_weight(KINDS["emb"], 0, emb)
+    got = m.predict(prompt, 20)
+    assert np.array_equal(got, want)
+    assert np.isfinite(m.logits()[0]).all() and np.isfinite(m.kv(1, 1, 20)).all()
+    m.close()
