@@ -1142,9 +1142,9 @@ struct StepRecorder {
             SLI_TRY(pg(m, w.qkv, (m->hq + 2 * m->hkv) * hd, D, f.hhi, f.hlo, eq, ps));
             PfAttnArgs<KT> aa{f.q, (const KT*)m->kc + ls, (const KT*)m->vc + ls, h, m->hq, m->hkv, m->T,
                               1.0f / sqrtf((float)hd)};
-            if constexpr (std::is_same<KT, __half>::value) {
+            if constexpr (std::is_same<KT, __half>::value && !F32) {
                 SLI_HIP(hd == 128 ? launch_pf_flash<128>(aa, ps, device_cus(), s) : launch_pf_flash<64>(aa, ps, device_cus(), s));
-            } else {  // fp32 cache: fp32 VALU, 64 chunk rows per workgroup
+            } else {  // fp32 VALU as the steps', 64 chunk rows per workgroup: a fp32 cache, or fp32 weights beside an fp16 one
                 const dim3 ag((M + kPaQB - 1) / kPaQB, m->hq);
                 if (hd == 128)
                     hipLaunchKernelGGL((pf_attn_kernel<KT, 128>), ag, dim3(256), 0, s, aa, ps);

@@ -18,7 +18,7 @@
 //   3. pf_flash_kernel (fp16 KV): block-causal attention against the cache rows 0 .. position (mha_kernel.cpp:36-77
 //      per query: s_t = q.k_t * scale, softmax, sum p_t v_t): S = K q^T on MFMA with q split hi/lo, online softmax in
 //      fp32, P V on MFMA with V read transposed (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the
-//      VALU form (fp32, 64-position query blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches.
+//      VALU form (fp32, 64-position query blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches and fp32 weights.
 // fp32 weights: the same GEMM on v_mfma_f32_16x16x4_f32 with fp32 activations (one image, stages of 32 k).
 // int8 weights: stages of 128 k; a depth that is 64 mod 128 (e.g. Llama-2-7B int8 down at TP 4, 2752) ends with
 // a half stage (pgemm_kernel).
