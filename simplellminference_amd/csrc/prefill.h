@@ -60,6 +60,17 @@ __device__ __forceinline__ void pf_split(float v, __half& hi, __half& lo) {
     lo = __float2half_rn(v - __half2float(hi));
 }
 
+// v as N fp16 terms, each the rounding of what the ones before leave: 2 carry 22 to 23 bits, 3 all 24 (down to the fp16
+// subnormal step 2^-24)
+template <int N>
+__device__ __forceinline__ void pf_terms(float v, __half (&t)[N][8], int e) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        t[i][e] = __float2half_rn(v);
+        v -= __half2float(t[i][e]);
+    }
+}
+
 // What a GEMM reads: fp16 hi + lo, or fp32 (beside fp32 weights)
 struct PfOut {
     __half *hi = nullptr, *lo = nullptr;
@@ -882,12 +893,12 @@ __device__ __forceinline__ void pa_tr_wait(uint2 (&x1)[4], uint2 (&x2)[4]) {
 // blocks of 16 QT query positions, a wave each (GQA: 4 heads read one tile; MHA: 4 position blocks do). K and V tiles of
 // 64 keys reach LDS by DMA, double-buffered, one barrier per tile: every key row is fetched once per 64 QT query rows.
 // Per tile a wave computes
-//   - Sᵀ = K Qᵀ: C[key][query] on v_mfma_f32_16x16x32_f16, A = K rows (exact fp16), B = Qᵀ as hi + lo fp16;
+//   - Sᵀ = K Qᵀ: C[key][query] on v_mfma_f32_16x16x32_f16, A = K rows (exact fp16), B = Qᵀ as TERMS fp16 images;
 //   - online softmax in base 2 (p = 2^(s c - m), one fma and one v_exp per score, its rounding that of the exponent);
 //     the row maximum over the 4 lane groups of a query, the row sum only at the end. p carries a factor 2^8, which
 //     divides out with the row sum: the lo halves of p >= 2^-21 stay normal fp16 numbers;
 //   - Oᵀ += Vᵀ Pᵀ: B = Pᵀ straight from the Sᵀ accumulators (lane l holds query l & 15, keys {4g .. 4g+3, 16+4g ..
-//     16+4g+3}, g = l >> 4 — the k order of the B operand), P as hi + lo; A = Vᵀ by ds_read_b64_tr_b16, whose 4-row
+//     16+4g+3}, g = l >> 4 — the k order of the B operand), P as TERMS images; A = Vᵀ by ds_read_b64_tr_b16, whose 4-row
 //     blocks are exactly those keys.
 // The latest (longest) position blocks are dispatched first. mha_kernel.cpp:36-77 per query. Bound by the matrix cores and
 // the softmax between them: Llama-3-8B, 3776 rows, 299 us a layer (785 TFLOP/s with hi + lo), where a workgroup per 16 rows
@@ -896,7 +907,7 @@ template <int HD>
 struct PfFlash {
     static constexpr int KT = 64, ROWB = HD * 2, IMG = KT * ROWB, CPR = ROWB / 16, PIECES = IMG / 1024;
 };
-template <int HD, int QT>
+template <int HD, int QT, int TERMS>
 __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, PfState ps, int GW) {
     using F = PfFlash<HD>;
     constexpr int ND = HD / 32, NT = HD / 16, NK = F::KT / 16, PPW = 2 * F::PIECES / 4;
@@ -912,7 +923,7 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
     const int last = min(ps.p0 + min(blk * RB + RB, ps.nv) - 1, a.T - 1);                   // the workgroup's
     const int wlast = i0 < ps.nv ? min(ps.p0 + min(i0 + 16 * QT, ps.nv) - 1, a.T - 1) : -1;  // the wave's
     const size_t qs = (size_t)a.hq * HD;
-    u32x4 qh[QT][ND], ql[QT][ND];
+    u32x4 qf[TERMS][QT][ND];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         const int row = seq * ps.rps + min(i0 + t * 16 + i16, ps.rps - 1);
@@ -921,11 +932,11 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
             const float4* qp = reinterpret_cast<const float4*>(a.q + (size_t)row * qs + (size_t)h * HD + db * 32 + g * 8);
             const float4 v0 = qp[0], v1 = qp[1];
             const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-            __half hh[8], hl[8];
+            __half ht[TERMS][8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) pf_split(f[e], hh[e], hl[e]);
-            qh[t][db] = *reinterpret_cast<const u32x4*>(hh);
-            ql[t][db] = *reinterpret_cast<const u32x4*>(hl);
+            for (int e = 0; e < 8; ++e) pf_terms(f[e], ht, e);
+#pragma unroll
+            for (int i = 0; i < TERMS; ++i) qf[i][t][db] = *reinterpret_cast<const u32x4*>(ht[i]);
         }
     }
     pf_float4 o[QT][NT];
@@ -977,16 +988,14 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
                 kf[kt] = *reinterpret_cast<const u32x4*>(kimg + r * F::ROWB + ((4 * db + g) ^ pa_swz_k(r, F::ROWB)) * 16);
             }
 #pragma unroll
-            for (int kt = 0; kt < NK; ++kt)
+            for (int i = 0; i < TERMS; ++i)
 #pragma unroll
-                for (int t = 0; t < QT; ++t) s[kt][t] = pf_mfma(kf[kt], qh[t][db], s[kt][t]);
+                for (int kt = 0; kt < NK; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < NK; ++kt)
-#pragma unroll
-                for (int t = 0; t < QT; ++t) s[kt][t] = pf_mfma(kf[kt], ql[t][db], s[kt][t]);
+                    for (int t = 0; t < QT; ++t) s[kt][t] = pf_mfma(kf[kt], qf[i][t][db], s[kt][t]);
         }
         // lane holds keys t0 + 16 kt + 4 g + r of query i0 + 16 t + i16
-        u32x4 ph[QT][NK / 2], pl[QT][NK / 2];
+        u32x4 pf[TERMS][QT][NK / 2];
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
             const int pos = ps.p0 + i0 + t * 16 + i16;
@@ -1012,15 +1021,15 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
             }
 #pragma unroll
             for (int kb = 0; kb < NK / 2; ++kb) {
-                __half hh[8], hl[8];
+                __half ht[TERMS][8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float p = __builtin_amdgcn_exp2f(fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, -mx[t])) * 256.0f;
                     l[t] += p;
-                    pf_split(p, hh[e], hl[e]);
+                    pf_terms(p, ht, e);
                 }
-                ph[t][kb] = *reinterpret_cast<const u32x4*>(hh);
-                pl[t][kb] = *reinterpret_cast<const u32x4*>(hl);
+#pragma unroll
+                for (int i = 0; i < TERMS; ++i) pf[i][t][kb] = *reinterpret_cast<const u32x4*>(ht[i]);
             }
         }
         // Vᵀ 16-d tile d: lane 16 g + 4 q + p addresses row (4 g + q) [+16] of the 32-key block, d 16 d + 4 p .. +3
@@ -1039,15 +1048,12 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
             }
             pa_tr_wait(x1, x2);
 #pragma unroll
-            for (int d = 0; d < NT; ++d)
+            for (int i = 0; i < TERMS; ++i)
 #pragma unroll
-                for (int t = 0; t < QT; ++t)
-                    o[t][d] = pf_mfma(u32x4{x1[d].x, x1[d].y, x2[d].x, x2[d].y}, ph[t][kb], o[t][d]);
+                for (int d = 0; d < NT; ++d)
 #pragma unroll
-            for (int d = 0; d < NT; ++d)
-#pragma unroll
-                for (int t = 0; t < QT; ++t)
-                    o[t][d] = pf_mfma(u32x4{x1[d].x, x1[d].y, x2[d].x, x2[d].y}, pl[t][kb], o[t][d]);
+                    for (int t = 0; t < QT; ++t)
+                        o[t][d] = pf_mfma(u32x4{x1[d].x, x1[d].y, x2[d].x, x2[d].y}, pf[i][t][kb], o[t][d]);
         }
     }
 #pragma unroll
@@ -1064,17 +1070,21 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
     }
 }
 
-// Heads and positions per workgroup and wave: 32 query positions per wave where that still gives every CU two workgroups,
-// 16 (twice as many workgroups, each key row read twice as often) below (511 rows of 32 heads: 256 workgroups, not 128).
+// Batches take three terms of q and p, as their steps do (attn_mfma.h); one sequence's prefill takes two. Heads and positions
+// per workgroup and wave: 32 query positions per wave where that still gives every CU two workgroups, 16 (twice as many
+// workgroups, each key row read twice as often) below (511 rows of 32 heads: 256 workgroups, not 128) and with three terms
+// at head_dim 128, where 32 spill 48 registers (8 prompts of 2000 of Llama-3-8B 480 ms, with 16 461; two terms 456).
 template <int HD>
 hipError_t launch_pf_flash(const PfAttnArgs<__half>& a, const PfState& ps, int cus, hipStream_t s) {
     const int G = a.hq / a.hkv, GW = G < 4 ? G : 4;
     const int ny = a.hkv * (G / GW);
     auto blocks = [&](int qt) { return (ps.nv + (4 / GW) * 16 * qt - 1) / ((4 / GW) * 16 * qt) * ps.nseq; };
-    if (blocks(2) * ny >= 2 * cus)
-        hipLaunchKernelGGL((pf_flash_kernel<HD, 2>), dim3(blocks(2), ny), dim3(256), 0, s, a, ps, GW);
+    const bool wide = blocks(2) * ny >= 2 * cus;
+    auto go = [&](auto kernel, int qt) { hipLaunchKernelGGL(kernel, dim3(blocks(qt), ny), dim3(256), 0, s, a, ps, GW); };
+    if (ps.nseq > 1)
+        HD == 64 && wide ? go(pf_flash_kernel<HD, HD == 64 ? 2 : 1, 3>, 2) : go(pf_flash_kernel<HD, 1, 3>, 1);
     else
-        hipLaunchKernelGGL((pf_flash_kernel<HD, 1>), dim3(blocks(1), ny), dim3(256), 0, s, a, ps, GW);
+        wide ? go(pf_flash_kernel<HD, 2, 2>, 2) : go(pf_flash_kernel<HD, 1, 2>, 1);
     return hipGetLastError();
 }
 

@@ -59,7 +59,7 @@ def _model(batch, w):
     return m
 
 
-@pytest.mark.parametrize("batch,w", [(1, "f32")])
+@pytest.mark.parametrize("batch,w", [(1, "f32"), (2, "f16")])
 def test_chunk_keeps_the_bits_of_the_steps(gpu, batch, w):
     m = _model(batch, w)
     r = np.random.default_rng(batch)
@@ -75,4 +75,23 @@ def test_chunk_keeps_the_bits_of_the_steps(gpu, batch, w):
     share = (got != want).mean()
     print("share of the second layer's rows that differ", share)
     assert share <= 5e-3
+    m.close()
+
+
+def test_batch_chunk_of_wide_waves(gpu):
+    """head_dim 64 and enough rows: 32 positions per wave with three terms. 1e-3 and one fp16 rounding of values up to 8, as in
+    the other batch tests."""
+    from simplellminference_amd.model import LlamaModel, LlamaModelConfig
+    n, B = 401, 8
+    m = LlamaModel(config=LlamaModelConfig(500, 64, 1024, 1024, 512, n + 3, 2, 16, 16, 1e-5, 1e4), w_dtype="f16", kv_dtype="f16",
+                   seed=9, batch=B).init()
+    r = np.random.default_rng(9)
+    prompts = [r.integers(0, 500, n).tolist() for _ in range(B)]
+    want, wl = m.predict_batch(prompts, n + 1, want_logits=True)
+    kv = [m.kv(1, which, n, seq=b) for b in range(B) for which in (0, 1)]
+    m.reset()
+    assert np.array_equal(m.predict_batch(prompts, n + 1), want)
+    assert np.abs(m.logits()[0] - wl[:, -1]).max() <= 1e-3
+    for a, b in zip(kv, [m.kv(1, which, n, seq=b) for b in range(B) for which in (0, 1)]):
+        assert np.abs(a - b).max() <= 2 ** -7
     m.close()
