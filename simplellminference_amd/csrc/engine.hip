@@ -1887,7 +1887,8 @@ static int set_state(sli_model* m, int seq, int32_t token, int32_t pos, int32_t 
     return SLI_OK;
 }
 
-static int set_prompt(sli_model* m, int seq, const int32_t* ids, int32_t n) {
+// fed: the prompt's tokens are the sequence's history too
+static int set_prompt(sli_model* m, int seq, const int32_t* ids, int32_t n, bool fed = false) {
     SLI_CHECK(m && ids, SLI_ERR_ARG, "null argument");
     SLI_CHECK(seq < m->B, SLI_ERR_RANGE, "sequence index out of range");
     SLI_CHECK(n >= 1 && n <= m->T, SLI_ERR_RANGE, "prompt length out of range");
@@ -1899,6 +1900,9 @@ static int set_prompt(sli_model* m, int seq, const int32_t* ids, int32_t n) {
         if (seq >= 0 && b != seq) continue;
         SLI_HIP(hipMemcpyAsync(m->prompt + (size_t)b * (m->T + 1), ids, sizeof(int32_t) * n, hipMemcpyHostToDevice,
                                m->stream));
+        if (fed)
+            SLI_HIP(hipMemcpyAsync(m->hist + (size_t)b * (m->T + 1), ids, sizeof(int32_t) * n, hipMemcpyHostToDevice,
+                                   m->stream));
     }
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, m->stream, m->st, m->hist, seq, m->B, m->T, 0, 0, 0, n);
     SLI_HIP(hipGetLastError());
@@ -2121,9 +2125,7 @@ extern "C" int sli_model_prefill_batch(sli_model* m, const int32_t* prompts, con
     for (int b = 0; b < m->B; ++b) {
         SLI_CHECK(lens[b] >= 1 && lens[b] <= ld && lens[b] <= m->T, SLI_ERR_RANGE, "prompt length out of range");
         const int32_t* p = prompts + (size_t)b * ld;
-        SLI_TRY(set_prompt(m, b, p, lens[b]));
-        SLI_HIP(hipMemcpyAsync(m->hist + (size_t)b * (m->T + 1), p, sizeof(int32_t) * lens[b], hipMemcpyHostToDevice,
-                               m->stream));
+        SLI_TRY(set_prompt(m, b, p, lens[b], true));
         if (lens[b] == 1) continue;
         slots.push_back(b);
         starts.push_back(0);
@@ -2146,8 +2148,7 @@ extern "C" int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n) {
         SLI_CHECK(ids[i] >= 0 && ids[i] < m->V, SLI_ERR_RANGE, "Token index is greater than vocab size.");
     if (m->bs) return sli_model_prefill_batch(m, ids, &n, n);
     SLI_HIP(hipSetDevice(m->c.device));
-    SLI_TRY(set_prompt(m, 0, ids, n));
-    SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
+    SLI_TRY(set_prompt(m, 0, ids, n, true));
     const bool chunks = n > 1 && sli_model_prefill_path(m);
     if (chunks) SLI_TRY(pf_ready(m));
     if (chunks && m->pf.cap) {
@@ -2169,10 +2170,7 @@ extern "C" int sli_tp_group_prefill(sli_tp_group* g, const int32_t* ids, int32_t
     SLI_CHECK(m0->B == 1, SLI_ERR_STATE, "prefill: batch-1 groups (a batch prefills through predict_batch)");
     SLI_CHECK(n >= 1 && n <= m0->T, SLI_ERR_RANGE, "prompt length out of range");
     SLI_HIP(hipSetDevice(g->device));
-    for (sli_model* m : g->ranks) {
-        SLI_TRY(set_prompt(m, 0, ids, n));
-        SLI_HIP(hipMemcpyAsync(m->hist, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, m->stream));
-    }
+    for (sli_model* m : g->ranks) SLI_TRY(set_prompt(m, 0, ids, n, true));
     int cap = n > 1 && sli_model_prefill_path(m0) ? kPfMaxChunk : 0;  // the smallest of the ranks'
     for (sli_model* m : g->ranks) {
         if (cap) SLI_TRY(pf_ready(m));
@@ -2311,10 +2309,10 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
         for (const PfState& c : pf_batch_chunks(m, n0)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
     }
     for (int b = 0; b < m->B; ++b) {
-        const int32_t* p = prompts + (size_t)b * ld;
+        const size_t row = (size_t)b * (m->T + 1);
         if (n0 > 0)
-            SLI_HIP(hipMemcpyAsync(m->hist + (size_t)b * (m->T + 1), p, sizeof(int32_t) * n0, hipMemcpyHostToDevice, m->stream));
-        SLI_TRY(set_state(m, b, p[n0], n0, 1));
+            SLI_HIP(hipMemcpyAsync(m->hist + row, m->prompt + row, sizeof(int32_t) * n0, hipMemcpyDeviceToDevice, m->stream));
+        SLI_TRY(set_state(m, b, prompts[(size_t)b * ld + n0], n0, 1));
     }
     const size_t per_step = (size_t)m->B * m->v_n;
     for (int t = n0; t < max_length; ++t) {  // model.cpp:157

@@ -105,8 +105,36 @@ def scratch_of_smaller_chunks(H):
     assert H.hh_live() == 0
 
 
+def callers_arrays_are_read(H):
+    """When a call that takes prompts returns, nothing is still to be copied out of the caller's arrays."""
+    from simplellminference_amd.model import TPGroup, preset
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    for kw in (dict(w_dtype="f32", kv_dtype="f32"), dict(w_dtype="f16")):
+        m = _llama(**kw)
+        for n in (1, 2, 20):
+            m.prefill(_prompts(m, n)[0])
+            assert H.hh_pending_host_reads() == 0, (kw, n)
+            m.set_prompt(_prompts(m, n)[0])
+            assert H.hh_pending_host_reads() == 0, (kw, n)
+        m.close()
+        g = TPGroup(preset("tiny-gqa"), 2, seed=1, **kw).init()
+        for n in (1, 20):
+            g.prefill([1] * n)
+            assert H.hh_pending_host_reads() == 0, ("group", kw, n)
+        g.close()
+    b = BlockSpec("attention", 2, 64, 64, kv_heads=1, scale=0.125, ff=128, ff_limit=7.0)
+    m = StackModel(StackSpec(64, 128, (b,) * 2, max_length=64), batch=2, seed=1).init()
+    for lens in ((1, 1), (1, 5), (3, 4)):
+        P = (ctypes.c_int32 * 10)(*range(10))
+        from simplellminference_amd._lib import call
+        call("sli_model_prefill_batch", m._h, P, (ctypes.c_int32 * 2)(*lens), 5)
+        assert H.hh_pending_host_reads() == 0, ("stack", lens)
+    m.close()
+
+
 # ---------------------------------------------------------------- the tests
-CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks"]
+CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
+         "callers_arrays_are_read"]
 
 
 @pytest.fixture(scope="module")
