@@ -269,6 +269,9 @@ int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out)
         HY_TRY(hy_alloc(s, (void**)&s->pg_ws, kPgWsBytes, false));
         HY_TRY(hy_new(s, &s->pg_cnt, kPgWsTiles));
     }
+    double w = 0.0, k = 0.0;
+    hy_step_bytes(s, 1, 0.0, &w, &k);
+    s->replays = w < kReplayBytes * (double)s->runs.size();
     return hy_allow_lds();
 }
 
@@ -797,8 +800,7 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
             const std::vector<int32_t>& want, float* logits_host, float* hidden_host) {
     const int n = (int)rows_in.size();
     SLI_CHECK(n >= 1 && n <= s->M && !segs.empty() && (int)segs.size() <= s->M, SLI_ERR_SHAPE, "pass: too many rows");
-    // a decode step runs its rows as they are, from a captured graph; a prompt pass is padded to the GEMM's row tiles and
-    // launched directly (its launches run longer than they take to enqueue, and every row count would be a graph)
+    // a decode step runs its rows as they are, from a captured graph; a prompt pass is padded to the GEMM's row tiles
     int M = s->f16 ? HyRec<__half>::rows_for(n) : n, kt = 0;
     SLI_CHECK(!one || n <= s->B, SLI_ERR_SHAPE, "pass: more sequences than slots");
     if (!one) {
@@ -820,13 +822,25 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
             SLI_HIP(hipMemcpy2DAsync(hidden_host + r * (size_t)n * s->D, sizeof(float) * s->D, s->x, sizeof(float) * s->Dp,
                                      sizeof(float) * s->D, n, hipMemcpyDeviceToHost, s->stream));
         }
-    } else if (!one) {
-        HY_TRY(HY_DISPATCH(s, M, one, msegs, kt, pass()));
     } else {
-        auto& g = s->graphs[M];
-        SLI_HIP(hipStreamSynchronize(s->stream));
-        HY_TRY(hy_capture(s, g, M, one, msegs, kt));
-        SLI_HIP(hipGraphLaunch(g.second, s->stream));
+        // (A prompt pass is launched directly the first time; replaying it saves a small stack the enqueueing, kReplayBytes.)
+        int gkt = 0;  // grid of a graph's expansion: a power of two, so that few graphs are captured
+        if (kt > 0) {
+            gkt = M / kLatTile + 1;
+            while (gkt < kt) gkt *= 2;
+            gkt = std::min(gkt, hy_key_tiles_max(s));
+        }
+        const bool keep = one || s->replays;
+        const auto at = std::make_pair(one ? 0 : 1 + gkt, M);
+        if (keep && (one || s->graphs.count(at))) {
+            auto& g = s->graphs[at];
+            SLI_HIP(hipStreamSynchronize(s->stream));
+            HY_TRY(hy_capture(s, g, M, one, msegs, gkt));
+            SLI_HIP(hipGraphLaunch(g.second, s->stream));
+        } else {
+            HY_TRY(HY_DISPATCH(s, M, one, msegs, kt, pass()));
+            if (keep) s->graphs[at];
+        }
     }
     if (!want.empty()) {
         const int nw = (int)want.size();

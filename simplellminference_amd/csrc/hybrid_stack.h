@@ -20,6 +20,11 @@ namespace sli {
         if (rc_ != SLI_OK) return rc_; \
     } while (0)
 
+// A prompt pass whose rows of launches recur is replayed from a graph where a run reads fewer weights than this: its launches
+// are over sooner than a busy host enqueues the next. Four blocks of width 256, 4 rows: 170 us replayed, 170 to 193
+// directly; eight sequential ones of width 1024 655 and 648 to 752; eight of width 2048 (84 MB a run) 447 and 434 to 464,
+// and above the graph saves nothing. The first pass of a row count is launched: a capture takes longer (0.1 to 0.4 ms).
+constexpr double kReplayBytes = 64e6;
 constexpr int kHyLogitRows = 256;  // wanted rows per pass of the output head
 constexpr int kHySection = 128;  // pairs: a GEMM row block (at most 256 rows) never straddles the two inputs
 
@@ -120,8 +125,10 @@ struct BlockStack {
     unsigned* bg_cnt = nullptr;
     size_t bg_ws_bytes = 0, bg_groups = 1;  // the most any projection needs (hy_bg_need)
     std::vector<void*> allocs;
-    // captured passes: {0, rows} of a decode step, {1 + key tile bucket, rows} of a prompt pass
-    std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // decode passes of `feed`, by row count
+    // captured passes of `feed`: {0, rows} of a decode step, {1 + grid of the expansion, rows} of a prompt pass (null:
+    // launched once so far)
+    std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+    bool replays = false;  // prompt passes too (kReplayBytes)
     float* pg_ws = nullptr;  // partial sums and arrival counters of the prompt GEMM (prefill.h PgIn)
     unsigned* pg_cnt = nullptr;
 };

@@ -455,6 +455,26 @@ def test_passes_repeat_bit_for_bit(gpu, dtype):
     m.close()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_replayed_prompt_passes(gpu, dtype):
+    """The second and later prompt passes of a row count are replays of a captured one: other tokens, slots, positions and
+    numbers of portions, decode passes in between, against the same passes launched one by one (as they are where the
+    residuals are asked for), bit for bit."""
+    t = R.random_tensors(PAIR, 31)
+    m, plain = (make(PAIR, t, dtype, 512, batch=3) for _ in range(2))
+    at = [0, 0, 0]
+    for i, entries in enumerate([{0: 40}, {1: 61}, {0: 33, 2: 20}, {0: 1, 1: 1}, {2: 64}, {0: 90, 1: 30}, {2: 100}, {1: 1},
+                                 {0: 128}, {1: 41}, {2: 9, 0: 7, 1: 31}, {1: 200}, {2: 230}, {0: 65}]):
+        ids = [tokens(n, PAIR["vocab"], seed=100 * i + b) for b, n in entries.items()]
+        args = list(entries), [at[b] for b in entries], ids, [[n - 1] for n in entries.values()]
+        got, want = m.feed(*args), plain.feed(*args, want_hidden=True)[0]
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (i, entries)
+        for b, n in entries.items():
+            at[b] += n
+    m.close()
+    plain.close()
+
+
 # ---------------------------------------------------------------- the framework's entry points
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_greedy_generation(gpu, dtype):

@@ -132,9 +132,32 @@ def callers_arrays_are_read(H):
     m.close()
 
 
+def small_stacks_replay_their_prompts(H):
+    """A prompt pass of a small block stack launches the first time its row count comes and is a graph from then on; a large one
+    always launches."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+
+    def spec(D, arrangement):
+        b = dict(parallel=BlockSpec("attention", D // 64, 64, 64, kv_heads=D // 128, scale=0.125, ff=D, ff_limit=7.0),
+                 sequential=BlockSpec("latent", D // 64, 64, 64, scale=0.125, kv_rank=64, window=32, ff=D, experts=4, top=2))
+        return StackSpec(64, D, (b[arrangement],) * 2, max_length=300, arrangement=arrangement,
+                         positions=300 if arrangement == "sequential" else 0)
+    for arrangement, D, small in (("parallel", 256, True), ("sequential", 256, True), ("parallel", 3072, False)):
+        m = StackModel(spec(D, arrangement), batch=2, seed=1).init()
+        for n in (20, 100, 200):
+            counts = []
+            for _ in range(3):
+                had = H.hh_launches(), H.hh_graph_launches()
+                m.feed([0], [0], [[1] * n])
+                counts.append((H.hh_launches() - had[0], H.hh_graph_launches() - had[1]))
+            assert counts[0][0] > 10 and counts[0][1] == 0
+            assert counts[1:] == ([(0, 1)] * 2 if small else [counts[0]] * 2), (arrangement, D, n, counts)
+        m.close()
+
+
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
-         "callers_arrays_are_read"]
+         "callers_arrays_are_read", "small_stacks_replay_their_prompts"]
 
 
 @pytest.fixture(scope="module")
