@@ -1053,31 +1053,7 @@ struct StepRecorder {
     // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); the last prompt
     // position runs as an ordinary decode step. Phases as record_phase: 2l = qkv, attention, wo; 2l+1 =
     // gate/up, down; under tensor parallelism each ends with the all-reduce of the chunk's residual rows.
-    // The GEMM tilings (prefill.h PgCfg<BM, WR, S, AT, SA>), each with the time of one stage of a workgroup when every CU
-    // has one, in us (tools/pgemm_lab, one MI355X, 7B shapes): f(PgCfg<...>{}, us). The launch takes the one whose plan
-    // (prefill.h pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth) costs
-    // least. 192-row tiles of 96 chunk rows: q/k/v 33 and gate/up 51 us at 96 rows, where 128 rows take 43 and 72; of 64
-    // rows 27 and 47 (int8 25 and 41) against 30 and 51 (28 and 48) of 128- and 256-row tiles. Measured at 512
-    // rows, q/k/v | gate/up | wo | down in us: 112 | 202 | 44 | 96, against 144 | 263 | 122 | 122 of two 256-row chunks
-    // with one workgroup per tile; 64 rows int8 26 | 44 | 15 | 24 against 46 | 48 | 42 | 42.
-    // fp32, 74 rows, in the engine: 158 | 276 | 54 | 132 (gate/up: 63 TFLOP/s in padded rows of the matrix cores' 151).
-    template <class F>
-    static void pg_each(F&& f) {
-        if constexpr (std::is_same<WT, float>::value) {
-            f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.3f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 1.3f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.2f);
-            f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
-        } else if constexpr (std::is_same<WT, int8_t>::value) {
-            f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.15f), f(PgCfg<96, 4, 2, 2>{}, 1.6f);
-            f(PgCfg<64, 4, 2, 3>{}, 1.4f), f(PgCfg<64, 4, 2, 2>{}, 1.2f), f(PgCfg<64, 4, 3, 2>{}, 1.27f);
-            f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
-        } else {
-            f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
-            f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);
-            f(PgCfg<96, 4, 2, 3, 4>{}, 1.05f), f(PgCfg<96, 4, 2, 2, 4>{}, 0.85f);
-            f(PgCfg<64, 4, 3, 3>{}, 0.85f), f(PgCfg<64, 4, 3, 2>{}, 0.65f), f(PgCfg<64, 4, 4, 2>{}, 0.72f), f(PgCfg<64, 2, 4, 2>{}, 0.52f);
-            f(PgCfg<32, 4, 4, 3>{}, 0.66f), f(PgCfg<32, 4, 4, 2>{}, 0.6f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
-        }
-    }
+    // one GEMM over a chunk's rows: the tiling (prefill.h pg_tilings) whose plan costs least over the rows padded to its BM
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
                   const PfState& st) {
@@ -1085,7 +1061,7 @@ struct StepRecorder {
         in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
         float best = INFINITY;
         int pick = 0, i = 0;
-        pg_each([&](auto cfg, float us) {
+        pg_tilings<WT>([&](auto cfg, float us) {
             using Geo = PgGeo<decltype(cfg), WT>;
             const int M = (in.valid + Geo::BM - 1) / Geo::BM * Geo::BM;
             // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
@@ -1097,7 +1073,7 @@ struct StepRecorder {
         });
         hipError_t err = hipSuccess;
         i = 0;
-        pg_each([&](auto cfg, float) {
+        pg_tilings<WT>([&](auto cfg, float) {
             if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
         });
         SLI_HIP(err);
@@ -1106,7 +1082,7 @@ struct StepRecorder {
     template <class Epi>
     static int allow_pg(sli_model*) {
         hipError_t err = hipSuccess;
-        pg_each([&](auto cfg, float) {
+        pg_tilings<WT>([&](auto cfg, float) {
             const hipError_t e = pgemm_allow_lds<Epi, decltype(cfg), WT>();
             if (e != hipSuccess) err = e;
         });

@@ -64,14 +64,14 @@ struct HyProj {
             in.ws = s->pg_ws, in.cnt = s->pg_cnt;
             float best = INFINITY;
             int pick = 0, i = 0;
-            pg_each(M, [&](auto cfg, float us) {
+            pg_row_tilings(M, [&](auto cfg, float us) {
                 const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true);
                 if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
                 ++i;
             });
             hipError_t err = hipSuccess;
             i = 0;
-            pg_each(M, [&](auto cfg, float) {
+            pg_row_tilings(M, [&](auto cfg, float) {
                 if (i++ == pick) err = launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, u0}, PfState{}, st());
             });
             SLI_HIP(err);
@@ -80,24 +80,12 @@ struct HyProj {
             return fail(SLI_ERR_ARG, "prompt GEMM: fp16 weights");
         }
     }
-    // Tilings (their row count divides M), each with the time of one stage of a workgroup when the chip is full of them, in
-    // us (tools/pgemm_lab, LAB_ONE); the launch takes the one whose plan (prefill.h pg_plan) costs least. At 34304 x 4096
-    // and 4096 x 15104, us, the tiles of the last round cut over the depth | whole tiles: 1024 rows 369 | 401 and 161 |
-    // 196, 256 rows 116 | 129 and 56 | 112, 64 rows 65 | 75 and 30 | 79.
-    template <class F>
-    static void pg_each(int M, F&& f) {
-        if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
-        if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.2f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
-        if (M % 64 == 0) f(PgCfg<64, 4, 4, 2, 0, 1>{}, 0.57f), f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.56f);
-        if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.75f);
-        if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.9f);
-    }
     template <class Epi>
     static int allow() {
         if constexpr (F16) {
             hipError_t err = hipSuccess;
             for (int M : {32, 256})
-                pg_each(M, [&](auto cfg, float) {
+                pg_row_tilings(M, [&](auto cfg, float) {
                     const hipError_t e = pgemm_allow_lds<PgPair<Epi>, decltype(cfg), __half>();
                     if (e != hipSuccess) err = e;
                 });

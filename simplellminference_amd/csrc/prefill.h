@@ -763,6 +763,44 @@ hipError_t pgemm_allow_lds() {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)PgGeo<Cfg, WT>::LDS);
 }
 
+// The tilings of the Llama prompts, f(PgCfg<...>{}, us): us weighs a stage of the tiling, about what it takes with the chip
+// full of whole tiles that share their weight rows (tools/pgemm_lab stages, profiles/pgemm_tilings.txt): fp16 within 8 %, but
+// the 192 x 32 tile 0.54; int8 4 to 19 % below; fp32 2.96, 2.58, 1.63, 1.06, 1.95, the 96-row tile at half its time. A launch
+// takes the one whose plan (pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth)
+// costs least. Llama-2-7B, q/k/v | gate/up | wo | down, us (the same file): the best plan against the best tiling in whole
+// tiles: 512 rows 105 | 208 | 44 | 93 against 105 | 230 | 45 | 117; 64 rows 29 | 47 | 14 | 28 against 41 | 50 | 25 | 61; int8
+// 64 rows 26 | 41 | 15 | 25 against 34 | 47 | 27 | 67. The 192-row tiles: 96 rows gate/up 52, where 128 rows take 63 and 68;
+// 64 rows, against 128-row tiles, gate/up 47 | 50 (int8 41 | 47), q/k/v 29 | 32 (26 | 28).
+template <typename WT, class F>
+void pg_tilings(F&& f) {
+    if constexpr (std::is_same<WT, float>::value) {
+        f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.3f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 1.3f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.2f);
+        f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
+    } else if constexpr (std::is_same<WT, int8_t>::value) {
+        f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.15f), f(PgCfg<96, 4, 2, 2>{}, 1.6f);
+        f(PgCfg<64, 4, 2, 3>{}, 1.4f), f(PgCfg<64, 4, 2, 2>{}, 1.2f);
+        f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
+    } else {
+        f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
+        f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);
+        f(PgCfg<96, 4, 2, 3, 4>{}, 1.05f), f(PgCfg<96, 4, 2, 2, 4>{}, 0.85f);
+        f(PgCfg<64, 4, 3, 3>{}, 0.85f), f(PgCfg<64, 4, 3, 2>{}, 0.65f);
+        f(PgCfg<32, 4, 4, 3>{}, 0.66f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
+    }
+}
+
+// The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.91; 1.03,
+// 1.10, 0.71; 0.41; 0.45; 0.61. 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 349 | 381 and
+// 149 | 184, 256 rows 113 | 121 and 55 | 80, 64 rows 65 | 76 and 34 | 76.
+template <class F>
+void pg_row_tilings(int M, F&& f) {
+    if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.2f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
+    if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.56f);
+    if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.75f);
+    if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.9f);
+}
+
 // ---------------------------------------------------------------- 3. block-causal attention
 // grid (rows / 64, hq); 4 waves x 16 queries; lane l: query l & 15 of the wave, dims [c * HD/4, (c+1) * HD/4) with
 // c = l >> 4. Scores: the 4 lanes of a query add their quarter dot products (xor 16 / 32 exchanges); every lane
