@@ -8,6 +8,7 @@
 #include <functional>
 #include <map>
 #include <set>
+#include <string>
 #include <vector>
 
 namespace {
@@ -34,6 +35,9 @@ size_t room = (size_t)-1, used = 0;
 std::map<int, int> mallocs_on, attributes_on;
 std::map<void*, size_t> live;
 std::set<Stream*> streams;
+std::map<const void*, std::string> kernels;
+std::set<std::string> launched;
+std::string names;
 
 int done(int e) {
     if (e != kOk) last_error = e;
@@ -68,6 +72,17 @@ int hh_attributes_on(int d) { return attributes_on[d]; }
 int hh_live() { return (int)live.size(); }
 void hh_fail_at(int k) { fail_at = k < 0 ? -1 : mallocs + k; }  // the k-th allocation from now (0: the next) fails
 void hh_room(size_t n) { room = n ? used + n : (size_t)-1; }    // bytes left to allocate (0: no limit)
+const char* hh_launched() {  // the kernels launched or recorded since the last call, one name a line
+    names.clear();
+    for (auto& n : launched) names += n + "\n";
+    launched.clear();
+    return names.c_str();
+}
+const char* hh_kernels() {  // those that the loaded libraries hold
+    names.clear();
+    for (auto& k : kernels) names += k.second + "\n";
+    return names.c_str();
+}
 int hh_pending_host_reads() {
     int n = 0;
     for (Stream* s : streams) n += s->host_reads;
@@ -145,10 +160,11 @@ int hipGraphDestroy(void* g) { return free(g), kOk; }
 int hipGraphExecDestroy(void* e) { return free(e), kOk; }
 int hipGraphLaunch(void*, void*) { return ++graph_launches, kOk; }
 int hipFuncSetAttribute(const void*, int, int) { return ++attributes_on[current], kOk; }
-int hipLaunchKernel(const void*, Dim3, Dim3, void**, size_t, void* st) {
+int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void* st) {
     Stream* s = (Stream*)st;
     if (s && s->device != current) ++wrong_device;
     if (!s || !s->capturing) ++launches;
+    launched.insert(kernels[f]);
     return kOk;
 }
 int __hipPushCallConfiguration(Dim3 g, Dim3 b, size_t sh, void* s) { return config = {g, b, sh, s}, kOk; }
@@ -156,7 +172,9 @@ int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* sh, void** s) {
     return *g = config.g, *b = config.b, *sh = config.sh, *s = config.s, kOk;
 }
 void** __hipRegisterFatBinary(const void*) { return (void**)malloc(8); }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+    kernels[f] = name;
+}
 void __hipUnregisterFatBinary(void** m) { free(m); }
 int hipEventCreate(void** e) { return *e = malloc(1), kOk; }
 int hipEventDestroy(void* e) { return free(e), kOk; }

@@ -315,6 +315,21 @@ def test_prompt_past_one_pass(gpu, dtype):
     m.close()
 
 
+@pytest.mark.parametrize("n", [33, 65, 129, 257, 700, 1025, 1153, 2048, 2049])
+def test_row_counts_of_a_pass(gpu, n):
+    """Prompt passes of every tile height with padding rows, up to a whole pass of 2048 and one row more: the last positions'
+    logits as when the tokens before them come in portions of other row counts."""
+    c = stack(blk(heads=4, dim=64, vdim=64, kv_rank=64, window=100, ff=136), blk(experts=0, heads=3, dim=32, vdim=40, window=0),
+              width=192, positions=2112, vocab=203)
+    m = make(c, R.random_tensors(c, 22), "bfloat16")
+    ids, cut = tokens(n, c["vocab"], n), max(0, n - 40)
+    whole = m.feed([0], [0], [ids], [list(range(cut, n))])
+    for p in range(0, cut, 480):
+        m.feed([0], [p], [ids[p:min(cut, p + 480)]])
+    close(whole, m.feed([0], [cut], [ids[cut:]], [list(range(n - cut))]), "bfloat16")
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("lens", [(5, 70, 33), (1, 2, 3, 130, 64, 31, 32, 97), tuple(range(3, 14))])
 def test_batches_of_unequal_requests(gpu, lens, dtype):

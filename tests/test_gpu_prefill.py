@@ -5,8 +5,9 @@ teacher-forces the prompt one token per forward (model.cpp:157-165); the oracle'
 the bar is the oracle's predict: greedy token ids bit-exact, logits of every computed position within 1e-3,
 and the K/V rows the prefill writes within the fp16 cache rounding.
 
-The launches of a chunk run 32, 64 or a multiple of 128 rows: the prompt lengths below cover each, padding rows, and
-GEMMs whose last round of tiles is cut over the depth.
+The row-wise launches of a chunk run a multiple of 32 rows, and each GEMM pads them to its own tiles (32, 64, 96 or 128
+chunk rows): the prompt lengths below cover padding rows, GEMMs whose last round of tiles is cut over the depth, every
+tiling, and a second chunk.
 """
 import numpy as np
 import pytest
@@ -46,7 +47,7 @@ def _check(gtok, glog, otok, olog, n, tol=1e-3):
 @pytest.mark.parametrize("name", ["tiny", "tiny-gqa"])
 @pytest.mark.parametrize("n", [1, 2, 9, 33, 63])
 def test_prefill_predict_matches_oracle(gpu, oracle, name, n):
-    """Short prompts (n - 1 prefilled positions = 0, 1, 8, 32, 62: chunk sizes 32 and 64, padding rows),
+    """Short prompts (n - 1 prefilled positions = 0, 1, 8, 32, 62: 32 and 64 rows, padding rows),
     then greedy up to the context end."""
     cfg, om, gm = _pair(oracle, name)
     prompt = _prompt(n, cfg.vocab_size)
@@ -60,7 +61,7 @@ def test_prefill_predict_matches_oracle(gpu, oracle, name, n):
 
 @pytest.mark.parametrize("n", [129, 200, 257, 300])
 def test_prefill_long_prompts(gpu, oracle, n):
-    """Prompts of 129..300 tokens: launches of 128, 256 and 384 rows, GQA."""
+    """Prompts of 129..300 tokens: 128, 224, 256 and 320 rows, GQA."""
     cfg, om, gm = _pair(oracle, "tiny-gqa", max_length=320)
     prompt = _prompt(n, cfg.vocab_size)
     steps = n + 12
@@ -103,7 +104,7 @@ def test_prefill_llama7b_shape(gpu, oracle):
 @pytest.mark.timeout(400)
 def test_prefill_llama7b_shape_long(gpu, oracle):
     """Llama-2-7B layer shapes (2 layers; vocab cut to 512 so the CPU oracle stays in budget), a 140-token
-    prompt: one 256-row chunk with 117 padding rows, hd 128, 4096 x 11008 projections."""
+    prompt: 139 rows, padded to 160 and to the GEMMs' tiles, hd 128, 4096 x 11008 projections."""
     cfg, om, gm = _pair(oracle, "llama2-7b", seed=1, num_hidden_layers=2, max_length=160, vocab_size=512)
     prompt = _prompt(140, cfg.vocab_size)
     otok, olog = om.predict(prompt, 144)
@@ -156,8 +157,8 @@ def test_prefill_f32_weights_teacher_forces(gpu, oracle):
 
 
 def test_prefill_twice_reuses_graphs(gpu, oracle):
-    """A second prompt on the same model (graphs already captured, other chunk sizes) gives the oracle's
-    tokens too: the chunk position and count come from device memory, not from the capture."""
+    """A second and a third prompt on the same model, of other row counts, give the oracle's tokens too: over the first one's
+    cache rows and scratch, and with the same decode graph."""
     cfg, om, gm = _pair(oracle, "tiny-gqa", max_length=320)
     for n in (70, 260, 5):
         prompt = _prompt(n, cfg.vocab_size, seed=11)
@@ -253,3 +254,83 @@ def test_prefill_attention_groups(gpu, hd, heads, kvh, n):
     m.close()
     assert np.array_equal(tok, ref)
     assert np.abs(log - lref).max() <= 1e-3
+
+
+# (weights, shape, batch, prompt): between them every tiling of the prompt GEMMs runs (test_host_runtime.py looks)
+TILING_SHAPES = [("f16", "llama2-7b", 1, 10), ("f16", "llama2-7b", 1, 74), ("f16", "llama2-7b", 1, 200),
+                 ("f16", "llama3-8b", 1, 104), ("f16", "llama3-8b", 1, 200), ("f16", "llama2-7b", 2, 400),
+                 ("i8", "llama2-7b", 1, 10), ("i8", "llama2-7b", 1, 50), ("i8", "llama2-7b", 1, 74), ("i8", "llama2-7b", 1, 130),
+                 ("i8", "llama3-8b", 1, 130), ("i8", "llama3-8b", 1, 200), ("f32", "llama2-7b", 1, 18),
+                 ("f32", "llama2-7b", 1, 50), ("f32", "llama2-7b", 1, 74), ("f32", "llama3-8b", 1, 20), ("f32", "llama3-8b", 1, 104)]
+
+
+def tiling_model(w, name, batch):
+    from simplellminference_amd.model import LlamaModel, preset
+    return LlamaModel(config=preset(name, num_hidden_layers=2, vocab_size=500, max_length=416), w_dtype=w,
+                      kv_dtype="f32" if w == "f32" else "f16", seed=12, batch=batch).init()
+
+
+def tiling_run(m, prompts, length, steps):
+    """Prompts through the chunks, or (steps) through the decode step."""
+    if m.batch > 1:
+        return m.predict_batch(prompts, length, want_logits=steps)
+    if steps or m.w_dtype == 0:  # (fp32: predict's chunk)
+        return m.predict(prompts[0], length, want_logits=steps)
+    return m.predict_prefill(prompts[0], length)
+
+
+@pytest.mark.parametrize("w,name,batch,n", TILING_SHAPES)
+def test_prefill_every_tiling(gpu, w, name, batch, n):
+    """Two layers of real width against the decode steps: fp16 and int8 logits within the 8e-4 of their norm that an fp16
+    cache's roundings either way make, fp32 within 2e-6 (sums of up to 14336 products in another order). The second layer's
+    cache rows follow from the first's, whose values round either way: within one fp16 rounding of the largest, and in norm
+    below 2^-12 (2^-11 / sqrt 3 would be every value rounded the other way). fp32 rows: 2^-14."""
+    m = tiling_model(w, name, batch)
+    prompts = [_prompt(n + b, m.config.vocab_size)[b:] for b in range(batch)]
+    want, wl = tiling_run(m, prompts, n + 1, True)
+    rows = lambda: [m.kv(1, which, n, seq=b) for b in range(batch) for which in (0, 1)]
+    kv = rows()
+    wl = (wl if batch == 1 else wl.swapaxes(0, 1))[-1]
+    m.reset()
+    got = tiling_run(m, prompts, n + 1, False)
+    log = m.logits()[0]
+    assert np.array_equal(got, want)
+    assert np.linalg.norm(log - wl) <= (2e-6 if w == "f32" else 8e-4) * np.linalg.norm(wl)
+    for a, b in zip(rows(), kv):
+        d = np.abs(a - b).max()
+        assert d <= (2.0 ** -14 if w == "f32" else 2.0 ** -10 * np.abs(b).max())
+        assert np.linalg.norm(a - b) <= 2.0 ** -12 * np.linalg.norm(b)
+    m.close()
+
+
+@pytest.mark.parametrize("w,kv", [("f16", "f16"), ("i8", "f16"), ("f16", "f32"), ("f32", "f32"), ("f32", "f16")])
+@pytest.mark.parametrize("n", [4098, 4130])
+def test_prompt_past_one_chunk(gpu, w, kv, n):
+    """Prompts of 4097 and 4129 positions: a second chunk of 1 and of 33 rows, whose queries see the first one's cache rows.
+    The bars of this file (fp32: 1e-4)."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset("tiny-gqa", max_length=4200), w_dtype=w, kv_dtype=kv, seed=3).init()
+    prompt = _prompt(n, m.config.vocab_size)
+    want = m.predict_prefill(prompt, n + 6) if w == "f32" else m.predict(prompt, n + 6)  # the decode steps
+    log, rows = m.logits()[0], [m.kv(1, which, n)[4090:] for which in (0, 1)]
+    m.reset()
+    got = m.predict(prompt, n + 6) if w == "f32" else m.predict_prefill(prompt, n + 6)
+    assert np.array_equal(got, want)
+    assert np.abs(m.logits()[0] - log).max() <= (1e-4 if (w, kv) == ("f32", "f32") else 1e-3)
+    for a, b in zip([m.kv(1, which, n)[4090:] for which in (0, 1)], rows):
+        assert np.abs(a - b).max() <= (1e-4 if kv == "f32" and w == "f32" else 2 ** -7)
+    m.close()
+
+
+def test_prompt_past_one_chunk_tp_group(gpu):
+    """The same of an in-process group of two ranks, against one rank."""
+    from simplellminference_amd.model import LlamaModel, TPGroup, preset
+    cfg, n = preset("tiny-gqa", max_length=4200), 4130
+    prompt = _prompt(n, cfg.vocab_size)
+    m = LlamaModel(config=cfg, w_dtype="f16", kv_dtype="f16", seed=3).init()
+    want = m.predict_prefill(prompt, n + 6)
+    m.close()
+    g = TPGroup(cfg, 2, w_dtype="f16", kv_dtype="f16", seed=3).init()
+    got = g.predict_prefill(prompt, n + 6)
+    g.close()
+    assert np.array_equal(np.asarray(got).reshape(-1)[:n + 6], want)

@@ -535,3 +535,29 @@ def test_replayed_prompt_passes(gpu, dtype):
             at[b] += n
     m.close()
     plain.close()
+
+
+# prompts of a 4096-wide block: between them every tiling of the stacks' prompt GEMMs runs (test_host_runtime.py looks)
+TILING_ROWS = [20, 33, 129, 700]
+
+
+def wide_model():
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    return StackModel(StackSpec(203, 4096, (BlockSpec("attention", 4, 64, 64, kv_heads=2, scale=0.125, ff=8192, ff_limit=7.0),),
+                                taps=4, residual_mult=0.4, max_length=800), batch=1, seed=4).init()
+
+
+@pytest.mark.parametrize("n", TILING_ROWS)
+def test_every_tiling_of_a_pass(gpu, n):
+    """Whole prompts against the same in portions of 64 rows and single steps."""
+    m = wide_model()
+    ids = tokens(n, vocab=203, seed=n)
+    want = list(range(n - 3, n))
+    whole = m.feed([0], [0], [ids], [want])
+    p = 0
+    while p < n - 3:
+        e = min(n - 3, p + 64)
+        m.feed([0], [p], [ids[p:e]])
+        p = e
+    close(whole, np.concatenate([m.feed([0], [i], [[ids[i]]], [[0]]) for i in want]), "bfloat16")
+    m.close()

@@ -5,6 +5,7 @@ Each case runs in a process of its own (the runtime replaces HIP for the whole p
 """
 import ctypes
 import os
+import re
 import subprocess
 import sys
 
@@ -155,9 +156,43 @@ def small_stacks_replay_their_prompts(H):
         m.close()
 
 
+def _tilings(names):
+    """(weight type, tiling) of the prompt GEMM instances among kernel names."""
+    out = set()
+    for n in names.decode().split():
+        g = re.search(r"pgemm_kernel.*PgCfgI((?:L[ib]\d+E)+)E+(a|f|6__half|DF16_|S\d*_)EE", n)
+        if g:
+            cfg = tuple(int(v) for v in re.findall(r"L[ib](\d+)E", g[1]))
+            if not cfg[6]:  # (not the grouped ones: the expert rows' and the latent expansion's)
+                out.add((g[2] if g[2] in "af" else "half", cfg))
+    return out
+
+
+def every_tiling_is_tested(H):
+    """The shapes that the GPU tests name run every tiling that the library holds."""
+    from tests import test_gpu_prefill as P, test_gpu_stack as S
+    H.hh_launched()
+    run = set()
+    for w, name, batch, n in P.TILING_SHAPES:
+        m = P.tiling_model(w, name, batch)
+        H.hh_launched()
+        P.tiling_run(m, [[1] * n] * batch, n + 1, False)
+        run |= _tilings(H.hh_launched())
+        m.close()
+    m = S.wide_model()
+    for n in S.TILING_ROWS:
+        H.hh_launched()
+        m.feed([0], [0], [[1] * n])
+        run |= _tilings(H.hh_launched())
+    m.close()
+    held = _tilings(H.hh_kernels())
+    assert len(held) > 20 and run == held, sorted(held - run)
+
+
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
-         "callers_arrays_are_read", "small_stacks_replay_their_prompts"]
+         "callers_arrays_are_read", "small_stacks_replay_their_prompts",
+         "every_tiling_is_tested"]
 
 
 @pytest.fixture(scope="module")
@@ -182,5 +217,6 @@ if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     H = ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)  # before libsli.so: its references to HIP end here
     H.hh_room.argtypes = [ctypes.c_size_t]
+    H.hh_launched.restype = H.hh_kernels.restype = ctypes.c_char_p
     globals()[sys.argv[1]](H)
     print("ok", sys.argv[1])
