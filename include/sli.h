@@ -66,8 +66,8 @@ int sli_stream_sync(sli_stream_t stream);
 int sli_matmul(const float* x, const void* w, int w_dtype, const float* w_row_scale, float* y, int32_t rows,
                int32_t cols, float scale, sli_stream_t stream);
 
-/* Batched projection for B sequences decoding in lockstep (the reference is batch 1; this serves
- * SURVEY.md §8 config C4): y[b][r] = sum_c x[b][c] * W[r][c] for b < batch <= 8, on MFMA
+/* Batched projection for B sequences decoding in lockstep (the reference is batch 1):
+ * y[b][r] = sum_c x[b][c] * W[r][c] for b < batch <= 8, on MFMA
  * (v_mfma_f32_16x16x32_f16; the fp32 input is carried as fp16 hi + lo columns). x [batch][cols] fp32, W
  * [rows][cols] fp16 (SLI_DT_F16 only), y [batch][rows] fp32, cols % 32 == 0. The workspace
  * (sli_matmul_batch_workspace_bytes, 0 = unsupported shape) holds split-K partials and counters. */
@@ -138,7 +138,7 @@ typedef struct sli_model sli_model;
 
 /* Tensor-parallel shard plan (host only, no device needed): the window of the full reference-layout
  * tensor `kind` (sli_synth.h) that rank cfg->tp_rank holds, and where it lands in the rank's fused
- * buffer. Megatron split (SURVEY.md §8(e)): wq/wk/wv/gate/up by output rows (heads / FFN columns),
+ * buffer. Megatron split: wq/wk/wv/gate/up by output rows (heads / FFN columns),
  * wo/down by input columns, embedding and norms replicated, LM head = embedding rows [vocab_lo,
  * vocab_lo + vocab_n). */
 typedef struct {
@@ -202,7 +202,9 @@ int sli_model_get_state_seq(sli_model* m, int32_t seq, int32_t* pos, int32_t* to
  * multi-process tensor parallelism every rank calls it, the chunk's residual rows all-reduced over RCCL
  * twice per layer), filling the K/V cache; the state is left at
  * (token ids[n-1], position n-1, advancing, prompt = ids), so the next sli_model_step yields the first
- * greedy token exactly as the reference's token-by-token predict (model.cpp:157-165) would. */
+ * greedy token exactly as the reference's token-by-token predict (model.cpp:157-165) would.
+ * The chunks' scratch (about 93 KB a position of a 7B model, and 64 MB) is allocated by the first call that runs one. Where
+ * 4096 positions do not fit, chunks are smaller, and where none fits the prompt goes through the decode step. */
 int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n);
 /* Which path sli_model_prefill takes for this model: 1 = chunked MFMA GEMMs (prefill.h), 0 = the decode step,
  * teacher-forced (fp32 weights, batch > 1, unsupported shapes, or a TP rank without an RCCL communicator). */
@@ -228,7 +230,7 @@ int sli_model_get_history(sli_model* m, int32_t seq, int32_t n, int32_t* out);
  * 128 whose per-workgroup shares fit (the TP-4 / TP-8 shards of Llama-2-7B); otherwise SLI_ERR_STATE with the
  * reason. Under tensor parallelism it needs the one-shot buffers and SLI_ALLREDUCE_FUSED_WG (ranks on distinct
  * devices), or no communicator (SLI_DEBUG_NOCOMM). Not for the ranks of an in-process group.
- * (Round 5 removed the opt-in persistent one-launch step, mode 1; sli_model_set_exec(1) returns SLI_ERR_ARG.) */
+ * (Mode 1, an opt-in persistent one-launch step, is gone; sli_model_set_exec(1) returns SLI_ERR_ARG.) */
 enum { SLI_EXEC_LAUNCHES = 0, SLI_EXEC_PERSIST = 2 };
 int sli_model_set_exec(sli_model* m, int32_t mode);
 int sli_model_get_exec(sli_model* m, int32_t* mode);
@@ -244,7 +246,9 @@ int sli_model_sync(sli_model* m);
 int sli_model_get_logits(sli_model* m, float* host, int32_t n, int32_t* vocab_lo);
 /* LlamaModel::predict on token ids: tokens_out[t] = token fed at position t; logits_out optional
  * [max_length][local vocab]. batch > 1: every sequence gets the prompt, tokens_out is [batch][max_length]
- * and logits_out [max_length][batch][local vocab]. */
+ * and logits_out [max_length][batch][local vocab].
+ * Without logits_out, one rank with fp32 weights, or with fp16 weights and batch > 1, runs the positions before the shortest
+ * prompt's last (from 8 on) as sli_model_prefill's chunks, in the precision of its steps; the rest, and all else, steps. */
 int sli_model_predict(sli_model* m, const int32_t* prompt, int32_t n_prompt, int32_t max_length,
                       int32_t* tokens_out, float* logits_out);
 /* predict for batch sequences with their own prompts: prompts [batch][ld] (sequence b's first lens[b]
@@ -259,10 +263,10 @@ int sli_model_get_kv_seq(sli_model* m, int32_t seq, int32_t layer, int32_t which
  * dequantised with its row scales). */
 int sli_model_get_weight(sli_model* m, int32_t kind, int32_t index, float* host, int64_t n);
 int sli_model_stream(sli_model* m, sli_stream_t* out);
-/* Algorithmic HBM bytes of one step on this rank (weights, KV at the current position) — SURVEY.md §8(d). */
+/* Algorithmic HBM bytes of one step on this rank (weights, KV at the current position). */
 int sli_model_step_bytes(sli_model* m, double* weight_bytes, double* kv_bytes);
 /* ---------------------------------------------------------------- in-process tensor parallelism
- * The SURVEY.md §4 item-5 "fake communicator" (the reference drives one device, model.cpp:247-256):
+ * A "fake communicator" (the reference drives one device, model.cpp:247-256):
  * tp_size rank models of cfg (cfg->tp_rank is ignored; rank r gets the sli_tp_plan shard of rank r)
  * on cfg->device, sharing one stream and stepped in lockstep by one captured hipGraph. Every all-reduce
  * of the multi-GPU step (the residual-stream sum after wo and down, the argmax-key MAX after the LM
@@ -363,7 +367,7 @@ int sli_model_time_gemv(sli_model* m, int32_t iters, double* avg_us, double* byt
 int sli_model_time_steps(sli_model* m, int32_t iters, double* avg_us);
 /* Per-kernel-family probe: for each family f (sli_kernel_family) replays that family's launches of one
  * step `iters` times between HIP events on the model's stream; us[f] = mean device time per launch,
- * bytes[f] = algorithmic HBM bytes per launch (SURVEY.md §8(d): the weight matrix (+ int8 row scales),
+ * bytes[f] = algorithmic HBM bytes per launch (the weight matrix (+ int8 row scales),
  * or K and V of the live context for attention), launches[f] = launches per step. Arrays of
  * SLI_FAM_COUNT. */
 typedef enum { SLI_FAM_QKV = 0, SLI_FAM_ATTN, SLI_FAM_WO, SLI_FAM_GU, SLI_FAM_DOWN, SLI_FAM_LM, SLI_FAM_COUNT } sli_kernel_family;
@@ -371,7 +375,7 @@ int sli_model_time_families(sli_model* m, int32_t iters, double* us, double* byt
 /* The measured streaming-read floor of the same launches: for each family, a pure read kernel (no
  * arithmetic, 16-byte non-temporal loads, one 1024-thread workgroup per CU) over exactly the buffers that
  * family's launches stream (each layer's weight matrix; K and V of the layer for attention, the
- * allocated context), replayed the same way; us[f] = mean device µs per launch (SURVEY §8(d): the
+ * allocated context), replayed the same way; us[f] = mean device µs per launch (the
  * fraction of a measured stream-copy bandwidth). */
 int sli_model_time_stream(sli_model* m, int32_t iters, double* us);
 /* Test hook (no device needed): runs the bounded-wait policy of comm_wait.h against mocked probes. mode 0: a

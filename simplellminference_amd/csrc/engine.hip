@@ -2,7 +2,7 @@
 // (source/model/model.cpp:40-140) and decode loop (:142-187) as a fused, graph-captured HIP step,
 // sharded Megatron-style over tp_size ranks (one process per GPU) with RCCL all-reduces.
 //
-// Per layer, five streaming launches replace the reference's ~18 (SURVEY.md §3.3):
+// Per layer, five streaming launches replace the reference's ~18:
 //   1. RMSNorm ⊕ [wq;wk;wv] GEMV ⊕ RoPE ⊕ K/V cache write        (model.cpp:52-67)
 //   2. attention partials (split context)   3. combine           (model.cpp:70-78)
 //   4. wo GEMV ⊕ residual add  [+ all-reduce under TP]           (model.cpp:80-90)
@@ -139,7 +139,7 @@ struct sli_model {
     } tl;
 };
 
-// In-process tensor parallelism (the "fake communicator"): tp_size rank models on
+// In-process tensor parallelism (a "fake communicator"): tp_size rank models on
 // one device share one stream and one captured graph that steps them in lockstep; every all-reduce is a
 // device-side reduction over the ranks' buffers in rank order (the ranks' kernels are the multi-GPU
 // ones, so the sharded engine itself is what the group tests run).
@@ -485,7 +485,7 @@ constexpr int kDeferBatched = 2;
 
 // ---------------------------------------------------------------- the layer stack as one persistent launch
 // (SLI_EXEC_PERSIST, tp_layers.h). Taken for batch-1 fp16 models at head_dim 128 whose per-workgroup shares fit the
-// kernel's LDS partial buffer: the TP-4 / TP-8 shards of Llama-2-7B (C2), not the unsharded 7B.
+// kernel's LDS partial buffer: the TP-4 / TP-8 shards of Llama-2-7B, not the unsharded 7B.
 static int tpl_nwg() { return gemv_max_blocks(); }
 
 static int tpl_check(const sli_model* m, std::string* why) {
@@ -1656,7 +1656,7 @@ static int create_model(const sli_model_config* cfg, const void* comm_id, sli_tp
     if (B > 1 && (rc = SLI_DISPATCH(m, prepare, m)) != SLI_OK) return bail(rc);
     if ((rc = sli_model_reset(m)) != SLI_OK) return bail(rc);
 
-    // Debug switches (tests only, DESIGN.md §6): SLI_DEBUG_FORCE_COMM=1 runs the tensor-parallel step
+    // Debug switches (tests only): SLI_DEBUG_FORCE_COMM=1 runs the tensor-parallel step
     // (partials + RCCL all-reduces) on a 1-rank communicator; SLI_DEBUG_NOCOMM=1 builds a tp_size>1
     // shard without a communicator (weight-placement checks; its logits are not meaningful).
     const bool force_comm = !group && c.tp_size == 1 && std::getenv("SLI_DEBUG_FORCE_COMM") != nullptr;
@@ -1980,7 +1980,8 @@ static std::vector<PfState> pf_batch_chunks(const sli_model* m, int n) {
 // Positions of a batch's prompts that sli_model_predict_batch runs as chunks before its steps (0: all of them as steps):
 // what every prompt has and the steps need not produce. A chunk costs two or three steps whatever it holds, so short
 // prompts stay with the steps; so do single sequences with fp16 or int8 weights, whose step keeps activations in fp32
-// where a chunk splits them in two fp16 terms (fp32 weights multiply fp32 activations in both).
+// where a chunk splits them in two fp16 terms. Fp32 weights multiply fp32 activations in both and attend in fp32 in both; the
+// rows of a batch are two fp16 terms to the projections and three to the attention in both.
 static int pf_predict_positions(const sli_model* m, const int32_t* lens, int max_length) {
     if (m->partial || (m->B == 1 && m->c.w_dtype != SLI_DT_F32) || !pf_supported(m)) return 0;
     const int n = std::min(*std::min_element(lens, lens + m->B), max_length) - 1;
@@ -2221,7 +2222,7 @@ int sli_model_get_history(sli_model* m, int32_t seq, int32_t n, int32_t* out) {
 int sli_model_set_exec(sli_model* m, int32_t mode) {
     SLI_CHECK(m, SLI_ERR_ARG, "null model");
     SLI_CHECK(mode == SLI_EXEC_LAUNCHES || mode == SLI_EXEC_PERSIST, SLI_ERR_ARG,
-              "unknown execution mode (the persistent one-launch step, mode 1, was removed in round 5: DESIGN.md §9)");
+              "unknown execution mode (the persistent one-launch step, mode 1, is gone)");
     if (mode == SLI_EXEC_PERSIST) {
         std::string why;
         SLI_CHECK(tpl_check(m, &why), SLI_ERR_STATE, "persistent layers: " + why);

@@ -48,7 +48,7 @@ __device__ __forceinline__ void store2(__half* p, const float* v) {
 // OT: element type of the feed-forward product in the output projection's input.
 template <typename KT, typename OT>
 struct HyIn {
-    static constexpr bool kRolled = true;  // (prefill.h; 1024 rows, 34304 x 4096: 497 us with the tiles indexed in scratch, 404 for 1152 rows now)
+    static constexpr bool kRolled = true;  // (prefill.h; 34304 x 4096: 497 us for 1024 rows with the tiles indexed in scratch, 391 for 1152 so)
     int retention;
     int H, G, dim, vdim, hpq, hpv;   // hpq / hpv: pairs per q,k / v,g head
     int e_q, e_k, e_v, e_g, u1p, ff;  // pair ranges

@@ -23,8 +23,8 @@ __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + expf
 
 // ---------------------------------------------------------------- epilogues
 // Row sections start at multiples of 4 rows, so four consecutive rows never straddle two of them.
-struct SeqIn {
-    static constexpr bool kRolled = true;  // (prefill.h)  // [q | latent | gate ; residual gate]
+struct SeqIn {  // [q | latent | gate ; residual gate]
+    static constexpr bool kRolled = true;  // (prefill.h PgRolled)
     int Hq, dim, hq_ld;       // query rows; values and stride of a head in q
     int r_kv, R, Rp, r_g, Hv, r_rg, D, ld;
     float *q, *lat, *gate, *rg;

@@ -10,20 +10,21 @@
 //      is read from HBM once per BM positions (the decode step reads it once per position). Operands are staged
 //      through an S-deep LDS ring by LDS-DMA (global_load_lds_dwordx4: one 1-KiB fragment image per
 //      wave-instruction, read back conflict-free by ds_read_b128), S - 1 stages in flight behind a counted
-//      vmcnt and a raw s_barrier (cdna_hip_programming.md §5 "Pipelining across barriers"), or the weight images
+//      vmcnt and a raw s_barrier, or the weight images
 //      in a deeper ring of their own (PgCfg::SA); the fragment reads of the next k-block are issued ahead of the
 //      current k-block's MFMAs. Fused epilogues:
 //      RoPE + K/V cache rows + q (model.cpp:52-67), residual add (:86-90, :124-128), SwiGLU (:111-115,
 //      written straight as the down projection's hi/lo operand);
 //   3. pf_flash_kernel (fp16 KV): block-causal attention against the cache rows 0 .. position (mha_kernel.cpp:36-77
-//      per query: s_t = q.k_t * scale, softmax, sum p_t v_t): S = K q^T on MFMA with q split hi/lo, online softmax in
-//      fp32, P V on MFMA with V read transposed (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the
+//      per query: s_t = q.k_t * scale, softmax, sum p_t v_t): S = K q^T on MFMA with q in two fp16 terms (batches:
+//      three), online softmax in fp32, P V on MFMA with V read transposed (ds_read_b64_tr_b16) from LDS-DMA'd K/V tiles; pf_attn_kernel, the
 //      VALU form (fp32, 64-position query blocks, K/V tiles of 64 positions in LDS), serves fp32 KV caches and fp32 weights.
 // fp32 weights: the same GEMM on v_mfma_f32_16x16x4_f32 with fp32 activations (one image, stages of 32 k).
 // int8 weights: stages of 128 k; a depth that is 64 mod 128 (e.g. Llama-2-7B int8 down at TP 4, 2752) ends with
 // a half stage (pgemm_kernel).
-// The launches of a chunk go to the stream one by one (its start position and valid count are kernel arguments): each
-// runs longer than it takes to enqueue, so a captured graph would only add its capture to a model's first prompt.
+// The launches of a chunk go to the stream one by one (its start position and valid count are kernel arguments): at the
+// widths of a 7B model each runs longer than it takes to enqueue, and a captured graph would add its capture to a model's
+// first prompt.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -33,8 +34,9 @@
 
 namespace sli {
 
-// Prompt positions per weight pass. The activations of a chunk (at 4096 rows of a 7B model 0.6 GB) are small beside the
-// weights, and every chunk pays a partial last round of tiles per GEMM (pg_plan) and reads the weights once.
+// Prompt positions per weight pass. The activations of a chunk (at 4096 rows of a 7B model 0.4 GB) are small beside the
+// weights, and every chunk pays a partial last round of tiles per GEMM (pg_plan) and reads the weights once. Where that does
+// not fit beside the model, chunks are smaller (engine.hip pf_ready).
 constexpr int kPfMaxChunk = 4096;
 constexpr int kPgGroup = 8;        // position blocks that an XCD takes through its row blocks together
 

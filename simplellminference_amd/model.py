@@ -1,7 +1,7 @@
 """``LlamaModel`` — Python mirror of the reference's model::LlamaModel (include/model/model.h:59-89)
 over the fused, graph-captured HIP decode step of libsli.so (engine.hip).
 
-Differences from the reference, all deliberate and documented in DESIGN.md:
+Differences from the reference, all deliberate:
   * the model shape is a runtime ``LlamaModelConfig`` (the reference hard-codes config.h:5-17 and
     copies it back in read_model_file, model.cpp:219-230);
   * ``predict`` takes token ids, or text when a ``tokenizer_path`` is given (``encode.SPELayer`` over the Python
@@ -38,7 +38,7 @@ class LlamaModelConfig:
 
 
 PRESETS = {
-    # BASELINE.json configs[0]: tiny-llama shape (2 layers, d=256, 4 heads), greedy 32 tokens
+    # tiny-llama shape (2 layers, d=256, 4 heads), greedy 32 tokens
     "tiny": LlamaModelConfig(512, 64, 256, 256, 768, 64, 2, 4, 4, 1e-5, 10000.0),
     "tiny-gqa": LlamaModelConfig(512, 64, 256, 128, 768, 64, 2, 4, 2, 1e-5, 10000.0),
     # tiny shapes wide enough for tensor parallelism over 8 ranks (heads and kv heads divisible by 8)
@@ -47,9 +47,9 @@ PRESETS = {
     # small head_dim-128 shapes for the persistent layer stack (tp_layers.h: head_dim 128, per-CU shares that fit)
     "small-h128": LlamaModelConfig(1000, 128, 1024, 1024, 2816, 512, 2, 8, 8, 1e-5, 10000.0),
     "small-h128-gqa": LlamaModelConfig(1000, 128, 1024, 512, 2816, 512, 2, 8, 4, 1e-5, 10000.0),
-    # configs[1..3]: Llama-2 7B (public model card shape), ctx 2048
+    # Llama-2 7B (public model card shape), ctx 2048
     "llama2-7b": LlamaModelConfig(32000, 128, 4096, 4096, 11008, 2048, 32, 32, 32, 1e-5, 10000.0),
-    # configs[4]: Llama-3 8B (GQA), ctx 4096
+    # Llama-3 8B (GQA), ctx 4096
     "llama3-8b": LlamaModelConfig(128256, 128, 4096, 1024, 14336, 4096, 32, 32, 8, 1e-5, 500000.0),
     # the reference's own hard-coded default (config.h:5-17, Llama-3.2-3B shape)
     "reference-default": LlamaModelConfig(),
@@ -370,7 +370,7 @@ def comm_id() -> bytes:
 
 
 class TPGroup:
-    """In-process tensor parallelism (sli_tp_group; SURVEY.md §4 item 5): ``tp_size`` rank engines on one
+    """In-process tensor parallelism (sli_tp_group): ``tp_size`` rank engines on one
     device, stepped in lockstep by one graph whose all-reduces are device-side reductions over the ranks'
     buffers. ``ranks[r]`` is a borrowed ``LlamaModel`` of rank r (weights, state, logits shard)."""
 

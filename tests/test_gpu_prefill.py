@@ -1,4 +1,4 @@
-"""Prompt prefill (sli_model_prefill; SURVEY.md §8(f)2): the prompt's positions 0..n-2 run through the
+"""Prompt prefill (sli_model_prefill): the prompt's positions 0..n-2 run through the
 layers in chunks of up to 4096 positions — every projection one MFMA GEMM over the chunk, attention
 block-causal over the cache — then decoding continues from the last prompt token. The reference
 teacher-forces the prompt one token per forward (model.cpp:157-165); the oracle's predict does the same, so
