@@ -11,8 +11,8 @@
 //      through an S-deep LDS ring by LDS-DMA (global_load_lds_dwordx4: one 1-KiB fragment image per
 //      wave-instruction, read back conflict-free by ds_read_b128), S - 1 stages in flight behind a counted
 //      vmcnt and a raw s_barrier, or the weight images
-//      in a deeper ring of their own (PgCfg::SA); the fragment reads of the next k-block are issued ahead of the
-//      current k-block's MFMAs. Fused epilogues:
+//      in a deeper ring of their own (PgCfg::SA); the fragment reads of the next k-block and the next stage's DMA are
+//      spread between the current k-block's MFMAs. Fused epilogues:
 //      RoPE + K/V cache rows + q (model.cpp:52-67), residual add (:86-90, :124-128), SwiGLU (:111-115,
 //      written straight as the down projection's hi/lo operand);
 //   3. pf_flash_kernel (fp16 KV): block-causal attention against the cache rows 0 .. position (mha_kernel.cpp:36-77
@@ -28,6 +28,7 @@
 #pragma once
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "step_state.h"
@@ -155,16 +156,13 @@ static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* 
 // LDS-DMA of one 1-KiB fragment image: lane i's 16 bytes at gsrc land at LDS byte lds + 16 i (inline asm: the
 // compiler neither counts nor drains it; the kernel counts its own vmcnt).
 __device__ __forceinline__ void pf_dma(const void* gsrc, unsigned lds) {
-    unsigned keep;
     asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
+        "s_mov_b32 m0, %1\n\t"
         "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep)
+        "global_load_lds_dwordx4 %0, off"
+        :
         : "v"(gsrc), "s"(lds)
-        : "memory");
+        : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void pf_wait_vm() {
@@ -209,9 +207,8 @@ struct PgIn {
 // Epilogue contract: row(t, i) = weight row of 16-row tile t's row i (i < 16, always valid); store(t, i0, m, v)
 // gets the fp32 sums of tile rows i0 .. i0+3 (i0 % 4 == 0) for chunk row m.
 // AT_: 16-row weight tiles per wave (2: a wave's 32 rows; 4: 64 rows, so every B fragment read from LDS feeds twice
-// the MFMAs). The fragment reads of k-block j + 1 are issued before the MFMAs of k-block j (two register sets),
-// across the stage barrier too, and every hi MFMA of a k-block goes ahead of its lo MFMAs (no back-to-back MFMAs on one
-// accumulator).
+// the MFMAs). The fragment reads of k-block j + 1 run beside the MFMAs of k-block j (two register sets), across the stage
+// barrier too.
 // SA_ > 0: the weight (A) images get a ring of their own, SA_ stages deep (SA_ - 1 issued ahead), and
 // the activation (B) images a 2-stage ring (one ahead): the A bytes come from HBM (read once per chunk), the B bytes
 // from L2, so only A needs the deep prefetch, and B, the larger image, does not pay for it in LDS.
@@ -299,6 +296,17 @@ __device__ __forceinline__ void pg_wait_stages(int later) {
     }
 }
 
+// f(std::integral_constant<int, 0>{}) .. f(<N - 1>): indices that are constants whatever the unroller makes of a loop
+template <int N, class F, int... I>
+__device__ __forceinline__ void pg_for_seq(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void pg_for(F&& f) {
+    pg_for_seq<N>(f, std::make_integer_sequence<int, N>{});
+}
+#define PG_INLINE __attribute__((always_inline))
+
 // Epilogues with a member kRolled = true are looped over a wave's tiles instead of unrolled
 template <class Epi, class = void>
 struct PgRolled : std::false_type {};
@@ -375,7 +383,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             if constexpr (HALF) adv[j] = Geo::B_ROW, back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
         }
     }
-    auto piece = [&](int j, unsigned dst, bool tail) {
+    auto piece = [&](int j, unsigned dst, bool tail) PG_INLINE {
         if constexpr (HALF) {
             pf_dma(src[j] - (tail ? back[j] : 0), dst);
             src[j] += adv[j];
@@ -384,26 +392,23 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             src[j] += Geo::A_ROW;
         }
     };
-    auto issue = [&](int s) {
-        const unsigned dst = ring + (unsigned)((s % S) * Geo::STAGE);
-        const bool tail = half_tail && s == ns - 1;
-#pragma unroll
-        for (int j = 0; j < Geo::DPW; ++j) piece(j, dst + (unsigned)((wave * Geo::DPW + j) * 1024), tail);
-    };
-
-    // split rings: A stage s in slot s % SA at ring, B stage s in slot s % 2 behind the A ring
+    // One ring: stage s in slot s % S. Split rings: A stage s in slot s % SA at ring, B stage s in slot s % 2 behind the A ring.
     const unsigned ring_b = ring + (unsigned)(Geo::SA * Geo::A_BYTES);
-    auto issue_a = [&](int s) {
-        const unsigned dst = ring + (unsigned)((s % (Geo::SA ? Geo::SA : 1)) * Geo::A_BYTES);
-        const bool tail = half_tail && s == ns - 1;
-#pragma unroll
-        for (int j = 0; j < Geo::DPA; ++j) piece(j, dst + (unsigned)((wave * Geo::DPA + j) * 1024), tail);
-    };
-    auto issue_b = [&](int s) {
-        const unsigned dst = ring_b + (unsigned)((s & 1) * Geo::B_BYTES);
-        const bool tail = half_tail && s == ns - 1;
-#pragma unroll
-        for (int j = 0; j < Geo::DPB; ++j) piece(Geo::DPA + j, dst + (unsigned)((wave * Geo::DPB + j) * 1024), tail);
+    // piece j of what iteration s issues: stage s + S - 1, or A stage s + SA - 1 (j < DPA) and B stage s + 1. Issue order:
+    // B pieces first (j counts from them).
+    constexpr int SAN = Geo::SA ? Geo::SA : 1;
+    auto dma = [&](int j, int s) PG_INLINE {
+        if constexpr (Geo::SA == 0) {
+            const int t = s + S - 1;
+            piece(j, ring + (unsigned)((t % S) * Geo::STAGE + (wave * Geo::DPW + j) * 1024), half_tail && t == ns - 1);
+        } else if (j < Geo::DPB) {
+            const int t = s + 1;
+            piece(Geo::DPA + j, ring_b + (unsigned)((t & 1) * Geo::B_BYTES + (wave * Geo::DPB + j) * 1024), half_tail && t == ns - 1);
+        } else {
+            const int t = s + SAN - 1;
+            piece(j - Geo::DPB, ring + (unsigned)((t % SAN) * Geo::A_BYTES + (wave * Geo::DPA + j - Geo::DPB) * 1024),
+                  half_tail && t == ns - 1);
+        }
     };
     constexpr int AT = Geo::AT;
     pf_float4 acc[AT][Geo::WPT];
@@ -416,63 +421,90 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     const int kg = lane >> 4, r16 = lane & 15;
     const int sa = pg_swz(r16, Geo::A_ROW), sb = pg_swz(r16, Geo::B_ROW);
     if constexpr (Geo::SA == 0) {
-        for (int s = 0; s < S - 1 && s < ns; ++s) issue(s);
-    } else {  // the schedule of iterations -(SA - 1) .. -1: B(i + 1), then A(i + SA - 1)
-        for (int i = 1 - Geo::SA; i < 0; ++i) {
-            if (i + 1 >= 0 && i + 1 < ns) issue_b(i + 1);
-            if (i + Geo::SA - 1 >= 0 && i + Geo::SA - 1 < ns) issue_a(i + Geo::SA - 1);
-        }
-    }
-    // fragments of k-block kb of stage buffer st (A images at st, B images at stb) into (af, bh, bl)
-    auto read_frags = [&](const char* st, const char* stb, int kb, u32x4(&af)[AT], u32x4(&bh)[Geo::WPT],
-                          u32x4(&bl)[Geo::WPT]) {
 #pragma unroll
-        for (int a = 0; a < AT; ++a) {
-            const char* img = st + (wr * AT + a) * Geo::A_IMG + r16 * Geo::A_ROW;
-            if constexpr (sizeof(WT) != 1) {
-                af[a] = *reinterpret_cast<const u32x4*>(img + ((4 * kb + kg) ^ sa) * 16);
-            } else {
-                const int off = ((2 * kb + (kg >> 1)) ^ sa) * 16 + 8 * (kg & 1);
-                af[a] = pg_i8_to_f16(*reinterpret_cast<const uint2*>(img + off));
+        for (int i = 1 - S; i < 0; ++i)
+            if (i + S - 1 < ns) {
+#pragma unroll
+                for (int j = 0; j < Geo::DPW; ++j) dma(j, i);
+            }
+    } else {  // the schedule of iterations -(SA - 1) .. -1: B(i + 1), then A(i + SA - 1)
+#pragma unroll
+        for (int i = 1 - Geo::SA; i < 0; ++i) {
+            if (i + 1 >= 0 && i + 1 < ns) {
+#pragma unroll
+                for (int j = 0; j < Geo::DPB; ++j) dma(j, i);
+            }
+            if (i + Geo::SA - 1 < ns) {
+#pragma unroll
+                for (int j = Geo::DPB; j < Geo::DPW; ++j) dma(j, i);
             }
         }
-#pragma unroll
-        for (int b = 0; b < Geo::WPT; ++b) {
+    }
+    // Fragments of a k-block: AT of the weights, NB WPT of the activations
+    struct Frags {
+        u32x4 a[AT], b[Geo::WPT][Geo::NB];
+    };
+    // read r of k-block kb of stage buffer st (A images at st, B images at stb): the weights' first
+    auto read_frag = [&](int r, const char* st, const char* stb, int kb, Frags& f) PG_INLINE {
+        if (r < AT) {
+            const char* img = st + (wr * AT + r) * Geo::A_IMG + r16 * Geo::A_ROW;
+            if constexpr (sizeof(WT) != 1) {
+                f.a[r] = *reinterpret_cast<const u32x4*>(img + ((4 * kb + kg) ^ sa) * 16);
+            } else {
+                const int off = ((2 * kb + (kg >> 1)) ^ sa) * 16 + 8 * (kg & 1);
+                f.a[r] = pg_i8_to_f16(*reinterpret_cast<const uint2*>(img + off));
+            }
+        } else {
+            const int u = r - AT, b = u / Geo::NB, t = u % Geo::NB;
             const int pt = wp * Geo::WPT + b;
-            const char* img = stb + (Geo::NB * pt) * Geo::B_IMG + r16 * Geo::B_ROW + ((4 * kb + kg) ^ sb) * 16;
-            bh[b] = *reinterpret_cast<const u32x4*>(img);
-            if constexpr (Geo::NB == 2) bl[b] = *reinterpret_cast<const u32x4*>(img + Geo::B_IMG);
+            const char* img = stb + (Geo::NB * pt + t) * Geo::B_IMG + r16 * Geo::B_ROW + ((4 * kb + kg) ^ sb) * 16;
+            f.b[b][t] = *reinterpret_cast<const u32x4*>(img);
         }
     };
-    auto mfmas = [&](const u32x4(&af)[AT], const u32x4(&bh)[Geo::WPT], const u32x4(&bl)[Geo::WPT]) {
-        if constexpr (Geo::F32) {  // lane group kg holds k 4 kg .. +3 of the 16-k block: MFMA e takes k 4 kg + e of each
+    constexpr int NR = AT + Geo::NB * Geo::WPT;   // reads of a k-block
+    constexpr int NSL = Geo::NB * Geo::WPT;       // slices of a k-block: AT MFMAs each
+    auto slice_mfma = [&](int i, const Frags& f) PG_INLINE {
+        const int b = i / Geo::NB, t = i % Geo::NB;
+        if constexpr (Geo::F32) {
 #pragma unroll
-            for (int b = 0; b < Geo::WPT; ++b)
+            for (int a = 0; a < AT; ++a) {
+                pf_float4 p[4];
 #pragma unroll
-                for (int a = 0; a < AT; ++a) {
-                    pf_float4 p[4];
+                for (int e = 0; e < 4; ++e)
+                    p[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(f.a[a][e]), __uint_as_float(f.b[b][t][e]),
+                                                                pf_float4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                acc[a][b] += (p[0] + p[1]) + (p[2] + p[3]);
+            }
+        } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        p[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(af[a][e]), __uint_as_float(bh[b][e]),
-                                                                    pf_float4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    acc[a][b] += (p[0] + p[1]) + (p[2] + p[3]);
-                }
-            return;
+            for (int a = 0; a < AT; ++a) acc[a][b] = pf_mfma(f.a[a], f.b[b][t], acc[a][b]);
         }
-#pragma unroll
-        for (int b = 0; b < Geo::WPT; ++b)
-#pragma unroll
-            for (int a = 0; a < AT; ++a) acc[a][b] = pf_mfma(af[a], bh[b], acc[a][b]);
-        if constexpr (Geo::NB == 2) {
-#pragma unroll
-            for (int b = 0; b < Geo::WPT; ++b)
-#pragma unroll
-                for (int a = 0; a < AT; ++a) acc[a][b] = pf_mfma(af[a], bl[b], acc[a][b]);
-        }
+    };
+    // MFMAs of fragments f in slices of AT (one activation fragment each), between them the reads of the next k-block into n
+    // and DMA pieces j0 .. j1 - 1 of iteration s: a wave issues them in the 12 cycles that an MFMA holds the matrix pipe
+    // after its issue. The order is fixed (sched_barrier, every 4 MFMAs or more): left to itself the compiler gathered a
+    // set's reads behind the MFMAs they should run beside, each wait for LDS then stood open, and the 16 DMA pieces stood
+    // in front. 512 rows, 7B q/k/v | gate/up | wo | down: 109 | 207 | 45 | 96 -> 93 | 181 | 42 | 84 us; 2048 rows 413 | 754 |
+    // 130 | 373 -> 377 | 670 | 109 | 327 (1260 TFLOP/s). The clock then falls from 2.0 to 1.66 GHz (MFMAs on random data
+    // alone hold 1.74 PFLOP/s): more waves, s_setprio and 128-row wave tiles measured the same.
+    auto phase = [&](const Frags& f, Frags& n, const char* st, const char* stb, auto KB, auto J0, auto J1, int s) PG_INLINE {
+        constexpr int RS = NSL > 1 ? NSL - 1 : 1;  // slices with reads
+        constexpr int kb = decltype(KB)::value, j0 = decltype(J0)::value, j1 = decltype(J1)::value;
+        pg_for<NSL>([&](auto I) PG_INLINE {
+            constexpr int i = decltype(I)::value;
+            if constexpr (kb >= 0 && i < RS) {
+                constexpr int r0 = NR * i / RS, r1 = NR * (i + 1) / RS;
+                pg_for<r1 - r0>([&](auto R) PG_INLINE { read_frag(r0 + R, st, stb, kb, n); });
+            }
+            constexpr int d0 = j0 + (j1 - j0) * i / NSL, d1 = j0 + (j1 - j0) * (i + 1) / NSL;
+            slice_mfma(i, f);
+            pg_for<d1 - d0>([&](auto J) PG_INLINE { dma(d0 + J, s); });
+            if constexpr ((i + 1) % (AT < 4 ? 4 / AT : 1) == 0 || i == NSL - 1) __builtin_amdgcn_sched_barrier(0);
+        });
     };
     constexpr bool TWO = Geo::FOLD > 0;
     pf_float4 tot[TWO ? AT : 1][TWO ? Geo::WPT : 1] = {};
-    auto fold = [&](auto& to, auto& from) {
+    auto fold = [&](auto& to, auto& from) PG_INLINE {
 #pragma unroll
         for (int a = 0; a < AT; ++a)
 #pragma unroll
@@ -482,49 +514,95 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             }
     };
     const bool live = Cfg::GR || pb * BM + wp * Geo::WPT * 16 < in.valid;  // (wave-uniform)
-    {
-        // set X holds even k-blocks, set Y odd ones (KBS is even; an int8 half stage has KBS / 2 = 2): per stage
-        // read(0) -> X, MFMA(Y: the previous stage's last k-block), read(1) -> Y, MFMA(X), ... The stage barrier
-        // follows this wave's lgkmcnt(0), so the previous stage's buffer is free for the DMA issued after it while
-        // its last fragments wait in registers.
-        static_assert(KBS % 2 == 0, "k-blocks per stage");
-        u32x4 xa[AT], xh[Geo::WPT], xl[Geo::WPT], ya[AT], yh[Geo::WPT], yl[Geo::WPT];
+    // before iteration s: stage s landed, every wave is done with the buffers that iteration s issues into
+    auto stage_begin = [&](int s) {
+        if constexpr (Geo::SA == 0) {
+            pg_wait_stages<Geo::DPW>(min(S - 2, ns - 1 - s));
+        } else {
+            // B(s) was the first load of iteration s - 1; only that iteration's A pieces (if it issued any) were
+            // issued after it, and A(s) before it
+            if (s + Geo::SA - 2 < ns)
+                pf_wait_vm<Geo::DPA>();
+            else
+                pf_wait_vm<0>();
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+    // pieces that iteration s issues
+    auto pieces = [&](int s) {
+        if constexpr (Geo::SA == 0)
+            return s + S - 1 < ns ? Geo::DPW : 0;
+        else
+            return s + Geo::SA - 1 < ns ? Geo::DPW : s + 1 < ns ? Geo::DPB : 0;
+    };
+    auto bufs = [&](int s, const char*& st, const char*& stb) {
+        if constexpr (Geo::SA == 0) {
+            st = pg_smem + (size_t)(s % S) * Geo::STAGE;
+            stb = st + Geo::A_BYTES;
+        } else {
+            st = pg_smem + (size_t)(s % Geo::SA) * Geo::A_BYTES;
+            stb = pg_smem + (size_t)Geo::SA * Geo::A_BYTES + (size_t)(s & 1) * Geo::B_BYTES;
+        }
+    };
+    static_assert(KBS % 2 == 0, "k-blocks per stage");
+    if (!live) {
         for (int s = 0; s < ns; ++s) {
-            const char *st, *stb;
-            if constexpr (Geo::SA == 0) {
-                pg_wait_stages<Geo::DPW>(min(S - 2, ns - 1 - s));
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_s_barrier();
-                if (s + S - 1 < ns) issue(s + S - 1);
-                st = pg_smem + (size_t)(s % S) * Geo::STAGE;
-                stb = st + Geo::A_BYTES;
-            } else {
-                // B(s) was the first load of iteration s - 1; only that iteration's A pieces (if it issued any) were
-                // issued after it, and A(s) before it
-                if (s + Geo::SA - 2 < ns)
-                    pf_wait_vm<Geo::DPA>();
-                else
-                    pf_wait_vm<0>();
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_s_barrier();
-                if (s + 1 < ns) issue_b(s + 1);
-                if (s + Geo::SA - 1 < ns) issue_a(s + Geo::SA - 1);
-                st = pg_smem + (size_t)(s % Geo::SA) * Geo::A_BYTES;
-                stb = pg_smem + (size_t)Geo::SA * Geo::A_BYTES + (size_t)(s & 1) * Geo::B_BYTES;
-            }
-            const int kbs = (half_tail && s == ns - 1) ? KBS / 2 : KBS;  // wave-uniform, even
+            stage_begin(s);
+            const int np = pieces(s);
 #pragma unroll
-            for (int kb = 0; kb < KBS; kb += 2) {
-                if (kb >= kbs || !live) break;
-                read_frags(st, stb, kb, xa, xh, xl);
-                if (s > 0 || kb > 0) mfmas(ya, yh, yl);
-                read_frags(st, stb, kb + 1, ya, yh, yl);
-                mfmas(xa, xh, xl);
+            for (int j = 0; j < Geo::DPW; ++j)
+                if (j < np) dma(j, s);
+        }
+    } else {
+        // Set X holds even k-blocks, set Y odd ones (an int8 half stage has KBS / 2 = 2): per stage MFMA(Y: the previous
+        // stage's last k-block) beside read(0) -> X, MFMA(X) beside read(1) -> Y, ... The stage barrier follows this wave's
+        // lgkmcnt(0), so the previous stage's buffer is free for the DMA issued after it while its last fragments wait in
+        // registers.
+        Frags X, Y;
+        // one iteration; P: pieces it issues
+        auto iter = [&](int s, auto P, auto first) PG_INLINE {
+            constexpr int NP = decltype(P)::value;
+            constexpr bool FIRST = decltype(first)::value;
+            const char *st, *stb;
+            stage_begin(s);
+            bufs(s, st, stb);
+            constexpr std::integral_constant<int, 0> q0;
+            constexpr std::integral_constant<int, NP / KBS> q1;
+            constexpr std::integral_constant<int, 2 * NP / KBS> q2;
+            if constexpr (FIRST) {
+                pg_for<NR>([&](auto R) PG_INLINE { read_frag(R, st, stb, 0, X); });
+                pg_for<q1>([&](auto J) PG_INLINE { dma(J, s); });
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                phase(Y, X, st, stb, q0, q0, q1, s);
+            }
+            phase(X, Y, st, stb, std::integral_constant<int, 1>{}, q1, q2, s);
+            if constexpr (KBS == 4) {
+                constexpr std::integral_constant<int, 3 * NP / KBS> q3;
+                if (NP > 0 || !(half_tail && s == ns - 1)) {
+                    phase(Y, X, st, stb, std::integral_constant<int, 2>{}, q2, q3, s);
+                    phase(X, Y, st, stb, std::integral_constant<int, 3>{}, q3, std::integral_constant<int, NP>{}, s);
+                }
             }
             if constexpr (TWO)
                 if (s % (Geo::FOLD / Geo::KS) == Geo::FOLD / Geo::KS - 1) fold(tot, acc);
-        }
-        if (live) mfmas(ya, yh, yl);
+        };
+        constexpr std::integral_constant<int, Geo::DPW> full;
+        constexpr std::integral_constant<int, Geo::SA ? Geo::DPB : 0> part;
+        constexpr std::integral_constant<int, 0> none;
+        constexpr int AHEAD = Geo::SA ? Geo::SA - 1 : S - 1;
+        constexpr std::true_type yes;
+        constexpr std::false_type no;
+        int s = 0;
+        if (AHEAD < ns) iter(s++, full, yes);
+        else if (part.value && 1 < ns) iter(s++, part, yes);
+        else iter(s++, none, yes);
+        for (; s + AHEAD < ns; ++s) iter(s, full, no);
+        if constexpr (part.value > 0)
+            for (; s + 1 < ns; ++s) iter(s, part, no);
+        for (; s < ns; ++s) iter(s, none, no);
+        phase(Y, X, nullptr, nullptr, std::integral_constant<int, -1>{}, none, none, 0);
         if constexpr (TWO) fold(acc, tot);
     }
     if (nsp > 1) {
