@@ -334,8 +334,10 @@ __device__ __forceinline__ bool attn_publish(const AttnArgs<KT>& a, int kvh, int
         }
         return false;
     }
-    // Workgroup partial: the WAVES slice states merged in LDS, published write-through (sc1) so the
-    // head's last-arriving workgroup can read it from any XCD without a fence pair
+    const int ns = min(pos / (WAVES * PPW) + 1, a.max_splits);  // live workgroups of this kv head
+    // Workgroup partial: the WAVES slice states merged in LDS. The only live split of its head (a context up to PPWG) is the
+    // head's output: the merge's weight is e^0, so o / L is what attn_merge would store, without the drain, the arrival and
+    // the read back (32 fp32 heads of 128 at 75 to 95 positions: 10.2 -> 7.2 us). Otherwise published write-through (sc1) so the head's last-arriving workgroup can read it from any XCD without a fence pair
     // (MI355X_MICROARCH.md, hand-off table row 1: sc1 stores, drained, one agent-scope add per
     // workgroup behind a workgroup barrier, sc1 loads by the last adder after the barrier it joins).
     for (int i = threadIdx.x; i < G * HD; i += 64 * WAVES) {
@@ -350,6 +352,10 @@ __device__ __forceinline__ bool attn_publish(const AttnArgs<KT>& a, int kvh, int
             o = fmaf(c, sh[w][g][d], o);
             L = fmaf(c, sh[w][g][HD + 1], L);
         }
+        if (ns == 1) {
+            __hip_atomic_store(a.out + (size_t)(kvh * G + g) * HD + d, o / L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            continue;
+        }
         float* dst = a.part + ((size_t)(kvh * G + g) * a.max_splits + wgs) * (HD + kAttnPartPad);
         __hip_atomic_store(dst + d, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (d == 0) {
@@ -357,9 +363,9 @@ __device__ __forceinline__ bool attn_publish(const AttnArgs<KT>& a, int kvh, int
             __hip_atomic_store(dst + HD + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+    if (ns == 1) return false;  // uniform
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains before the arrival
     __syncthreads();
-    const int ns = min(pos / (WAVES * PPW) + 1, a.max_splits);  // live workgroups of this kv head
     if (threadIdx.x == 0) {
         const unsigned prev = __hip_atomic_fetch_add(a.counters + kvh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last = prev == (unsigned)(ns - 1);

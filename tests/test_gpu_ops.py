@@ -182,6 +182,13 @@ def test_mha(gpu, oracle, kv_dtype, T, hd, H, Hkv, layer, pos):
     _close(got.cpu().numpy(), want, rtol=1e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("hd,pos", [(128, 0), (128, 126), (128, 127), (128, 128), (64, 254), (64, 255), (64, 256)])
+@pytest.mark.parametrize("H,Hkv", [(2, 2), (4, 2), (8, 2), (8, 1)])
+def test_mha_one_context_split(gpu, oracle, hd, pos, H, Hkv):
+    """Around the positions of one workgroup (fp32: 128 of head_dim 128, 256 of 64): the only split is the output."""
+    test_mha(gpu, oracle, "f32", 300, hd, H, Hkv, 1, pos)
+
+
 def test_swiglu_add(gpu, oracle):
     torch = gpu
     from simplellminference_amd import ops
