@@ -46,12 +46,17 @@ constexpr int bg_step_width(int tpw) { return tpw == 1 ? 2 : 4; }
 // A plan whose waves own 6 or 7 k-blocks of every tile (C4 down: K 14336 over 4 splits, 7; the prefill's
 // Llama-2 down: K 11008 over 4 splits, 6) streams each tile as ONE 7-vector step instead of 4 + 3 / 4 + 2
 // (clamped duplicates in the second step): C4 down 31.6 -> 29.4 us, 512-token prefill +1.5 %.
+// 5 k-blocks likewise as one 5-vector step (a block stack's 2048 x 10240 at 6 rows, 4 splits of 2 tiles with both in flight:
+// 18.6 -> 14.6 us; as 4 + 1 the plan was 5 splits of 3 tiles).
 #ifndef SLI_BG_U7_FROM
 #define SLI_BG_U7_FROM 6
 #endif
-inline bool bg_seven_blocks(int splits, int K) {
-    const int bpw = ((((K >> 5) + splits - 1) / splits) + kBgWaves - 1) / kBgWaves;
-    return bpw >= SLI_BG_U7_FROM && bpw <= 7;
+inline int bg_wave_blocks(int splits, int K) { return ((((K >> 5) + splits - 1) / splits) + kBgWaves - 1) / kBgWaves; }
+// The step of a plan without the fused RMS
+inline int bg_width(int splits, int K, int tpw) {
+    const int bpw = bg_wave_blocks(splits, K);
+    if (tpw == 1) return bg_step_width(tpw);
+    return bpw >= SLI_BG_U7_FROM && bpw <= 7 ? 7 : bpw == 5 ? 5 : bg_step_width(tpw);
 }
 
 struct BgIn {
@@ -110,7 +115,7 @@ inline BgPlan bg_plan(int ntiles, int K, int B, bool norm, int cus = 256, bool s
             const int rounds = (wgs + cus - 1) / cus;
             int blocks = kbs;
             if (steps) {
-                const int bpw = (kbs + kBgWaves - 1) / kBgWaves, w = bg_seven_blocks(s, K) ? 7 : bg_step_width(tpw);
+                const int bpw = bg_wave_blocks(s, K), w = bg_width(s, K, tpw);
                 blocks = kBgWaves * w * ((bpw + w - 1) / w);
             }
             double per_wg = (double)tpw * blocks + 0.25 * kbs * B / 8.0 + 40.0;
@@ -414,10 +419,17 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
             const int j = it >> 6, i = (it >> 3) & 7, b = it & 7;
             if (b >= B) continue;
             float v0 = 0.0f, v1 = 0.0f;
-            for (int sp = 0; sp < S; ++sp) {  // split order: deterministic
-                const unsigned o = (unsigned)((j * S + sp) * 128);
-                v0 += bg_load_sc1(base, bytes, 4u * (o + i * 8 + b));
-                v1 += bg_load_sc1(base, bytes, 4u * (o + (i + 8) * 8 + b));
+            for (int s0 = 0; s0 < S; s0 += 8) {  // split order: deterministic; 8 splits' loads in flight (that launch 19.6 -> 18.6 us)
+                float p0[8], p1[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const unsigned o = (unsigned)((j * S + min(s0 + u, S - 1)) * 128);
+                    p0[u] = bg_load_sc1(base, bytes, 4u * (o + i * 8 + b));
+                    p1[u] = bg_load_sc1(base, bytes, 4u * (o + (i + 8) * 8 + b));
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (s0 + u < S) v0 += p0[u], v1 += p1[u];
             }
             epi.store(t0 + j, i, b, v0, v1, keys);
         }
@@ -602,9 +614,11 @@ hipError_t bg_allow_lds() {
         const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&bgemm_kernel<Epi, NORM, 2>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kBgLdsMax);
         if (!NORM) {
+            const hipError_t e5 = hipFuncSetAttribute(reinterpret_cast<const void*>(&bgemm_kernel<Epi, NORM, 5>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kBgLdsMax);
             const hipError_t e7 = hipFuncSetAttribute(reinterpret_cast<const void*>(&bgemm_kernel<Epi, NORM, 7>),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBgLdsMax);
-            if (e7 != hipSuccess) return e7;
+            if (e5 != hipSuccess || e7 != hipSuccess) return e5 != hipSuccess ? e5 : e7;
         }
         return e4 != hipSuccess ? e4 : e2;
     }();
@@ -619,14 +633,16 @@ hipError_t launch_bgemm(const __half* W, const BgIn& in_, const Epi& epi, const 
     in.splits = p.splits;
     const dim3 grid(p.groups * p.splits);
     if (in.norm_w && p.splits != 1) return hipErrorInvalidValue;  // the fused RMS runs on one split only
-    const bool u2 = bg_step_width(p.tpw) == 2;
-    if (in.norm_w && u2)
+    const int u = in.norm_w ? bg_step_width(p.tpw) : bg_width(p.splits, in.K, p.tpw);
+    if (in.norm_w && u == 2)
         hipLaunchKernelGGL((bgemm_kernel<Epi, true, 2>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);
     else if (in.norm_w)
         hipLaunchKernelGGL((bgemm_kernel<Epi, true, 4>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);
-    else if (u2)
+    else if (u == 2)
         hipLaunchKernelGGL((bgemm_kernel<Epi, false, 2>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);
-    else if (bg_seven_blocks(p.splits, in.K))
+    else if (u == 5)
+        hipLaunchKernelGGL((bgemm_kernel<Epi, false, 5>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);
+    else if (u == 7)
         hipLaunchKernelGGL((bgemm_kernel<Epi, false, 7>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);
     else
         hipLaunchKernelGGL((bgemm_kernel<Epi, false, 4>), grid, dim3(kBgThreads), p.lds, s, W, in, epi);

@@ -53,6 +53,14 @@ def test_matmul_batch_exact_integers(gpu, rows, cols, batch):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("rows,cols,batch", [(8200, 2080, 8), (8200, 2560, 5), (8200, 2592, 3),
+                                             (16, 16384, 8), (48, 9216, 6), (64, 4640, 1)])
+def test_matmul_batch_steps_of_five_and_many_splits(gpu, rows, cols, batch):
+    """A wave's 5 k-blocks of a tile as one step (and the 6 beside them), and merges of more splits than one round of loads
+    holds. Small integers: sums are exact in any order."""
+    test_matmul_batch_exact_integers(gpu, rows, cols, batch)
+
+
 @pytest.mark.parametrize("name", ["tiny", "tiny-gqa"])
 @pytest.mark.parametrize("kv", ["f16", "f32"])
 def test_batch_predict_parity(gpu, oracle, name, kv):
