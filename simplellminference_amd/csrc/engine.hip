@@ -615,6 +615,11 @@ constexpr int kPfPad = 128;
 template <typename WT, typename KT>
 struct StepRecorder {
     static constexpr bool NT = true;  // streamed-once weights: non-temporal loads
+    // Vectors per lane and step of the one-row wo GEMV: a fp32 row has twice a fp16 row's vectors, and two steps of 8 keep
+    // 16 KiB of a wave in flight, a whole row of 4096 (4096 x 4096: 15.7 -> 12.8 us against two of 2). The down GEMV's two
+    // steps of 6 hold 12 KiB already (8: 30.5 -> 30.9 us).
+    static constexpr bool F32 = std::is_same<WT, float>::value;
+    static constexpr int kUWo = F32 ? 8 : 2;
     static int gemv_qkv(sli_model* m, int l) {
         const LayerW& w = m->layers[l];
         GemvIn in{m->x, m->norms + (size_t)(2 * l) * m->D, m->c.eps, m->D};
@@ -662,11 +667,11 @@ struct StepRecorder {
         if (!m->wo_merge) {  // the attention merged its splits into attn: a plain input
             GemvIn in{m->attn, nullptr, 0.0f, m->hq * m->hd};
             if (fused_ar(m)) {
-                SLI_HIP((launch_gemv_u<WT, 1, 2, NT>((const WT*)w.wo, in, push_epi(m, w.wo_s, 0), m->D, m->stream)));
+                SLI_HIP((launch_gemv_u<WT, 1, kUWo, NT>((const WT*)w.wo, in, push_epi(m, w.wo_s, 0), m->D, m->stream)));
                 return SLI_OK;
             }
             EpiStore<1> e{tp ? m->xpart : m->x, (!tp || m->c.tp_rank == 0) ? m->x : nullptr, w.wo_s, 1.0f, m->D};
-            SLI_HIP((launch_gemv_u<WT, 1, 2, NT>((const WT*)w.wo, in, e, m->D, m->stream)));
+            SLI_HIP((launch_gemv_u<WT, 1, kUWo, NT>((const WT*)w.wo, in, e, m->D, m->stream)));
             return SLI_OK;
         }
         GemvIn in{m->attn, nullptr, 0.0f, m->hq * m->hd};

@@ -39,6 +39,20 @@ def test_tiny_predict_parity(gpu, oracle, name, w, kv, tol):
     gm.close()
 
 
+@pytest.mark.parametrize("heads", [5, 20, 32, 33])
+def test_fp32_output_projection_widths(gpu, oracle, heads):
+    """fp32 output projections of 640 to 4224 columns: under, at and past a step of 2048, split over the columns or not. The
+    bar is test_tiny_predict_parity's."""
+    D = 128 * heads
+    om, gm = _models(oracle, "small-h128-gqa", "f32", "f32", hidden_size=D, num_attention_heads=heads,
+                     num_key_value_heads=heads, kv_hidden_size=D, num_hidden_layers=1)
+    otok, olog = om.predict(PROMPT, 6)
+    gtok, glog = gm.predict(PROMPT, 6, want_logits=True)
+    assert np.array_equal(gtok, otok)
+    assert np.abs(glog - olog).max() <= 1e-4
+    gm.close()
+
+
 def test_forward_is_idempotent_and_matches_predict(gpu, oracle):
     om, gm = _models(oracle, "tiny-gqa", "f16", "f16")
     toks, logits = gm.predict(PROMPT, 12, want_logits=True)
