@@ -632,16 +632,39 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         for (int a = 0; a < AT; ++a)
 #pragma unroll
             for (int b = 0; b < Geo::WPT; ++b) acc[a][b] = pf_float4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int q = 0; q < nsp; ++q) {
-            const auto rs = __builtin_amdgcn_make_buffer_rsrc(tw + (size_t)q * TILE * 4, 0, bytes, 0x00020000);
+        // A split's partials come from memory: several splits' loads are in flight together (16 float4 of a thread), or the
+        // merge takes a round trip each. 45 tokens of an int8 7B prompt 1.013 -> 1.023 times as fast as one by one.
+        if constexpr (NV <= 16) {
+            constexpr int QB = 16 / NV;
+            const auto rs = __builtin_amdgcn_make_buffer_rsrc(tw, 0, bytes * nsp, 0x00020000);
+            for (int q0 = 0; q0 < nsp; q0 += QB) {
+                u32x4 p[QB][NV];
 #pragma unroll
-            for (int a = 0; a < AT; ++a) {
+                for (int i = 0; i < QB; ++i)
 #pragma unroll
-                for (int b = 0; b < Geo::WPT; ++b)
-                    acc[a][b] += __builtin_bit_cast(
-                        pf_float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                       rs, 16u * ((a * Geo::WPT + b) * Geo::THREADS + threadIdx.x), 0, 16));
-                asm volatile("" ::: "memory");  // (one tile row's loads in flight: more would spill at 256 columns)
+                    for (int j = 0; j < NV; ++j)
+                        p[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16u * threadIdx.x + 16u * Geo::THREADS * j,
+                                                                        bytes * min(q0 + i, nsp - 1), 16);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < QB; ++i)
+                    if (q0 + i < nsp) {
+#pragma unroll
+                        for (int j = 0; j < NV; ++j) acc[j / Geo::WPT][j % Geo::WPT] += __builtin_bit_cast(pf_float4, p[i][j]);
+                    }
+            }
+        } else {
+            for (int q = 0; q < nsp; ++q) {
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(tw + (size_t)q * TILE * 4, 0, bytes, 0x00020000);
+#pragma unroll
+                for (int a = 0; a < AT; ++a) {
+#pragma unroll
+                    for (int b = 0; b < Geo::WPT; ++b)
+                        acc[a][b] += __builtin_bit_cast(
+                            pf_float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rs, 16u * ((a * Geo::WPT + b) * Geo::THREADS + threadIdx.x), 0, 16));
+                    asm volatile("" ::: "memory");  // (one tile row's loads in flight: more would spill at 256 columns)
+                }
             }
         }
     }
