@@ -347,6 +347,15 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     constexpr bool HALF = sizeof(WT) == 1;
     const bool half_tail = HALF && (in.K % Geo::KS) != 0 && s0 + ns == nsk;
     const int nt = in.N >> 4;       // row tiles
+    // Row blocks start their walk of the depth at different stages, rot on, and wrap around: rows of fp16 weights lie 8 KiB
+    // and more apart, and workgroups that all walk from the same column reach less of the memory's rate (likely a few channels at a time). Where
+    // one row block's weights are read once (a chunk of one position block): with more, their activations no longer fit the
+    // L2 side by side (256 rows, gate/up 92.7 -> 94.7 us); up to two splits, more of them start apart already (down at 96
+    // rows 34.8 -> 38.9); 128 weight rows and more (tiles of 64, two on a CU, 28672 x 4096 at 32 rows 52.4 -> 60.1). 7B
+    // gate/up at 32 | 64 | 96 rows 45.5 | 50.0 | 53.4 -> 37.0 | 42.5 | 48.8 us, a stack's 34304 x 4096 at 128 82.9 -> 71.6.
+    // int8 rows are half as long and its walk is not bound by memory: 39.2 -> 39.1.
+    constexpr bool ROT = sizeof(WT) == 2 && !Cfg::GR && BM <= 128 && Geo::BN >= 128;
+    const int rot = ROT && PB == 1 && nsp <= 2 ? rb % ns : 0, wrap = ns - 1 - rot;  // stage t: (t + rot) % ns of the range
     const unsigned ring = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)pg_smem;
 
     // this wave's DMA instructions d in [wave*DPW, (wave+1)*DPW): stage bytes [1024 d, 1024 (d + 1)). Lane i
@@ -368,7 +377,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const int r = (off % Geo::A_IMG) / Geo::A_ROW + lane / 8;
             const int c = (lane % 8) ^ pg_swz(r, Geo::A_ROW);
             const int row = epi.row(min(t, nt - 1), r);
-            src[j] = reinterpret_cast<const char*>(in.W) + (size_t)row * in.K * sizeof(WT) + c * 16 + (size_t)s0 * Geo::A_ROW;
+            src[j] = reinterpret_cast<const char*>(in.W) + (size_t)row * in.K * sizeof(WT) + c * 16 + (size_t)(s0 + rot) * Geo::A_ROW;
             if constexpr (HALF) adv[j] = Geo::A_ROW, back[j] = c >= 4 ? Geo::A_ROW / 2 : 0;
         } else {
             constexpr int cpr = Geo::B_ROW / 16;
@@ -379,17 +388,17 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const __half* B = Geo::NB == 2 ? ((u & 1) ? in.Blo : in.Bhi) : rb * Geo::BN >= in.row_b2 ? in.Bhi2 : in.Bhi;
             int m = pb * BM + pt * 16 + r;
             if constexpr (Cfg::GR) m = in.grp.rowmap ? in.grp.rowmap[m] : tile.y + pt * 16 + r;
-            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * (Geo::F32 ? 4 : 2) + c * 16 + (size_t)s0 * Geo::B_ROW;
+            src[j] = reinterpret_cast<const char*>(B) + (size_t)m * in.K * (Geo::F32 ? 4 : 2) + c * 16 + (size_t)(s0 + rot) * Geo::B_ROW;
             if constexpr (HALF) adv[j] = Geo::B_ROW, back[j] = c >= cpr / 2 ? Geo::B_ROW / 2 : 0;
         }
     }
-    auto piece = [&](int j, unsigned dst, bool tail) PG_INLINE {
+    auto piece = [&](int j, unsigned dst, int t) PG_INLINE {  // of stage t
         if constexpr (HALF) {
-            pf_dma(src[j] - (tail ? back[j] : 0), dst);
+            pf_dma(src[j] - (half_tail && t == ns - 1 ? back[j] : 0), dst);
             src[j] += adv[j];
         } else {
             pf_dma(src[j], dst);
-            src[j] += Geo::A_ROW;
+            src[j] += ROT && t == wrap ? Geo::A_ROW - ns * Geo::A_ROW : Geo::A_ROW;
         }
     };
     // One ring: stage s in slot s % S. Split rings: A stage s in slot s % SA at ring, B stage s in slot s % 2 behind the A ring.
@@ -400,14 +409,13 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     auto dma = [&](int j, int s) PG_INLINE {
         if constexpr (Geo::SA == 0) {
             const int t = s + S - 1;
-            piece(j, ring + (unsigned)((t % S) * Geo::STAGE + (wave * Geo::DPW + j) * 1024), half_tail && t == ns - 1);
+            piece(j, ring + (unsigned)((t % S) * Geo::STAGE + (wave * Geo::DPW + j) * 1024), t);
         } else if (j < Geo::DPB) {
             const int t = s + 1;
-            piece(Geo::DPA + j, ring_b + (unsigned)((t & 1) * Geo::B_BYTES + (wave * Geo::DPB + j) * 1024), half_tail && t == ns - 1);
+            piece(Geo::DPA + j, ring_b + (unsigned)((t & 1) * Geo::B_BYTES + (wave * Geo::DPB + j) * 1024), t);
         } else {
             const int t = s + SAN - 1;
-            piece(j - Geo::DPB, ring + (unsigned)((t % SAN) * Geo::A_BYTES + (wave * Geo::DPA + j - Geo::DPB) * 1024),
-                  half_tail && t == ns - 1);
+            piece(j - Geo::DPB, ring + (unsigned)((t % SAN) * Geo::A_BYTES + (wave * Geo::DPA + j - Geo::DPB) * 1024), t);
         }
     };
     constexpr int AT = Geo::AT;
