@@ -876,21 +876,24 @@ hipError_t pgemm_allow_lds() {
 
 // The tilings of the Llama prompts, f(PgCfg<...>{}, us): us weighs a stage of the tiling, about what it takes with the chip
 // full of whole tiles that share their weight rows (tools/pgemm_lab stages, profiles/pgemm_tilings.txt): fp16 within 8 %, but
-// the 192 x 32 tile 0.54; int8 4 to 19 % below; fp32 2.96, 2.58, 1.63, 1.06, 1.95, the 96-row tile at half its time. A launch
+// the 192 x 32 tile 0.54; int8 4 to 14 % below; fp32 2.96, 2.58, 1.63, 1.06, 1.95, the 96-row tile at half its time. A launch
 // takes the one whose plan (pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth)
 // costs least. Llama-2-7B, q/k/v | gate/up | wo | down, us (the same file): the best plan against the best tiling in whole
 // tiles: 512 rows 105 | 208 | 44 | 93 against 105 | 230 | 45 | 117; 64 rows 29 | 47 | 14 | 28 against 41 | 50 | 25 | 61; int8
 // 64 rows 26 | 41 | 15 | 25 against 34 | 47 | 27 | 67. The 192-row tiles: 96 rows gate/up 52, where 128 rows take 63 and 68;
 // 64 rows, against 128-row tiles, gate/up 47 | 50 (int8 41 | 47), q/k/v 29 | 32 (26 | 28).
+// The int8 tilings with a weight ring of their own (SA 3 or 5) have two to four stages of the weights in flight instead of
+// one to two; 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
+// 50.6; 32 rows (192 x 32 against 256 x 32 in one ring): gate/up 33.3 -> 29.9.
 template <typename WT, class F>
 void pg_tilings(F&& f) {
     if constexpr (std::is_same<WT, float>::value) {
         f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.3f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 1.3f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.2f);
         f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
     } else if constexpr (std::is_same<WT, int8_t>::value) {
-        f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.15f), f(PgCfg<96, 4, 2, 2>{}, 1.6f);
-        f(PgCfg<64, 4, 2, 3>{}, 1.4f), f(PgCfg<64, 4, 2, 2>{}, 1.2f);
-        f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
+        f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.05f), f(PgCfg<96, 4, 2, 2, 3>{}, 1.37f);
+        f(PgCfg<64, 4, 2, 3, 3>{}, 1.42f), f(PgCfg<64, 4, 2, 2, 3>{}, 1.1f);
+        f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 2, 3, 5>{}, 1.17f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
     } else {
         f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
         f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);

@@ -213,6 +213,23 @@ def test_prefill_splits_match_decode(gpu, w, n):
         assert np.abs(a - b).max() <= 2 ** -7
 
 
+@pytest.mark.parametrize("n", [20, 66, 131, 200, 290])
+def test_prefill_int8_half_last_stage_of_split_rings(gpu, n):
+    """int8 depths that end in a half stage (1088 = 8.5 x 128, 11072 = 86.5 x 128) in the tilings whose weights have a ring of
+    their own, against the decode steps; test_prefill_splits_match_decode's bounds."""
+    from simplellminference_amd.model import LlamaModel, preset
+    cfg = preset("tiny", max_length=320, hidden_size=1088, num_attention_heads=17, num_key_value_heads=17, kv_hidden_size=1088,
+                 intermediate_size=11072)
+    m = LlamaModel(config=cfg, w_dtype="i8", kv_dtype="f16", seed=6).init()
+    prompt = _prompt(n, cfg.vocab_size)
+    ref = m.predict(prompt, n + 3, want_logits=True)
+    m.reset()
+    tok, log = m.predict_prefill(prompt, n + 3, want_logits=True)
+    m.close()
+    assert np.array_equal(tok, ref[0])
+    assert np.abs(log[n - 1:] - ref[1][n - 1:]).max() <= 1e-3
+
+
 @pytest.mark.parametrize("n", [97, 98, 161, 193, 194, 290])
 def test_prefill_rows_of_each_tiling(gpu, n):
     """Row counts around multiples of 96: every GEMM of a chunk pads to its own tile (96 rows where that is cheaper than 64
@@ -260,7 +277,7 @@ def test_prefill_attention_groups(gpu, hd, heads, kvh, n):
 TILING_SHAPES = [("f16", "llama2-7b", 1, 10), ("f16", "llama2-7b", 1, 74), ("f16", "llama2-7b", 1, 200),
                  ("f16", "llama3-8b", 1, 104), ("f16", "llama3-8b", 1, 200), ("f16", "llama2-7b", 2, 400),
                  ("i8", "llama2-7b", 1, 10), ("i8", "llama2-7b", 1, 50), ("i8", "llama2-7b", 1, 74), ("i8", "llama2-7b", 1, 130),
-                 ("i8", "llama3-8b", 1, 130), ("i8", "llama3-8b", 1, 200), ("f32", "llama2-7b", 1, 18),
+                 ("i8", "llama3-8b", 1, 120), ("i8", "llama3-8b", 1, 130), ("i8", "llama3-8b", 1, 200), ("f32", "llama2-7b", 1, 18),
                  ("f32", "llama2-7b", 1, 50), ("f32", "llama2-7b", 1, 74), ("f32", "llama3-8b", 1, 20), ("f32", "llama3-8b", 1, 104)]
 
 
