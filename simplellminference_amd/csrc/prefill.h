@@ -904,12 +904,13 @@ void pg_tilings(F&& f) {
 }
 
 // The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.91; 1.03,
-// 1.10, 0.71; 0.41; 0.45; 0.61. 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 349 | 381 and
+// 0.71; 0.41; 0.45; 0.61. (Two workgroups of 128 x 128 on a CU were third at every size, 2048 x 10240 at 1024 rows 56.2
+// where 128 x 256 takes 52.5.) 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 349 | 381 and
 // 149 | 184, 256 rows 113 | 121 and 55 | 80, 64 rows 65 | 76 and 34 | 76.
 template <class F>
 void pg_row_tilings(int M, F&& f) {
     if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
-    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.2f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
     if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.56f);
     if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.75f);
     if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.9f);
