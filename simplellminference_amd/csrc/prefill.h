@@ -875,13 +875,13 @@ hipError_t pgemm_allow_lds() {
 }
 
 // The tilings of the Llama prompts, f(PgCfg<...>{}, us): us weighs a stage of the tiling, about what it takes with the chip
-// full of whole tiles that share their weight rows (tools/pgemm_lab stages, profiles/pgemm_tilings.txt): fp16 within 8 %, but
-// the 192 x 32 tile 0.54; int8 4 to 14 % below; fp32 2.96, 2.58, 1.63, 1.06, 1.95, the 96-row tile at half its time. A launch
+// full of whole tiles that share their weight rows (tools/pgemm_lab stages, profiles/pgemm_tilings.txt): fp16 1.60,
+// 1.53, 1.22, 0.89, 0.92, 0.73, 0.70, 0.53, 0.47, 0.37, 8 to 29 % below the listed times, which lie between these and those of weights read once; int8
+// within 8 %; fp32 2.84, 2.56, 1.52, 1.04, 1.90, the 96-row tile at half its time. A launch
 // takes the one whose plan (pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth)
 // costs least. Llama-2-7B, q/k/v | gate/up | wo | down, us (the same file): the best plan against the best tiling in whole
-// tiles: 512 rows 105 | 208 | 44 | 93 against 105 | 230 | 45 | 117; 64 rows 29 | 47 | 14 | 28 against 41 | 50 | 25 | 61; int8
-// 64 rows 26 | 41 | 15 | 25 against 34 | 47 | 27 | 67. The 192-row tiles: 96 rows gate/up 52, where 128 rows take 63 and 68;
-// 64 rows, against 128-row tiles, gate/up 47 | 50 (int8 41 | 47), q/k/v 29 | 32 (26 | 28).
+// tiles: 512 rows 91 | 176 | 40 | 84 against 91 | 187 | 40 | 108; 64 rows 29 | 42 | 13 | 28 against 40 | 46 | 20 | 56; int8
+// 64 rows 25 | 36 | 15 | 24 against 32 | 45 | 26 | 65. 96 rows gate/up 49, where 128 rows take 58.
 // The int8 tilings with a weight ring of their own (SA 3 or 5) have two to four stages of the weights in flight instead of
 // one to two; 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
 // 50.6; 32 rows (192 x 32 against 256 x 32 in one ring): gate/up 33.3 -> 29.9.
@@ -903,10 +903,10 @@ void pg_tilings(F&& f) {
     }
 }
 
-// The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.91; 1.03,
-// 0.71; 0.41; 0.45; 0.61. (Two workgroups of 128 x 128 on a CU were third at every size, 2048 x 10240 at 1024 rows 56.2
-// where 128 x 256 takes 52.5.) 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 349 | 381 and
-// 149 | 184, 256 rows 113 | 121 and 55 | 80, 64 rows 65 | 76 and 34 | 76.
+// The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.71; 0.94,
+// 0.53; 0.36; 0.41; 0.56. (Two workgroups of 128 x 128 on a CU were third at every size, 2048 x 10240 at 1024 rows 56.2
+// where 128 x 256 takes 52.5.) 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 328 | 353 and
+// 131 | 146, 256 rows 108 | 118 and 53 | 74, 64 rows 63 | 74 and 33 | 74.
 template <class F>
 void pg_row_tilings(int M, F&& f) {
     if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
