@@ -904,13 +904,14 @@ void pg_tilings(F&& f) {
 }
 
 // The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.71; 0.94,
-// 0.53; 0.36; 0.41; 0.56. (Two workgroups of 128 x 128 on a CU were third at every size, 2048 x 10240 at 1024 rows 56.2
-// where 128 x 256 takes 52.5.) 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 328 | 353 and
-// 131 | 146, 256 rows 108 | 118 and 53 | 74, 64 rows 63 | 74 and 33 | 74.
+// 1.06, 0.53; 0.36; 0.41; 0.56. 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 328 | 353 and
+// 131 | 146, 256 rows 108 | 118 and 53 | 74, 64 rows 63 | 74 and 33 | 74. Two workgroups of 128 x 128 on a CU are the fastest
+// where tiles twice as wide leave half a round empty: 3072 x 11264 at 768 rows 76, the others 86 and more; 11264 x 1024 at
+// 1408 rows 39, the others 46.
 template <class F>
 void pg_row_tilings(int M, F&& f) {
     if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
-    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.2f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
     if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.56f);
     if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.75f);
     if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.9f);
