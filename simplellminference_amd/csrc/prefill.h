@@ -495,6 +495,10 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     // in front. 512 rows, 7B q/k/v | gate/up | wo | down: 109 | 207 | 45 | 96 -> 93 | 181 | 42 | 84 us; 2048 rows 413 | 754 |
     // 130 | 373 -> 377 | 670 | 109 | 327 (1260 TFLOP/s). The clock then falls from 2.0 to 1.66 GHz (MFMAs on random data
     // alone hold 1.74 PFLOP/s): more waves, s_setprio and 128-row wave tiles measured the same.
+    // PAIR: where a second workgroup runs on the CU and the ring has two stages, the order is the compiler's and the DMA goes
+    // first: the other workgroup's MFMAs run beside the reads, and the next stage needs all of the time there is to land
+    // (128 x 128 of a stack, 5120 x 18944 at 1536 rows: 315 -> 283 us).
+    constexpr bool PAIR = Geo::SA == 0 && S == 2 && 2 * Geo::LDS <= 160 * 1024;
     auto phase = [&](const Frags& f, Frags& n, const char* st, const char* stb, auto KB, auto J0, auto J1, int s) PG_INLINE {
         constexpr int RS = NSL > 1 ? NSL - 1 : 1;  // slices with reads
         constexpr int kb = decltype(KB)::value, j0 = decltype(J0)::value, j1 = decltype(J1)::value;
@@ -507,7 +511,7 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             constexpr int d0 = j0 + (j1 - j0) * i / NSL, d1 = j0 + (j1 - j0) * (i + 1) / NSL;
             slice_mfma(i, f);
             pg_for<d1 - d0>([&](auto J) PG_INLINE { dma(d0 + J, s); });
-            if constexpr ((i + 1) % (AT < 4 ? 4 / AT : 1) == 0 || i == NSL - 1) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!PAIR && ((i + 1) % (AT < 4 ? 4 / AT : 1) == 0 || i == NSL - 1)) __builtin_amdgcn_sched_barrier(0);
         });
     };
     constexpr bool TWO = Geo::FOLD > 0;
@@ -568,6 +572,16 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         // lgkmcnt(0), so the previous stage's buffer is free for the DMA issued after it while its last fragments wait in
         // registers.
         Frags X, Y;
+        // Of an iteration's np pieces, those issued before phase i. What must land within the stage that issues it goes out
+        // early: a split ring's activations in the first phase, all of a two-stage ring in the first half. Spread over the whole
+        // stage the last of them were waited for at its end (96 x 128 tiles of fp16, 4096 x 11008 at 384 rows: 84.5 -> 79.4 us;
+        // 256 x 256 of a stack, 34304 x 4096 at 2048 rows: 550 -> 530).
+        constexpr auto due = [](int i, int np) constexpr {
+            const int early = np < Geo::DPB ? np : Geo::DPB;
+            if (PAIR || i == 0) return PAIR ? np : 0;
+            if (Geo::SA) return early + i * (np - early) / KBS;
+            return S > 2 ? i * np / KBS : 2 * i < KBS ? (2 * i * np + KBS - 1) / KBS : np;
+        };
         // one iteration; P: pieces it issues
         auto iter = [&](int s, auto P, auto first) PG_INLINE {
             constexpr int NP = decltype(P)::value;
@@ -575,19 +589,20 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             const char *st, *stb;
             stage_begin(s);
             bufs(s, st, stb);
-            constexpr std::integral_constant<int, 0> q0;
-            constexpr std::integral_constant<int, NP / KBS> q1;
-            constexpr std::integral_constant<int, 2 * NP / KBS> q2;
+            constexpr std::integral_constant<int, due(0, NP)> q0;
+            constexpr std::integral_constant<int, due(1, NP)> q1;
+            constexpr std::integral_constant<int, due(2, NP)> q2;
+            if constexpr (PAIR) pg_for<NP>([&](auto J) PG_INLINE { dma(J, s); });
             if constexpr (FIRST) {
                 pg_for<NR>([&](auto R) PG_INLINE { read_frag(R, st, stb, 0, X); });
-                pg_for<q1>([&](auto J) PG_INLINE { dma(J, s); });
+                pg_for<q1 - q0>([&](auto J) PG_INLINE { dma(q0 + J, s); });
                 __builtin_amdgcn_sched_barrier(0);
             } else {
-                phase(Y, X, st, stb, q0, q0, q1, s);
+                phase(Y, X, st, stb, std::integral_constant<int, 0>{}, q0, q1, s);
             }
             phase(X, Y, st, stb, std::integral_constant<int, 1>{}, q1, q2, s);
             if constexpr (KBS == 4) {
-                constexpr std::integral_constant<int, 3 * NP / KBS> q3;
+                constexpr std::integral_constant<int, due(3, NP)> q3;
                 if (NP > 0 || !(half_tail && s == ns - 1)) {
                     phase(Y, X, st, stb, std::integral_constant<int, 2>{}, q2, q3, s);
                     phase(X, Y, st, stb, std::integral_constant<int, 3>{}, q3, std::integral_constant<int, NP>{}, s);
