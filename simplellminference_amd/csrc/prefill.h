@@ -347,15 +347,18 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     constexpr bool HALF = sizeof(WT) == 1;
     const bool half_tail = HALF && (in.K % Geo::KS) != 0 && s0 + ns == nsk;
     const int nt = in.N >> 4;       // row tiles
-    // Row blocks start their walk of the depth at different stages, rot on, and wrap around: rows of fp16 weights lie 8 KiB
-    // and more apart, and workgroups that all walk from the same column reach less of the memory's rate (likely a few channels at a time). Where
-    // one row block's weights are read once (a chunk of one position block): with more, their activations no longer fit the
-    // L2 side by side (256 rows, gate/up 92.7 -> 94.7 us); up to two splits, more of them start apart already (down at 96
-    // rows 34.8 -> 38.9); 128 weight rows and more (tiles of 64, two on a CU, 28672 x 4096 at 32 rows 52.4 -> 60.1). 7B
-    // gate/up at 32 | 64 | 96 rows 45.5 | 50.0 | 53.4 -> 37.0 | 42.5 | 48.8 us, a stack's 34304 x 4096 at 128 82.9 -> 71.6.
-    // int8 rows are half as long and its walk is not bound by memory: 39.2 -> 39.1.
+    // Row blocks start their walk of the depth at different stages, rot on, and wrap around: workgroups that all walk from the
+    // same column reach less of the memory's rate where rows of fp16 weights lie a multiple of 8 KiB apart (likely a few
+    // channels at a time), of 4 KiB with one activation image. 22016 x 4096 at 32 | 64 | 96 rows 47.3 | 51.1 | 53.9 -> 36.7 |
+    // 41.5 | 45.8 us, a stack's 22528 x 2048 at 32 rows 23.4 -> 21.1; other distances lose by it: 27648 x 5120 at 96 rows 78.8
+    // -> 82.2, 16384 x 2048 (two images) at 64 19.6 -> 20.7, a stack's 25600 x 3072 at 128 42.5 -> 43.8. Where one row block's
+    // weights are read once (a chunk of one position block): with more, their activations no longer fit the L2 side by side
+    // (256 rows, gate/up 92.7 -> 94.7); up to two splits, more of them start apart already (down at 96 rows 34.8 -> 38.9); 128
+    // weight rows and more (tiles of 64, two on a CU, 28672 x 4096 at 32 rows 52.4 -> 60.1). int8 rows are half as long and
+    // their walk is not bound by memory: 39.2 -> 39.1.
     constexpr bool ROT = sizeof(WT) == 2 && !Cfg::GR && BM <= 128 && Geo::BN >= 128;
-    const int rot = ROT && PB == 1 && nsp <= 2 ? rb % ns : 0, wrap = ns - 1 - rot;  // stage t: (t + rot) % ns of the range
+    const bool apart = in.K % (Geo::NB == 2 ? 4096 : 2048) == 0;
+    const int rot = ROT && PB == 1 && nsp <= 2 && apart ? rb % ns : 0, wrap = ns - 1 - rot;  // stage t: (t + rot) % ns of the range
     const unsigned ring = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)pg_smem;
 
     // this wave's DMA instructions d in [wave*DPW, (wave+1)*DPW): stage bytes [1024 d, 1024 (d + 1)). Lane i

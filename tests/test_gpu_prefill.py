@@ -273,6 +273,30 @@ def test_prefill_attention_groups(gpu, hd, heads, kvh, n):
     assert np.abs(log - lref).max() <= 1e-3
 
 
+@pytest.mark.parametrize("width,ff,n", [(4096, 192, 20), (4096, 11008, 66), (4096, 2048, 97), (4096, 11008, 128), (4096, 11008, 129),
+                                        (8192, 1024, 33), (4160, 2048, 97), (2048, 8192, 66)])
+def test_prefill_rotated_walk(gpu, width, ff, n):
+    """Chunks of one position block at 4096 and 8192 columns, whose row blocks start apart in the depth: fewer and more of them
+    than stages (64, 128), whole tiles and two splits, a last row block of a few rows; 129 positions and widths that keep the
+    order. Against the decode steps: the cache rows of one layer, bounds of test_prefill_every_tiling."""
+    from simplellminference_amd.model import LlamaModel, preset
+    cfg = preset("tiny", max_length=160, hidden_size=width, num_attention_heads=width // 64, num_key_value_heads=width // 64,
+                 kv_hidden_size=width, intermediate_size=ff)
+    m = LlamaModel(config=cfg, w_dtype="f16", kv_dtype="f16", seed=8).init()
+    prompt = _prompt(n, cfg.vocab_size)
+    want = m.predict(prompt, n + 1)
+    lw, kv = m.logits()[0], [m.kv(1, which, n) for which in (0, 1)]
+    m.reset()
+    got = m.predict_prefill(prompt, n + 1)
+    log = m.logits()[0]
+    assert np.array_equal(got, want)
+    assert np.linalg.norm(log - lw) <= 8e-4 * np.linalg.norm(lw)
+    for a, b in zip([m.kv(1, which, n) for which in (0, 1)], kv):
+        assert np.abs(a - b).max() <= 2.0 ** -10 * np.abs(b).max()
+        assert np.linalg.norm(a - b) <= 2.0 ** -12 * np.linalg.norm(b)
+    m.close()
+
+
 # (weights, shape, batch, prompt): between them every tiling of the prompt GEMMs runs (test_host_runtime.py looks)
 TILING_SHAPES = [("f16", "llama2-7b", 1, 10), ("f16", "llama2-7b", 1, 74), ("f16", "llama2-7b", 1, 200),
                  ("f16", "llama3-8b", 1, 104), ("f16", "llama3-8b", 1, 200), ("f16", "llama2-7b", 2, 400),

@@ -547,6 +547,12 @@ def wide_model():
                                 taps=4, residual_mult=0.4, max_length=800), batch=1, seed=4).init()
 
 
+@pytest.mark.parametrize("n", [66, 100, 128])
+def test_pass_of_one_position_block(gpu, n):
+    """Passes of 128 rows, whose row blocks start their walk of 4096 columns apart."""
+    test_every_tiling_of_a_pass(gpu, n)
+
+
 @pytest.mark.parametrize("n", TILING_ROWS)
 def test_every_tiling_of_a_pass(gpu, n):
     """Whole prompts against the same in portions of 64 rows and single steps."""
