@@ -615,11 +615,19 @@ constexpr int kPfPad = 128;
 template <typename WT, typename KT>
 struct StepRecorder {
     static constexpr bool NT = true;  // streamed-once weights: non-temporal loads
-    // Vectors per lane and step of the one-row wo GEMV: a fp32 row has twice a fp16 row's vectors, and two steps of 8 keep
-    // 16 KiB of a wave in flight, a whole row of 4096 (4096 x 4096: 15.7 -> 12.8 us against two of 2). The down GEMV's two
-    // steps of 6 hold 12 KiB already (8: 30.5 -> 30.9 us).
-    static constexpr bool F32 = std::is_same<WT, float>::value;
-    static constexpr int kUWo = F32 ? 8 : 2;
+    // The one-row wo GEMV. Two steps of 2 vectors a lane; fp32 rows of whole 2048-column steps of 8 (16 KiB of a wave) where a
+    // wave has two of them or more: 4096 x 4096 16.5 -> 13.0 us, 8192 x 2048 16.5 -> 13.1. With fewer, or steps partly past the
+    // row's end, 8 vectors lose: 4096 x 512 (a TP-8 rank) 5.5 -> 6.2, 4096 x 2048 7.8 -> 9.9, 4096 x 3072 10.3 -> 10.7. (The down
+    // GEMV's two steps of 6 hold 12 KiB already: 8 vectors 30.5 -> 30.9 us.)
+    template <class Epi>
+    static hipError_t wo_row(sli_model* m, const void* W, const GemvIn& in, const Epi& e) {
+        if constexpr (std::is_same<WT, float>::value) {
+            const int waves = gemv_max_blocks() * (kGemvThreads / 64);
+            if (in.cols % 2048 == 0 && (long)m->D * (in.cols / 2048) >= 2L * waves)
+                return launch_gemv_u<WT, 1, 8, NT>((const WT*)W, in, e, m->D, m->stream);
+        }
+        return launch_gemv_u<WT, 1, 2, NT>((const WT*)W, in, e, m->D, m->stream);
+    }
     static int gemv_qkv(sli_model* m, int l) {
         const LayerW& w = m->layers[l];
         GemvIn in{m->x, m->norms + (size_t)(2 * l) * m->D, m->c.eps, m->D};
@@ -667,11 +675,11 @@ struct StepRecorder {
         if (!m->wo_merge) {  // the attention merged its splits into attn: a plain input
             GemvIn in{m->attn, nullptr, 0.0f, m->hq * m->hd};
             if (fused_ar(m)) {
-                SLI_HIP((launch_gemv_u<WT, 1, kUWo, NT>((const WT*)w.wo, in, push_epi(m, w.wo_s, 0), m->D, m->stream)));
+                SLI_HIP(wo_row(m, w.wo, in, push_epi(m, w.wo_s, 0)));
                 return SLI_OK;
             }
             EpiStore<1> e{tp ? m->xpart : m->x, (!tp || m->c.tp_rank == 0) ? m->x : nullptr, w.wo_s, 1.0f, m->D};
-            SLI_HIP((launch_gemv_u<WT, 1, kUWo, NT>((const WT*)w.wo, in, e, m->D, m->stream)));
+            SLI_HIP(wo_row(m, w.wo, in, e));
             return SLI_OK;
         }
         GemvIn in{m->attn, nullptr, 0.0f, m->hq * m->hd};

@@ -210,10 +210,31 @@ def stack_prompts_take_the_fast_tilings(H):
         m.close()
 
 
+def fp32_output_projection_steps(H):
+    """A fp32 output projection reads 8 vectors a lane and step only where a wave has two whole such steps (of 2048 columns):
+    one rank of 4096 columns, not the ranks of 512 to 2048 of a group, nor a width that they do not divide."""
+    from simplellminference_amd.model import LlamaModel, TPGroup, preset
+    kw = dict(w_dtype="f32", kv_dtype="f32", seed=1)
+    steps = lambda: set(re.findall(r"gemv_kernelIfLi1ELi(\d)ELb1ENS_8EpiStore", H.hh_launched().decode()))
+    for heads, tp, want in ((32, 1, 8), (32, 2, 2), (32, 8, 2), (24, 1, 2), (64, 4, 8), (64, 8, 2)):
+        cfg = preset("tiny", max_length=2048, vocab_size=64, head_dim=128, hidden_size=128 * heads, num_attention_heads=heads,
+                     num_key_value_heads=heads, kv_hidden_size=128 * heads, num_hidden_layers=1, intermediate_size=256)
+        H.hh_launched()
+        if tp == 1:
+            m = LlamaModel(config=cfg, **kw).init()
+            m.step()
+        else:
+            m = TPGroup(cfg, tp, **kw).init()
+            m.step()
+        # (a down projection's steps are 6)
+        assert {int(v) for v in steps()} - {6, 1} == {want}, (heads, tp, want)
+        m.close()
+
+
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts",
-         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings"]
+         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "fp32_output_projection_steps"]
 
 
 @pytest.fixture(scope="module")
