@@ -900,9 +900,11 @@ hipError_t pgemm_allow_lds() {
 // costs least. Llama-2-7B, q/k/v | gate/up | wo | down, us (the same file): the best plan against the best tiling in whole
 // tiles: 512 rows 91 | 176 | 40 | 84 against 91 | 187 | 40 | 108; 64 rows 29 | 42 | 13 | 28 against 40 | 46 | 20 | 56; int8
 // 64 rows 25 | 36 | 15 | 24 against 32 | 45 | 26 | 65. 96 rows gate/up 49, where 128 rows take 58.
-// The int8 tilings with a weight ring of their own (SA 3 or 5) have two to four stages of the weights in flight instead of
-// one to two; 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
-// 50.6; 32 rows (192 x 32 against 256 x 32 in one ring): gate/up 33.3 -> 29.9.
+// The int8 tilings with a weight ring of their own (SA 3) have two stages of the weights in flight instead of one (a wave waits
+// for its loads in order, so for all weights issued before the activations it needs: a deeper ring holds stages that have
+// landed); 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
+// 50.6; 32 rows: q/k/v 17.8 us with 3 slots, 19.5 with 5, gate/up 25.3 and 26.4. 256 x 32 in one ring stays for very wide
+// outputs: 28672 x 4096 at 9 rows 27.6, the next 30.4.
 template <typename WT, class F>
 void pg_tilings(F&& f) {
     if constexpr (std::is_same<WT, float>::value) {
@@ -911,7 +913,7 @@ void pg_tilings(F&& f) {
     } else if constexpr (std::is_same<WT, int8_t>::value) {
         f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.05f), f(PgCfg<96, 4, 2, 2, 3>{}, 1.37f);
         f(PgCfg<64, 4, 2, 3, 3>{}, 1.42f), f(PgCfg<64, 4, 2, 2, 3>{}, 1.1f);
-        f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 2, 3, 5>{}, 1.17f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
+        f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 2, 3, 3>{}, 1.12f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
     } else {
         f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
         f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);
