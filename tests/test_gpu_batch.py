@@ -53,11 +53,16 @@ def test_matmul_batch_exact_integers(gpu, rows, cols, batch):
     assert np.array_equal(got, want)
 
 
+# (rows, cols, batch) -> blocks of a step: waves with 5 k-blocks of a tile (or 4 and 5, unevenly), 6, 7 and 4
+STEP_SHAPES = {(2048, 10240, 1): 5, (2048, 10240, 6): 5, (2048, 10240, 8): 5, (2048, 8224, 3): 5, (2048, 8416, 8): 5,
+               (2048, 10272, 8): 7, (2048, 14336, 1): 7, (2048, 8192, 6): 4}
+
+
 @pytest.mark.parametrize("rows,cols,batch", [(8200, 2080, 8), (8200, 2560, 5), (8200, 2592, 3),
-                                             (16, 16384, 8), (48, 9216, 6), (64, 4640, 1)])
+                                             (16, 16384, 8), (48, 9216, 6), (64, 4640, 1)] + list(STEP_SHAPES))
 def test_matmul_batch_steps_of_five_and_many_splits(gpu, rows, cols, batch):
-    """A wave's 5 k-blocks of a tile as one step (and the 6 beside them), and merges of more splits than one round of loads
-    holds. Small integers: sums are exact in any order."""
+    """A wave's 5, 6 or 7 k-blocks of a tile as one step (STEP_SHAPES; test_host_runtime.py looks that they run), and merges of 3
+    and 4 splits and of 9 and 16, more than one round of loads holds. Small integers: sums are exact in any order."""
     test_matmul_batch_exact_integers(gpu, rows, cols, batch)
 
 

@@ -567,3 +567,23 @@ def test_every_tiling_of_a_pass(gpu, n):
         p = e
     close(whole, np.concatenate([m.feed([0], [i], [[ids[i]]], [[0]]) for i in want]), "bfloat16")
     m.close()
+
+
+def narrow_model(batch):
+    """One block of width 2048 whose output projection has 10240 columns: five k-blocks a wave in a decode pass of 2 rows and
+    more (test_host_runtime.py looks)."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    return StackModel(StackSpec(203, 2048, (BlockSpec("attention", 32, 64, 64, kv_heads=8, scale=0.125, ff=8192, ff_limit=7.0),),
+                                taps=4, residual_mult=0.4, max_length=40), batch=batch, seed=4).init()
+
+
+@pytest.mark.parametrize("batch", [2, 6, 8])
+def test_decode_pass_with_steps_of_five(gpu, batch):
+    """Rows of a decode pass together against the same rows one at a time, whose projections are the row-wise ones."""
+    m = narrow_model(batch)
+    ids = [tokens(4, vocab=203, seed=b) for b in range(batch)]
+    m.feed(range(batch), [0] * batch, [i[:3] for i in ids], [[]] * batch)
+    got = m.feed(range(batch), [3] * batch, [i[3:] for i in ids], [[0]] * batch)
+    alone = np.concatenate([m.feed([b], [3], [ids[b][3:]], [[0]]) for b in range(batch)])
+    m.close()
+    close(got, alone, "bfloat16")

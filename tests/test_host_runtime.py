@@ -231,10 +231,35 @@ def fp32_output_projection_steps(H):
         m.close()
 
 
+def steps_of_the_batched_projection(H):
+    """The shapes that the GPU tests name run the steps that they name."""
+    from simplellminference_amd import _lib
+    from tests import test_gpu_batch as B, test_gpu_stack as S
+    ran = lambda tag: {int(v) for v in re.findall(r"bgemm_kernel\w*" + tag + r"\w*?ELb0ELi(\d)E", H.hh_launched().decode())}
+    H.hh_launched()
+    for (rows, cols, batch), step in B.STEP_SHAPES.items():
+        n = _lib.load().sli_matmul_batch_workspace_bytes(rows, cols, batch)
+        buf = [ctypes.c_void_p() for _ in range(4)]
+        for p, size in zip(buf, (4 * batch * cols, 2 * rows * cols, 4 * batch * rows, n)):
+            assert H.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0
+        x, w, y, ws = buf
+        _lib.call("sli_matmul_batch", x, w, _lib.DT_F16, y, rows, cols, batch, ws, n, None)
+        assert ran("BgEpiStore") == {step}, (rows, cols, batch)
+        for p in buf:
+            H.hipFree(p)
+    for batch in (2, 6, 8):
+        m = S.narrow_model(batch)
+        H.hh_launched()
+        m.feed(range(batch), [0] * batch, [[1]] * batch, [[0]] * batch)
+        assert ran("HyOut") == {5}, batch
+        m.close()
+
+
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts",
-         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "fp32_output_projection_steps"]
+         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "fp32_output_projection_steps",
+         "steps_of_the_batched_projection"]
 
 
 @pytest.fixture(scope="module")
