@@ -337,7 +337,8 @@ __device__ __forceinline__ bool attn_publish(const AttnArgs<KT>& a, int kvh, int
     const int ns = min(pos / (WAVES * PPW) + 1, a.max_splits);  // live workgroups of this kv head
     // Workgroup partial: the WAVES slice states merged in LDS. The only live split of its head (a context up to PPWG) is the
     // head's output: the merge's weight is e^0, so o / L is what attn_merge would store, without the drain, the arrival and
-    // the read back (32 fp32 heads of 128 at 75 to 95 positions: 10.2 -> 7.2 us). Otherwise published write-through (sc1) so the head's last-arriving workgroup can read it from any XCD without a fence pair
+    // the read back (32 fp32 heads of 128 at 75 to 95 positions: 10.2 -> 7.2 us). Otherwise published write-through (sc1) so
+    // the head's last-arriving workgroup can read it from any XCD without a fence pair
     // (MI355X_MICROARCH.md, hand-off table row 1: sc1 stores, drained, one agent-scope add per
     // workgroup behind a workgroup barrier, sc1 loads by the last adder after the barrier it joins).
     for (int i = threadIdx.x; i < G * HD; i += 64 * WAVES) {
@@ -363,7 +364,10 @@ __device__ __forceinline__ bool attn_publish(const AttnArgs<KT>& a, int kvh, int
             __hip_atomic_store(dst + HD + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    if (ns == 1) return false;  // uniform
+    if (ns == 1) {  // uniform
+        if (a.stamps && threadIdx.x == 0) a.stamps[blockIdx.x * 4 + 2] = __builtin_amdgcn_s_memrealtime();
+        return false;
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave drains before the arrival
     __syncthreads();
     if (threadIdx.x == 0) {
