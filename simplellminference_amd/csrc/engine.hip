@@ -1080,8 +1080,8 @@ struct StepRecorder {
             // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
             // in 16 ranges and more
             if (st.nseq > 1 && Geo::FOLD == 0) us = INFINITY;
-            const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true);
-            if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
+            const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true, us);
+            if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
             ++i;
         });
         hipError_t err = hipSuccess;

@@ -65,8 +65,8 @@ struct HyProj {
             float best = INFINITY;
             int pick = 0, i = 0;
             pg_row_tilings(M, [&](auto cfg, float us) {
-                const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true);
-                if (p.cost * us < best) best = p.cost * us, pick = i, in.full = p.full, in.splits = p.splits;
+                const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true, us, PgRolled<PgPair<Epi>>::value);
+                if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits;
                 ++i;
             });
             hipError_t err = hipSuccess;

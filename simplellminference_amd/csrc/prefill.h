@@ -847,30 +847,37 @@ struct PgEpiResid {  // y[m][row] = resid[m][row] + sum * row scale (matmul_kern
 struct PgPlan {
     int full = 0x7fffffff, splits = 1;  // PgIn
     int slots = 0;                      // per XCD
-    float cost = 0.0f;                  // in stages of the tiling
+    float us = 0.0f;
 };
 constexpr size_t kPgWsBytes = 64u << 20;  // partial sums of a launch at most
 constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
+// stage: us of a stage of the tiling (pg_tilings). Around its walk of the depth a workgroup takes 2 us and 6 for 128 KiB of sums
+// (a 128 x 256 tile): dispatch, the ring's first stages, the epilogue; a cut round 2 us, 0.6 for each split and 1.5 for each
+// split's and two more 128 KiB: the partial sums' way out and back. These and the stage times are fitted together, so that the
+// plan that costs least is the fastest one: over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken takes
+// 1.1 % longer than the fastest, of int8 0.4, of fp32 0.7, of block stacks 1.9 % (tools/pgemm_lab prints both).
+// rolled: a looped epilogue (kRolled) takes time by the tiles a wave loops over: a stack's 25600 x 3072 at 384 rows 100.6 us in
+// 128 x 256 tiles (16 a wave), 95.9 in 128 x 128 (8), with a plain epilogue 84 and 90. 0.5 us each is what picks best.
 template <class Cfg, typename WT>
-PgPlan pg_plan(int N, int K, int M, int cus, bool ws) {
+PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled = false) {
     using Geo = PgGeo<Cfg, WT>;
     const int nrb = (N + Geo::BN - 1) / Geo::BN, nx = (nrb + 7) / 8 * (M / Geo::BM);
     const int ns = (K + Geo::KS - 1) / Geo::KS;
     const int occ = (int)((160 * 1024) / Geo::LDS), cpx = std::max(1, cus / 8) * occ;
-    // entry and exit of a workgroup, and a split's share of the partial sums' way out and back, in stages
-    constexpr float kEdge = 5.0f;
-    const float part = 1.2f * (float)(16 * Geo::AT * Geo::WPT * Geo::THREADS) / (float)Geo::STAGE;
+    constexpr float kTile = 16.0f * Geo::AT * Geo::WPT * Geo::THREADS / 131072.0f, kEdge = 2.0f + 6.0f * kTile;
+    const float epi = rolled ? 0.5f * Geo::AT * Geo::WPT : 0.0f;
     PgPlan best;
     best.slots = nx;
-    best.cost = (float)((nx + cpx - 1) / cpx) * ((float)ns + kEdge);
+    best.us = (float)((nx + cpx - 1) / cpx) * ((float)ns * stage + kEdge + epi);
     const int full = nx / cpx * cpx, tail = nx - full;
     for (int S : {2, 3, 4, 5, 6, 8, 10, 12, 16}) {
         if (!ws || tail == 0 || ns < 4 * S || 8 * tail > kPgWsTiles ||
             (size_t)8 * tail * S * 16 * Geo::AT * Geo::WPT * Geo::THREADS > kPgWsBytes)
             break;
-        const float c = (float)(full / cpx) * ((float)ns + kEdge) +
-                        (float)((tail * S + cpx - 1) / cpx) * ((float)(ns + S - 1) / (float)S + kEdge) + part * (float)(S + 2);
-        if (c < best.cost) best = PgPlan{full, S, full + tail * S, c};
+        const float us = (float)(full / cpx) * ((float)ns * stage + kEdge + epi) +
+                         (float)((tail * S + cpx - 1) / cpx) * ((float)(ns + S - 1) / (float)S * stage + kEdge) + 2.0f +
+                         0.6f * (float)S + 1.5f * kTile * (float)(S + 2) + epi;
+        if (us < best.us) best = PgPlan{full, S, full + tail * S, us};
     }
     return best;
 }
@@ -892,14 +899,12 @@ hipError_t pgemm_allow_lds() {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)PgGeo<Cfg, WT>::LDS);
 }
 
-// The tilings of the Llama prompts, f(PgCfg<...>{}, us): us weighs a stage of the tiling, about what it takes with the chip
-// full of whole tiles that share their weight rows (tools/pgemm_lab stages, profiles/pgemm_tilings.txt): fp16 1.60,
-// 1.53, 1.22, 0.89, 0.92, 0.73, 0.70, 0.53, 0.47, 0.37, 8 to 29 % below the listed times, which lie between these and those of weights read once; int8
-// within 8 %; fp32 2.84, 2.56, 1.52, 1.04, 1.90, the 96-row tile at half its time. A launch
-// takes the one whose plan (pg_plan: rounds over the rows padded to its BM, and the last round's tiles cut over the depth)
-// costs least. Llama-2-7B, q/k/v | gate/up | wo | down, us (the same file): the best plan against the best tiling in whole
-// tiles: 512 rows 91 | 176 | 40 | 84 against 91 | 187 | 40 | 108; 64 rows 29 | 42 | 13 | 28 against 40 | 46 | 20 | 56; int8
-// 64 rows 25 | 36 | 15 | 24 against 32 | 45 | 26 | 65. 96 rows gate/up 49, where 128 rows take 58.
+// The tilings of the Llama prompts, f(PgCfg<...>{}, us): us is a stage of the tiling as pg_plan counts it. A launch takes the
+// tiling whose plan costs least (rounds over the rows padded to its BM, the last round's tiles cut over the depth).
+// Llama-2-7B, q/k/v | gate/up | wo | down, us, what the plan takes against the best tiling in whole tiles
+// (profiles/pgemm_tilings.txt): 512 rows 83 | 155 | 39 | 79 against 83 | 160 | 40 | 106; 64 rows 30 | 44 | 13 | 28 against 39 |
+// 46 | 20 | 55; int8 64 rows 26 | 35 | 14 | 25 against 30 | 38 | 25 | 61; fp32 96 rows 145 | 238 | 54 | 122 against 194 | 328 |
+// 97 | 256.
 // The int8 tilings with a weight ring of their own (SA 3) have two stages of the weights in flight instead of one (a wave waits
 // for its loads in order, so for all weights issued before the activations it needs: a deeper ring holds stages that have
 // landed); 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
@@ -908,33 +913,33 @@ hipError_t pgemm_allow_lds() {
 template <typename WT, class F>
 void pg_tilings(F&& f) {
     if constexpr (std::is_same<WT, float>::value) {
-        f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.3f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 1.3f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.2f);
-        f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.05f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.9f);
+        f(PgCfg<128, 4, 4, 2, 0, 1>{}, 2.29f), f(PgCfg<96, 2, 4, 2, 0, 1>{}, 2.22f), f(PgCfg<64, 4, 4, 2, 0, 1>{}, 1.22f);
+        f(PgCfg<32, 2, 6, 2, 0, 1>{}, 1.08f), f(PgCfg<32, 2, 4, 4, 0, 1>{}, 1.53f);
     } else if constexpr (std::is_same<WT, int8_t>::value) {
-        f(PgCfg<128, 4, 2, 2>{}, 1.95f), f(PgCfg<96, 4, 2, 3>{}, 2.05f), f(PgCfg<96, 4, 2, 2, 3>{}, 1.37f);
-        f(PgCfg<64, 4, 2, 3, 3>{}, 1.42f), f(PgCfg<64, 4, 2, 2, 3>{}, 1.1f);
-        f(PgCfg<32, 4, 3, 4>{}, 1.35f), f(PgCfg<32, 4, 4, 2>{}, 0.9f), f(PgCfg<32, 4, 2, 3, 3>{}, 1.12f), f(PgCfg<32, 2, 4, 2>{}, 0.72f);
+        f(PgCfg<128, 4, 2, 2>{}, 1.57f), f(PgCfg<96, 4, 2, 3>{}, 1.64f), f(PgCfg<96, 4, 2, 2, 3>{}, 1.18f);
+        f(PgCfg<64, 4, 2, 3, 3>{}, 1.32f), f(PgCfg<64, 4, 2, 2, 3>{}, 1.01f);
+        f(PgCfg<32, 4, 3, 4>{}, 1.33f), f(PgCfg<32, 4, 4, 2>{}, 0.99f), f(PgCfg<32, 4, 2, 3, 3>{}, 1.02f), f(PgCfg<32, 2, 4, 2>{}, 1.03f);
     } else {
-        f(PgCfg<128, 4, 2, 4, 3>{}, 1.73f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 1.8f);
-        f(PgCfg<128, 4, 2, 3, 4>{}, 1.4f), f(PgCfg<128, 4, 2, 2, 4>{}, 1.08f);
-        f(PgCfg<96, 4, 2, 3, 4>{}, 1.05f), f(PgCfg<96, 4, 2, 2, 4>{}, 0.85f);
-        f(PgCfg<64, 4, 3, 3>{}, 0.85f), f(PgCfg<64, 4, 3, 2>{}, 0.65f);
-        f(PgCfg<32, 4, 4, 3>{}, 0.66f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
+        f(PgCfg<128, 4, 2, 4, 3>{}, 0.95f), f(PgCfg<128, 4, 2, 4, 3, 2, false, true>{}, 0.98f);
+        f(PgCfg<128, 4, 2, 3, 4>{}, 0.88f), f(PgCfg<128, 4, 2, 2, 4>{}, 0.67f);
+        f(PgCfg<96, 4, 2, 3, 4>{}, 0.76f), f(PgCfg<96, 4, 2, 2, 4>{}, 0.64f);
+        f(PgCfg<64, 4, 3, 3>{}, 0.58f), f(PgCfg<64, 4, 3, 2>{}, 0.5f);
+        f(PgCfg<32, 4, 4, 3>{}, 0.44f), f(PgCfg<32, 2, 4, 2>{}, 0.42f);
     }
 }
 
-// The tilings of block-stack prompts (one fp16 image; their row count divides M). With the chip full (as above): 1.71; 0.94,
-// 1.06, 0.53; 0.36; 0.41; 0.56. 34304 x 4096 and 4096 x 15104, us, best plan | best whole tiles: 1024 rows 328 | 353 and
-// 131 | 146, 256 rows 108 | 118 and 53 | 74, 64 rows 63 | 74 and 33 | 74. Two workgroups of 128 x 128 on a CU are the fastest
-// where tiles twice as wide leave half a round empty: 3072 x 11264 at 768 rows 76, the others 86 and more; 11264 x 1024 at
-// 1408 rows 39, the others 46.
+// The tilings of block-stack prompts (one fp16 image; their row count divides M). 34304 x 4096 and 4096 x 15104,
+// us, as above: 1024 rows 272 | 127 against 300 | 142; 256 rows 106 | 52 against 116 | 73; 64 rows 62 | 32 against 73 | 75.
+// Two workgroups of 128 x 128 on a CU are the fastest where tiles twice as wide leave half a round empty: 3072 x 11264 at 768
+// rows 75, the others 86 and more; 11264 x 1024 at 1408 rows 40, the others 46. The 32-row tiles read weights and little else,
+// whatever a stage takes alone: theirs are the values that pick the faster one at 32 rows.
 template <class F>
 void pg_row_tilings(int M, F&& f) {
-    if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.85f);
-    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 1.15f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.2f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.77f);
-    if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.56f);
-    if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.75f);
-    if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.9f);
+    if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.3f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 0.76f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.05f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.52f);
+    if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.49f);
+    if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.42f);
+    if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.4f);
 }
 
 // ---------------------------------------------------------------- 3. block-causal attention

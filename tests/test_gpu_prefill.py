@@ -302,7 +302,8 @@ TILING_SHAPES = [("f16", "llama2-7b", 1, 10), ("f16", "llama2-7b", 1, 74), ("f16
                  ("f16", "llama3-8b", 1, 104), ("f16", "llama3-8b", 1, 200), ("f16", "llama2-7b", 2, 400),
                  ("i8", "llama2-7b", 1, 10), ("i8", "llama2-7b", 1, 50), ("i8", "llama2-7b", 1, 74), ("i8", "llama2-7b", 1, 130),
                  ("i8", "llama3-8b", 1, 120), ("i8", "llama3-8b", 1, 130), ("i8", "llama3-8b", 1, 200), ("f32", "llama2-7b", 1, 18),
-                 ("f32", "llama2-7b", 1, 50), ("f32", "llama2-7b", 1, 74), ("f32", "llama3-8b", 1, 20), ("f32", "llama3-8b", 1, 104)]
+                 ("f32", "llama2-7b", 1, 50), ("f32", "llama2-7b", 1, 74), ("f32", "llama3-8b", 1, 20), ("f32", "llama3-8b", 1, 104),
+                 ("i8", "llama3-8b", 1, 10), ("i8", "small-h128", 1, 10)]
 
 
 def tiling_model(w, name, batch):

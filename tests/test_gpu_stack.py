@@ -553,10 +553,21 @@ def test_pass_of_one_position_block(gpu, n):
     test_every_tiling_of_a_pass(gpu, n)
 
 
+def middle_model():
+    """A 3072-wide block, whose output projection takes the 128 x 128 tiling at 768 rows (test_host_runtime.py looks)."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    return StackModel(StackSpec(203, 3072, (BlockSpec("attention", 24, 128, 128, kv_heads=24, scale=0.1, ff=8192, ff_limit=7.0),),
+                                taps=4, residual_mult=0.4, max_length=800), batch=1, seed=4).init()
+
+
+def test_pairs_of_workgroups(gpu):
+    test_every_tiling_of_a_pass(gpu, 700, middle_model)
+
+
 @pytest.mark.parametrize("n", TILING_ROWS)
-def test_every_tiling_of_a_pass(gpu, n):
+def test_every_tiling_of_a_pass(gpu, n, model=wide_model):
     """Whole prompts against the same in portions of 64 rows and single steps."""
-    m = wide_model()
+    m = model()
     ids = tokens(n, vocab=203, seed=n)
     want = list(range(n - 3, n))
     whole = m.feed([0], [0], [ids], [want])

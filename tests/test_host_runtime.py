@@ -181,12 +181,13 @@ def every_tiling_is_tested(H):
         P.tiling_run(m, [[1] * n] * batch, n + 1, False)
         run |= _tilings(H.hh_launched())
         m.close()
-    m = S.wide_model()
-    for n in S.TILING_ROWS:
-        H.hh_launched()
-        m.feed([0], [0], [[1] * n])
-        run |= _tilings(H.hh_launched())
-    m.close()
+    for model, rows in ((S.wide_model, S.TILING_ROWS), (S.middle_model, [700])):
+        m = model()
+        for n in rows:
+            H.hh_launched()
+            m.feed([0], [0], [[1] * n])
+            run |= _tilings(H.hh_launched())
+        m.close()
     held = _tilings(H.hh_kernels())
     assert len(held) > 20 and run == held, sorted(held - run)
 
@@ -207,6 +208,28 @@ def stack_prompts_take_the_fast_tilings(H):
         m.feed([0], [0], [[1] * n])
         ran = _tilings(H.hh_launched(), "HyOut")
         assert len(ran) == 1 and {(c[0], c[1], c[3]) for _, c in ran} <= fast, (D, n, ran)
+        m.close()
+
+
+# Prompts of Llama-2-7B: (weights, positions through the chunk, epilogue) -> (BM, WR, AT) of the tilings, each within 4 % of the
+# fastest at its best split. us of that tiling | of the one that stale stage times took: fp16 512 rows wo 39 | 43, down 79 | 103;
+# 64 rows down 28 | 33; int8 96 rows gate/up 45 | 54; fp32 512 rows gate/up 1024 | 1350, 96 rows gate/up 238 | 294
+PROMPT_TILES = {("f16", 512, "PgEpiResid"): {(128, 4, 2), (128, 4, 4)}, ("f16", 64, "PgEpiResid"): {(32, 2, 2), (64, 4, 2)},
+                ("i8", 96, "PgEpiSwiGLU"): {(96, 4, 3)}, ("f32", 512, "PgEpiSwiGLU"): {(128, 4, 2)},
+                ("f32", 96, "PgEpiSwiGLU"): {(32, 2, 4)}}
+
+
+def prompts_take_the_fast_tilings(H):
+    """The plans of a prompt's GEMMs take tilings that were within 4 % of the fastest."""
+    from tests import test_gpu_prefill as P
+    from simplellminference_amd.model import LlamaModel, preset
+    for (w, n, epi), fast in PROMPT_TILES.items():
+        m = LlamaModel(config=preset("llama2-7b", num_hidden_layers=1, vocab_size=500, max_length=600), w_dtype=w,
+                       kv_dtype="f32" if w == "f32" else "f16", seed=1).init()
+        H.hh_launched()
+        P.tiling_run(m, [[1] * (n + 1)], n + 1, False)
+        ran = {(c[0], c[1], c[3]) for _, c in _tilings(H.hh_launched(), epi)}
+        assert ran == fast, (w, n, epi, ran)
         m.close()
 
 
@@ -258,8 +281,8 @@ def steps_of_the_batched_projection(H):
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts",
-         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "fp32_output_projection_steps",
-         "steps_of_the_batched_projection"]
+         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
+         "fp32_output_projection_steps", "steps_of_the_batched_projection"]
 
 
 @pytest.fixture(scope="module")

@@ -1,7 +1,8 @@
 // pgemm_lab — the tilings of the prompt GEMM (csrc/prefill.h pg_tilings, pg_row_tilings):
 //   pgemm_lab M [splits ...]  device time per launch at M rows of the 7B projections (HIP events, 20 launches, weights
 //                             streamed from HBM), issued MFMA TFLOP/s, a spot check of 64 outputs against a host fp64 sum.
-//                             splits 0 = the plan, 1 = whole tiles, n = the last round's tiles cut into n
+//                             splits 0 = the plan, 1 = whole tiles, n = the last round's tiles cut into n. Each projection
+//                             ends with the tiling that the engine takes, its time and the fastest
 //   pgemm_lab stages          time of one stage of every tiling with the chip full of whole tiles (two rounds over a depth
 //                             of 8192), weights read once (one position block) and shared by eight, beside the listed one
 // LAB_W: f16 (default), i8, f32, or one (a single fp16 image: the block stacks' tilings).
@@ -110,18 +111,22 @@ static void release(Bufs<WT>& b) {
 
 static float* g_ws;
 static unsigned* g_cnt;
-// force: splits of every tile (0: the plan)
+struct Timed {
+    std::string tag;
+    double us = 1e30;
+};
+// rows are padded to the tiling's; force: splits of the last round's tiles (0: the plan); returns the time and what it is of
 template <class Cfg, typename WT>
-static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force = 0) {
+static Timed run(const char* name, Bufs<WT>& b, const Shape& sh, int rows, int force, float stage) {
     using Geo = PgGeo<Cfg, WT>;
-    if (M % Geo::BM) return;
-    PgPlan pl = pg_plan<Cfg, WT>(sh.N, sh.K, M, 256, true);
+    const int M = (rows + Geo::BM - 1) / Geo::BM * Geo::BM;
+    PgPlan pl = pg_plan<Cfg, WT>(sh.N, sh.K, M, 256, true, stage);
     if (force) {
         const int nx = ((sh.N + Geo::BN - 1) / Geo::BN + 7) / 8 * (M / Geo::BM), f = nx / (32 * (160 * 1024 / Geo::LDS)) * (32 * (160 * 1024 / Geo::LDS));
         if (force == 1) pl.full = 0x7fffffff, pl.splits = 1, pl.slots = nx;
         else pl.full = f, pl.splits = force, pl.slots = f + (nx - f) * force;
-        if ((size_t)8 * (nx - f) * force * 16 * Geo::AT * Geo::WPT * Geo::THREADS > kPgWsBytes || (sh.K + Geo::KS - 1) / Geo::KS < force) return;
-        if (force > 1 && nx == f) return;
+        if ((size_t)8 * (nx - f) * force * 16 * Geo::AT * Geo::WPT * Geo::THREADS > kPgWsBytes || (sh.K + Geo::KS - 1) / Geo::KS < force) return {};
+        if (force > 1 && nx == f) return {};
     }
     char tag[96];
     snprintf(tag, sizeof tag, "%s full %d S %d", name, pl.full > 100000 ? -1 : pl.full, pl.splits);
@@ -138,7 +143,7 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
     double maxrel = 0.0;
     uint64_t s = 777;
     for (int i = 0; i < 64; ++i) {
-        const int m = rng(s) % M, row = rng(s) % sh.N;
+        const int m = rng(s) % rows, row = rng(s) % sh.N;
         double ref = 0.0, mag = 0.0;
         for (int k = 0; k < sh.K; ++k) {
             double w;
@@ -175,6 +180,7 @@ static void run(const char* name, Bufs<WT>& b, const Shape& sh, int M, int force
     fflush(stdout);
     CK(hipEventDestroy(e0));
     CK(hipEventDestroy(e1));
+    return {tag, us};
 }
 
 template <class Cfg>
@@ -194,10 +200,19 @@ static void each(bool one, int M, F&& f) {
 template <typename WT>
 static void sweep(const Shape& sh, int M, const std::vector<int>& forces, bool one) {
     Bufs<WT> b;
-    make(b, sh.N, sh.K, M);
-    each<WT>(one, M, [&](auto cfg, float) {
-        for (int f : forces) run<decltype(cfg), WT>(name_of(cfg).c_str(), b, sh, M, f);
+    make(b, sh.N, sh.K, M + 128);
+    Timed pick, best;
+    float least = INFINITY;
+    each<WT>(one, M, [&](auto cfg, float us) {
+        using Cfg = decltype(cfg);
+        for (int f : forces) {
+            const Timed t = run<Cfg, WT>(name_of(cfg).c_str(), b, sh, M, f, us);
+            if (t.us < best.us) best = t;
+            const float p = pg_plan<Cfg, WT>(sh.N, sh.K, (M + Cfg::BM - 1) / Cfg::BM * Cfg::BM, 256, true, us).us;
+            if (f == 0 && p < least) least = p, pick = t;
+        }
     });
+    printf("%-5s taken: %s %.1f us (%.1f planned); fastest: %s %.1f us\n", sh.name, pick.tag.c_str(), pick.us, least, best.tag.c_str(), best.us);
     release(b);
 }
 
