@@ -1079,7 +1079,7 @@ struct StepRecorder {
             const int M = (in.valid + Geo::BM - 1) / Geo::BM * Geo::BM;
             // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
             // in 16 ranges and more
-            if (st.nseq > 1 && Geo::FOLD == 0) us = INFINITY;
+            if (Geo::FOLD == 0 && (st.nseq > 1 || !pg_one_chain(N, K, in.valid))) us = INFINITY;
             const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true, us);
             if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
             ++i;

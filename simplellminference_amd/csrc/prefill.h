@@ -154,7 +154,8 @@ static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* 
 
 // ---------------------------------------------------------------- 2. the GEMM
 // LDS-DMA of one 1-KiB fragment image: lane i's 16 bytes at gsrc land at LDS byte lds + 16 i (inline asm: the
-// compiler neither counts nor drains it; the kernel counts its own vmcnt).
+// compiler neither counts nor drains it; the kernel counts its own vmcnt). m0 is named as written, so the compiler sets it
+// anew for its own uses.
 __device__ __forceinline__ void pf_dma(const void* gsrc, unsigned lds) {
     asm volatile(
         "s_mov_b32 m0, %1\n\t"
@@ -211,7 +212,9 @@ struct PgIn {
 // barrier too.
 // SA_ > 0: the weight (A) images get a ring of their own, SA_ stages deep (SA_ - 1 issued ahead), and
 // the activation (B) images a 2-stage ring (one ahead): the A bytes come from HBM (read once per chunk), the B bytes
-// from L2, so only A needs the deep prefetch, and B, the larger image, does not pay for it in LDS.
+// from L2, so only A needs the longer prefetch, and B, the larger image, does not pay for it in LDS. Loads are waited for in
+// order and every stage's activations are waited for, so a weight stage has two iterations to land whatever SA_ is: a fourth
+// slot holds a stage that has landed.
 // NB_: activation images per position: 2 (fp16 hi + lo, two MFMAs per product) or 1 (fp16 activations).
 // GR_: row blocks with weights of their own (PgGroups; one image).
 // FO_: short chains (PgGeo::FOLD) for a 64 x 64 wave tile too.
@@ -493,11 +496,11 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
     };
     // MFMAs of fragments f in slices of AT (one activation fragment each), between them the reads of the next k-block into n
     // and DMA pieces j0 .. j1 - 1 of iteration s: a wave issues them in the 12 cycles that an MFMA holds the matrix pipe
-    // after its issue. The order is fixed (sched_barrier, every 4 MFMAs or more): left to itself the compiler gathered a
-    // set's reads behind the MFMAs they should run beside, each wait for LDS then stood open, and the 16 DMA pieces stood
-    // in front. 512 rows, 7B q/k/v | gate/up | wo | down: 109 | 207 | 45 | 96 -> 93 | 181 | 42 | 84 us; 2048 rows 413 | 754 |
-    // 130 | 373 -> 377 | 670 | 109 | 327 (1260 TFLOP/s). The clock then falls from 2.0 to 1.66 GHz (MFMAs on random data
-    // alone hold 1.74 PFLOP/s): more waves, s_setprio and 128-row wave tiles measured the same.
+    // after its issue. The order is fixed (sched_barrier, every 4 MFMAs or, of slices of 3, every 3): left to itself the
+    // compiler gathered a set's reads behind the MFMAs they should run beside, each wait for LDS then stood open, and the 16
+    // DMA pieces stood in front. 128 x 192 tiles, 7B q/k/v | gate/up at 512 rows 92 | 188 -> 83 | 166 us; 128 x 256, gate/up
+    // at 2048 rows 754 -> 670 (1260 TFLOP/s). The clock then falls from 2.0 to 1.66 GHz (MFMAs on random data alone hold 1.74
+    // PFLOP/s): more waves, s_setprio and 128-row wave tiles measured the same.
     // PAIR: where a second workgroup runs on the CU and the ring has two stages, the order is the compiler's and the DMA goes
     // first: the other workgroup's MFMAs run beside the reads, and the next stage needs all of the time there is to land
     // (128 x 128 of a stack, 5120 x 18944 at 1536 rows: 315 -> 283 us).
@@ -898,6 +901,12 @@ hipError_t pgemm_allow_lds() {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(&pgemm_kernel<Epi, Cfg, WT>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)PgGeo<Cfg, WT>::LDS);
 }
+
+// Where a prompt's GEMM may sum in one chain over its depth or split (PgGeo::FOLD 0: the 128 x 256 tiling, 4 % faster than with
+// short chains): what long prompts spend their time on, gate/up from 769 rows and depths of 8192 and more from 1537. Llama-2-7B,
+// relative error of the logits against float64, so | wherever it is the fastest: 512 tokens 4.4e-5 | 4.9e-5, 700 4.1e-5 |
+// 5.8e-5, 1025 4.0e-5 | 4.8e-5, 2000 4.5e-5 | 4.5e-5.
+inline bool pg_one_chain(int N, int K, int rows) { return (N >= 16384 && rows > 768) || (K >= 8192 && rows > 1536); }
 
 // The tilings of the Llama prompts, f(PgCfg<...>{}, us): us is a stage of the tiling as pg_plan counts it. A launch takes the
 // tiling whose plan costs least (rounds over the rows padded to its BM, the last round's tiles cut over the depth).

@@ -303,12 +303,12 @@ TILING_SHAPES = [("f16", "llama2-7b", 1, 10), ("f16", "llama2-7b", 1, 74), ("f16
                  ("i8", "llama2-7b", 1, 10), ("i8", "llama2-7b", 1, 50), ("i8", "llama2-7b", 1, 74), ("i8", "llama2-7b", 1, 130),
                  ("i8", "llama3-8b", 1, 120), ("i8", "llama3-8b", 1, 130), ("i8", "llama3-8b", 1, 200), ("f32", "llama2-7b", 1, 18),
                  ("f32", "llama2-7b", 1, 50), ("f32", "llama2-7b", 1, 74), ("f32", "llama3-8b", 1, 20), ("f32", "llama3-8b", 1, 104),
-                 ("i8", "llama3-8b", 1, 10), ("i8", "small-h128", 1, 10)]
+                 ("i8", "llama3-8b", 1, 10), ("i8", "small-h128", 1, 10), ("f16", "llama2-7b", 1, 800)]
 
 
-def tiling_model(w, name, batch):
+def tiling_model(w, name, batch, n=400):
     from simplellminference_amd.model import LlamaModel, preset
-    return LlamaModel(config=preset(name, num_hidden_layers=2, vocab_size=500, max_length=416), w_dtype=w,
+    return LlamaModel(config=preset(name, num_hidden_layers=2, vocab_size=500, max_length=max(400, n) + 16), w_dtype=w,
                       kv_dtype="f32" if w == "f32" else "f16", seed=12, batch=batch).init()
 
 
@@ -327,7 +327,7 @@ def test_prefill_every_tiling(gpu, w, name, batch, n):
     cache's roundings either way make, fp32 within 2e-6 (sums of up to 14336 products in another order). The second layer's
     cache rows follow from the first's, whose values round either way: within one fp16 rounding of the largest, and in norm
     below 2^-12 (2^-11 / sqrt 3 would be every value rounded the other way). fp32 rows: 2^-14."""
-    m = tiling_model(w, name, batch)
+    m = tiling_model(w, name, batch, n)
     prompts = [_prompt(n + b, m.config.vocab_size)[b:] for b in range(batch)]
     want, wl = tiling_run(m, prompts, n + 1, True)
     rows = lambda: [m.kv(1, which, n, seq=b) for b in range(batch) for which in (0, 1)]

@@ -176,7 +176,7 @@ def every_tiling_is_tested(H):
     H.hh_launched()
     run = set()
     for w, name, batch, n in P.TILING_SHAPES:
-        m = P.tiling_model(w, name, batch)
+        m = P.tiling_model(w, name, batch, n)
         H.hh_launched()
         P.tiling_run(m, [[1] * n] * batch, n + 1, False)
         run |= _tilings(H.hh_launched())
@@ -233,6 +233,20 @@ def prompts_take_the_fast_tilings(H):
         m.close()
 
 
+def short_prompts_sum_in_short_chains(H):
+    """GEMMs that sum in one chain over the depth: none up to 769 tokens, gate/up alone up to 1537, then down too."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset("llama2-7b", num_hidden_layers=1, vocab_size=500, max_length=2100), seed=1).init()
+    chain = lambda names, epi: any(c[3] == 4 and c[5] == 2 and not c[7] for _, c in _tilings(names, epi))
+    for n, gate_up, down in ((513, False, False), (701, False, False), (769, False, False), (1025, True, False),
+                             (1537, True, False), (2049, True, True)):
+        H.hh_launched()
+        m.prefill([1] * n)
+        names = H.hh_launched()
+        assert (chain(names, "PgEpiSwiGLU"), chain(names, "PgEpiResid"), chain(names, "PgEpiQKV")) == (gate_up, down, False), n
+    m.close()
+
+
 def fp32_output_projection_steps(H):
     """A fp32 output projection reads 8 vectors a lane and step only where a wave has two whole such steps (of 2048 columns):
     one rank of 4096 columns, not the ranks of 512 to 2048 of a group, nor a width that they do not divide."""
@@ -282,6 +296,7 @@ def steps_of_the_batched_projection(H):
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
+         "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
 
 

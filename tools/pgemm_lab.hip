@@ -207,6 +207,7 @@ static void sweep(const Shape& sh, int M, const std::vector<int>& forces, bool o
         using Cfg = decltype(cfg);
         for (int f : forces) {
             const Timed t = run<Cfg, WT>(name_of(cfg).c_str(), b, sh, M, f, us);
+            if (!one && PgGeo<Cfg, WT>::FOLD == 0 && !pg_one_chain(sh.N, sh.K, M)) continue;  // (listed, not taken)
             if (t.us < best.us) best = t;
             const float p = pg_plan<Cfg, WT>(sh.N, sh.K, (M + Cfg::BM - 1) / Cfg::BM * Cfg::BM, 256, true, us).us;
             if (f == 0 && p < least) least = p, pick = t;
