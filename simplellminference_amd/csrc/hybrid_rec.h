@@ -64,14 +64,15 @@ struct HyProj {
             in.ws = s->pg_ws, in.cnt = s->pg_cnt;
             float best = INFINITY;
             int pick = 0, i = 0;
-            pg_row_tilings(M, [&](auto cfg, float us) {
-                const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true, us, PgRolled<PgPair<Epi>>::value);
+            constexpr bool rolled = PgRolled<PgPair<Epi>>::value;
+            pg_row_tilings(M, rolled, [&](auto cfg, float us) {
+                const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true, us, rolled);
                 if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits;
                 ++i;
             });
             hipError_t err = hipSuccess;
             i = 0;
-            pg_row_tilings(M, [&](auto cfg, float) {
+            pg_row_tilings(M, rolled, [&](auto cfg, float) {
                 if (i++ == pick) err = launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, u0}, PfState{}, st());
             });
             SLI_HIP(err);
@@ -85,7 +86,7 @@ struct HyProj {
         if constexpr (F16) {
             hipError_t err = hipSuccess;
             for (int M : {32, 256})
-                pg_row_tilings(M, [&](auto cfg, float) {
+                pg_row_tilings(M, false, [&](auto cfg, float) {
                     const hipError_t e = pgemm_allow_lds<PgPair<Epi>, decltype(cfg), __half>();
                     if (e != hipSuccess) err = e;
                 });

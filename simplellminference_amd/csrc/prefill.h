@@ -860,7 +860,8 @@ constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
 // plan that costs least is the fastest one: over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken takes
 // 1.1 % longer than the fastest, of int8 0.4, of fp32 0.7, of block stacks 1.9 % (tools/pgemm_lab prints both).
 // rolled: a looped epilogue (kRolled) takes time by the tiles a wave loops over: a stack's 25600 x 3072 at 384 rows 100.6 us in
-// 128 x 256 tiles (16 a wave), 95.9 in 128 x 128 (8), with a plain epilogue 84 and 90. 0.5 us each is what picks best.
+// 128 x 256 tiles (16 a wave), 95.9 in 128 x 128 (8), with a plain epilogue 84 and 90. 0.7 us each, shared by the workgroups of
+// a CU, is what picks best.
 template <class Cfg, typename WT>
 PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled = false) {
     using Geo = PgGeo<Cfg, WT>;
@@ -868,7 +869,7 @@ PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled =
     const int ns = (K + Geo::KS - 1) / Geo::KS;
     const int occ = (int)((160 * 1024) / Geo::LDS), cpx = std::max(1, cus / 8) * occ;
     constexpr float kTile = 16.0f * Geo::AT * Geo::WPT * Geo::THREADS / 131072.0f, kEdge = 2.0f + 6.0f * kTile;
-    const float epi = rolled ? 0.5f * Geo::AT * Geo::WPT : 0.0f;
+    const float epi = rolled ? 0.7f * Geo::AT * Geo::WPT / (float)occ : 0.0f;
     PgPlan best;
     best.slots = nx;
     best.us = (float)((nx + cpx - 1) / cpx) * ((float)ns * stage + kEdge + epi);
@@ -941,12 +942,13 @@ void pg_tilings(F&& f) {
 // us, as above: 1024 rows 272 | 127 against 300 | 142; 256 rows 106 | 52 against 116 | 73; 64 rows 62 | 32 against 73 | 75.
 // Two workgroups of 128 x 128 on a CU are the fastest where tiles twice as wide leave half a round empty: 3072 x 11264 at 768
 // rows 75, the others 86 and more; 11264 x 1024 at 1408 rows 40, the others 46. The 32-row tiles read weights and little else,
-// whatever a stage takes alone: theirs are the values that pick the faster one at 32 rows.
+// whatever a stage takes alone: theirs are the values that pick the faster one at 32 rows. With a looped epilogue (rolled) pairs
+// of 128 x 128 gain less: 22528 x 2048 at 768 rows 117 us where 128 x 256 takes 106.
 template <class F>
-void pg_row_tilings(int M, F&& f) {
+void pg_row_tilings(int M, bool rolled, F&& f) {
     if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.3f);
-    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 0.76f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, 1.05f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.52f);
-    if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.49f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 0.76f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, rolled ? 1.3f : 1.05f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.52f);
+    if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.46f);
     if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.42f);
     if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.4f);
 }

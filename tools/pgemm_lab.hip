@@ -193,7 +193,7 @@ static std::string name_of(Cfg) {
 template <typename WT, class F>
 static void each(bool one, int M, F&& f) {
     if constexpr (sizeof(WT) == 2)
-        if (one) return M ? pg_row_tilings(M, f) : (pg_row_tilings(32, f), pg_row_tilings(256, f));
+        if (one) return M ? pg_row_tilings(M, false, f) : (pg_row_tilings(32, false, f), pg_row_tilings(256, false, f));
     pg_tilings<WT>(f);
 }
 
