@@ -857,8 +857,9 @@ constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
 // stage: us of a stage of the tiling (pg_tilings). Around its walk of the depth a workgroup takes 2 us and 6 for 128 KiB of sums
 // (a 128 x 256 tile): dispatch, the ring's first stages, the epilogue; a cut round 2 us, 0.6 for each split and 1.5 for each
 // split's and two more 128 KiB: the partial sums' way out and back. These and the stage times are fitted together, so that the
-// plan that costs least is the fastest one: over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken takes
-// 1.1 % longer than the fastest, of int8 0.4, of fp32 0.7, of block stacks 1.9 % (tools/pgemm_lab prints both).
+// plan that costs least is the fastest one, and are no times of their own (a large product's stages last longer: the clock
+// falls). Over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken lasts 1.1 % longer than the fastest, of
+// int8 0.4, of fp32 0.8, of block stacks 2 % (tools/pgemm_lab prints both).
 // rolled: a looped epilogue (kRolled) takes time by the tiles a wave loops over: a stack's 25600 x 3072 at 384 rows 100.6 us in
 // 128 x 256 tiles (16 a wave), 95.9 in 128 x 128 (8), with a plain epilogue 84 and 90. 0.7 us each, shared by the workgroups of
 // a CU, is what picks best.
@@ -912,9 +913,9 @@ inline bool pg_one_chain(int N, int K, int rows) { return (N >= 16384 && rows > 
 // The tilings of the Llama prompts, f(PgCfg<...>{}, us): us is a stage of the tiling as pg_plan counts it. A launch takes the
 // tiling whose plan costs least (rounds over the rows padded to its BM, the last round's tiles cut over the depth).
 // Llama-2-7B, q/k/v | gate/up | wo | down, us, what the plan takes against the best tiling in whole tiles
-// (profiles/pgemm_tilings.txt): 512 rows 83 | 155 | 39 | 79 against 83 | 160 | 40 | 106; 64 rows 30 | 44 | 13 | 28 against 39 |
-// 46 | 20 | 55; int8 64 rows 26 | 35 | 14 | 25 against 30 | 38 | 25 | 61; fp32 96 rows 145 | 238 | 54 | 122 against 194 | 328 |
-// 97 | 256.
+// (profiles/pgemm_tilings.txt): 512 rows 86 | 187 | 38 | 88 against 86 | 183 | 40 | 110; 64 rows 28 | 42 | 13 | 28 against 39 |
+// 46 | 19 | 56; int8 64 rows 24 | 36 | 15 | 24 against 32 | 41 | 26 | 65; fp32 96 rows 157 | 248 | 56 | 137 against 194 | 335 |
+// 98 | 260. In the engine (profiles/prompt_7b_f16_512_kernel_stats.csv) 512 rows take 97 | 184 | 44 | 95.
 // The int8 tilings with a weight ring of their own (SA 3) have two stages of the weights in flight instead of one (a wave waits
 // for its loads in order, so for all weights issued before the activations it needs: a deeper ring holds stages that have
 // landed); 64 rows: gate/up 39.1 -> 36.2, q/k/v 24.8 -> 24.4, down 25.2 -> 23.7; 192 rows: q/k/v of 96 x 128 tiles 54.8 ->
@@ -939,7 +940,7 @@ void pg_tilings(F&& f) {
 }
 
 // The tilings of block-stack prompts (one fp16 image; their row count divides M). 34304 x 4096 and 4096 x 15104,
-// us, as above: 1024 rows 272 | 127 against 300 | 142; 256 rows 106 | 52 against 116 | 73; 64 rows 62 | 32 against 73 | 75.
+// us, as above: 1024 rows 321 | 138 against 352 | 147; 256 rows 108 | 53 against 120 | 73; 64 rows 64 | 34 against 75 | 74.
 // Two workgroups of 128 x 128 on a CU are the fastest where tiles twice as wide leave half a round empty: 3072 x 11264 at 768
 // rows 75, the others 86 and more; 11264 x 1024 at 1408 rows 40, the others 46. The 32-row tiles read weights and little else,
 // whatever a stage takes alone: theirs are the values that pick the faster one at 32 rows. With a looped epilogue (rolled) pairs
@@ -947,7 +948,8 @@ void pg_tilings(F&& f) {
 template <class F>
 void pg_row_tilings(int M, bool rolled, F&& f) {
     if (M % 256 == 0) f(PgCfg<256, 4, 2, 4, 0, 1>{}, 1.3f);
-    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 0.76f), f(PgCfg<128, 4, 2, 2, 0, 1>{}, rolled ? 1.3f : 1.05f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.52f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 3, 4, 0, 1>{}, 0.76f), f(PgCfg<128, 2, 3, 4, 0, 1>{}, 0.52f);
+    if (M % 128 == 0) f(PgCfg<128, 4, 2, 2, 0, 1>{}, rolled ? 1.3f : 1.05f);
     if (M % 64 == 0) f(PgCfg<64, 2, 4, 2, 0, 1>{}, 0.46f);
     if (M < 64) f(PgCfg<32, 2, 4, 2, 0, 1>{}, 0.42f);
     if (M % 64 != 0) f(PgCfg<32, 2, 4, 4, 0, 1>{}, 0.4f);
