@@ -35,6 +35,7 @@
 #include "prefill.h"
 #include "qkv_attn.h"
 #include "rope_table.h"
+#include "small_launch.h"
 #include "step_state.h"
 #include "tp_layers.h"
 
@@ -137,6 +138,14 @@ struct sli_model {
         unsigned* epoch = nullptr;
         sli::tl_u2** xg = nullptr;
     } tl;
+    // predict's greedy loop as one launch (small_model.h): granules and weight table (null: the model takes the steps)
+    struct Small {
+        sli::sm_u2* g = nullptr;
+        const void** w = nullptr;
+        size_t granules = 0;
+        int nwg = 0;
+        unsigned tag = 4;  // the next launch's first tag
+    } sm;
 };
 
 // In-process tensor parallelism (a "fake communicator"): tp_size rank models on
@@ -608,6 +617,65 @@ static int tpl_launch(sli_model* m) {
     return SLI_OK;
 }
 
+// ---------------------------------------------------------------- a small model's greedy loop as one launch
+// Workgroups, of which every one sweeps every edge: 256-wide fp32 preset, us a step with 16 | 32 | 64 | 128 of them 39.7 | 27.4 |
+// 28.4 | 35.9, 512-wide 86 | 49 | 34.3 | 32.2. The graph's steps take 68.7 and 68.2. Models of 1024 take 77 as launches and 92 here
+// (a wave's rows of an op no longer fit its LDS), so they keep them.
+constexpr int kSmWgs = 64;
+// K of a head's context, which each of its workgroups reads: at 1000 positions of 64 (fp32) a step takes 6 us longer than at 36,
+// at 2048 about 24 and the launches are as fast soon after.
+constexpr size_t kSmMaxKey = 512 << 10;
+
+// Scratch at creation, tens of KB, where the model takes that path (null otherwise)
+static int small_alloc(sli_model* m) {
+    const int wd = m->c.w_dtype;
+    if (m->B != 1 || m->partial || m->group || m->bs || wd == SLI_DT_I8 || m->D > kSmMaxD || m->Il > kSmMaxI || m->D % 8 || m->Il % 8) return SLI_OK;
+    int J = 1;
+    while (m->hq * J * 2 <= kSmWgs) J *= 2;
+    const int nwg = m->hq * J, hd = m->hd;
+    if (nwg > kSmWgs || m->D < nwg || m->Il < nwg || nwg > device_cus()) return SLI_OK;
+    m->sm.granules = (size_t)(m->hq + 2 * m->hkv) * hd + (size_t)m->hq * m->D + m->Il + m->D + 2 * nwg;
+    SLI_TRY(model_alloc(m, (void**)&m->sm.g, 8 * m->sm.granules));
+    SLI_HIP(hipMemset(m->sm.g, 0, 8 * m->sm.granules));
+    std::vector<const void*> w;
+    for (const LayerW& l : m->layers) w.insert(w.end(), {l.qkv, l.wo, l.gu, l.down});
+    const void** wt = nullptr;
+    SLI_TRY(model_alloc(m, (void**)&wt, sizeof(void*) * w.size()));
+    SLI_HIP(hipMemcpy(wt, w.data(), sizeof(void*) * w.size(), hipMemcpyHostToDevice));
+    SLI_HIP(small_allow(wd, m->c.kv_dtype, hd));
+    m->sm.w = wt;
+    m->sm.nwg = nwg;
+    return SLI_OK;
+}
+
+// Whether positions below `length` take that launch
+static bool small_takes(const sli_model* m, int length) {
+    return m->sm.w && m->exec == SLI_EXEC_LAUNCHES && (size_t)length * m->hd * m->kvbytes <= kSmMaxKey;
+}
+
+// n steps from the device's state on, as one launch
+static int small_steps(sli_model* m, int n) {
+    const unsigned need = 4u * (unsigned)n * (unsigned)(m->L + 1);
+    if (m->sm.tag + need < m->sm.tag) {  // (the tags wrap: none of the old ones may be left)
+        SLI_HIP(hipMemsetAsync(m->sm.g, 0, 8 * m->sm.granules, m->stream));
+        m->sm.tag = 4;
+    }
+    SmArgs a{};
+    a.D = m->D, a.hq = m->hq, a.hkv = m->hkv, a.hd = m->hd, a.I = m->Il, a.L = m->L, a.T = m->T, a.V = m->V, a.nwg = m->sm.nwg;
+    a.act_mode = m->c.act_mode, a.n = n, a.eps = m->c.eps, a.scale = 1.0f / sqrtf((float)m->hd);
+    a.w = m->sm.w, a.emb = m->emb, a.norms = m->norms, a.kc = m->kc, a.vc = m->vc, a.sin_t = m->sin_t, a.cos_t = m->cos_t;
+    a.st = m->st, a.prompt = m->prompt, a.hist = m->hist, a.logits = m->logits;
+    a.g_qkv = m->sm.g;
+    a.g_wo = a.g_qkv + (size_t)(m->hq + 2 * m->hkv) * m->hd;
+    a.g_act = a.g_wo + (size_t)m->hq * m->D;
+    a.g_x = a.g_act + m->Il;
+    a.g_key = a.g_x + m->D;
+    a.tag0 = m->sm.tag;
+    m->sm.tag += need;
+    SLI_HIP(small_launch(a, m->c.w_dtype, m->c.kv_dtype, m->hd, m->stream));
+    return SLI_OK;
+}
+
 // rows of the row-wise launches for a chunk of n rows. A GEMM pads them to its own tiles: the buffers have kPfPad more.
 static int pf_rows(int n) { return (n + 31) / 32 * 32; }
 constexpr int kPfPad = 128;
@@ -1066,9 +1134,9 @@ struct StepRecorder {
     // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); the last prompt
     // position runs as an ordinary decode step. Phases as record_phase: 2l = qkv, attention, wo; 2l+1 =
     // gate/up, down; under tensor parallelism each ends with the all-reduce of the chunk's residual rows.
-    // kv_only: the last layer. Nothing reads its residual rows, so it ends with the K and V rows that the cache keeps (the
-    // attention, wo, gate/up and down of one layer in 32: 512 tokens of Llama-2-7B 17.01 -> 16.57 ms). A model of one layer, which only serves
-    // to look at that layer's launches, runs it whole.
+    // kv_only: the last layer. Nothing reads its residual rows, so it ends with the K and V rows that the cache keeps (no
+    // attention, wo, gate/up and down of one layer in 32: 512 tokens of Llama-2-7B 17.01 -> 16.57 ms). A model of one layer,
+    // which only serves to look at that layer's launches, runs it whole.
     // one GEMM over a chunk's rows: the tiling (prefill.h pg_tilings) whose plan costs least over the rows padded to its BM
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
@@ -1699,6 +1767,7 @@ static int create_model(const sli_model_config* cfg, const void* comm_id, sli_tp
     m->wo_merge = m->B == 1 ? wo_merges(m) : 1;
     m->wo_ks = wo_ksplit(m);
     if (m->wo_ks > 1 && (rc = model_alloc(m, (void**)&m->wo_part, sizeof(float) * m->wo_ks * D)) != SLI_OK) return bail(rc);
+    if ((rc = small_alloc(m)) != SLI_OK) return bail(rc);
     *out = m;
     return SLI_OK;
 }
@@ -2303,6 +2372,7 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     }
     // (the prompt positions' logits come from the steps)
     int n0 = logits_out || m->bs ? 0 : pf_predict_positions(m, lens, max_length);
+    const bool wants_chunks = n0 > 0;
     if (n0 > 0) SLI_TRY(pf_ready(m));
     if (m->pf.cap == 0) n0 = 0;
     if (n0 > 0) {
@@ -2315,6 +2385,18 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
         SLI_TRY(set_state(m, b, prompts[(size_t)b * ld + n0], n0, 1));
     }
     const size_t per_step = (size_t)m->B * m->v_n;
+    // (scratch that did not fit leaves the steps; so does a wait that gave up, which happens where other work keeps the
+    // launch's workgroups from running together)
+    bool loop = small_takes(m, max_length) && !logits_out && (n0 > 0 || !wants_chunks);
+    if (loop) {
+        SLI_TRY(small_steps(m, max_length - n0));
+        DevState d{};
+        SLI_HIP(hipMemcpyAsync(&d, m->st, sizeof(d), hipMemcpyDeviceToHost, m->stream));
+        SLI_HIP(hipMemcpyAsync(tokens_out, m->hist, sizeof(int32_t) * max_length, hipMemcpyDeviceToHost, m->stream));
+        SLI_TRY(wait_stream(m));
+        if (!(d.error & kSmErrWait)) return d.error ? check_device_errors(m) : SLI_OK;
+        SLI_TRY(set_state(m, 0, prompts[n0], n0, 1));
+    }
     for (int t = n0; t < max_length; ++t) {  // model.cpp:157
         SLI_TRY(sli_model_step(m));
         if (logits_out) SLI_TRY(sli_model_get_logits(m, logits_out + (size_t)t * per_step, (int32_t)per_step, nullptr));

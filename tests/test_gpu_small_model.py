@@ -1,0 +1,54 @@
+"""The greedy loop of a small model as one launch (csrc/small_model.h) against the same model's steps, launch by launch, which
+test_gpu_model.py holds to the oracle. Both compute in fp32 and differ in the order of their sums only."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(w, kv, **over):
+    from simplellminference_amd.model import LlamaModel, preset
+    return LlamaModel(config=preset("tiny-gqa", **over), w_dtype=w, kv_dtype=kv, seed=5).init()
+
+
+# heads of 64 and 128, one to eight queries a kv head, widths whose rows are no whole pieces, an FFN wider than the width, heads
+# that do not divide 64
+SHAPES = {"tiny": {}, "h128": dict(head_dim=128, hidden_size=512, kv_hidden_size=256, num_attention_heads=4, num_key_value_heads=2,
+                                   intermediate_size=1032, vocab_size=700),
+          "h8": dict(hidden_size=512, kv_hidden_size=64, num_attention_heads=8, num_key_value_heads=1, intermediate_size=2048),
+          "h6": dict(hidden_size=384, kv_hidden_size=192, num_attention_heads=6, num_key_value_heads=3, intermediate_size=520,
+                     num_hidden_layers=3, vocab_size=333),
+          "h1": dict(hidden_size=64, kv_hidden_size=64, num_attention_heads=1, num_key_value_heads=1, intermediate_size=72,
+                     num_hidden_layers=1, vocab_size=50)}
+
+
+@pytest.mark.parametrize("w,kv", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("f32", "f16")])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_loop_matches_steps(gpu, shape, w, kv):
+    m = _model(w, kv, max_length=150, **SHAPES[shape])
+    V = m.config.vocab_size
+    # one step; a prompt alone; past the keys of one pass (16 to 64) and of several; up to the last position
+    for n, length in ((1, 1), (3, 3), (2, 18), (7, 34), (5, 66), (4, 131), (1, 150)):
+        ids = [(13 * i + n) % V for i in range(n)]
+        want, wl = m.predict(ids, length, want_logits=True)
+        kv_want = [m.kv(m.config.num_hidden_layers - 1, which, length) for which in (0, 1)]
+        m.reset()
+        for _ in range(2):
+            assert np.array_equal(m.predict(ids, length), want), (n, length)
+            log = m.logits()[0]
+            # fp32 sums in another order (1e-6 of the norm); an fp16 cache rounds K and V either way (2^-11 of a value)
+            assert np.linalg.norm(log - wl[-1]) <= (5e-6 if kv == "f32" else 5e-4) * np.linalg.norm(wl[-1]), (n, length)
+            for which in (0, 1):
+                d = np.abs(m.kv(m.config.num_hidden_layers - 1, which, length) - kv_want[which]).max()
+                assert d <= (2e-5 if kv == "f32" else 1e-2), (n, length, which)
+        assert m.state()["pos"] == min(length, 149) and m.state()["error"] == 0
+    m.close()
+
+
+def test_context_beyond_the_loop(gpu):
+    """Contexts on both sides of the rule (512 KiB of a head's keys) give the same tokens."""
+    m = _model("f32", "f32", max_length=2100)
+    want = m.predict([3, 1, 4], 2100, want_logits=True)[0]
+    assert np.array_equal(m.predict([3, 1, 4], 2048), want[:2048])
+    assert np.array_equal(m.predict([3, 1, 4], 2049), want[:2049])
+    m.close()

@@ -156,6 +156,18 @@ def small_stacks_replay_their_prompts(H):
         m.close()
 
 
+def small_models_predict_in_one_launch(H):
+    """predict of a narrow model without logits is one launch; a wider one, a long context and int8 weights take the steps."""
+    for kw, n, steps in ((dict(w_dtype="f32", kv_dtype="f32"), 30, 0), (dict(w_dtype="f16"), 30, 0), (dict(w_dtype="i8"), 30, 30),
+                         (dict(w_dtype="f16", preset="tiny-h8"), 30, 0), (dict(w_dtype="f16", preset="small-h128"), 30, 30),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(max_length=2100)), 2049, 2049)):
+        m = _llama(**kw)
+        had = H.hh_graph_launches()
+        m.predict([1, 2, 3], n)
+        assert H.hh_graph_launches() - had == steps, (kw, n)
+        m.close()
+
+
 def _tilings(names, epilogue=""):
     """(weight type, tiling) of the prompt GEMM instances among kernel names, of one epilogue or all."""
     out = set()
@@ -294,7 +306,7 @@ def steps_of_the_batched_projection(H):
 
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
-         "callers_arrays_are_read", "small_stacks_replay_their_prompts",
+         "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
          "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
