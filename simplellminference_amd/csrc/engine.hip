@@ -113,6 +113,7 @@ struct sli_model {
         __half *hhi = nullptr, *hlo = nullptr, *ahi = nullptr, *alo = nullptr;
         float* ws = nullptr;                    // partial sums of the tiles that a GEMM cuts over its depth (PgIn::ws)
         unsigned* cnt = nullptr;
+        sli::PfPart part;                       // partial sums in ws that the next norm adds to x (PgIn::defer)
         int cap = 0;                            // positions of a chunk at most (0: none of this is allocated)
     } pf;
     // tensor-parallel all-reduce: SLI_ALLREDUCE_RCCL (ncclAllReduce) or SLI_ALLREDUCE_ONESHOT (oneshot.h)
@@ -677,6 +678,7 @@ static int small_steps(sli_model* m, int n) {
 }
 
 // rows of the row-wise launches for a chunk of n rows. A GEMM pads them to its own tiles: the buffers have kPfPad more.
+constexpr int kPfDeferRows = 128;  // rows of a chunk up to which wo and down leave cut sums to the next norm
 static int pf_rows(int n) { return (n + 31) / 32 * 32; }
 constexpr int kPfPad = 128;
 
@@ -1140,7 +1142,7 @@ struct StepRecorder {
     // one GEMM over a chunk's rows: the tiling (prefill.h pg_tilings) whose plan costs least over the rows padded to its BM
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
-                  const PfState& st) {
+                  const PfState& st, PfPart* part = nullptr) {
         PgIn<WT> in{(const WT*)W, hi, lo, N, K, 0};
         in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
         float best = INFINITY;
@@ -1155,6 +1157,13 @@ struct StepRecorder {
             if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
             ++i;
         });
+        // part: the launch may leave its sums to the next norm, where they are few (a merge in the GEMM is its last workgroups'
+        // store, arrival and load; in the norm it is a load): 45 rows of Llama-2-7B, wo and down with their norms 51.3 -> 46.6
+        // us, int8 46.4 -> 43.5, 100 rows 64.8 -> 61.5; at 511 rows nothing is left of it
+        if (part && in.full == 0 && in.splits > 1 && in.valid <= kPfDeferRows && (size_t)in.splits * in.M * N * sizeof(float) <= kPgWsBytes) {
+            in.defer = true;
+            *part = PfPart{in.ws, in.splits, (size_t)in.M * N, e.rscale};
+        }
         hipError_t err = hipSuccess;
         i = 0;
         pg_tilings<WT>([&](auto cfg, float) {
@@ -1194,8 +1203,11 @@ struct StepRecorder {
         PgEpiResid er{tp ? f.xpart : f.x, (!tp || m->c.tp_rank == 0) ? f.x : nullptr, nullptr, D, D};
         constexpr bool F32 = std::is_same<WT, float>::value;
         const PfOut h = F32 ? PfOut{nullptr, nullptr, (float*)f.hhi} : PfOut{f.hhi, f.hlo};
-        hipLaunchKernelGGL(pf_norm_split_kernel, dim3(M), dim3(256), 0, s, f.x, m->norms + (size_t)p * D, h, D, m->c.eps);
+        if (p == 0) f.part = {};
+        const auto norm = M <= kPfDeferRows ? &pf_norm_split_kernel<512> : &pf_norm_split_kernel<256>;
+        hipLaunchKernelGGL(norm, dim3(M), dim3(M <= kPfDeferRows ? 512 : 256), 0, s, f.x, m->norms + (size_t)p * D, h, D, m->c.eps, f.part);
         SLI_HIP(hipGetLastError());
+        f.part = {};
         if (p % 2 == 0) {
             const size_t ls = (size_t)l * m->B * m->hkv * m->T * hd;
             PgEpiQKV<KT> eq{f.q, (KT*)m->kc + ls, (KT*)m->vc + ls, w.qkv_s, m->sin_t, m->cos_t, m->hq, m->hkv, hd, m->T};
@@ -1218,12 +1230,12 @@ struct StepRecorder {
             }
             SLI_HIP(hipGetLastError());
             er.rscale = w.wo_s;
-            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, ps);
+            return pg(m, w.wo, D, QD, f.hhi, f.hlo, er, ps, tp ? nullptr : &f.part);
         }
         PgEpiSwiGLU eg{F32 ? PfOut{nullptr, nullptr, (float*)f.ahi} : PfOut{f.ahi, f.alo}, w.gu_s, m->Il, m->c.act_mode};
         SLI_TRY(pg(m, w.gu, 2 * m->Il, D, f.hhi, f.hlo, eg, ps));
         er.rscale = w.down_s;
-        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, ps);
+        return pg(m, w.down, D, m->Il, f.ahi, f.alo, er, ps, tp ? nullptr : &f.part);
     }
     static int record_prefill(sli_model* m, const PfState& ps) {
         const int M = pf_rows(ps.nseq == 1 ? ps.nv : ps.nseq * ps.rps);

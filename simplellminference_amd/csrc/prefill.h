@@ -109,41 +109,71 @@ __global__ void __launch_bounds__(256) pf_embed_kernel(PfState ps, const int32_t
     for (int i = threadIdx.x; i < D; i += 256) x[(size_t)m * D + i] = to_f32(emb[(size_t)tok * D + i]) * s;
 }
 
+// Partial sums of a GEMM that the next norm adds up (PgIn::defer): x += (part[0] + .. + part[n - 1]) * rscale, in x
+struct PfPart {
+    const float* part = nullptr;  // [n][rows][D]
+    int n = 0;
+    size_t stride = 0;  // rows D
+    const float* rscale = nullptr;
+};
+
 // one workgroup per chunk row: h = (x * 1/rms) * w (rms_kernel.cpp:12-22) or plain x (w == nullptr), as hi/lo.
 // The row is held in registers (a float4 per thread and pass; D % 4 == 0, D <= 8192): one read of x, 8-byte
-// hi / lo stores.
-static __global__ void __launch_bounds__(256) pf_norm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                           PfOut out, int D, float eps) {
-    constexpr int MAXV = 8;  // float4 per thread: D <= 8192
+// hi / lo stores. 512 threads a row for few rows (pp: more loads in flight: 45 rows 1 us less), 256 else.
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS) pf_norm_split_kernel(float* __restrict__ x, const float* __restrict__ w, PfOut out,
+                                                                int D, float eps, PfPart pp) {
+    constexpr int MAXV = 8192 / 4 / THREADS;  // float4 per thread: D <= 8192
+    constexpr int PB = 8;                     // partial sums in flight
     const int m = blockIdx.x;
-    const float* xr = x + (size_t)m * D;
+    float* xr = x + (size_t)m * D;
     const int n4 = D / 4;
     float4 v[MAXV], wv[MAXV];
     float ss = 0.0f;
     // the norm weights are loaded with x, not after the reduction: one memory round trip fewer
     const float4* w4 = reinterpret_cast<const float4*>(w ? w : xr);
 #pragma unroll
-    for (int j = 0; j < MAXV; ++j)
-        if (j * 256 + (int)threadIdx.x < n4) {
-            v[j] = reinterpret_cast<const float4*>(xr)[j * 256 + threadIdx.x];
-            wv[j] = w4[j * 256 + threadIdx.x];
+    for (int j = 0; j < MAXV; ++j) {
+        const int i = j * THREADS + (int)threadIdx.x;
+        if (i < n4) {
+            v[j] = reinterpret_cast<const float4*>(xr)[i];
+            wv[j] = w4[i];
+            if (pp.n) {
+                const float4* p4 = reinterpret_cast<const float4*>(pp.part + (size_t)m * D) + i;
+                const float4 sc = pp.rscale ? reinterpret_cast<const float4*>(pp.rscale)[i] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                for (int q0 = 0; q0 < pp.n; q0 += PB) {
+                    float4 t[PB];
+#pragma unroll
+                    for (int q = 0; q < PB; ++q) t[q] = p4[(size_t)min(q0 + q, pp.n - 1) * (pp.stride / 4)];
+#pragma unroll
+                    for (int q = 0; q < PB; ++q)
+                        if (q0 + q < pp.n) s.x += t[q].x, s.y += t[q].y, s.z += t[q].z, s.w += t[q].w;
+                }
+                if (pp.rscale) s.x *= sc.x, s.y *= sc.y, s.z *= sc.z, s.w *= sc.w;
+                v[j].x += s.x, v[j].y += s.y, v[j].z += s.z, v[j].w += s.w;
+                reinterpret_cast<float4*>(xr)[i] = v[j];
+            }
             ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
         }
+    }
     float inv = 1.0f;
     if (w) {
         ss = wave_sum(ss);
-        __shared__ float red[4];
+        __shared__ float red[THREADS / 64];
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
         __syncthreads();
-        const float t = red[0] + red[1] + red[2] + red[3];
+        float t = red[0];
+#pragma unroll
+        for (int k = 1; k < THREADS / 64; ++k) t += red[k];
         const float tep = t / (float)D;      // rms_kernel.cpp:17
         const float rms = sqrtf(tep + eps);  // :18
         inv = 1.0f / rms;                    // :19
     }
 #pragma unroll
     for (int j = 0; j < MAXV; ++j)
-        if (j * 256 + (int)threadIdx.x < n4) {
-            const int i = (j * 256 + threadIdx.x) * 4;
+        if (j * THREADS + (int)threadIdx.x < n4) {
+            const int i = (j * THREADS + threadIdx.x) * 4;
             const float f[4] = {v[j].x, v[j].y, v[j].z, v[j].w}, g[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
             float y[4];
 #pragma unroll
@@ -195,6 +225,8 @@ struct PgIn {
     int full = 0x7fffffff, splits = 1;
     float* ws = nullptr;
     unsigned* cnt = nullptr;
+    // (epilogues with kDefer, where every tile is cut) the sums stay partial: ws [split][M][N], for the launch that reads them
+    bool defer = false;
     int valid = 0x7fffffff;  // chunk rows from here on are padding: a wave that holds only such rows multiplies nothing
 };
 
@@ -309,6 +341,12 @@ __device__ __forceinline__ void pg_for(F&& f) {
     pg_for_seq<N>(f, std::make_integer_sequence<int, N>{});
 }
 #define PG_INLINE __attribute__((always_inline))
+
+// Epilogues with a member kDefer = true may leave a cut round's sums partial (PgIn::defer): row i of tile t is t * 16 + i
+template <class Epi, class = void>
+struct PgDefers : std::false_type {};
+template <class Epi>
+struct PgDefers<Epi, std::enable_if_t<Epi::kDefer>> : std::true_type {};
 
 // Epilogues with a member kRolled = true are looped over a wave's tiles instead of unrolled
 template <class Epi, class = void>
@@ -634,6 +672,23 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         phase(Y, X, nullptr, nullptr, std::integral_constant<int, -1>{}, none, none, 0);
         if constexpr (TWO) fold(acc, tot);
     }
+    const int i0 = 4 * (lane >> 4);  // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15
+    if constexpr (PgDefers<Epi>::value) {
+        if (nsp > 1 && in.defer) {
+            if (!live) return;
+#pragma unroll
+            for (int a = 0; a < AT; ++a) {
+                const int t = rb * Geo::NA + wr * AT + a;
+                if (t >= nt) continue;
+#pragma unroll
+                for (int b = 0; b < Geo::WPT; ++b) {
+                    const int m = pb * BM + (wp * Geo::WPT + b) * 16 + r16;
+                    *reinterpret_cast<pf_float4*>(in.ws + ((size_t)sp * in.M + m) * in.N + t * 16 + i0) = acc[a][b];
+                }
+            }
+            return;
+        }
+    }
     if (nsp > 1) {
         // Partial sums go out write-through (sc1); the tile's last workgroup to arrive adds them in split order (the
         // same sum whichever arrives last) and runs the epilogue.
@@ -697,8 +752,6 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             }
         }
     }
-    // C[i][n] of a 16x16 tile: lane l holds rows 4 (l >> 4) + r, column l & 15
-    const int i0 = 4 * (lane >> 4);
     if constexpr (PgRolled<Epi>::value) {
         // an epilogue too large to be unrolled over the tiles: a loop over them, the sums indexed in the ring's LDS
         // (indexed registers would live in scratch)
@@ -828,6 +881,7 @@ struct PgEpiResid {  // y[m][row] = resid[m][row] + sum * row scale (matmul_kern
     const float* resid;  // the residual stream (tensor-parallel ranks > 0: null, their partial has none)
     const float* rscale;
     int nrows, ld;
+    static constexpr bool kDefer = true;
     __device__ int row(int t, int i) const { return min(t * 16 + i, nrows - 1); }
     __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
         const int row = t * 16 + i0;  // rows row .. row + 3 (nrows % 16 == 0: the host's check)

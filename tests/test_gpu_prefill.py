@@ -345,6 +345,28 @@ def test_prefill_every_tiling(gpu, w, name, batch, n):
     m.close()
 
 
+@pytest.mark.parametrize("w", ["f16", "i8", "f32"])
+def test_prefill_sums_left_to_the_norm(gpu, w):
+    """wo and down of chunks up to 128 rows leave cut sums (int8: unscaled) to the next norm, of 129 rows they merge them: three
+    layers, so that both hand over, in chunks on both sides. Bars as above; a third layer's cache rows follow from two."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset("llama2-7b", num_hidden_layers=3, vocab_size=500, max_length=140), w_dtype=w,
+                   kv_dtype="f32" if w == "f32" else "f16", seed=4).init()
+    for n in (10, 47, 129, 130):
+        prompt = _prompt(n, 500)
+        want, wl = tiling_run(m, [prompt], n + 1, True)
+        kv = [m.kv(2, which, n) for which in (0, 1)]
+        m.reset()
+        got = tiling_run(m, [prompt], n + 1, False)
+        assert np.array_equal(got, want), n
+        assert np.linalg.norm(m.logits()[0] - wl[-1]) <= (2e-6 if w == "f32" else 8e-4) * np.linalg.norm(wl[-1]), n
+        for which in (0, 1):
+            a, b = m.kv(2, which, n), kv[which]
+            assert np.linalg.norm(a - b) <= 2.0 ** -11 * np.linalg.norm(b), n
+        m.reset()
+    m.close()
+
+
 @pytest.mark.parametrize("w,kv", [("f16", "f16"), ("i8", "f16"), ("f16", "f32"), ("f32", "f32"), ("f32", "f16")])
 @pytest.mark.parametrize("n", [4098, 4130])
 def test_prompt_past_one_chunk(gpu, w, kv, n):
