@@ -532,6 +532,23 @@ struct HyRec : HyProj<WT> {
         e.rows = s->rows;
         return e;
     }
+    // Portions are cut so that a pass of M rows has about two workgroups a CU, into groups of 128 tokens and more, where their
+    // mean is three groups: side by side two workgroups a CU take 5.9 us a chunk instead of 4.1 and the first launch 3.2, so less
+    // is not saved (six portions of 17 to 300 tokens, 64 workgroups each: whole 42.5 us, cut at 128 44). 1025 tokens of 16 heads
+    // of 128 x 256: 137 us whole, 53 + 29 cut at 288.
+    template <int KD>
+    void ret_chunks(RetArgs a) const {
+        using G = RcGeo<KD>;
+        const int base = a.nsl * a.H, ng = 2 * device_cus() / base;
+        const int gt = std::max(kRetGroup, ng > 0 ? (M / ng + kRcTok - 1) / kRcTok * kRcTok : M);
+        const int np = M / gt;
+        const size_t bytes = (size_t)(np + msegs) * base * a.dim * kRetCols * sizeof(float);
+        if (M >= 3 * gt * msegs && bytes <= kPgWsBytes) {
+            a.gt = gt, a.nparts = np, a.part = s->pg_ws;
+            hipLaunchKernelGGL((ret_chunk_kernel<KD, true>), dim3(a.nsl, a.H, np), dim3(256), G::LDS_STATE, st(), a);
+        }
+        hipLaunchKernelGGL((ret_chunk_kernel<KD>), dim3(a.nsl, a.H, a.gt ? np + msegs : msegs), dim3(256), G::LDS, st(), a);
+    }
     template <typename OT>
     int mixer(const HyLayer& l, const HyRun& r) const {
         const sli_block_desc& d = l.d;
@@ -542,13 +559,13 @@ struct HyRec : HyProj<WT> {
         if (one)
             hipLaunchKernelGGL(ret_step_kernel, dim3(l.nsl, d.heads, M), dim3(256), 0, st(), a);
         else if (kd == 32)
-            hipLaunchKernelGGL(ret_chunk_kernel<32>, sg, dim3(256), RcGeo<32>::LDS, st(), a);
+            ret_chunks<32>(a);
         else if (kd == 64)
-            hipLaunchKernelGGL(ret_chunk_kernel<64>, sg, dim3(256), RcGeo<64>::LDS, st(), a);
+            ret_chunks<64>(a);
         else if (kd == 128)
-            hipLaunchKernelGGL(ret_chunk_kernel<128>, sg, dim3(256), RcGeo<128>::LDS, st(), a);
+            ret_chunks<128>(a);
         else if (kd == 256)
-            hipLaunchKernelGGL(ret_chunk_kernel<256>, sg, dim3(256), RcGeo<256>::LDS, st(), a);
+            ret_chunks<256>(a);
         else
             hipLaunchKernelGGL(ret_scan_kernel, sg, dim3(256), ret_scan_lds(d.dim), st(), a);
         SLI_HIP(hipGetLastError());
@@ -814,7 +831,7 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
     SLI_HIP(hipMemcpyAsync(s->rows, rows.data(), sizeof(RowRef) * M, hipMemcpyHostToDevice, s->stream));
     SLI_HIP(hipMemcpyAsync(s->segs, segs.data(), sizeof(SegRef) * ns, hipMemcpyHostToDevice, s->stream));
     SLI_HIP(hipMemcpyAsync(s->nsegs, &ns, sizeof(ns), hipMemcpyHostToDevice, s->stream));
-    const int msegs = one ? M : std::min(s->B, M / kHyTile);
+    const int msegs = one ? M : s->replays ? std::min(s->B, M / kHyTile) : ns;  // (a replayed pass has other portions)
     if (hidden_host) {  // eager, with a copy after every run
         HY_TRY(HY_DISPATCH(s, M, one, msegs, kt, embed()));
         for (size_t r = 0; r < s->runs.size(); ++r) {

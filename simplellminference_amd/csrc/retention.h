@@ -28,6 +28,10 @@ struct RetArgs {
     const int32_t* nsegs;
     int H, dim, vdim, nsl;
     float* ssq = nullptr;  // [M][H][nsl] sums of o^2 over a slice (step form, nullable)
+    // chunk form: portions cut into groups of gt tokens (0: whole) that run side by side; states between them in part
+    // [slot][H][nsl][dim][kRetCols]: the groups but each portion's last, then per portion the state it starts from
+    int gt = 0, nparts = 0;
+    float* part = nullptr;
 };
 
 __device__ __forceinline__ float* ret_slice(const RetArgs& a, int slot, int h, int sl) {

@@ -171,6 +171,33 @@ def test_retention_alone_long(gpu, dtype):
     m.close()
 
 
+@pytest.mark.parametrize("first", [0, 1, 100])
+@pytest.mark.parametrize("n", [384, 385, 511, 513, 640])
+def test_retention_cut_into_groups(gpu, n, first):
+    """Passes whose portion is cut (groups of 128 tokens): ends of groups and one past them, from the start and from a state that
+    an earlier pass left, whose last group writes what the first one starts from; then tokens one by one from the state left."""
+    c = stack(ret(heads=2, dim=40, vdim=72, rot_dims=32, decay=(0.97, 0.9995), ff=0), width=64)
+    t = R.random_tensors(c, 19)
+    ids = tokens(first + n + 2, c["vocab"], n)
+    m = make(c, t, "bfloat16", 800)
+    cuts = ([first] if first else []) + [first + n, first + n + 1]
+    close(pieces(m, ids, cuts), R.forward(c, t, ids)[0], "bfloat16")
+    m.close()
+
+
+def test_retention_groups_of_two_portions(gpu):
+    """One portion of six groups beside one of a single group, from states of different ages."""
+    c = stack(ret(heads=2, dim=64, vdim=64, decay=(0.99, 0.9995), ff=0), width=64)
+    t = R.random_tensors(c, 23)
+    a, b = tokens(760, c["vocab"], 1), tokens(110, c["vocab"], 2)
+    m = make(c, t, "bfloat16", 800, batch=2)
+    m.feed([0, 1], [0, 0], [a[:30], b[:7]])
+    out = m.feed([0, 1], [30, 7], [a[30:], b[7:]], [list(range(730)), list(range(103))])
+    close(out[:730], R.forward(c, t, a)[0][30:], "bfloat16")
+    close(out[730:], R.forward(c, t, b)[0][7:], "bfloat16")
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_feed_forward_clamp_alone(gpu, dtype):
     c = stack(dict(att(ff=64, ff_limit=0.5)), taps=1)
