@@ -640,13 +640,9 @@ struct HyRec : HyProj<WT> {
                 if (!one && l.hd <= 128) {
                     const PfAttnArgs<__half> pa{l.q, (const __half*)r.kc, (const __half*)r.vc, {cat<OT>(l), nullptr},
                                                 d.heads, d.kv_heads, s->T, d.scale};
-                    const PfRowsArgs px{s->rows, l.r1, l.r2, l.sink, l.Kp, d.vdim};
-                    const dim3 gr(M / 16, d.heads);
-                    if (l.hd == 64)
-                        hipLaunchKernelGGL((pf_attn_mfma_kernel<64, 1>), gr, dim3(256), 0, st(), pa, px);
-                    else
-                        hipLaunchKernelGGL((pf_attn_mfma_kernel<128, 1>), gr, dim3(256), 0, st(), pa, px);
-                    SLI_HIP(hipGetLastError());
+                    const PfPortions px{s->segs, s->nsegs, l.r1, l.r2, l.sink, l.Kp, d.vdim};
+                    SLI_HIP(l.hd == 64 ? launch_pf_flash_rows<64>(pa, px, M, msegs, device_cus(), st())
+                                       : launch_pf_flash_rows<128>(pa, px, M, msegs, device_cus(), st()));
                     return SLI_OK;
                 }
             }

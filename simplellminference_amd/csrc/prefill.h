@@ -1097,7 +1097,8 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
     }
 }
 
-// ---- 3b. the packed rows of block-stack models, on MFMA (fp16 cache). A workgroup = 16 rows (queries) of one head;
+// ---- 3b. windowed attention over expanded keys of the block stacks' latent attention, on MFMA. A workgroup = 16 rows (queries)
+// of one head;
 // its 4 waves split the key range into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o)
 // through LDS at the end; per tile as pf_flash_kernel, with K and V in the wave's own images.
 template <int HD>
@@ -1153,8 +1154,17 @@ template <int HD>
 struct PfFlash {
     static constexpr int KT = 64, ROWB = HD * 2, IMG = KT * ROWB, CPR = ROWB / 16, PIECES = IMG / 1024;
 };
-template <int HD, int QT, int TERMS>
-__global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, PfState ps, int GW) {
+// ROWS: the rows are packed portions of several sequences (step_state.h SegRef; the caches hold one [hkv][T][HD] block per
+// sequence slot), with a distance bias and a sink per head (attn_rows.h) and one fp16 output [M][ldo] of vdim dims per head.
+// 1025 rows of 32 heads of 128: 85 us as a workgroup per 16 rows and head, now 51.
+struct PfPortions {
+    const SegRef* segs = nullptr;
+    const int32_t* nsegs = nullptr;
+    const float *r1 = nullptr, *r2 = nullptr, *sink = nullptr;  // [hq]
+    int ldo = 0, vdim = 0;
+};
+template <int HD, int QT, int TERMS, bool ROWS = false>
+__global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, PfState ps, int GW, PfPortions x) {
     using F = PfFlash<HD>;
     constexpr int ND = HD / 32, NT = HD / 16, NK = F::KT / 16, PPW = 2 * F::PIECES / 4;
     __shared__ __attribute__((aligned(1024))) char sm[2 * 2 * F::IMG];
@@ -1163,7 +1173,22 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
     const int G = a.hq / a.hkv, ng = G / GW, kvh = blockIdx.y / ng;
     const int h = kvh * G + (blockIdx.y - kvh * ng) * GW + wave % GW;
     const int RB = (4 / GW) * 16 * QT;  // query positions per workgroup
-    const int bx = gridDim.x - 1 - blockIdx.x, blk = bx / ps.nseq, seq = bx - blk * ps.nseq;
+    const int bx = gridDim.x - 1 - blockIdx.x;
+    int blk, seq, row0;
+    if constexpr (ROWS) {  // block bx of the portions' blocks
+        int i = 0;
+        const int n = *x.nsegs;
+        for (blk = bx; i < n; ++i) {
+            const int nb = (x.segs[i].n + RB - 1) / RB;
+            if (blk < nb) break;
+            blk -= nb;
+        }
+        if (i >= n) return;  // (uniform)
+        const SegRef sg = x.segs[i];
+        seq = sg.slot, row0 = sg.row0, ps.p0 = sg.pos0, ps.nv = ps.rps = sg.n;
+    } else {
+        blk = bx / ps.nseq, seq = bx - blk * ps.nseq, row0 = seq * ps.rps;
+    }
     if (blk * RB >= ps.nv) return;  // (uniform) only padding rows
     const int i0 = blk * RB + (wave / GW) * 16 * QT;
     const int last = min(ps.p0 + min(blk * RB + RB, ps.nv) - 1, a.T - 1);                   // the workgroup's
@@ -1172,7 +1197,7 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
     u32x4 qf[TERMS][QT][ND];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-        const int row = seq * ps.rps + min(i0 + t * 16 + i16, ps.rps - 1);
+        const int row = row0 + min(i0 + t * 16 + i16, ps.rps - 1);
 #pragma unroll
         for (int db = 0; db < ND; ++db) {
             const float4* qp = reinterpret_cast<const float4*>(a.q + (size_t)row * qs + (size_t)h * HD + db * 32 + g * 8);
@@ -1210,6 +1235,7 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
     };
     const float c2 = a.scale * 1.44269504088896340736f;
     const int nt = last / F::KT + 1;
+    const float bias1 = ROWS ? x.r1[h] : 0.0f, bias2 = ROWS ? x.r2[h] : 0.0f;
     issue(0);
     for (int tt = 0; tt < nt; ++tt) {
         pf_wait_vm<0>();
@@ -1245,6 +1271,19 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
             const int pos = ps.p0 + i0 + t * 16 + i16;
+            if constexpr (ROWS) {  // the scores in base 2, less the bias of their distance (keys past the query: any number)
+#pragma unroll
+                for (int kt = 0; kt < NK; ++kt) s[kt][t] *= c2;
+                if (bias1 != 0.0f) {
+#pragma unroll
+                    for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float dist = (float)max(pos - (t0 + kt * 16 + 4 * g + r), 0);
+                            s[kt][t][r] -= bias1 * __builtin_amdgcn_logf(fmaf(bias2, dist, 1.0f));  // (log2)
+                        }
+                }
+            }
             if (t0 + F::KT - 1 > ps.p0 + i0 + t * 16) {  // (wave-uniform) the diagonal
 #pragma unroll
                 for (int kt = 0; kt < NK; ++kt)
@@ -1256,7 +1295,7 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
 #pragma unroll
             for (int kt = 0; kt < NK; ++kt)
                 cmax = fmaxf(cmax, fmaxf(fmaxf(s[kt][t][0], s[kt][t][1]), fmaxf(s[kt][t][2], s[kt][t][3])));
-            cmax = max_xor32(max_xor16(cmax)) * c2;
+            cmax = max_xor32(max_xor16(cmax)) * (ROWS ? 1.0f : c2);
             const float mn = fmaxf(mx[t], cmax);
             if (__any(mn > mx[t])) {  // (key 0 is seen by every row: the maximum is finite from the first tile on)
                 const float corr = __builtin_amdgcn_exp2f(mx[t] - mn);
@@ -1270,7 +1309,8 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
                 __half ht[TERMS][8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, -mx[t])) * 256.0f;
+                    const float p = __builtin_amdgcn_exp2f(ROWS ? s[2 * kb + (e >> 2)][t][e & 3] - mx[t]
+                                                                : fmaf(s[2 * kb + (e >> 2)][t][e & 3], c2, -mx[t])) * 256.0f;
                     l[t] += p;
                     pf_terms(p, ht, e);
                 }
@@ -1305,7 +1345,28 @@ __global__ void __launch_bounds__(256, 2) pf_flash_kernel(PfAttnArgs<__half> a, 
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         const int i = i0 + t * 16 + i16;
-        const float inv = 1.0f / sum_xor32(sum_xor16(l[t]));
+        const float ls = sum_xor32(sum_xor16(l[t]));
+        if constexpr (ROWS) {
+            const float sk = x.sink[h] * 1.44269504088896340736f, M = fmaxf(mx[t], sk), f = __builtin_amdgcn_exp2f(mx[t] - M);
+            const float inv = f / (ls * f + 256.0f * __builtin_amdgcn_exp2f(sk - M));
+            if (i >= ps.nv) continue;
+            __half* dst = a.out.hi + (size_t)(row0 + i) * x.ldo + (size_t)h * x.vdim;
+#pragma unroll
+            for (int d = 0; d < NT; ++d) {
+                const int d0 = d * 16 + 4 * g;
+                const __half y[4] = {__float2half_rn(o[t][d][0] * inv), __float2half_rn(o[t][d][1] * inv),
+                                     __float2half_rn(o[t][d][2] * inv), __float2half_rn(o[t][d][3] * inv)};
+                if (x.vdim % 4 == 0 && d0 < x.vdim) {
+                    *reinterpret_cast<uint2*>(dst + d0) = *reinterpret_cast<const uint2*>(y);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (d0 + r < x.vdim) dst[d0 + r] = y[r];
+                }
+            }
+            continue;
+        }
+        const float inv = 1.0f / ls;
         if (i >= ps.nv) continue;
 #pragma unroll
         for (int d = 0; d < NT; ++d) {  // lane holds d = 16 d + 4 g + r of query i
@@ -1326,7 +1387,7 @@ hipError_t launch_pf_flash(const PfAttnArgs<__half>& a, const PfState& ps, int c
     const int ny = a.hkv * (G / GW);
     auto blocks = [&](int qt) { return (ps.nv + (4 / GW) * 16 * qt - 1) / ((4 / GW) * 16 * qt) * ps.nseq; };
     const bool wide = blocks(2) * ny >= 2 * cus;
-    auto go = [&](auto kernel, int qt) { hipLaunchKernelGGL(kernel, dim3(blocks(qt), ny), dim3(256), 0, s, a, ps, GW); };
+    auto go = [&](auto kernel, int qt) { hipLaunchKernelGGL(kernel, dim3(blocks(qt), ny), dim3(256), 0, s, a, ps, GW, PfPortions{}); };
     if (ps.nseq > 1)
         HD == 64 && wide ? go(pf_flash_kernel<HD, HD == 64 ? 2 : 1, 3>, 2) : go(pf_flash_kernel<HD, 1, 3>, 1);
     else
@@ -1334,20 +1395,30 @@ hipError_t launch_pf_flash(const PfAttnArgs<__half>& a, const PfState& ps, int c
     return hipGetLastError();
 }
 
-// ROWS: the rows are packed portions of several sequences (step_state.h RowRef; a 16-row group belongs to one portion,
-// its valid rows first), with a distance bias and a sink per head (attn_rows.h) and one fp16 output [M][ldo] of vdim
-// dims per head; the caches hold one [hkv][T][HD] block per sequence slot.
-// ROWS 2: no bias and no sink; a query sees the last `window` positions up to its own, position t's K and V are row
-// t + koff[row / 32] of one [hkv][T][HD] block (latent.h expands them), and the output is multiplied by gate [M][hq vdim].
+// The portions of a pass of M rows, msegs of them at most
+template <int HD>
+hipError_t launch_pf_flash_rows(const PfAttnArgs<__half>& a, const PfPortions& x, int M, int msegs, int cus, hipStream_t s) {
+    const int G = a.hq / a.hkv, GW = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1, ny = a.hkv * (G / GW);
+    auto blocks = [&](int qt) { return M / ((4 / GW) * 16 * qt) + msegs; };
+    if ((M / ((4 / GW) * 32)) * ny >= 2 * cus)
+        hipLaunchKernelGGL((pf_flash_kernel<HD, 2, 2, true>), dim3(blocks(2), ny), dim3(256), 0, s, a, PfState{}, GW, x);
+    else
+        hipLaunchKernelGGL((pf_flash_kernel<HD, 1, 2, true>), dim3(blocks(1), ny), dim3(256), 0, s, a, PfState{}, GW, x);
+    return hipGetLastError();
+}
+
+// Windowed: the rows are packed portions (step_state.h RowRef; a 16-row group belongs to one portion, its valid rows first); a
+// query sees the last `window` positions up to its own, position t's K and V are row t + koff[row / 32] of one [hkv][T][HD]
+// block (latent.h expands them), and the output, one fp16 row [M][ldo] of vdim dims per head, is multiplied by gate
+// [M][hq vdim].
 struct PfRowsArgs {
     const RowRef* rows = nullptr;
-    const float *r1 = nullptr, *r2 = nullptr, *sink = nullptr;  // [hq]
     int ldo = 0, vdim = 0;
     int window = 0;
     const int32_t* koff = nullptr;
     const float* gate = nullptr;
 };
-template <int HD, int ROWS>
+template <int HD>
 __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, PfRowsArgs x) {
     using G = PaGeo<HD>;
     constexpr int ND = HD / 32, NT = HD / 16;  // 32-d blocks (S), 16-d tiles (O)
@@ -1357,27 +1428,14 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
     const int g = lane >> 4, i16 = lane & 15;
     const int h = blockIdx.y, kvh = h / (a.hq / a.hkv);
     const int mq = blockIdx.x * 16 + i16;  // this lane's query (chunk row)
-    int pos, last, slot = 0;  // last: the group's last query position
-    int kmin = 0, koff = 0, tile0 = 0;
-    bool live = true;
     const RowRef r0 = x.rows[blockIdx.x * 16];
     if (r0.slot < 0) return;  // (uniform) a group of padding rows
-    slot = r0.slot;
-    live = x.rows[mq].slot >= 0;
-    pos = r0.pos + i16;
-    last = r0.pos + (int)__popcll(__ballot(live)) / 4 - 1;  // (a row is the query of 4 lanes)
-    if constexpr (ROWS == 2) {
-        slot = 0;
-        kmin = max(0, r0.pos - x.window + 1);  // the first key any row of the group sees
-        koff = x.koff[blockIdx.x >> 1];
-        tile0 = kmin / 32;
-    }
+    const bool live = x.rows[mq].slot >= 0;
+    const int pos = r0.pos + i16;
+    const int last = r0.pos + (int)__popcll(__ballot(live)) / 4 - 1;  // the group's last query (a row is the query of 4 lanes)
+    const int kmin = max(0, r0.pos - x.window + 1);  // the first key any row of the group sees
+    const int koff = x.koff[blockIdx.x >> 1], tile0 = kmin / 32;
     const int kmax = last;  // cache rows past it are read as this one (their scores are masked)
-    float bias1 = 0.0f, bias2 = 0.0f;
-    if constexpr (ROWS == 1) {
-        bias1 = x.r1[h];
-        bias2 = x.r2[h];
-    }
     const int ntiles = last / 32 + 1;
     const size_t qs = (size_t)a.hq * HD;
     // Qᵀ as the B operand: lane l = query l & 15, d = 32 db + 8 g .. +8, fp32 -> hi + lo
@@ -1400,8 +1458,8 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
     char* kimg = sm + wave * G::WAVE;
     const unsigned kbase = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)kimg;
     const unsigned vbase = kbase + G::IMG;
-    const __half* kc = a.kc + ((size_t)slot * a.hkv + kvh) * a.T * HD;
-    const __half* vc = a.vc + ((size_t)slot * a.hkv + kvh) * a.T * HD;
+    const __half* kc = a.kc + (size_t)kvh * a.T * HD;
+    const __half* vc = a.vc + (size_t)kvh * a.T * HD;
     for (int tt = tile0 + wave; tt < ntiles; tt += 4) {
         const int t0 = tt * 32;
         // K pieces 0 .. P/2-1, V pieces P/2 .. P-1; lane i of a piece: row (piece rows) + i / CPR, physical
@@ -1412,7 +1470,7 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
             const int jj = isv ? j - G::PIECES / 2 : j;
             const int r = jj * (1024 / G::ROWB) + lane / G::CPR;
             const int c = (lane % G::CPR) ^ (isv ? pa_swz_v(r, G::ROWB) : pa_swz_k(r, G::ROWB));
-            const int kr = ROWS == 2 ? max(min(t0 + r, kmax), kmin) + koff : min(t0 + r, kmax);
+            const int kr = max(min(t0 + r, kmax), kmin) + koff;
             const __half* src = (isv ? vc : kc) + (size_t)kr * HD + c * 8;
             pf_dma(src, (isv ? vbase : kbase) + (unsigned)(jj * 1024));
         }
@@ -1439,9 +1497,8 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int key = t0 + kt * 16 + 4 * g + r;
-                float sc = sacc[kt][r] * a.scale;
-                if constexpr (ROWS == 1) sc -= bias1 * __logf(1.0f + bias2 * (float)(pos - key));
-                const bool see = key <= pos && (ROWS != 2 || key > pos - x.window);
+                const float sc = sacc[kt][r] * a.scale;
+                const bool see = key <= pos && key > pos - x.window;
                 const float v = see ? sc : -INFINITY;
                 sv[kt * 4 + r] = v;
                 cmax = fmaxf(cmax, v);
@@ -1504,10 +1561,6 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
         M = fmaxf(M, m4[w]);
     }
     float L = 0.0f;
-    if constexpr (ROWS == 1) {
-        M = fmaxf(M, x.sink[h]);
-        L = expf(x.sink[h] - M);
-    }
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         w4[w] = m4[w] == -INFINITY ? 0.0f : expf(m4[w] - M);
@@ -1522,12 +1575,10 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
         const int d0 = t * 16 + 4 * g;
         __half* dst = a.out.hi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
         if (!live) continue;
-        if constexpr (ROWS == 2) {
-            const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
+        const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (d0 + r < x.vdim) acc[r] *= gt[r];
-        }
+        for (int r = 0; r < 4; ++r)
+            if (d0 + r < x.vdim) acc[r] *= gt[r];
         if (x.vdim % 4 == 0 && d0 < x.vdim) {
             const __half hv[4] = {__float2half_rn(acc[0] * inv), __float2half_rn(acc[1] * inv),
                                   __float2half_rn(acc[2] * inv), __float2half_rn(acc[3] * inv)};

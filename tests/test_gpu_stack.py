@@ -522,6 +522,26 @@ def test_errors_come_from_the_host(gpu):
         StackModel(StackSpec(8, 8, (BlockSpec("attention", 3, 4, 4, kv_heads=2),))).init()
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 4, 128, 128), (4, 2, 64, 64), (8, 2, 128, 100), (3, 1, 40, 30)])
+def test_attention_blocks_of_portions(gpu, heads, kv, dim, vdim):
+    """Prompt attention over portions of one pass: blocks of 16 to 64 rows end inside portions, each portion starts at a position
+    of its own (key tiles of 64: below, at and past one), with biases and sinks; vdim not whole 4s."""
+    c = stack(att(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, ff=0), width=64)
+    t = R.random_tensors(c, 31)
+    lens, firsts = (17, 70, 130, 33), (0, 5, 64, 121)
+    ids = [tokens(f + n, c["vocab"], n) for n, f in zip(lens, firsts)]
+    m = make(c, t, "bfloat16", 300, batch=4)
+    for i, f in enumerate(firsts):
+        if f:
+            m.feed([i], [0], [ids[i][:f]])
+    out = m.feed(range(4), firsts, [x[f:] for x, f in zip(ids, firsts)], [list(range(n)) for n in lens])
+    p = 0
+    for x, n, f in zip(ids, lens, firsts):
+        close(out[p:p + n], R.forward(c, t, x)[0][f:], "bfloat16", f"portion of {n}")
+        p += n
+    m.close()
+
+
 @pytest.mark.parametrize("n", [33, 65, 129, 257, 300, 700, 1025, 2048, 2049])
 def test_row_counts_of_a_pass(gpu, n):
     """Prompt passes of every tile height with padding rows, a launch's last tiles cut over the depth (narrow outputs: all of
