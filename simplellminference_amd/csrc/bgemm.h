@@ -75,11 +75,15 @@ struct BgIn {
     // 16-byte A operand at l * 16 — one wave load is one contiguous KiB (8 full 128-B lines) instead of 16 rows x
     // 64 B (16 half lines). 0: W row-major [rows][K] (the op-level entry, tools/bgemm_lab)
     int tiled = 0;
+    // tiles from tile2 on read x2 (two projections of equal depth in one launch): groups [0, groups1) take the tiles below it
+    const float* x2 = nullptr;
+    int tile2 = 0x7fffffff, groups1 = 0x7fffffff;
 };
 
 // ---------------------------------------------------------------- host-side plan
 struct BgPlan {
     int ntiles = 0, tpw = 1, splits = 1, groups = 0;
+    int tile2 = 0x7fffffff, groups1 = 0x7fffffff;  // BgIn
     size_t lds = 0;
 };
 
@@ -96,7 +100,8 @@ inline size_t bg_lds_bytes(int K, int splits, int tpw) {
 // steps (row-major weights): a wave's blocks of a tile are priced as the whole steps they take, and a split's publish and
 // merge at 3 us. At 8 rows of 4096 columns 544 tiles took 20.5 us in one split and 30.4 us in four, 257 tiles 14.8 us and
 // (five) 21.5 us.
-inline BgPlan bg_plan(int ntiles, int K, int B, bool norm, int cus = 256, bool steps = false) {
+// nt1 > 0: the first nt1 tiles and the others have inputs of their own, so no workgroup takes tiles of both.
+inline BgPlan bg_plan(int ntiles, int K, int B, bool norm, int cus = 256, bool steps = false, int nt1 = 0) {
     const int nkb = K / 32;
     BgPlan best;
     double best_cost = 1e30;
@@ -110,7 +115,7 @@ inline BgPlan bg_plan(int ntiles, int K, int B, bool norm, int cus = 256, bool s
         if (kbs * 32 > kBgMaxStageK) continue;  // staging registers
         for (int tpw = 1; tpw <= 64; ++tpw) {
             if (bg_lds_bytes(K, s, tpw) > (size_t)kBgLdsMax) break;
-            const int groups = (ntiles + tpw - 1) / tpw;
+            const int g1 = (nt1 + tpw - 1) / tpw, groups = g1 + (ntiles - nt1 + tpw - 1) / tpw;
             const int wgs = groups * s;
             const int rounds = (wgs + cus - 1) / cus;
             int blocks = kbs;
@@ -129,9 +134,10 @@ inline BgPlan bg_plan(int ntiles, int K, int B, bool norm, int cus = 256, bool s
                 best.tpw = tpw;
                 best.splits = s;
                 best.groups = groups;
+                if (nt1 > 0) best.tile2 = nt1, best.groups1 = g1;
                 best.lds = bg_lds_bytes(K, s, tpw);
             }
-            if (groups == 1) break;
+            if (tpw >= ntiles) break;
         }
     }
     return best;
@@ -203,8 +209,10 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
     const int kbs_max = (nkb + S - 1) / S;
     float* P = reinterpret_cast<float*>(bg_smem + kBgScratch + (size_t)kbs_max * 1024);  // [2][16 waves][16][8]
     float* R = P + 2 * kBgWaves * 128;                                                 // [tpw][16][8]
-    const int t0 = g * in.tpw;
-    const int ntg = min(in.tpw, in.ntiles - t0);  // this workgroup's tiles (uniform)
+    const bool second = g >= in.groups1;
+    const int t0 = second ? in.tile2 + (g - in.groups1) * in.tpw : g * in.tpw;
+    const int ntg = min(in.tpw, (second ? in.ntiles : min(in.ntiles, in.tile2)) - t0);  // this workgroup's tiles (uniform)
+    const float* x = second ? in.x2 : in.x;
     const int wb0 = kb0 + (wave * nkbs) / kBgWaves;  // this wave's blocks of every tile
     const int wnb = kb0 + ((wave + 1) * nkbs) / kBgWaves - wb0;
     const int per_wave_max = (nkbs + kBgWaves - 1) / kBgWaves;
@@ -243,7 +251,7 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
     for (int n = 0; n < kBgNH; ++n) {
         const int blk = wb0 + max(min(2 * n + wbo, wnb - 1), 0);  // clamped into the row, never a branch
         const int k8 = min(blk, nkb - 1) * 4 + wq;
-        const float4* xp = reinterpret_cast<const float4*>(in.x + (size_t)sbc * K + (size_t)k8 * 8);
+        const float4* xp = reinterpret_cast<const float4*>(x + (size_t)sbc * K + (size_t)k8 * 8);
         xa[n][0] = kStage ? xp[0] : make_float4(0.f, 0.f, 0.f, 0.f);
         xa[n][1] = kStage ? xp[1] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
@@ -631,6 +639,7 @@ hipError_t launch_bgemm(const __half* W, const BgIn& in_, const Epi& epi, const 
     in.ntiles = p.ntiles;
     in.tpw = p.tpw;
     in.splits = p.splits;
+    in.tile2 = p.tile2, in.groups1 = p.groups1;
     const dim3 grid(p.groups * p.splits);
     if (in.norm_w && p.splits != 1) return hipErrorInvalidValue;  // the fused RMS runs on one split only
     const int u = in.norm_w ? bg_step_width(p.tpw) : bg_width(p.splits, in.K, p.tpw);

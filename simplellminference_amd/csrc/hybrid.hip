@@ -76,11 +76,12 @@ static int hy_attn_splits(int T) { return std::max(kAmMaxSplits, (T + 64 * kAmWg
 
 static int hy_allow_lds();
 
-// the batched projections of np pairs over K columns: their workspace (every row count; the head takes any number of wanted rows)
-int hy_bg_need(BlockStack* s, int np, int K) {
+// the batched projections of np pairs (and np2 of a second input) over K columns: their workspace (every row count; the head takes any number of wanted rows)
+int hy_bg_need(BlockStack* s, int np, int K, int np2) {
     if (!s->f16 || np == 0) return SLI_OK;
     for (int b = 1; b <= kBgMaxBatch; ++b) {
-        const BgPlan p = bg_plan((np + 7) / 8, K, b, false, gemv_max_blocks(), true);
+        const int nt = (np + 7) / 8, nt2 = (np2 + 7) / 8;
+        const BgPlan p = bg_plan(nt + nt2, K, b, false, gemv_max_blocks(), true, nt2 ? nt : 0);
         SLI_CHECK(p.groups > 0, SLI_ERR_SHAPE, "stack: no tiling of a batched projection fits");
         s->bg_ws_bytes = std::max(s->bg_ws_bytes, bg_part_bytes(p));
         s->bg_groups = std::max(s->bg_groups, (size_t)p.groups);
@@ -190,8 +191,7 @@ static int par_create(BlockStack* s) {
         if (l.d.mixer == SLI_MIX_ATTENTION)
             part = std::max(part, (size_t)Bp * l.d.heads * hy_attn_splits(s->T) * (l.hd + kAttnPartPad)),
             ncnt = std::max(ncnt, (size_t)Bp * l.d.heads);
-        HY_TRY(hy_bg_need(s, l.e_g, s->Dp));
-        HY_TRY(hy_bg_need(s, l.d.ff, s->Dp));
+        HY_TRY(hy_bg_need(s, l.e_g, s->Dp, l.d.ff));
         HY_TRY(hy_bg_need(s, (s->D + 1) / 2, l.Kp));
     }
     HY_TRY(hy_new(s, &s->part, part));
@@ -500,7 +500,7 @@ template <typename WT>
 struct HyRec : HyProj<WT> {
     using KT = WT;  // fp16 weights with an fp16 cache, fp32 with fp32
     using P = HyProj<WT>;
-    using P::F16, P::GV, P::s, P::M, P::one, P::msegs, P::key_tiles, P::st, P::path, P::rows_for, P::project, P::pgemm;
+    using P::F16, P::GV, P::s, P::M, P::one, P::msegs, P::key_tiles, P::st, P::path, P::rows_for, P::project, P::project2, P::pgemm;
     template <class Epi>
     static int allow() { return P::template allow<Epi>(); }
     template <typename OT>
@@ -703,8 +703,12 @@ struct HyRec : HyProj<WT> {
             else
                 HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei));
         } else {
-            HY_TRY(project(l.win, s->c1, s->Dp, l.e_g, 0, ei));
-            if (l.d.ff > 0) HY_TRY(project(l.win, s->c2, s->Dp, l.d.ff, l.u1p, ei));
+            if (l.d.ff > 0 && path(M, s->Dp) == P::BG) {
+                HY_TRY(project2(l.win, s->c1, s->c2, s->Dp, l.e_g, l.u1p, l.d.ff, ei));
+            } else {
+                HY_TRY(project(l.win, s->c1, s->Dp, l.e_g, 0, ei));
+                if (l.d.ff > 0) HY_TRY(project(l.win, s->c2, s->Dp, l.d.ff, l.u1p, ei));
+            }
         }
         HY_TRY(mixer<OT>(l, r));
         if constexpr (std::is_same<OT, float>::value) {
@@ -767,6 +771,7 @@ struct HyRec : HyProj<WT> {
     }
     static int allow_all() {
         HY_TRY((allow<HyIn<KT, float>>()));
+        SLI_HIP((bg_allow_lds<BgPair2<HyIn<KT, float>>, false>()));
         HY_TRY((allow<HyIn<KT, __half>>()));
         HY_TRY((allow<HyOut>()));
         return allow<HyLogits>();

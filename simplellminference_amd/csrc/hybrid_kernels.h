@@ -264,6 +264,21 @@ struct BgPair {  // bgemm.h: tile rows i and i + 8 are pair 8 t + i
     __device__ void finish(unsigned long long*, int, int) const {}
 };
 
+// Pairs [0, n1) and [u1, u1 + n2), the second from tile nt1 on (BgIn::tile2)
+template <class Epi>
+struct BgPair2 {
+    Epi e;
+    int n1, n2, u1, nt1;
+    __device__ int pair(int t, int i) const { return t < nt1 ? min(8 * t + i, n1 - 1) : u1 + min(8 * (t - nt1) + i, n2 - 1); }
+    __device__ int row(int t, int i) const { return 2 * pair(t, i & 7) + (i >> 3); }
+    __device__ void pre_a(int, int, int) {}
+    __device__ void pre_b() {}
+    __device__ void store(int t, int i, int b, float v0, float v1, unsigned long long*) const {
+        if (t < nt1 ? 8 * t + i < n1 : 8 * (t - nt1) + i < n2) e.pair(pair(t, i), b, v0, v1);
+    }
+    __device__ void finish(unsigned long long*, int, int) const {}
+};
+
 template <class Epi>
 struct PgPair {  // prefill.h: plain 16-row tiles, 4 consecutive rows per store
     static constexpr bool kRolled = PgRolled<Epi>::value;

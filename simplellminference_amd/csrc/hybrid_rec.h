@@ -55,6 +55,24 @@ struct HyProj {
         SLI_HIP((launch_rows_gemm<WT, Epi>(w, (const float*)X, K, npairs, u0, M, e, st())));
         return SLI_OK;
     }
+    // 2 .. 8 rows: pairs [0, n1) of X and [u1, u1 + n2) of X2 in one launch. 6 rows of 2048 columns, a block's 9728 and 11264
+    // pairs in the mean: two launches 25.6 us, one 22.8; a decode pass of 16 blocks for 2 | 3 | 5 | 8 sequences 1020 | 1084 | 1220 |
+    // 1413 us -> 982 | 1045 | 1187 | 1375.
+    template <class Epi>
+    int project2(const void* W, const void* X, const void* X2, int K, int n1, int u1, int n2, const Epi& e) const {
+        if constexpr (F16) {
+            BgIn in{};
+            in.x = (const float*)X, in.x2 = (const float*)X2;
+            in.K = K, in.B = M;
+            in.ws = s->bg_ws, in.counters = s->bg_cnt;
+            const int nt1 = (n1 + 7) / 8, nt2 = (n2 + 7) / 8;
+            SLI_HIP((launch_bgemm((const WT*)W, in, BgPair2<Epi>{e, n1, n2, u1, nt1},
+                                  bg_plan(nt1 + nt2, K, M, false, gemv_max_blocks(), true, nt1), st())));
+            return SLI_OK;
+        } else {
+            return fail(SLI_ERR_ARG, "batched projection: fp16 weights");
+        }
+    }
     // pairs [0, split) read X, pairs [split, npairs) X2 (split: a multiple of kHySection; X2 null: one input)
     template <class Epi>
     int pgemm(const WT* w, const __half* X, const __half* X2, int split, int K, int npairs, int u0, const Epi& e) const {

@@ -140,8 +140,8 @@ int hy_new(BlockStack* s, T** p, size_t n) {
     return hy_alloc(s, reinterpret_cast<void**>(p), sizeof(T) * n);
 }
 
-// creation: reserve the workspace of the batched projections of np pairs over K columns
-int hy_bg_need(BlockStack* s, int np, int K);
+// creation: reserve the workspace of the batched projections of np pairs (and np2 of a second input) over K columns
+int hy_bg_need(BlockStack* s, int np, int K, int np2 = 0);
 
 // where a tensor's elements come from: host memory, or (host null) a generator on the device
 struct HySrcRand {  // uniform in (-amp, amp) by element index

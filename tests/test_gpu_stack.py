@@ -635,6 +635,21 @@ def narrow_model(batch):
                                 taps=4, residual_mult=0.4, max_length=40), batch=batch, seed=4).init()
 
 
+@pytest.mark.parametrize("batch", [2, 8])
+@pytest.mark.parametrize("heads,ff,width", [(1, 5, 64), (3, 37, 96), (5, 1030, 1056), (8, 8200, 256)])
+def test_both_inputs_of_a_batched_block(gpu, batch, heads, ff, width):
+    """Mixer and feed-forward pairs that end inside 16-row tiles, one and several workgroups each, tiles of many pairs: decode
+    passes of several sequences as the same tokens one sequence at a time."""
+    c = stack(att(heads=heads, kv_heads=1, dim=24, vdim=20, ff=ff), ret(heads=heads, dim=20, vdim=12, rot_dims=8, ff=ff), width=width)
+    t = R.random_tensors(c, 41)
+    ids = [tokens(4, c["vocab"], b) for b in range(batch)]
+    m = make(c, t, "bfloat16", 16, batch=batch)
+    got = np.stack([m.feed(range(batch), [i] * batch, [[x[i]] for x in ids], [[0]] * batch) for i in range(4)])
+    for b, x in enumerate(ids):
+        close(got[:, b], R.forward(c, t, x)[0], "bfloat16", f"sequence {b}")
+    m.close()
+
+
 @pytest.mark.parametrize("batch", [2, 6, 8])
 def test_decode_pass_with_steps_of_five(gpu, batch):
     """Rows of a decode pass together against the same rows one at a time, whose projections are the row-wise ones."""

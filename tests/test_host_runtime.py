@@ -168,6 +168,19 @@ def small_models_predict_in_one_launch(H):
         m.close()
 
 
+def batched_inputs_share_a_launch(H):
+    """A decode pass of a block with a feed-forward projects both of its inputs in one launch; without one there is one input."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    for ff, want in ((300, "BgPair2"), (0, "BgPair")):
+        b = BlockSpec("attention", 5, 64, 64, kv_heads=1, scale=0.1, ff=ff, ff_limit=7.0)
+        m = StackModel(StackSpec(64, 256, (b,) * 2, taps=4, max_length=32), batch=3, seed=1).init()
+        H.hh_launched()
+        m.feed(range(3), [0] * 3, [[1]] * 3, [[0]] * 3)
+        ran = set(re.findall(r"bgemm_kernelINS_\d+(BgPair2?)INS_4HyIn", H.hh_launched().decode()))
+        assert ran == {want}, (ff, ran)
+        m.close()
+
+
 def _tilings(names, epilogue=""):
     """(weight type, tiling) of the prompt GEMM instances among kernel names, of one epilogue or all."""
     out = set()
@@ -307,6 +320,7 @@ def steps_of_the_batched_projection(H):
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
+         "batched_inputs_share_a_launch",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
          "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
