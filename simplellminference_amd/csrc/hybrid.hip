@@ -198,6 +198,50 @@ static int par_create(BlockStack* s) {
     return hy_new(s, &s->attn_cnt, ncnt);
 }
 
+// Copies of the weights in the batched projection's fragment layout, where several sequences may decode together: a wave reads one
+// KiB in a piece instead of 16 rows x 64 bytes. 6 rows of a 2048-wide stack, a block's projections 22.8 + 14.7 -> 17.9 + 12.2 us; a
+// decode pass of 16 blocks for 2 | 8 sequences 982 | 1375 -> 867 | 1233. They take as much memory as the weights, so they are
+// allocated last, where they fit with 1 GiB to spare, or the row-major matrices are streamed (SLI_DEBUG_BG_ROWMAJOR: always, tests).
+static void hy_alloc_tiles(BlockStack* s) {
+    if (!s->f16 || s->B < 2 || s->seq || std::getenv("SLI_DEBUG_BG_ROWMAJOR")) return;
+    std::vector<std::pair<void**, size_t>> want;
+    for (HyLayer& l : s->layers) {
+        want.push_back({&l.win_t, bg_tiled_bytes((l.e_g + 7) / 8 + ((int)l.d.ff + 7) / 8, s->Dp)});
+        want.push_back({&l.wout_t, bg_tiled_bytes(((s->D + 1) / 2 + 7) / 8, l.Kp)});
+    }
+    want.push_back({&s->head_t, bg_tiled_bytes(((s->V + 1) / 2 + 7) / 8, s->Dp)});
+    size_t need = 0, free_b = 0, total_b = 0;
+    for (const auto& p : want) need += p.second;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < need + ((size_t)1 << 30)) return;
+    const size_t n0 = s->allocs.size();
+    for (const auto& p : want) {
+        if (hipMalloc(p.first, p.second) != hipSuccess) {  // none of them then
+            (void)hipGetLastError();
+            for (size_t i = n0; i < s->allocs.size(); ++i) (void)hipFree(s->allocs[i]);
+            s->allocs.resize(n0);
+            for (const auto& q : want) *q.first = nullptr;
+            return;
+        }
+        s->allocs.push_back(*p.first);
+    }
+    s->tiled = true;
+}
+static int hy_sync_tiles(BlockStack* s) {
+    if (!s->tiled) return SLI_OK;
+    typedef HyIn<__half, float> In;
+    for (const HyLayer& l : s->layers) {
+        const int nt1 = (l.e_g + 7) / 8, nt2 = ((int)l.d.ff + 7) / 8, no = (s->D + 1) / 2;
+        if (l.d.ff > 0)
+            SLI_HIP(launch_bg_tile((const __half*)l.win, s->Dp, nt1 + nt2, BgPair2<In>{{}, l.e_g, (int)l.d.ff, l.u1p, nt1}, l.win_t, s->stream));
+        else
+            SLI_HIP(launch_bg_tile((const __half*)l.win, s->Dp, nt1, BgPair<In>{{}, l.e_g, 0}, l.win_t, s->stream));
+        SLI_HIP(launch_bg_tile((const __half*)l.wout, l.Kp, (no + 7) / 8, BgPair<HyOut>{{}, no, 0}, l.wout_t, s->stream));
+    }
+    const int nh = (s->V + 1) / 2;
+    SLI_HIP(launch_bg_tile((const __half*)s->head, s->Dp, (nh + 7) / 8, BgPair<HyLogits>{{}, nh, 0}, s->head_t, s->stream));
+    return SLI_OK;
+}
+
 int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out) {
     const sli_stack_config& c = *cfg;
     SLI_CHECK(c.vocab > 0 && c.width > 0 && c.n_blocks > 0 && c.blocks && c.max_len > 0 && c.batch > 0, SLI_ERR_SHAPE,
@@ -272,6 +316,7 @@ int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out)
     double w = 0.0, k = 0.0;
     hy_step_bytes(s, 1, 0.0, &w, &k);
     s->replays = w < kReplayBytes * (double)s->runs.size();
+    hy_alloc_tiles(s);
     return hy_allow_lds();
 }
 
@@ -491,6 +536,7 @@ int hy_prepare(BlockStack* s) {
     SLI_HIP(hipMemcpy(s->fnorm, g.data(), sizeof(float) * Dp, hipMemcpyHostToDevice));
     for (int d = 0; d < s->D; ++d) g[d] = (float)(g[d] * std::sqrt((double)s->D / Dp));
     SLI_HIP(hipMemcpy(s->fnorm_p, g.data(), sizeof(float) * Dp, hipMemcpyHostToDevice));
+    HY_TRY(hy_sync_tiles(s));
     s->dirty = false;
     return SLI_OK;
 }
@@ -704,9 +750,9 @@ struct HyRec : HyProj<WT> {
                 HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei));
         } else {
             if (l.d.ff > 0 && path(M, s->Dp) == P::BG) {
-                HY_TRY(project2(l.win, s->c1, s->c2, s->Dp, l.e_g, l.u1p, l.d.ff, ei));
+                HY_TRY(project2(l.win, s->c1, s->c2, s->Dp, l.e_g, l.u1p, l.d.ff, ei, l.win_t));
             } else {
-                HY_TRY(project(l.win, s->c1, s->Dp, l.e_g, 0, ei));
+                HY_TRY(project(l.win, s->c1, s->Dp, l.e_g, 0, ei, l.win_t));
                 if (l.d.ff > 0) HY_TRY(project(l.win, s->c2, s->Dp, l.d.ff, l.u1p, ei));
             }
         }
@@ -720,7 +766,7 @@ struct HyRec : HyProj<WT> {
             }
         }
         const HyOut eo{s->x, s->Dp, s->D, s->c.residual_mult};
-        return project(l.wout, cat<OT>(l), l.Kp, (s->D + 1) / 2, 0, eo);
+        return project(l.wout, cat<OT>(l), l.Kp, (s->D + 1) / 2, 0, eo, l.wout_t);
     }
     int embed() const {
         hipLaunchKernelGGL(hy_embed_kernel<WT>, dim3(M), dim3(256), 0, st(), s->rows, (const WT*)s->emb, (const WT*)s->pos,
@@ -741,7 +787,7 @@ struct HyRec : HyProj<WT> {
         hipLaunchKernelGGL(norm_rows_kernel<OT>, dim3(n), dim3(256), 0, st(), s->x, idx, s->fnorm, (OT*)s->xl, s->D, s->Dp,
                            s->c.eps);
         SLI_HIP(hipGetLastError());
-        return project(s->head, s->xl, s->Dp, (s->V + 1) / 2, 0, HyLogits{y, s->V, n});
+        return project(s->head, s->xl, s->Dp, (s->V + 1) / 2, 0, HyLogits{y, s->V, n}, s->head_t);
     }
     int pass() const {
         HY_TRY(embed());

@@ -30,7 +30,7 @@ struct HyProj {
     static int rows_for(int n) { return F16 && n > kBgMaxBatch ? pad_to(n, kHyTile) : n; }
 
     template <class Epi>
-    int project(const void* W, const void* X, int K, int npairs, int u0, const Epi& e) const {
+    int project(const void* W, const void* X, int K, int npairs, int u0, const Epi& e, const void* Wt = nullptr) const {
         const WT* w = (const WT*)W + (size_t)2 * u0 * K;
         const Path p = path(M, K);
         if (p == GV) {
@@ -47,7 +47,8 @@ struct HyProj {
                 in.ws = s->bg_ws;
                 in.counters = s->bg_cnt;
                 const BgPlan pl = bg_plan((npairs + 7) / 8, K, M, false, gemv_max_blocks(), true);
-                SLI_HIP((launch_bgemm(w, in, BgPair<Epi>{e, npairs, u0}, pl, st())));
+                in.tiled = Wt != nullptr;  // (Wt: the copy from pair u0 on)
+                SLI_HIP((launch_bgemm(Wt ? (const WT*)Wt : w, in, BgPair<Epi>{e, npairs, u0}, pl, st())));
                 return SLI_OK;
             }
             if (p == PG) return pgemm(w, (const __half*)X, nullptr, 0, K, npairs, u0, e);
@@ -59,14 +60,15 @@ struct HyProj {
     // pairs in the mean: two launches 25.6 us, one 22.8; a decode pass of 16 blocks for 2 | 3 | 5 | 8 sequences 1020 | 1084 | 1220 |
     // 1413 us -> 982 | 1045 | 1187 | 1375.
     template <class Epi>
-    int project2(const void* W, const void* X, const void* X2, int K, int n1, int u1, int n2, const Epi& e) const {
+    int project2(const void* W, const void* X, const void* X2, int K, int n1, int u1, int n2, const Epi& e, const void* Wt) const {
         if constexpr (F16) {
             BgIn in{};
             in.x = (const float*)X, in.x2 = (const float*)X2;
             in.K = K, in.B = M;
             in.ws = s->bg_ws, in.counters = s->bg_cnt;
             const int nt1 = (n1 + 7) / 8, nt2 = (n2 + 7) / 8;
-            SLI_HIP((launch_bgemm((const WT*)W, in, BgPair2<Epi>{e, n1, n2, u1, nt1},
+            in.tiled = Wt != nullptr;
+            SLI_HIP((launch_bgemm((const WT*)(Wt ? Wt : W), in, BgPair2<Epi>{e, n1, n2, u1, nt1},
                                   bg_plan(nt1 + nt2, K, M, false, gemv_max_blocks(), true, nt1), st())));
             return SLI_OK;
         } else {

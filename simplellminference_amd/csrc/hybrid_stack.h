@@ -38,6 +38,7 @@ struct HyLayer {
     int nsl = 0;  // retention: state slices per head
     int rot = -1;
     void *win = nullptr, *wout = nullptr;
+    void *win_t = nullptr, *wout_t = nullptr;  // the same in the batched projection's fragment layout (BlockStack::tiled)
     float *f1 = nullptr, *f2 = nullptr, *r1 = nullptr, *r2 = nullptr, *sink = nullptr, *decay = nullptr;
     // the output projection's input and the attention query rows, one buffer per shape: their padding columns are never
     // written, so they stay zero
@@ -112,6 +113,8 @@ struct BlockStack {
     std::vector<float> fgain;  // one gain, or one per channel
     std::map<std::string, bool> want;  // tensor -> placed
     bool dirty = true;
+    bool tiled = false;     // decode passes of several sequences stream copies in the fragment layout (bgemm.h BgIn::tiled)
+    void* head_t = nullptr;
     // activations of a pass
     RowRef* rows = nullptr;
     SegRef* segs = nullptr;

@@ -635,11 +635,15 @@ def narrow_model(batch):
                                 taps=4, residual_mult=0.4, max_length=40), batch=batch, seed=4).init()
 
 
+@pytest.mark.parametrize("tiled", [True, False])
 @pytest.mark.parametrize("batch", [2, 8])
-@pytest.mark.parametrize("heads,ff,width", [(1, 5, 64), (3, 37, 96), (5, 1030, 1056), (8, 8200, 256)])
-def test_both_inputs_of_a_batched_block(gpu, batch, heads, ff, width):
-    """Mixer and feed-forward pairs that end inside 16-row tiles, one and several workgroups each, tiles of many pairs: decode
-    passes of several sequences as the same tokens one sequence at a time."""
+@pytest.mark.parametrize("heads,ff,width", [(1, 5, 64), (3, 37, 96), (5, 1030, 1056), (8, 8200, 256), (2, 0, 70)])
+def test_both_inputs_of_a_batched_block(gpu, monkeypatch, tiled, batch, heads, ff, width):
+    """Mixer and feed-forward pairs that end inside 16-row tiles, one and several workgroups each, tiles of many pairs, from the
+    fragment-layout copies and from the matrices: decode passes of several sequences against the oracle; then with a weight
+    replaced, of which the copies must not keep the old one."""
+    if not tiled:
+        monkeypatch.setenv("SLI_DEBUG_BG_ROWMAJOR", "1")
     c = stack(att(heads=heads, kv_heads=1, dim=24, vdim=20, ff=ff), ret(heads=heads, dim=20, vdim=12, rot_dims=8, ff=ff), width=width)
     t = R.random_tensors(c, 41)
     ids = [tokens(4, c["vocab"], b) for b in range(batch)]
@@ -647,6 +651,12 @@ def test_both_inputs_of_a_batched_block(gpu, batch, heads, ff, width):
     got = np.stack([m.feed(range(batch), [i] * batch, [[x[i]] for x in ids], [[0]] * batch) for i in range(4)])
     for b, x in enumerate(ids):
         close(got[:, b], R.forward(c, t, x)[0], "bfloat16", f"sequence {b}")
+    for name in ("l0.mix.v", "l1.mix.o", "head"):
+        t[name] = -0.5 * t[name]
+        m.set_tensor(name, t[name])
+    out = m.feed(range(batch), [0] * batch, [[x[0]] for x in ids], [[0]] * batch)
+    for b, x in enumerate(ids):
+        close(out[b], R.forward(c, t, x[:1])[0][0], "bfloat16", f"replaced, sequence {b}")
     m.close()
 
 
