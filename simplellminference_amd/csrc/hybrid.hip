@@ -226,8 +226,8 @@ static void hy_alloc_tiles(BlockStack* s) {
     }
     s->tiled = true;
 }
-static int hy_sync_tiles(BlockStack* s) {
-    if (!s->tiled) return SLI_OK;
+int hy_sync_tiles(BlockStack* s) {
+    if (!s->tiled || !s->tiles_dirty) return SLI_OK;
     typedef HyIn<__half, float> In;
     for (const HyLayer& l : s->layers) {
         const int nt1 = (l.e_g + 7) / 8, nt2 = ((int)l.d.ff + 7) / 8, no = (s->D + 1) / 2;
@@ -239,6 +239,7 @@ static int hy_sync_tiles(BlockStack* s) {
     }
     const int nh = (s->V + 1) / 2;
     SLI_HIP(launch_bg_tile((const __half*)s->head, s->Dp, (nh + 7) / 8, BgPair<HyLogits>{{}, nh, 0}, s->head_t, s->stream));
+    s->tiles_dirty = false;
     return SLI_OK;
 }
 
@@ -536,8 +537,8 @@ int hy_prepare(BlockStack* s) {
     SLI_HIP(hipMemcpy(s->fnorm, g.data(), sizeof(float) * Dp, hipMemcpyHostToDevice));
     for (int d = 0; d < s->D; ++d) g[d] = (float)(g[d] * std::sqrt((double)s->D / Dp));
     SLI_HIP(hipMemcpy(s->fnorm_p, g.data(), sizeof(float) * Dp, hipMemcpyHostToDevice));
-    HY_TRY(hy_sync_tiles(s));
     s->dirty = false;
+    s->tiles_dirty = true;
     return SLI_OK;
 }
 
@@ -872,6 +873,11 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
         for (const SegRef& g : segs) kt += seq_key_tiles(s, g.pos0, g.n);
         SLI_CHECK(kt <= hy_key_tiles_max(s), SLI_ERR_SHAPE, "pass: too many expanded rows");
     }
+    // passes and heads that run the batched projection (HyProj::path): one row does where a depth is past the GEMV's
+    int deep = s->Dp;
+    for (const HyLayer& l : s->layers) deep = std::max(deep, l.Kp);
+    const auto batched = [](int k, int K) { return k >= (K > kGemvMaxCols ? 1 : 2) && k <= kBgMaxBatch; };
+    if ((one && batched(M, deep)) || batched((int)(want.size() % kHyLogitRows), s->Dp)) HY_TRY(hy_sync_tiles(s));
     std::vector<RowRef> rows(rows_in);
     rows.resize(M, RowRef{-1, 0, 0, 0});
     const int32_t ns = (int32_t)segs.size();

@@ -113,7 +113,9 @@ struct BlockStack {
     std::vector<float> fgain;  // one gain, or one per channel
     std::map<std::string, bool> want;  // tensor -> placed
     bool dirty = true;
-    bool tiled = false;     // decode passes of several sequences stream copies in the fragment layout (bgemm.h BgIn::tiled)
+    // decode passes of several sequences stream copies in the fragment layout (bgemm.h BgIn::tiled), built before the first one
+    // after weights were placed (hy_sync_tiles)
+    bool tiled = false, tiles_dirty = true;
     void* head_t = nullptr;
     // activations of a pass
     RowRef* rows = nullptr;
