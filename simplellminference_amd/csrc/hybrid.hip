@@ -767,7 +767,12 @@ struct HyRec : HyProj<WT> {
             }
         }
         const HyOut eo{s->x, s->Dp, s->D, s->c.residual_mult};
-        return project(l.wout, cat<OT>(l), l.Kp, (s->D + 1) / 2, 0, eo, l.wout_t);
+        if constexpr (!std::is_same<OT, float>::value) {
+            // (x and its input have rows to spare: rows past M are computed where that is faster, and read by nobody)
+            return pgemm((const WT*)l.wout, cat<OT>(l), nullptr, 0, l.Kp, (s->D + 1) / 2, 0, eo, s->M);
+        } else {
+            return project(l.wout, cat<OT>(l), l.Kp, (s->D + 1) / 2, 0, eo, l.wout_t);
+        }
     }
     int embed() const {
         hipLaunchKernelGGL(hy_embed_kernel<WT>, dim3(M), dim3(256), 0, st(), s->rows, (const WT*)s->emb, (const WT*)s->pos,

@@ -77,22 +77,28 @@ struct HyProj {
     }
     // pairs [0, split) read X, pairs [split, npairs) X2 (split: a multiple of kHySection; X2 null: one input)
     template <class Epi>
-    int pgemm(const WT* w, const __half* X, const __half* X2, int split, int K, int npairs, int u0, const Epi& e) const {
+    int pgemm(const WT* w, const __half* X, const __half* X2, int split, int K, int npairs, int u0, const Epi& e, int spare = 0) const {
         if constexpr (F16) {
             PgIn<__half> in{w, X, nullptr, pad_to(2 * npairs, 16), K, M};
             if (X2) in.Bhi2 = X2, in.row_b2 = 2 * split;
             in.ws = s->pg_ws, in.cnt = s->pg_cnt;
             float best = INFINITY;
-            int pick = 0, i = 0;
+            int pick = 0;
             constexpr bool rolled = PgRolled<PgPair<Epi>>::value;
-            pg_row_tilings(M, rolled, [&](auto cfg, float us) {
-                const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, M, device_cus(), true, us, rolled);
-                if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits;
-                ++i;
-            });
+            // spare: rows there are. Tiles of 256 rows over more rows than there are to do may be faster than tiles of 128: 4096 x
+            // 15104 at 1152 rows 191 us, at 1280 rows 169.
+            for (int m : {M, pad_to(M, 256)}) {
+                int i = 0;
+                if (m > M && m > spare) break;
+                pg_row_tilings(m, rolled, [&](auto cfg, float us) {
+                    const PgPlan p = pg_plan<decltype(cfg), __half>(in.N, K, m, device_cus(), true, us, rolled);
+                    if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits, in.M = m;
+                    ++i;
+                });
+            }
             hipError_t err = hipSuccess;
-            i = 0;
-            pg_row_tilings(M, rolled, [&](auto cfg, float) {
+            int i = 0;
+            pg_row_tilings(in.M, rolled, [&](auto cfg, float) {
                 if (i++ == pick) err = launch_pgemm<PgPair<Epi>, decltype(cfg), __half>(in, PgPair<Epi>{e, npairs, u0}, PfState{}, st());
             });
             SLI_HIP(err);
