@@ -79,61 +79,72 @@ struct EpiParts<E, std::void_t<decltype(E::kParts)>> {
     static constexpr bool value = E::kParts;
 };
 
+// Staged by the first waves, four float4 a thread, as many as the input fills (4096 columns: 4 of the 16): a wave's 16-byte load costs
+// the CU's load unit 16 cycles whether its lanes hold new columns or repeat the last, and the weights queue behind it. All 16
+// waves loading four rounds of x and of the norm weights before, us: 12288 x 4096 int8 13.2 -> 11.9, fp16 18.1 -> 17.7; 4096 x
+// 11008 int8 11.6 -> 10.8, fp16 16.5 -> 16.3. (The branches are uniform, and no wait crosses them but the waves' own.)
 template <int G>
 struct XStage {
     float4 xr[kGemvStageV4];
     float4 wr[kGemvStageV4];
+    int nt = 0;  // threads that stage: whole waves, the first ones, four float4 each
     __device__ __forceinline__ void issue(const GemvIn& in) {
-        const int tid = threadIdx.x, nt = kGemvThreads, n4 = in.cols >> 2;
+        const int tid = threadIdx.x, n4 = in.cols >> 2;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        nt = ((n4 + kGemvStageV4 - 1) / kGemvStageV4 + 63) & ~63;
+        if (wave * 64 >= nt) return;  // (uniform)
         const float4* x4 = reinterpret_cast<const float4*>(in.x);
-        // unconditional (clamped) loads: a load under a branch would make the weight waits conservative
-        const float4* w4 = reinterpret_cast<const float4*>(in.norm_w ? in.norm_w : in.x);
 #pragma unroll
-        for (int k = 0; k < kGemvStageV4; ++k) {
-            xr[k] = x4[min(tid + k * nt, n4 - 1)];
-            wr[k] = w4[min(tid + k * nt, n4 - 1)];
+        for (int k = 0; k < kGemvStageV4; ++k) xr[k] = x4[min(tid + k * nt, n4 - 1)];
+        if (in.norm_w) {
+            const float4* w4 = reinterpret_cast<const float4*>(in.norm_w);
+#pragma unroll
+            for (int k = 0; k < kGemvStageV4; ++k) wr[k] = w4[min(tid + k * nt, n4 - 1)];
         }
     }
-    // x (optionally RMS-normalised, rms_kernel.cpp:5-23) into LDS; the caller then barriers. Stores are
-    // unconditional too (clamped rounds rewrite the last vector with its own value).
+    // x (optionally RMS-normalised, rms_kernel.cpp:5-23) into LDS; the caller then barriers. (Clamped rounds rewrite the last
+    // vector with its own value.)
     __device__ __forceinline__ void commit(float* smem, const GemvIn& in) {
         float* red = smem;
         float4* xs4 = reinterpret_cast<float4*>(smem + kGemvLdsHead);
-        const int tid = threadIdx.x, nt = kGemvThreads, n4 = in.cols >> 2;
+        const int tid = threadIdx.x, n4 = in.cols >> 2;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const bool mine = wave * 64 < nt;
         if (in.norm_w == nullptr) {
+            if (mine) {
 #pragma unroll
-            for (int k = 0; k < kGemvStageV4; ++k) xs4[xswz<G>(min(tid + k * nt, n4 - 1))] = xr[k];
+                for (int k = 0; k < kGemvStageV4; ++k) xs4[xswz<G>(min(tid + k * nt, n4 - 1))] = xr[k];
+            }
             return;
         }
-        float ss = 0.0f;
+        if (mine) {
+            float ss = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kGemvStageV4; ++k) {
-            const float m = tid + k * nt < n4 ? 1.0f : 0.0f;
-            ss += m * (xr[k].x * xr[k].x);
-            ss += m * (xr[k].y * xr[k].y);
-            ss += m * (xr[k].z * xr[k].z);
-            ss += m * (xr[k].w * xr[k].w);
+            for (int k = 0; k < kGemvStageV4; ++k) {
+                const float m = tid + k * nt < n4 ? 1.0f : 0.0f;
+                ss += m * (xr[k].x * xr[k].x);
+                ss += m * (xr[k].y * xr[k].y);
+                ss += m * (xr[k].z * xr[k].z);
+                ss += m * (xr[k].w * xr[k].w);
+            }
+            ss = wave_sum(ss);
+            if ((tid & 63) == 0) red[wave] = ss;
         }
-        ss = wave_sum(ss);
-        if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
-        if (tid == 0) {
+        if (mine) {
             float t = 0.0f;
             for (int w = 0; w < (nt >> 6); ++w) t += red[w];
-            const float tep = t / (float)in.cols;  // rms_kernel.cpp:17
-            const float rms = sqrtf(tep + in.eps);  // :18
-            red[32] = 1.0f / rms;                   // :19
-        }
-        __syncthreads();
-        const float inv = red[32];
+            const float tep = t / (float)in.cols;         // rms_kernel.cpp:17
+            const float inv = 1.0f / sqrtf(tep + in.eps);  // :18-19
 #pragma unroll
-        for (int k = 0; k < kGemvStageV4; ++k) {  // :20-22  y = (x * inv) * w
-            float4 o;
-            o.x = (xr[k].x * inv) * wr[k].x;
-            o.y = (xr[k].y * inv) * wr[k].y;
-            o.z = (xr[k].z * inv) * wr[k].z;
-            o.w = (xr[k].w * inv) * wr[k].w;
-            xs4[xswz<G>(min(tid + k * nt, n4 - 1))] = o;
+            for (int k = 0; k < kGemvStageV4; ++k) {  // :20-22  y = (x * inv) * w
+                float4 o;
+                o.x = (xr[k].x * inv) * wr[k].x;
+                o.y = (xr[k].y * inv) * wr[k].y;
+                o.z = (xr[k].z * inv) * wr[k].z;
+                o.w = (xr[k].w * inv) * wr[k].w;
+                xs4[xswz<G>(min(tid + k * nt, n4 - 1))] = o;
+            }
         }
     }
 };
@@ -172,9 +183,11 @@ struct XStageMerge {
             const int ub = (int)(((unsigned)(blockIdx.x * nw) * (unsigned)(am.ksplit * am.kunits)) / (unsigned)(gridDim.x * nw));
             h0 = (ub / am.kunits) * (in.cols / am.hd);
         }
+        pos = *am.pos_dev;
+        // no input of this wave's (uniform; 2048 columns of a K-split wo at 7B: 8 of 16 waves, fp16 9.4 -> 8.7 us, int8 7.9 -> 7.4)
+        if (__builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) >= in.cols >> 2) return;
         const int f = min((int)threadIdx.x, (in.cols >> 2) - 1);  // the first round of the input
         const int d4 = f % (am.hd >> 2);
-        pos = *am.pos_dev;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const float* r = row(f, s);

@@ -72,6 +72,23 @@ def test_matmul_i8_weights(gpu, oracle, rows, cols):
     _close(got, want, rtol=1e-4, atol=1e-4)
 
 
+# gemv.h XStage: the input is staged by the waves it fills at four float4 a thread; columns on both sides of a wave's 1024, one row
+# and the widest input a launch stages
+@pytest.mark.parametrize("cols", [8, 1016, 1024, 1032, 4088, 4104, 15360, 16320])
+@pytest.mark.parametrize("rows", [1, 33])
+def test_matmul_staging_edges(gpu, rows, cols):
+    torch = gpu
+    from simplellminference_amd import ops
+    r = _rng(rows + cols)
+    x = r.standard_normal(cols).astype(np.float32)
+    w = (r.standard_normal((rows, cols)) / np.sqrt(cols)).astype(np.float16)
+    w64 = w.astype(np.float64)
+    want, mag = w64 @ x, np.abs(w64) @ np.abs(x)
+    for t in (np.float16, np.float32):
+        got = ops.matmul(_t(torch, x), _t(torch, w.astype(t))).cpu().numpy()
+        assert np.all(np.abs(got - want) <= 4 * np.finfo(np.float32).eps * np.sqrt(cols) * mag), (t, np.abs(got - want).max())
+
+
 @pytest.mark.parametrize("dim", [256, 4096, 3072, 1000])
 def test_rmsnorm(gpu, oracle, dim):
     torch = gpu
