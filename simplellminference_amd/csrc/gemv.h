@@ -284,15 +284,11 @@ struct XStageSum {
         ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
         __syncthreads();
-        if (tid == 0) {
-            float t = 0.0f;
-            for (int w = 0; w < (kGemvThreads >> 6); ++w) t += red[w];
-            const float tep = t / (float)in.cols;  // rms_kernel.cpp:17
-            const float rms = sqrtf(tep + in.eps);  // :18
-            red[32] = 1.0f / rms;                   // :19
-        }
-        __syncthreads();
-        const float inv = red[32];
+        float t = 0.0f;
+#pragma unroll
+        for (int w = 0; w < (kGemvThreads >> 6); ++w) t += red[w];
+        const float tep = t / (float)in.cols;          // rms_kernel.cpp:17
+        const float inv = 1.0f / sqrtf(tep + in.eps);  // :18-19
         float4 o;  // :20-22  y = (x * inv) * w
         o.x = (v.x * inv) * wr.x;
         o.y = (v.y * inv) * wr.y;
@@ -367,7 +363,11 @@ inline size_t gemv_res_floats(int units, int grid, int R, int csplit = 1) {
 // for the first weight chunk (staged 4-6 us into a 10-30 us launch). The epilogue (residual reads,
 // RoPE, K/V writes, logits) runs once per workgroup after the loop, one thread per unit.
 // Prologue order: input loads, first weight chunk, input commit + barrier (see XStage).
-template <typename WT, int R, int U, bool NT, class Epi, class Stage, int NB = 2, bool SPLIT = false, bool OFFS = false>
+// ROWS: a unit's R rows are items of their own, so that the waves share a workgroup's rows and not its units (28672 x 4096, 56
+// units a workgroup: 7 rows a wave, where units give 3 or 4), and a step is one row's; the epilogue finds the unit's sums in
+// LDS as before, and a row's sum is the same, bit for bit. gemv_by_rows says where.
+template <typename WT, int R, int U, bool NT, class Epi, class Stage, int NB = 2, bool SPLIT = false, bool OFFS = false,
+          bool ROWS = false>
 __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvIn& in, Epi& epi, Stage& stage,
                                            float* smem) {
     const float* xs = smem + kGemvLdsHead;
@@ -390,10 +390,13 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
     // cpp chunks; the workgroup's (unit, part) items are balanced over its waves and the parts' row sums
     // are added in part order in the epilogue. CS = 1: one item per unit, the whole row per wave.
     const int CS = SPLIT ? in.csplit : 1;  // compile-time 1 unless the launch split the columns
+    static_assert(!ROWS || !SPLIT, "rows or column parts");
+    constexpr int SR = ROWS ? 1 : R;      // rows of an item
+    const int per = ROWS ? R : CS;        // items of a unit (Pos::p: its row or column part)
     constexpr bool PARTS = EpiParts<Epi>::value;
     static_assert(!PARTS || SPLIT, "parts need the split form");
     const int cpp = PARTS ? cpr : (cpr + CS - 1) / CS;  // chunks per part (a part past the row end is all masked)
-    const int ni = (ue - ub) * CS;       // the workgroup's items
+    const int ni = (ue - ub) * per;      // the workgroup's items
     // in.cw streaming waves share the items; a wave past them has none and repeats the loads of wave
     // (wave - cw)'s first steps (L2 hits on lines in flight), so no load sits behind a branch
     const int cw = in.cw;
@@ -421,7 +424,7 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
         int it, u, p, cc;
     };
     const int it_last = max(ie - 1, ib);
-    const Pos last{it_last, min(ub + it_last / CS, nunits - 1), it_last - (it_last / CS) * CS, cpp - 1};
+    const Pos last{it_last, min(ub + it_last / per, nunits - 1), it_last - (it_last / per) * per, cpp - 1};
     // A load past the wave's last step (its last round when the step count is not a multiple of NB, or the
     // first rounds of a wave with fewer than NB steps) reads the matrix's first chunk instead of repeating its
     // own last step: that repeat was issued after the first copy had landed, so it went back to HBM (int8
@@ -432,19 +435,23 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
 #define SLI_GEMV_DUP_LOADS 0
 #endif
     const Pos dummy = SLI_GEMV_DUP_LOADS ? last : Pos{0, 0, 0, 0};
-    auto load_step = [&](const Pos& q, u32x4 (&w)[U][R]) {
+    auto load_step = [&](const Pos& q, u32x4 (&w)[U][SR]) {
         const Pos& a = q.it > it_last ? dummy : q;
         int rows[R];
         if constexpr (PARTS)
             epi.rows_part(min(a.u, nunits - 1), a.p, rows);
         else
             epi.rows(min(a.u, nunits - 1), rows);
-        const int v = (PARTS ? a.cc : a.p * cpp + a.cc) * CV + lane;
+        const int v = (PARTS || ROWS ? a.cc : a.p * cpp + a.cc) * CV + lane;
+        if constexpr (ROWS) {
+#pragma unroll
+            for (int r = 1; r < R; ++r) rows[0] = a.p == r ? rows[r] : rows[0];
+        }
 #pragma unroll
         for (int j = 0; j < U; ++j) {
             const int vj = min(v + j * 64, nvec - 1);  // clamp, never branch around a load
 #pragma unroll
-            for (int r = 0; r < R; ++r)
+            for (int r = 0; r < SR; ++r)
                 w[j][r] = load16<NT>(reinterpret_cast<const char*>(W) + (size_t)rows[r] * row_bytes + (size_t)vj * 16);
         }
     };
@@ -452,28 +459,28 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
         if (++q.cc == cpp) {
             q.cc = 0;
             ++q.it;
-            if (++q.p == CS) {
+            if (++q.p == per) {
                 q.p = 0;
                 ++q.u;
             }
         }
     };
-    float acc[R];
+    float acc[SR];
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-    auto consume_step = [&](const Pos& q, const u32x4(&w)[U][R]) {
-        const int c = PARTS ? q.cc : q.p * cpp + q.cc;
+    for (int r = 0; r < SR; ++r) acc[r] = 0.0f;
+    auto consume_step = [&](const Pos& q, const u32x4(&w)[U][SR]) {
+        const int c = PARTS || ROWS ? q.cc : q.p * cpp + q.cc;
         const int v = c * CV + lane;
         const float* xp = PARTS ? xs + (size_t)q.p * in.cols : xs;
         if ((c + 1) * CV <= nvec)
-            gemv_chunk<WT, R, U>(w, xp, v, acc);
+            gemv_chunk<WT, SR, U>(w, xp, v, acc);
         else
-            gemv_chunk<WT, R, U, true>(w, xp, v, acc, nvec);
+            gemv_chunk<WT, SR, U, true>(w, xp, v, acc, nvec);
         if (q.cc == cpp - 1) {  // item complete: its R partial row sums go to LDS
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
+            for (int r = 0; r < SR; ++r) {
                 const float t = wave_sum(acc[r]);
-                if (lane == 0) res[((q.u - ub) * CS + q.p) * R + r] = t;
+                if (lane == 0) res[((q.u - ub) * per + q.p) * SR + r] = t;
                 acc[r] = 0.0f;
             }
         }
@@ -484,8 +491,8 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
     // duplicates one issued just before it (an in-flight miss to the same lines) and is never consumed;
     // no clamped load is ever issued after its data was consumed (a fresh HBM round trip at the end of
     // every wave).
-    u32x4 wbuf[NB][U][R];
-    const Pos first{ib, ub + ib / CS, ib - (ib / CS) * CS, 0};
+    u32x4 wbuf[NB][U][SR];
+    const Pos first{ib, ub + ib / per, ib - (ib / per) * per, 0};
     Pos lq = first;  // next step to load
     Pos cq = first;  // next step to consume
 #pragma unroll
@@ -541,12 +548,12 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
     }
 }
 
-template <typename WT, int R, int U, bool NT, class Epi, int NB = 2, bool SPLIT = false>
+template <typename WT, int R, int U, bool NT, class Epi, int NB = 2, bool SPLIT = false, bool ROWS = false>
 __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const WT* __restrict__ W, GemvIn in, Epi epi_in) {
     Epi epi = epi_in;  // mutable per-thread copy (EpiLogits keeps a running key)
     extern __shared__ __attribute__((aligned(16))) float smem[];
     XStage<Vec16<WT>::N / 4> stage;
-    gemv_block<WT, R, U, NT, Epi, XStage<Vec16<WT>::N / 4>, NB, SPLIT>(W, in, epi, stage, smem);
+    gemv_block<WT, R, U, NT, Epi, XStage<Vec16<WT>::N / 4>, NB, SPLIT, false, ROWS>(W, in, epi, stage, smem);
 }
 
 // the wo GEMV with its input merged from the attention's split partials (XStageMerge)
@@ -560,13 +567,13 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_merge_kernel(const WT* __re
 }
 
 // a GEMV whose input is x plus NP partial vectors (XStageSum)
-template <typename WT, int R, int U, bool NT, class Epi, int NP, int NB = 2>
+template <typename WT, int R, int U, bool NT, class Epi, int NP, int NB = 2, bool ROWS = false>
 __global__ void __launch_bounds__(kGemvThreads) gemv_sum_kernel(const WT* __restrict__ W, GemvIn in, Epi epi_in,
                                                                 const float* parts) {
     Epi epi = epi_in;
     extern __shared__ __attribute__((aligned(16))) float smem[];
     XStageSum<Vec16<WT>::N / 4, NP> stage{parts};
-    gemv_block<WT, R, U, NT, Epi, XStageSum<Vec16<WT>::N / 4, NP>, NB>(W, in, epi, stage, smem);
+    gemv_block<WT, R, U, NT, Epi, XStageSum<Vec16<WT>::N / 4, NP>, NB, false, false, ROWS>(W, in, epi, stage, smem);
 }
 
 // Row-by-row fallback for shapes the vector kernel cannot take (cols*sizeof(WT) not a multiple of 16
@@ -908,14 +915,15 @@ inline int gemv_blocks(int units, int csplit = 1) {
 // CU's share of the HBM stream stays under its per-CU fetch rate (gate/up: 230 workgroups, 31.4 -> 29.0 us,
 // C1 358 -> 368 tok/s; qkv at 1.5 units per wave would need 192 workgroups: measured slower, 17.9 -> 20.5 us;
 // profiles/r3_gemv_balance_ab.txt).
-inline int gemv_balanced_blocks(int units) {
-    const int b = gemv_blocks(units);
+// per: items of a unit (gemv_block ROWS: rows), of which a wave owns whole ones.
+inline int gemv_balanced_blocks(int units, int per = 1) {
+    const int b = gemv_blocks(units, per), items = units * per;
     const int w = kGemvThreads / 64;
-    const int k = (units + b * w - 1) / (b * w);  // most units of a wave at the full grid
-    const int g = (units + k * w - 1) / (k * w);
-    // only where the full grid's tail is real (>= 8 % more unit slots than units; the LM head's 2.4 % measured
+    const int k = (items + b * w - 1) / (b * w);  // most items of a wave at the full grid
+    const int g = (items + k * w - 1) / (k * w);
+    // only where the full grid's tail is real (>= 8 % more item slots than items; the LM head's 2.4 % measured
     // slower at 250 workgroups: 41.2 -> 43-44 us)
-    return (g < b && 8 * g >= 7 * b && 100LL * k * b * w >= 108LL * units) ? g : b;
+    return (g < b && 8 * g >= 7 * b && 100LL * k * b * w >= 108LL * items) ? g : b;
 }
 
 // Streaming waves per workgroup: with u units per workgroup and 16 waves, waves hold ceil(u / 16) or one
@@ -973,27 +981,54 @@ hipError_t launch_gemv_merge_ks(const WT* W, const GemvIn& in_, const Epi& epi, 
                        epi, am);
     return hipGetLastError();
 }
+// Vectors of a row in flight per lane and step where rows are streamed one by one (gemv_block ROWS), us at 12288 x 4096: int8
+// 10.4 with 2, 11.2 with 4; fp16 17.0 with 4, 18.6 with 8; fp32 32.7 with 4, 31.9 with 8.
+template <typename WT>
+constexpr int kGemvRowU = sizeof(WT) == 1 ? 2 : sizeof(WT) == 2 ? 4 : 8;
+// The share of the chip's wave slots that hold an item when no wave holds more than it must.
+inline float gemv_fill(int items) {
+    const int waves = gemv_max_blocks() * (kGemvThreads / 64);
+    return (float)items / ((float)((items + waves - 1) / waves) * waves);
+}
+// Units of two rows are streamed row by row (ROWS) where the units would need two column parts to give every wave an item, or where
+// rows fill a tenth more of the chip's waves: us, int8 | fp16 | fp32, pairs -> rows: 28672 x 4096 (fill 0.875 -> 1) 24.2 | 39.8 |
+// 75.3 -> 19.9 | 36.5 | 70.7; 12288 x 4096 (0.75 -> 1) 11.5 | 17.1 | 32.5 -> 10.4 | 17.0 | 31.9; where the fill is the same
+// 22016 x 4096 16.9 | 29.8 -> 16.1 | 29.6 alone but 17.4 | 28.98 -> 17.6 | 29.01 in a 7B step, and its 32000-row head 26.7 | 41.8 ->
+// 28.0 | 43.2. 16-bit pairs that have the whole chip stay (12288 in that step: 17.8, rows 17.9).
+template <typename WT, int R>
+inline bool gemv_by_rows(int units, int cs) {
+    if (R != 2 || cs > 2) return false;
+    if (cs == 2) return true;
+    if (sizeof(WT) == 2 && gemv_balanced_blocks(units) == gemv_max_blocks()) return false;
+    return gemv_fill(units * R) >= gemv_fill(units) + 0.1f;
+}
 template <typename WT, int R, int U, bool NT, class Epi, int NP, int NB = 2>
 hipError_t launch_gemv_sum(const WT* W, const GemvIn& in_, const Epi& epi, const float* parts, int units,
                            hipStream_t s) {
     if (in_.csplit != 1 || in_.cols > 4 * kGemvThreads) return hipErrorInvalidValue;  // XStageSum: one round
     GemvIn in = in_;
-    const int grid = gemv_balanced_blocks(units);
-    in.cw = gemv_wave_count<WT>(units, grid);
+    const bool by_rows = gemv_by_rows<WT, R>(units, 1);
+    const int per = by_rows ? R : 1, grid = gemv_balanced_blocks(units, per);
+    in.cw = gemv_wave_count<WT>(units * per, grid);
     const size_t lds = gemv_lds_bytes(in.cols) + sizeof(float) * gemv_res_floats(units, grid, R);
-    hipLaunchKernelGGL((gemv_sum_kernel<WT, R, U, NT, Epi, NP, NB>), dim3(grid), dim3(kGemvThreads), lds, s, W, in,
-                       epi, parts);
+    if (by_rows)
+        hipLaunchKernelGGL((gemv_sum_kernel<WT, R, kGemvRowU<WT>, NT, Epi, NP, NB, true>), dim3(grid), dim3(kGemvThreads), lds, s, W,
+                           in, epi, parts);
+    else
+        hipLaunchKernelGGL((gemv_sum_kernel<WT, R, U, NT, Epi, NP, NB>), dim3(grid), dim3(kGemvThreads), lds, s, W, in,
+                           epi, parts);
     return hipGetLastError();
 }
 
-template <typename WT, int R, int U, bool NT, class Epi, int NB = 2, bool SPLIT = false>
+template <typename WT, int R, int U, bool NT, class Epi, int NB = 2, bool SPLIT = false, bool ROWS = false>
 hipError_t launch_gemv(const WT* W, const GemvIn& in_, const Epi& epi, int units, hipStream_t s) {
     if (!SPLIT && in_.csplit != 1) return hipErrorInvalidValue;  // a split needs the SPLIT instantiation
     GemvIn in = in_;
-    const int grid = in.csplit == 1 ? gemv_balanced_blocks(units) : gemv_blocks(units, in.csplit);
-    in.cw = in.csplit == 1 ? gemv_wave_count<WT>(units, grid) : kGemvThreads / 64;
+    constexpr int per = ROWS ? R : 1;  // items of a unit
+    const int grid = in.csplit == 1 ? gemv_balanced_blocks(units, per) : gemv_blocks(units, in.csplit);
+    in.cw = in.csplit == 1 ? gemv_wave_count<WT>(units * per, grid) : kGemvThreads / 64;
     const size_t lds = gemv_lds_bytes(in.cols) + sizeof(float) * gemv_res_floats(units, grid, R, in.csplit);
-    hipLaunchKernelGGL((gemv_kernel<WT, R, U, NT, Epi, NB, SPLIT>), dim3(grid), dim3(kGemvThreads), lds, s, W, in,
+    hipLaunchKernelGGL((gemv_kernel<WT, R, U, NT, Epi, NB, SPLIT, ROWS>), dim3(grid), dim3(kGemvThreads), lds, s, W, in,
                        epi);
     return hipGetLastError();
 }
@@ -1023,11 +1058,18 @@ inline GemvSplit gemv_split(int units, int cols) {
     if (UW > 2 && need <= cpr(2)) return {need, 2};
     return {std::max(1, std::min(need, cpr(1))), 1};
 }
+template <typename WT>
+inline int gemv_u_blocks(int units, int cs) {  // launch_gemv_u's grid for two-row units
+    return gemv_by_rows<WT, 2>(units, cs) ? gemv_balanced_blocks(units, 2) : cs == 1 ? gemv_balanced_blocks(units) : gemv_blocks(units, cs);
+}
 template <typename WT, int R, int U, bool NT, class Epi>
 hipError_t launch_gemv_u(const WT* W, const GemvIn& in_, const Epi& epi, int units, hipStream_t s) {
     constexpr int UW = std::is_same<WT, int8_t>::value && U >= 2 ? U / 2 : U;
     GemvIn in = in_;
     const GemvSplit sp = gemv_split<WT, U>(units, in.cols);
+    if constexpr (R == 2) {
+        if (gemv_by_rows<WT, R>(units, sp.cs)) return launch_gemv<WT, R, kGemvRowU<WT>, NT, Epi, 2, false, true>(W, in, epi, units, s);
+    }
     in.csplit = sp.cs;
     if (sp.cs == 1) return launch_gemv<WT, R, UW, NT>(W, in, epi, units, s);
     if (sp.u == UW) return launch_gemv<WT, R, UW, NT, Epi, 2, true>(W, in, epi, units, s);

@@ -811,7 +811,7 @@ struct HyRec : HyProj<WT> {
             GemvIn in{s->x, s->fnorm_p, (float)((double)s->c.eps * s->D / s->Dp), s->Dp};
             const EpiLogits<2> e{y, keys, nullptr, s->V, 0, 0ull};
             const int units = (s->V + 1) / 2, cs = gemv_split<WT, 4>(units, s->Dp).cs;
-            *nkeys = cs == 1 ? gemv_balanced_blocks(units) : gemv_blocks(units, cs);  // launch_gemv's grid
+            *nkeys = gemv_u_blocks<WT>(units, cs);  // launch_gemv's grid
             SLI_HIP((launch_gemv_u<WT, 2, 4, true>((const WT*)s->head, in, e, units, st())));
             return SLI_OK;
         }

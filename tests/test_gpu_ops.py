@@ -89,6 +89,24 @@ def test_matmul_staging_edges(gpu, rows, cols):
         assert np.all(np.abs(got - want) <= 4 * np.finfo(np.float32).eps * np.sqrt(cols) * mag), (t, np.abs(got - want).max())
 
 
+# gemv.h gemv_by_rows: two-row units whose rows are streamed one by one (4096 waves: 4097 .. 8190 rows; 12287 and 28671, whose units
+# fill 3/4 and 7/8 of the waves' slots), an odd last row, rows shorter than a step and not a multiple of one
+@pytest.mark.parametrize("rows,cols", [(4097, 16), (4098, 1040), (6143, 4096), (8189, 272), (12287, 1040), (28671, 528)])
+def test_matmul_by_rows(gpu, rows, cols):
+    torch = gpu
+    from simplellminference_amd import ops
+    r = _rng(rows + cols)
+    x = r.standard_normal(cols).astype(np.float32)
+    q = r.integers(-127, 128, (rows, cols), dtype=np.int8)
+    s = (r.random(rows) * 0.01 + 0.001).astype(np.float32)
+    q64 = q.astype(np.float64)
+    lim = 4 * np.finfo(np.float32).eps * np.sqrt(cols) * (np.abs(q64) @ np.abs(x))
+    for t, sc in ((np.int8, s), (np.float16, None), (np.float32, None)):
+        got = ops.matmul(_t(torch, x), _t(torch, q.astype(t)), row_scale=None if sc is None else _t(torch, sc)).cpu().numpy()
+        k = 1.0 if sc is None else sc.astype(np.float64)
+        assert np.all(np.abs(got - (q64 @ x) * k) <= lim * k), t
+
+
 @pytest.mark.parametrize("dim", [256, 4096, 3072, 1000])
 def test_rmsnorm(gpu, oracle, dim):
     torch = gpu
