@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
     const int sbc = min(sb, B - 1);
     const int wq = lane & 3, wbo = (lane >> 2) & 1;  // per-wave staging: 8-k group, block offset
     float4 xa[kBgNH][2];
-    float4 wn[NORM ? kBgNH : 1][2];
+    u32x4 wnv{};  // float4 lane & 7 of the wave's block lane >> 3
 #ifdef BG_LAB_NOSTAGE  // tools/bgemm_lab only: no activation loads (an upper bound on what a ready image saves)
     constexpr bool kStage = false;
 #else
@@ -256,13 +256,8 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
         xa[n][1] = kStage ? xp[1] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if constexpr (NORM && kStage) {
-#pragma unroll
-        for (int n = 0; n < kBgNH; ++n) {
-            const int blk = wb0 + max(min(2 * n + wbo, wnb - 1), 0);
-            const float4* wp = reinterpret_cast<const float4*>(in.norm_w + (size_t)(min(blk, nkb - 1) * 4 + wq) * 8);
-            wn[n][0] = wp[0];
-            wn[n][1] = wp[1];
-        }
+        const int blk = min(wb0 + max(min(lane >> 3, wnb - 1), 0), nkb - 1);
+        wnv = reinterpret_cast<const u32x4*>(in.norm_w)[blk * 8 + (lane & 7)];
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -295,6 +290,19 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
     // ---- 3./4. this wave's blocks into LDS as B fragments (hi: column b, lo: 8 + b), visible to the
     // wave's own later reads after lgkmcnt(0); NORM: x * w staged, this wave's sum of x^2 to red[wave][b]
     float ss = 0.0f;
+    u32x4 wn[NORM ? kBgNH : 1][2];
+    if constexpr (NORM) {
+        // the wave's norm weights through its own first image block: one load instead of eight whose lanes hold the same 256
+        // bytes for every sequence (8 rows, 28672 | 6144 | 128256 x 4096: 38.8 | 13.3 | 162.8 -> 38.4 | 13.2 | 160.9 us)
+        u32x4* wl = img + (size_t)(wb0 - kb0) * 64;
+        if (wnb > 0) wl[lane] = wnv;  // (a wave without blocks has none of the image)
+        asm volatile("" ::: "memory");  // (a wave's LDS operations are in order; the lanes' are not the compiler's to reorder)
+#pragma unroll
+        for (int n = 0; n < kBgNH; ++n)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wn[n][h] = wl[(2 * n + wbo) * 8 + wq * 2 + h];
+        asm volatile("" ::: "memory");
+    }
 #pragma unroll
     for (int n = 0; n < kBgNH; ++n) {
         const int bw = 2 * n + wbo;
@@ -304,10 +312,8 @@ __global__ void __launch_bounds__(kBgThreads) bgemm_kernel(const __half* __restr
 #pragma unroll
             for (int e = 0; e < 8; ++e) v += y[e] * y[e];
             ss += bw < wnb ? v : 0.0f;
-            const float wv[8] = {wn[n][0].x, wn[n][0].y, wn[n][0].z, wn[n][0].w,
-                                 wn[n][1].x, wn[n][1].y, wn[n][1].z, wn[n][1].w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = bg_mul_rn(y[e], wv[e]);
+            for (int e = 0; e < 8; ++e) y[e] = bg_mul_rn(y[e], __uint_as_float(wn[n][e >> 2][e & 3]));
         }
         if (seq_live && bw < wnb) {
             u32x4 hi, lo;
