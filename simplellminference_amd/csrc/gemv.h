@@ -365,7 +365,7 @@ inline size_t gemv_res_floats(int units, int grid, int R, int csplit = 1) {
 // Prologue order: input loads, first weight chunk, input commit + barrier (see XStage).
 // ROWS: a unit's R rows are items of their own, so that the waves share a workgroup's rows and not its units (28672 x 4096, 56
 // units a workgroup: 7 rows a wave, where units give 3 or 4), and a step is one row's; the epilogue finds the unit's sums in
-// LDS as before, and a row's sum is the same, bit for bit. gemv_by_rows says where.
+// LDS as before. gemv_by_rows says where.
 template <typename WT, int R, int U, bool NT, class Epi, class Stage, int NB = 2, bool SPLIT = false, bool OFFS = false,
           bool ROWS = false>
 __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvIn& in, Epi& epi, Stage& stage,
@@ -465,18 +465,31 @@ __device__ __forceinline__ void gemv_block(const WT* __restrict__ W, const GemvI
             }
         }
     };
-    float acc[SR];
-#pragma unroll
-    for (int r = 0; r < SR; ++r) acc[r] = 0.0f;
+    // (ROWS: a step's second half has a sum of its own, so no chain is longer than a column part's was)
+    float acc[ROWS ? 2 : SR] = {};
     auto consume_step = [&](const Pos& q, const u32x4(&w)[U][SR]) {
         const int c = PARTS || ROWS ? q.cc : q.p * cpp + q.cc;
         const int v = c * CV + lane;
         const float* xp = PARTS ? xs + (size_t)q.p * in.cols : xs;
-        if ((c + 1) * CV <= nvec)
+        if constexpr (ROWS) {
+            typedef u32x4 Half[U / 2][1];
+            const Half &w0 = reinterpret_cast<const Half&>(w[0]), &w1 = reinterpret_cast<const Half&>(w[U / 2]);
+            if ((c + 1) * CV <= nvec) {
+                gemv_chunk<WT, 1, U / 2>(w0, xp, v, acc);
+                gemv_chunk<WT, 1, U / 2>(w1, xp, v + CV / 2, acc + 1);
+            } else {
+                gemv_chunk<WT, 1, U / 2, true>(w0, xp, v, acc, nvec);
+                gemv_chunk<WT, 1, U / 2, true>(w1, xp, v + CV / 2, acc + 1, nvec);
+            }
+        } else if ((c + 1) * CV <= nvec)
             gemv_chunk<WT, SR, U>(w, xp, v, acc);
         else
             gemv_chunk<WT, SR, U, true>(w, xp, v, acc, nvec);
         if (q.cc == cpp - 1) {  // item complete: its R partial row sums go to LDS
+            if constexpr (ROWS) {
+                acc[0] += acc[1];
+                acc[1] = 0.0f;
+            }
 #pragma unroll
             for (int r = 0; r < SR; ++r) {
                 const float t = wave_sum(acc[r]);
