@@ -687,7 +687,8 @@ struct StepRecorder {
     static constexpr bool NT = true;  // streamed-once weights: non-temporal loads
     // The one-row wo GEMV. Two steps of 2 vectors a lane; fp32 rows of whole 2048-column steps of 8 (16 KiB of a wave) where a
     // wave has two of them or more: 4096 x 4096 16.5 -> 13.0 us, 8192 x 2048 16.5 -> 13.1. With fewer, or steps partly past the
-    // row's end, 8 vectors lose: 4096 x 512 (a TP-8 rank) 5.5 -> 6.2, 4096 x 2048 7.8 -> 9.9, 4096 x 3072 10.3 -> 10.7. (The down
+    // row's end, 8 vectors lose: 4096 x 512 (a TP-8 rank) 5.5 -> 6.2, 4096 x 2048 7.8 -> 9.9, 4096 x 3072 10.3 -> 10.7. int8 takes
+    // steps of 1, of 2 in rows of whole 2048-column steps: a Llama-3 8B step 1944 -> 1934 us, 7B (rows cut in two) 1790 -> 1785. (The down
     // GEMV's two steps of 6 hold 12 KiB already: 8 vectors 30.5 -> 30.9 us.)
     template <class Epi>
     static hipError_t wo_row(sli_model* m, const void* W, const GemvIn& in, const Epi& e) {
@@ -696,6 +697,8 @@ struct StepRecorder {
             if (in.cols % 2048 == 0 && (long)m->D * (in.cols / 2048) >= 2L * waves)
                 return launch_gemv_u<WT, 1, 8, NT>((const WT*)W, in, e, m->D, m->stream);
         }
+        if constexpr (std::is_same<WT, int8_t>::value)
+            if (in.cols % 2048 == 0) return launch_gemv_u<WT, 1, 4, NT>((const WT*)W, in, e, m->D, m->stream);
         return launch_gemv_u<WT, 1, 2, NT>((const WT*)W, in, e, m->D, m->stream);
     }
     static int gemv_qkv(sli_model* m, int l) {
@@ -785,8 +788,15 @@ struct StepRecorder {
         // U vectors per lane per step; NB steps in flight while the merge staging runs: fp16 4 (every step of the
         // wave's rows at C1: wo 9.42 -> 8.97 us, +0.4 % tok/s; 3 is slower, 9.66), int8 2 (4 measured no faster)
         // (profiles/r4_wo_nb_ab.txt)
-        constexpr bool I8 = std::is_same<WT, int8_t>::value;
-        constexpr int UK = I8 ? 1 : 2, NBK = I8 ? 2 : 4;
+        // int8: one step of 2 a row where that is what the row holds (wo_row)
+        if constexpr (std::is_same<WT, int8_t>::value) {
+            if (in.cols % 2048 != 0) return launch_wo_ks<1, 2>(m, w, in, e, am, grid);
+            return launch_wo_ks<2, 2>(m, w, in, e, am, grid);
+        }
+        return launch_wo_ks<2, 4>(m, w, in, e, am, grid);
+    }
+    template <int UK, int NBK>
+    static int launch_wo_ks(sli_model* m, const LayerW& w, const GemvIn& in, const EpiKPart& e, const AttnMergeIn& am, int grid) {
         if (am.max_splits > 8)
             SLI_HIP((launch_gemv_merge_ks<WT, 1, UK, NT, EpiKPart, 16, NBK>((const WT*)w.wo, in, e, am, grid, m->stream)));
         else
