@@ -3,8 +3,8 @@
 //   * a distance bias: score(i, j) = (q_i . k_j) scale - r1_h ln(1 + r2_h (i - j));
 //   * a sink: the softmax denominator also holds exp(sink_h), which has no key, no value, no scale and no bias.
 // attn_rows_kernel is the form for every shape and element type (one wave per row and query head, fp32 sums); the
-// matrix-core forms of the same arithmetic are prefill.h pf_flash_kernel (ROWS) and attn_mfma.h, whose split partials
-// attn_sink_merge_kernel finishes.
+// matrix-core forms of the same arithmetic are prefill.h pf_flash_kernel (ROWS) and pf_attn_mfma_kernel, and attn_mfma.h,
+// whose split partials attn_sink_merge_kernel finishes.
 #pragma once
 #include "attention.h"
 #include "common.h"

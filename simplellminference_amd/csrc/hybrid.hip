@@ -687,6 +687,17 @@ struct HyRec : HyProj<WT> {
                 if (!one && l.hd <= 128) {
                     const PfAttnArgs<__half> pa{l.q, (const __half*)r.kc, (const __half*)r.vc, {cat<OT>(l), nullptr},
                                                 d.heads, d.kv_heads, s->T, d.scale};
+                    if (s->by_16) {
+                        PfRowsArgs px;
+                        px.rows = s->rows, px.r1 = l.r1, px.r2 = l.r2, px.sink = l.sink, px.ldo = l.Kp, px.vdim = d.vdim;
+                        const dim3 gr(M / 16, d.heads);
+                        if (l.hd == 64)
+                            hipLaunchKernelGGL((pf_attn_mfma_kernel<64, false>), gr, dim3(256), 0, st(), pa, px);
+                        else
+                            hipLaunchKernelGGL((pf_attn_mfma_kernel<128, false>), gr, dim3(256), 0, st(), pa, px);
+                        SLI_HIP(hipGetLastError());
+                        return SLI_OK;
+                    }
                     const PfPortions px{s->segs, s->nsegs, l.r1, l.r2, l.sink, l.Kp, d.vdim};
                     SLI_HIP(l.hd == 64 ? launch_pf_flash_rows<64>(pa, px, M, msegs, device_cus(), st())
                                        : launch_pf_flash_rows<128>(pa, px, M, msegs, device_cus(), st()));
@@ -883,6 +894,11 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
     for (const HyLayer& l : s->layers) deep = std::max(deep, l.Kp);
     const auto batched = [](int k, int K) { return k >= (K > kGemvMaxCols ? 1 : 2) && k <= kBgMaxBatch; };
     if ((one && batched(M, deep)) || batched((int)(want.size() % kHyLogitRows), s->Dp)) HY_TRY(hy_sync_tiles(s));
+    long groups = 0;  // (one choice for the pass, so that a replayed one has two forms and not one per set of layers)
+    for (const SegRef& g : segs) groups += (g.n + 15) / 16;
+    s->by_16 = true;
+    for (const HyLayer& l : s->layers)
+        if (l.d.mixer == SLI_MIX_ATTENTION && l.hd <= 128) s->by_16 = s->by_16 && pf_rows_by_16(groups, l.d.heads, l.hd, device_cus());
     std::vector<RowRef> rows(rows_in);
     rows.resize(M, RowRef{-1, 0, 0, 0});
     const int32_t ns = (int32_t)segs.size();
@@ -906,7 +922,7 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
             gkt = std::min(gkt, hy_key_tiles_max(s));
         }
         const bool keep = one || s->replays;
-        const auto at = std::make_pair(one ? 0 : 1 + gkt, M);
+        const auto at = std::make_pair(one ? 0 : 1 + 2 * gkt + s->by_16, M);
         if (keep && (one || s->graphs.count(at))) {
             auto& g = s->graphs[at];
             SLI_HIP(hipStreamSynchronize(s->stream));

@@ -467,9 +467,9 @@ struct SeqRec : HyProj<WT> {
             px.rows = s->rows, px.ldo = l.KA, px.vdim = d.vdim, px.window = l.window, px.koff = w.koff, px.gate = q().gate;
             const dim3 gr(M / 16, d.heads);
             if (l.hd == 64)
-                hipLaunchKernelGGL((pf_attn_mfma_kernel<64>), gr, dim3(256), 0, st(), pa, px);
+                hipLaunchKernelGGL((pf_attn_mfma_kernel<64, true>), gr, dim3(256), 0, st(), pa, px);
             else
-                hipLaunchKernelGGL((pf_attn_mfma_kernel<128>), gr, dim3(256), 0, st(), pa, px);
+                hipLaunchKernelGGL((pf_attn_mfma_kernel<128, true>), gr, dim3(256), 0, st(), pa, px);
             SLI_HIP(hipGetLastError());
             return SLI_OK;
         } else {

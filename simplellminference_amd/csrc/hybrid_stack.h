@@ -130,8 +130,9 @@ struct BlockStack {
     unsigned* bg_cnt = nullptr;
     size_t bg_ws_bytes = 0, bg_groups = 1;  // the most any projection needs (hy_bg_need)
     std::vector<void*> allocs;
-    // captured passes of `feed`: {0, rows} of a decode step, {1 + grid of the expansion, rows} of a prompt pass (null:
-    // launched once so far)
+    bool by_16 = false;  // the pass's prompt attention takes its portions by 16 rows (prefill.h pf_rows_by_16)
+    // captured passes of `feed`: {0, rows} of a decode step, {1 + 2 grid of the expansion + by_16, rows} of a prompt pass
+    // (null: launched once so far)
     std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
     bool replays = false;  // prompt passes too (kReplayBytes)
     float* pg_ws = nullptr;  // partial sums and arrival counters of the prompt GEMM (prefill.h PgIn)

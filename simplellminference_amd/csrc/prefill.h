@@ -1097,10 +1097,9 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
     }
 }
 
-// ---- 3b. windowed attention over expanded keys of the block stacks' latent attention, on MFMA. A workgroup = 16 rows (queries)
-// of one head;
-// its 4 waves split the key range into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o)
-// through LDS at the end; per tile as pf_flash_kernel, with K and V in the wave's own images.
+// ---- 3b. block stacks' packed portions by 16 rows (PfRowsArgs): passes of few rows (pf_rows_by_16), and windowed attention over
+// expanded keys of the latent attention, on MFMA. A workgroup = 16 rows (queries) of one head; its 4 waves split the key range
+// into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o) through LDS at the end; per tile as pf_flash_kernel, with K and V in the wave's own images.
 template <int HD>
 struct PaGeo {
     static constexpr int ROWB = HD * 2;          // bytes per image row
@@ -1156,7 +1155,7 @@ struct PfFlash {
 };
 // ROWS: the rows are packed portions of several sequences (step_state.h SegRef; the caches hold one [hkv][T][HD] block per
 // sequence slot), with a distance bias and a sink per head (attn_rows.h) and one fp16 output [M][ldo] of vdim dims per head.
-// 1025 rows of 32 heads of 128: 85 us as a workgroup per 16 rows and head, now 51.
+// 1025 rows of 32 heads of 128: 85 us as a workgroup per 16 rows and head, 51 here.
 struct PfPortions {
     const SegRef* segs = nullptr;
     const int32_t* nsegs = nullptr;
@@ -1407,18 +1406,28 @@ hipError_t launch_pf_flash_rows(const PfAttnArgs<__half>& a, const PfPortions& x
     return hipGetLastError();
 }
 
-// Windowed: the rows are packed portions (step_state.h RowRef; a 16-row group belongs to one portion, its valid rows first); a
-// query sees the last `window` positions up to its own, position t's K and V are row t + koff[row / 32] of one [hkv][T][HD]
-// block (latent.h expands them), and the output, one fp16 row [M][ldo] of vdim dims per head, is multiplied by gate
-// [M][hq vdim].
+// Where the portions take pf_attn_mfma_kernel instead: `groups` live groups of 16 rows in a pass, whose workgroups (heads of 128:
+// 2 a CU, of 64: 4) run side by side, each wave with a quarter of the keys, where a flash workgroup walks all of them. A layer, by
+// 16 rows | flash: 17 rows from position 15000 on, 8 query and 1 kv heads of 128, 233 | 384 us; 32 and 32 heads of 128, 256 rows
+// from 4000, 134 | 151; 32 and 8 heads of 64, 512 rows from 2000, 96 | 103. One more step of rows and flash leads: 512 rows of
+// the 32 of 128 227 | 211, 1024 of the 32 of 64 180 | 144. Over 1932 shapes (1 to 8 portions of 2 to 1024 rows, from position 0 to
+// 15000, 8 to 64 heads) no pass was slower by this rule than by 16 rows throughout.
+inline bool pf_rows_by_16(long groups, int heads, int hd, int cus) { return groups * heads <= (hd > 64 ? 2L : 4L) * cus; }
+
+// The rows are packed portions (step_state.h RowRef; a 16-row group belongs to one portion, its valid rows first); one fp16
+// output row [M][ldo] of vdim dims per head.
+// WINDOWED false: as pf_flash_kernel's ROWS: bias, sink, one [hkv][T][HD] cache block per sequence slot.
+// WINDOWED true: a query sees the last `window` positions up to its own, position t's K and V are row t + koff[row / 32] of one
+// [hkv][T][HD] block (latent.h expands them), and the output is multiplied by gate [M][hq vdim].
 struct PfRowsArgs {
     const RowRef* rows = nullptr;
+    const float *r1 = nullptr, *r2 = nullptr, *sink = nullptr;  // [hq]
     int ldo = 0, vdim = 0;
     int window = 0;
     const int32_t* koff = nullptr;
     const float* gate = nullptr;
 };
-template <int HD>
+template <int HD, bool WINDOWED>
 __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a, PfRowsArgs x) {
     using G = PaGeo<HD>;
     constexpr int ND = HD / 32, NT = HD / 16;  // 32-d blocks (S), 16-d tiles (O)
@@ -1433,8 +1442,9 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
     const bool live = x.rows[mq].slot >= 0;
     const int pos = r0.pos + i16;
     const int last = r0.pos + (int)__popcll(__ballot(live)) / 4 - 1;  // the group's last query (a row is the query of 4 lanes)
-    const int kmin = max(0, r0.pos - x.window + 1);  // the first key any row of the group sees
-    const int koff = x.koff[blockIdx.x >> 1], tile0 = kmin / 32;
+    const int kmin = WINDOWED ? max(0, r0.pos - x.window + 1) : 0;  // the first key any row of the group sees
+    const int koff = WINDOWED ? x.koff[blockIdx.x >> 1] : 0, tile0 = kmin / 32;
+    const float bias1 = WINDOWED ? 0.0f : x.r1[h], bias2 = WINDOWED ? 0.0f : x.r2[h];
     const int kmax = last;  // cache rows past it are read as this one (their scores are masked)
     const int ntiles = last / 32 + 1;
     const size_t qs = (size_t)a.hq * HD;
@@ -1458,8 +1468,8 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
     char* kimg = sm + wave * G::WAVE;
     const unsigned kbase = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)kimg;
     const unsigned vbase = kbase + G::IMG;
-    const __half* kc = a.kc + (size_t)kvh * a.T * HD;
-    const __half* vc = a.vc + (size_t)kvh * a.T * HD;
+    const size_t head = ((size_t)(WINDOWED ? 0 : r0.slot) * a.hkv + kvh) * a.T * HD;
+    const __half *kc = a.kc + head, *vc = a.vc + head;
     for (int tt = tile0 + wave; tt < ntiles; tt += 4) {
         const int t0 = tt * 32;
         // K pieces 0 .. P/2-1, V pieces P/2 .. P-1; lane i of a piece: row (piece rows) + i / CPR, physical
@@ -1497,8 +1507,9 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int key = t0 + kt * 16 + 4 * g + r;
-                const float sc = sacc[kt][r] * a.scale;
-                const bool see = key <= pos && key > pos - x.window;
+                float sc = sacc[kt][r] * a.scale;
+                if constexpr (!WINDOWED) sc -= bias1 * __logf(1.0f + bias2 * (float)(pos - key));
+                const bool see = key <= pos && (!WINDOWED || key > pos - x.window);
                 const float v = see ? sc : -INFINITY;
                 sv[kt * 4 + r] = v;
                 cmax = fmaxf(cmax, v);
@@ -1561,6 +1572,10 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
         M = fmaxf(M, m4[w]);
     }
     float L = 0.0f;
+    if constexpr (!WINDOWED) {
+        M = fmaxf(M, x.sink[h]);
+        L = expf(x.sink[h] - M);
+    }
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         w4[w] = m4[w] == -INFINITY ? 0.0f : expf(m4[w] - M);
@@ -1575,10 +1590,12 @@ __global__ void __launch_bounds__(256) pf_attn_mfma_kernel(PfAttnArgs<__half> a,
         const int d0 = t * 16 + 4 * g;
         __half* dst = a.out.hi + (size_t)mq * x.ldo + (size_t)h * x.vdim + d0;
         if (!live) continue;
-        const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
+        if constexpr (WINDOWED) {
+            const float* gt = x.gate + ((size_t)mq * a.hq + h) * x.vdim + d0;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (d0 + r < x.vdim) acc[r] *= gt[r];
+            for (int r = 0; r < 4; ++r)
+                if (d0 + r < x.vdim) acc[r] *= gt[r];
+        }
         if (x.vdim % 4 == 0 && d0 < x.vdim) {
             const __half hv[4] = {__float2half_rn(acc[0] * inv), __float2half_rn(acc[1] * inv),
                                   __float2half_rn(acc[2] * inv), __float2half_rn(acc[3] * inv)};

@@ -542,6 +542,50 @@ def test_attention_blocks_of_portions(gpu, heads, kv, dim, vdim):
     m.close()
 
 
+RAGGED = (1001, 700, 33, 250), (0, 5, 64, 121)  # 2048 rows with their padding
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim,lens,firsts", [
+    (32, 8, 64, 64, (2048,), (0,)), (32, 32, 128, 128, (2048,), (0,)), (32, 16, 128, 128, (1990,), (37,)), (32, 8, 64, 64, *RAGGED),
+    (32, 32, 128, 128, *RAGGED), (32, 16, 64, 60, *RAGGED), (32, 32, 128, 100, (256,), (70,)), (32, 32, 128, 100, (257,), (70,)),
+    (32, 8, 64, 50, (512,), (3,)), (32, 8, 64, 50, (513,), (3,)), (32, 16, 128, 128, (300, 150), (0, 500))])
+def test_attention_forms_agree(gpu, heads, kv, dim, vdim, lens, firsts):
+    """Prompt attention of many rows (64-key tiles shared by a workgroup: 32 and 16 positions a wave, heads of a kv head one, two
+    and four together, one portion and ragged ones, and the two sides of the rule that chooses it) against the same tokens in
+    portions of 32 to 256 rows, which take the form by 16 rows that the tests above hold to the oracle. Biases and sinks."""
+    c = stack(att(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, ff=0), width=64)
+    t = R.random_tensors(c, 31)
+    ids = [tokens(f + n, c["vocab"], n) for n, f in zip(lens, firsts)]
+    m = make(c, t, "bfloat16", 2112, batch=len(lens))
+    want = []
+    for i, x in enumerate(ids):
+        step = 32 if len(x) < 300 else 256
+        want.append(pieces(m, x, range(step, len(x), step), slot=i)[firsts[i]:])
+    for i, f in enumerate(firsts):
+        if f:
+            m.feed([i], [0], [ids[i][:f]])
+    out = m.feed(range(len(lens)), firsts, [x[f:] for x, f in zip(ids, firsts)], [list(range(n)) for n in lens])
+    p = 0
+    for w in want:
+        close(out[p:p + len(w)], w, "bfloat16", f"portion of {len(w)}")
+        p += len(w)
+    m.close()
+
+
+def test_replays_of_both_attention_forms(gpu):
+    """Passes of one row count whose portions take one attention form or the other are replays of passes of their own."""
+    c = stack(att(heads=48, kv_heads=48, dim=128, vdim=16, ff=0), width=64)
+    t = R.random_tensors(c, 37)
+    m, plain = (make(c, t, "bfloat16", 400, batch=8) for _ in range(2))
+    for i in range(3):
+        for slots, n in ((range(8), 2), ([i], 250)):  # 256 rows: 8 groups of 16 and 16 of them
+            args = slots, [0] * len(slots), [tokens(n, c["vocab"], 10 * i + b) for b in slots], [[n - 1]] * len(slots)
+            got, want = m.feed(*args), plain.feed(*args, want_hidden=True)[0]
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (i, n)
+    m.close()
+    plain.close()
+
+
 @pytest.mark.parametrize("n", [33, 65, 129, 257, 300, 700, 1025, 2048, 2049])
 def test_row_counts_of_a_pass(gpu, n):
     """Prompt passes of every tile height with padding rows, a launch's last tiles cut over the depth (narrow outputs: all of

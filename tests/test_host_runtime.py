@@ -181,6 +181,35 @@ def batched_inputs_share_a_launch(H):
         m.close()
 
 
+def attention_forms_of_a_prompt_pass(H):
+    """Prompt attention of a block stack: passes of few rows by 16 of them, others the flash form, wide where it fills the chip; one
+    graph a form."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+
+    def forms(m, slots, start, n):
+        H.hh_launched()
+        m.feed(range(slots), [start] * slots, [[1] * n] * slots)
+        return set(re.findall(r"(pf_flash_kernelILi\d+ELi\dELi2ELb1E|pf_attn_mfma_kernelILi\d+ELb0E)", H.hh_launched().decode()))
+    for hd, heads, kv, cases in ((64, 32, 8, ((2, 9, 0, "16"), (1, 512, 0, "16"), (1, 512, 1500, "16"), (1, 513, 0, "1"), (1, 1920, 0, "1"),
+                                              (1, 1921, 0, "2"), (3, 170, 0, "1"))),
+                                 (128, 32, 32, ((8, 32, 1000, "16"), (1, 256, 0, "16"), (1, 257, 0, "1"), (1, 2048, 0, "2"))),
+                                 (128, 8, 1, ((1, 1024, 0, "16"), (1, 1025, 0, "1")))):
+        b = BlockSpec("attention", heads, hd, hd, kv_heads=kv, scale=0.1)
+        m = StackModel(StackSpec(64, 3072, (b,) * 2, taps=4, max_length=2080), batch=8, seed=1).init()
+        for slots, n, start, form in cases:
+            want = f"pf_attn_mfma_kernelILi{hd}ELb0E" if form == "16" else f"pf_flash_kernelILi{hd}ELi{form}ELi2ELb1E"
+            assert forms(m, slots, start, n) == {want}, (hd, heads, kv, slots, n, start)
+        m.close()
+    b = BlockSpec("attention", 48, 128, 16, kv_heads=48, scale=0.1)
+    m = StackModel(StackSpec(64, 64, (b,), taps=4, max_length=300), batch=8, seed=1).init()
+    for again in range(2):  # 256 rows both: each form launches once, then is a graph
+        for slots, n in ((8, 2), (1, 250)):
+            had = H.hh_graph_launches()
+            ran = forms(m, slots, 0, n)
+            assert len(ran) == 1 and H.hh_graph_launches() - had == again, (slots, n, again, ran)
+    m.close()
+
+
 def _tilings(names, epilogue=""):
     """(weight type, tiling) of the prompt GEMM instances among kernel names, of one epilogue or all."""
     out = set()
@@ -320,7 +349,7 @@ def steps_of_the_batched_projection(H):
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
-         "batched_inputs_share_a_launch",
+         "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
          "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
