@@ -145,6 +145,7 @@ struct sli_model {
         const void** w = nullptr;
         size_t granules = 0;
         int nwg = 0;
+        float lost = 0.0f;  // small_lost_us
         unsigned tag = 4;  // the next launch's first tag
     } sm;
 };
@@ -626,6 +627,10 @@ constexpr int kSmWgs = 64;
 // K of a head's context, which each of its workgroups reads: at 1000 positions of 64 (fp32) a step takes 6 us longer than at 36,
 // at 2048 about 24 and the launches are as fast soon after.
 constexpr size_t kSmMaxKey = 512 << 10;
+// us a step that the launch saves, and a layer of it, and what a layer loses of it in the mean of a context of kSmMaxKey, fitted over
+// 492 shapes of 64 to 512 wide, 1 to 12 layers and vocabularies of 512 to 128256: none that the rule takes is slower than its
+// steps (small_lost_us says what they lose without it), and 20 that it leaves would be 5 % faster and more.
+constexpr float kSmSaves = 10.0f, kSmSavesLayer = 13.0f, kSmKeyLayer = 12.0f;
 
 // Scratch at creation, tens of KB, where the model takes that path (null otherwise)
 static int small_alloc(sli_model* m) {
@@ -646,12 +651,15 @@ static int small_alloc(sli_model* m) {
     SLI_HIP(small_allow(wd, m->c.kv_dtype, hd));
     m->sm.w = wt;
     m->sm.nwg = nwg;
+    m->sm.lost = small_lost_us(m->D, m->Il, m->L, m->V, (int)m->wbytes, nwg);
     return SLI_OK;
 }
 
 // Whether positions below `length` take that launch
 static bool small_takes(const sli_model* m, int length) {
-    return m->sm.w && m->exec == SLI_EXEC_LAUNCHES && (size_t)length * m->hd * m->kvbytes <= kSmMaxKey;
+    const size_t keys = (size_t)length * m->hd * m->kvbytes;
+    return m->sm.w && m->exec == SLI_EXEC_LAUNCHES && keys <= kSmMaxKey &&
+           m->sm.lost + m->L * (kSmKeyLayer * keys / kSmMaxKey) < kSmSaves + m->L * kSmSavesLayer;
 }
 
 // n steps from the device's state on, as one launch

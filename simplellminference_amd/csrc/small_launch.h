@@ -6,6 +6,8 @@
 namespace sli {
 
 constexpr int kSmMaxD = 512, kSmMaxI = 2048;   // model and FFN width
+constexpr int kSmThreads = 512, kSmWaves = kSmThreads / 64;
+constexpr int kSmWaveBytes = 8192;              // weights and norm weights that a wave asks for ahead
 constexpr int kSmErrWait = 64;                 // DevState::error
 typedef unsigned sm_u2 __attribute__((ext_vector_type(2)));
 
@@ -24,6 +26,18 @@ struct SmArgs {
     sm_u2 *g_qkv, *g_wo, *g_act, *g_x, *g_key;  // granules: (hq + 2 hkv) hd, hq D, I, D, 2 nwg
     unsigned tag0;         // the launch's tags are tag0 + (step (L + 1) + layer) 4 + edge (never one that was used before)
 };
+
+// us a step that the launch loses to rows which a wave cannot ask for ahead: it waits for each in turn, a head row of `each` KiB
+// 0.5 + 0.4 each, a gate/up pair 2.9. 256-wide fp32, two layers, us a step as launches | here: 512 tokens of vocabulary 69 | 26, 16384
+// 72 | 44, 32000 74 | 71, 128256 94 | 205; 512-wide 69 | 31, 75 | 67, 79 | 100, 109 | 371; 320-wide with 2048 units, 3 layers 92 | 96.
+inline float small_lost_us(int D, int I, int L, int V, int wbytes, int nwg) {
+    const int each = (D * wbytes + 1023) / 1024, ahead = kSmWaveBytes / 1024 - (D * 4 + 1023) / 1024, waves = nwg * kSmWaves;
+    auto late = [&](int items, int rows) {
+        const int n = (items + waves - 1) / waves - ahead / (rows * each);
+        return (float)(n > 0 ? n : 0);
+    };
+    return late(V, 1) * (0.5f + 0.4f * each) + L * 2.9f * late(I, 2);
+}
 
 // dtypes: SLI_DT_F32 or SLI_DT_F16 of the weights and of the cache. small_allow: once a process and device, before a launch.
 hipError_t small_allow(int wd, int kd, int hd);

@@ -4,7 +4,8 @@
 //
 // Why: a step of the 256-wide two-layer preset reads 7 MB (1 us), and its 13 graph launches of 2 to 8 us take 69. Here a step
 // has four all-to-all edges a layer and one for the token, each a store and a load through memory and what a workgroup does
-// between them, 3 us: 28 us a step, 36 greedy tokens in 1.0 ms instead of 2.5. The edges bound it.
+// between them, 3 us: 28 us a step, 36 greedy tokens in 1.0 ms instead of 2.5. The edges bound it (and, with large
+// vocabularies, the head's rows: small_launch.h small_lost_us).
 //
 // Structure: hq J workgroups of 8 waves, all resident; every workgroup holds the whole residual row and runs every op on its
 // share of the rows. An edge is 8-byte {value, tag} granules as in tp_layers.h: one sc1 store each, no flag, no drain;
@@ -28,8 +29,6 @@
 
 namespace sli {
 
-constexpr int kSmThreads = 512, kSmWaves = kSmThreads / 64;
-constexpr int kSmWaveBytes = 8192;              // weights and norm weights that a wave asks for ahead
 constexpr unsigned kSmSpin = 1u << 20;          // sweeps of one wait before it gives up
 struct alignas(16) SmSmem {
     float x[kSmMaxD], x1[kSmMaxD], act[kSmMaxI];

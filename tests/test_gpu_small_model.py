@@ -12,12 +12,13 @@ def _model(w, kv, **over):
 
 
 # heads of 64 and 128, one to eight queries a kv head, widths whose rows are no whole pieces, an FFN wider than the width, heads
-# that do not divide 64
+# that do not divide 64, a vocabulary of many more rows than a wave asks for ahead
 SHAPES = {"tiny": {}, "h128": dict(head_dim=128, hidden_size=512, kv_hidden_size=256, num_attention_heads=4, num_key_value_heads=2,
                                    intermediate_size=1032, vocab_size=700),
           "h8": dict(hidden_size=512, kv_hidden_size=64, num_attention_heads=8, num_key_value_heads=1, intermediate_size=2048),
           "h6": dict(hidden_size=384, kv_hidden_size=192, num_attention_heads=6, num_key_value_heads=3, intermediate_size=520,
                      num_hidden_layers=3, vocab_size=333),
+          "v20k": dict(vocab_size=20000),
           "h1": dict(hidden_size=64, kv_hidden_size=64, num_attention_heads=1, num_key_value_heads=1, intermediate_size=72,
                      num_hidden_layers=1, vocab_size=50)}
 

@@ -157,10 +157,21 @@ def small_stacks_replay_their_prompts(H):
 
 
 def small_models_predict_in_one_launch(H):
-    """predict of a narrow model without logits is one launch; a wider one, a long context and int8 weights take the steps."""
+    """predict of a narrow model without logits is one launch; a wider one, a long context and int8 weights take the steps, and so
+    does one whose vocabulary or feed-forward is too wide for what its layers save."""
+    wide = dict(hidden_size=512, num_attention_heads=8, num_key_value_heads=8, kv_hidden_size=512, intermediate_size=1024)
+    odd = dict(hidden_size=320, num_attention_heads=5, num_key_value_heads=5, kv_hidden_size=320, intermediate_size=2048, num_hidden_layers=3)
     for kw, n, steps in ((dict(w_dtype="f32", kv_dtype="f32"), 30, 0), (dict(w_dtype="f16"), 30, 0), (dict(w_dtype="i8"), 30, 30),
                          (dict(w_dtype="f16", preset="tiny-h8"), 30, 0), (dict(w_dtype="f16", preset="small-h128"), 30, 30),
-                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(max_length=2100)), 2049, 2049)):
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(max_length=2100)), 2049, 2049),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(vocab_size=20000)), 30, 0),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(vocab_size=32000)), 30, 30),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(vocab_size=32000, num_hidden_layers=8)), 30, 0),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(vocab_size=20000, max_length=2048)), 2048, 2048),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(wide, vocab_size=8192)), 30, 0),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=dict(wide, vocab_size=32000)), 30, 30),
+                         (dict(w_dtype="f16", over=dict(wide, vocab_size=128256, num_hidden_layers=8)), 30, 30),
+                         (dict(w_dtype="f32", kv_dtype="f32", over=odd), 30, 30)):
         m = _llama(**kw)
         had = H.hh_graph_launches()
         m.predict([1, 2, 3], n)
