@@ -147,6 +147,8 @@ struct sli_model {
         int nwg = 0;
         float lost = 0.0f;  // small_lost_us
         unsigned tag = 4;  // the next launch's first tag
+        unsigned spin = sli::kSmSpin;
+        bool gave_up = false;  // a launch did: this model takes the steps from then on
     } sm;
 };
 
@@ -652,13 +654,16 @@ static int small_alloc(sli_model* m) {
     m->sm.w = wt;
     m->sm.nwg = nwg;
     m->sm.lost = small_lost_us(m->D, m->Il, m->L, m->V, (int)m->wbytes, nwg);
+    // tests: waits that give up at once, tags about to wrap
+    if (const char* e = std::getenv("SLI_DEBUG_SMALL_SPIN")) m->sm.spin = (unsigned)std::strtoul(e, nullptr, 10);
+    if (const char* e = std::getenv("SLI_DEBUG_SMALL_TAG")) m->sm.tag = (unsigned)std::strtoul(e, nullptr, 10);
     return SLI_OK;
 }
 
 // Whether positions below `length` take that launch
 static bool small_takes(const sli_model* m, int length) {
     const size_t keys = (size_t)length * m->hd * m->kvbytes;
-    return m->sm.w && m->exec == SLI_EXEC_LAUNCHES && keys <= kSmMaxKey &&
+    return m->sm.w && !m->sm.gave_up && m->exec == SLI_EXEC_LAUNCHES && keys <= kSmMaxKey &&
            m->sm.lost + m->L * (kSmKeyLayer * keys / kSmMaxKey) < kSmSaves + m->L * kSmSavesLayer;
 }
 
@@ -680,6 +685,7 @@ static int small_steps(sli_model* m, int n) {
     a.g_x = a.g_act + m->Il;
     a.g_key = a.g_x + m->D;
     a.tag0 = m->sm.tag;
+    a.spin = m->sm.spin, a.look = m->sm.spin >= 1023 ? 1023 : 0;
     m->sm.tag += need;
     SLI_HIP(small_launch(a, m->c.w_dtype, m->c.kv_dtype, m->hd, m->stream));
     return SLI_OK;
@@ -2417,7 +2423,7 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     }
     const size_t per_step = (size_t)m->B * m->v_n;
     // (scratch that did not fit leaves the steps; so does a wait that gave up, which happens where other work keeps the
-    // launch's workgroups from running together)
+    // launch's workgroups from running together: it took a second, so no later call tries again)
     bool loop = small_takes(m, max_length) && !logits_out && (n0 > 0 || !wants_chunks);
     if (loop) {
         SLI_TRY(small_steps(m, max_length - n0));
@@ -2426,6 +2432,7 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
         SLI_HIP(hipMemcpyAsync(tokens_out, m->hist, sizeof(int32_t) * max_length, hipMemcpyDeviceToHost, m->stream));
         SLI_TRY(wait_stream(m));
         if (!(d.error & kSmErrWait)) return d.error ? check_device_errors(m) : SLI_OK;
+        m->sm.gave_up = true;
         SLI_TRY(set_state(m, 0, prompts[n0], n0, 1));
     }
     for (int t = n0; t < max_length; ++t) {  // model.cpp:157

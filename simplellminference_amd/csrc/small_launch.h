@@ -9,6 +9,7 @@ constexpr int kSmMaxD = 512, kSmMaxI = 2048;   // model and FFN width
 constexpr int kSmThreads = 512, kSmWaves = kSmThreads / 64;
 constexpr int kSmWaveBytes = 8192;              // weights and norm weights that a wave asks for ahead
 constexpr int kSmErrWait = 64;                 // DevState::error
+constexpr unsigned kSmSpin = 1u << 20;         // sweeps of one wait before it gives up
 typedef unsigned sm_u2 __attribute__((ext_vector_type(2)));
 
 struct SmArgs {
@@ -24,6 +25,7 @@ struct SmArgs {
     int32_t* hist;
     float* logits;
     sm_u2 *g_qkv, *g_wo, *g_act, *g_x, *g_key;  // granules: (hq + 2 hkv) hd, hq D, I, D, 2 nwg
+    unsigned spin, look;   // kSmSpin; a wait looks up from its sweeps every look + 1 of them (a power of two)
     unsigned tag0;         // the launch's tags are tag0 + (step (L + 1) + layer) 4 + edge (never one that was used before)
 };
 

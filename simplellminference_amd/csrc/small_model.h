@@ -20,7 +20,7 @@
 // A wave asks for its weight rows of the next op (LDS-DMA, its own 8 KiB) before it waits for that op's input. K and V rows of
 // earlier steps are read with sc1 loads: other XCDs wrote them.
 // Every wait is bounded: one that gives up sets DevState::error kSmErrWait, the workgroup skips every later wait, the others'
-// waits give up too and the grid drains; the host then runs the steps again as launches.
+// waits give up too and the grid drains; the host then runs the steps as launches, and every later call of the model's.
 #pragma once
 #include "common.h"
 #include "prefill.h"
@@ -29,7 +29,6 @@
 
 namespace sli {
 
-constexpr unsigned kSmSpin = 1u << 20;          // sweeps of one wait before it gives up
 struct alignas(16) SmSmem {
     float x[kSmMaxD], x1[kSmMaxD], act[kSmMaxI];
     float qkv[3 * 128];
@@ -48,7 +47,7 @@ __device__ __forceinline__ void sm_put(sm_u2* g, int i, float v, unsigned tag) {
 // N granules at element offsets off[], of a thread, until all carry `tag` (of lanes with !on: whatever they hold)
 template <int N>
 __device__ __forceinline__ void sm_wait(const sm_u2* g, const int (&off)[N], bool on, unsigned tag, float (&out)[N], SmSmem& sm,
-                                        DevState* st) {
+                                        const SmArgs& a) {
     const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<sm_u2*>(g), 0, 0x7fffffff, 0x00020000);
     for (unsigned pass = 0;; ++pass) {
         sm_u2 v[N];
@@ -61,10 +60,10 @@ __device__ __forceinline__ void sm_wait(const sm_u2* g, const int (&off)[N], boo
             out[j] = __uint_as_float(v[j].x);
         }
         if (!__any(on && miss) || sm.dead) return;
-        if ((pass & 1023u) == 1023u) {
-            const bool peer = (__hip_atomic_load(&st->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kSmErrWait) != 0;
-            if (peer || pass >= kSmSpin) {
-                __hip_atomic_fetch_or(&st->error, kSmErrWait, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((pass & a.look) == a.look) {
+            const bool peer = (__hip_atomic_load(&a.st->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kSmErrWait) != 0;
+            if (peer || pass >= a.spin) {
+                __hip_atomic_fetch_or(&a.st->error, kSmErrWait, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 sm.dead = 1;
                 return;
             }
@@ -218,7 +217,7 @@ __global__ void __launch_bounds__(kSmThreads) small_predict_kernel(SmArgs a) {
                 const int i = min(tid, 3 * HD - 1);
                 const int off[1] = {i < HD ? h * HD + i : i < 2 * HD ? (a.hq + kvh) * HD + i - HD : (a.hq + a.hkv + kvh) * HD + i - 2 * HD};
                 float v[1];
-                sm_wait<1>(a.g_qkv, off, true, tag, v, sm, a.st);
+                sm_wait<1>(a.g_qkv, off, true, tag, v, sm, a);
                 sm.qkv[i] = v[0];
             }
             __syncthreads();
@@ -312,7 +311,7 @@ __global__ void __launch_bounds__(kSmThreads) small_predict_kernel(SmArgs a) {
                     float v[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) off[j] = min(h0 + j, a.hq - 1) * D + i;
-                    sm_wait<4>(a.g_wo, off, true, tag + 1, v, sm, a.st);
+                    sm_wait<4>(a.g_wo, off, true, tag + 1, v, sm, a);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) s += h0 + j < a.hq ? v[j] : 0.0f;
                 }
@@ -337,7 +336,7 @@ __global__ void __launch_bounds__(kSmThreads) small_predict_kernel(SmArgs a) {
             for (int i0 = 0; i0 < I; i0 += 2 * kSmThreads) {
                 const int off[2] = {min(i0 + tid, I - 1), min(i0 + kSmThreads + tid, I - 1)};
                 float v[2];
-                sm_wait<2>(a.g_act, off, true, tag + 2, v, sm, a.st);
+                sm_wait<2>(a.g_act, off, true, tag + 2, v, sm, a);
                 sm.act[off[0]] = v[0], sm.act[off[1]] = v[1];
             }
             __syncthreads();
@@ -351,7 +350,7 @@ __global__ void __launch_bounds__(kSmThreads) small_predict_kernel(SmArgs a) {
             for (int i0 = 0; i0 < D; i0 += kSmThreads) {
                 const int off[1] = {min(i0 + tid, D - 1)};
                 float v[1];
-                sm_wait<1>(a.g_x, off, true, tag + 3, v, sm, a.st);
+                sm_wait<1>(a.g_x, off, true, tag + 3, v, sm, a);
                 sm.x[off[0]] = v[0];
             }
             __syncthreads();
@@ -385,7 +384,7 @@ __global__ void __launch_bounds__(kSmThreads) small_predict_kernel(SmArgs a) {
             const int i = min(i0 + lane, a.nwg - 1);
             const int off[2] = {2 * i, 2 * i + 1};
             float v[2];
-            sm_wait<2>(a.g_key, off, true, tag, v, sm, a.st);
+            sm_wait<2>(a.g_key, off, true, tag, v, sm, a);
             const unsigned long long k = (unsigned long long)__float_as_uint(v[1]) << 32 | __float_as_uint(v[0]);
             best = k > best ? k : best;
         }

@@ -46,6 +46,42 @@ def test_loop_matches_steps(gpu, shape, w, kv):
     m.close()
 
 
+@pytest.mark.parametrize("w", ["f32", "f16"])
+@pytest.mark.parametrize("shape", ["tiny", "h6"])
+def test_wait_that_gives_up(gpu, monkeypatch, shape, w):
+    """A launch whose waits give up at their first miss ends, and the call, like those after it, gives what the steps give."""
+    m = _model(w, w, max_length=150, **SHAPES[shape])
+    calls = [([(7 * i + n) % 300 for i in range(n)], length) for n, length in ((3, 40), (20, 150), (1, 1))]
+    want = []
+    for ids, length in calls:
+        tok, log = m.predict(ids, length, want_logits=True)
+        want.append((tok, log[-1], [m.kv(1, which, length) for which in (0, 1)]))
+    m.close()
+    monkeypatch.setenv("SLI_DEBUG_SMALL_SPIN", "0")
+    m = _model(w, w, max_length=150, **SHAPES[shape])
+    for (ids, length), (tok, log, kv) in zip(calls, want):
+        assert np.array_equal(m.predict(ids, length), tok), length
+        # fp32: prompts of 9 and more run as chunks, their sums in another order
+        assert np.linalg.norm(m.logits()[0] - log) <= (5e-6 if w == "f32" else 0) * np.linalg.norm(log), length
+        for which in (0, 1):
+            assert np.abs(m.kv(1, which, length) - kv[which]).max() <= (2e-5 if w == "f32" else 0), (length, which)
+        assert m.state() == dict(m.state(), pos=min(length, 149), error=0)
+    m.close()
+
+
+def test_tags_that_wrap(gpu, monkeypatch):
+    """Launches on both sides of the wrap of the granules' tags (36 of them a launch of 3 steps)."""
+    m = _model("f32", "f32", max_length=60)
+    want = [m.predict([5, 6], n, want_logits=True)[0] for n in (3, 3, 40)]
+    m.close()
+    monkeypatch.setenv("SLI_DEBUG_SMALL_TAG", str(2 ** 32 - 50))
+    m = _model("f32", "f32", max_length=60)
+    for w, n in zip(want, (3, 3, 40)):
+        assert np.array_equal(m.predict([5, 6], n), w), n
+        assert m.state()["error"] == 0
+    m.close()
+
+
 def test_context_beyond_the_loop(gpu):
     """Contexts on both sides of the rule (512 KiB of a head's keys) give the same tokens."""
     m = _model("f32", "f32", max_length=2100)
