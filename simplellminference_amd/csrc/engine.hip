@@ -1431,8 +1431,7 @@ static int record_stack(sli_model* m) {
 
 static int capture(sli_model* m) {
     if (m->bs) {
-        SLI_TRY(hy_prepare(m->bs));
-        if (m->B > 1) SLI_TRY(hy_sync_tiles(m->bs));
+        SLI_TRY(hy_prepare_step(m->bs, m->B));
         return capture_graph(m->stream, m->graph, m->graph_exec, [&]() { return record_stack(m); });
     }
     if (m->comm_dead) return fail(SLI_ERR_COMM, "the RCCL communicator was aborted by an earlier bounded wait");

@@ -30,8 +30,8 @@ int hy_init_synthetic(BlockStack* s, uint32_t seed);
 int hy_fill_context(BlockStack* s, uint32_t seed, int upto);
 // before a capture or an eager pass: every tensor is there, the folded coefficients and tables are uploaded
 int hy_prepare(BlockStack* s);
-// before decode passes of several sequences: their copies of the weights (BlockStack::tiled)
-int hy_sync_tiles(BlockStack* s);
+// the same before a model's decode step of B sequences, with the copies of the weights that it reads
+int hy_prepare_step(BlockStack* s, int B);
 int hy_runs(const BlockStack* s);
 // A prompt pass also expands cached rows (latent attention): what a portion of n tokens at pos0 adds, and the most a pass
 // may hold (one portion of kHyMaxRows rows always fits)

@@ -198,38 +198,46 @@ static int par_create(BlockStack* s) {
     return hy_new(s, &s->attn_cnt, ncnt);
 }
 
-// Copies of the weights in the batched projection's fragment layout, where several sequences may decode together: a wave reads one
+// Copies of the weights in the batched projection's fragment layout, where several sequences decode together: a wave reads one
 // KiB in a piece instead of 16 rows x 64 bytes. 6 rows of a 2048-wide stack, a block's projections 22.8 + 14.7 -> 17.9 + 12.2 us; a
-// decode pass of 16 blocks for 2 | 8 sequences 982 | 1375 -> 867 | 1233. They take as much memory as the weights, so they are
-// allocated last, where they fit with 1 GiB to spare, or the row-major matrices are streamed (SLI_DEBUG_BG_ROWMAJOR: always, tests).
-static void hy_alloc_tiles(BlockStack* s) {
+// decode pass of 16 blocks for 2 | 8 sequences 982 | 1375 -> 867 | 1233. They take as much memory as the weights, so the first pass
+// that reads them allocates them, the blocks' or the head's, once, where they take no more than a quarter of the free memory;
+// otherwise the row-major matrices are streamed (SLI_DEBUG_BG_ROWMAJOR: always, tests).
+static void hy_alloc_tiles(BlockStack* s, bool head) {
+    HyTiles& t = head ? s->head_tiles : s->layer_tiles;
+    if (t.asked) return;
+    t.asked = true;
     if (!s->f16 || s->B < 2 || s->seq || std::getenv("SLI_DEBUG_BG_ROWMAJOR")) return;
     std::vector<std::pair<void**, size_t>> want;
+    if (head) want.push_back({&s->head_t, bg_tiled_bytes(((s->V + 1) / 2 + 7) / 8, s->Dp)});
     for (HyLayer& l : s->layers) {
+        if (head) break;
         want.push_back({&l.win_t, bg_tiled_bytes((l.e_g + 7) / 8 + ((int)l.d.ff + 7) / 8, s->Dp)});
         want.push_back({&l.wout_t, bg_tiled_bytes(((s->D + 1) / 2 + 7) / 8, l.Kp)});
     }
-    want.push_back({&s->head_t, bg_tiled_bytes(((s->V + 1) / 2 + 7) / 8, s->Dp)});
     size_t need = 0, free_b = 0, total_b = 0;
     for (const auto& p : want) need += p.second;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < need + ((size_t)1 << 30)) return;
-    const size_t n0 = s->allocs.size();
-    for (const auto& p : want) {
-        if (hipMalloc(p.first, p.second) != hipSuccess) {  // none of them then
-            (void)hipGetLastError();
-            for (size_t i = n0; i < s->allocs.size(); ++i) (void)hipFree(s->allocs[i]);
-            s->allocs.resize(n0);
-            for (const auto& q : want) *q.first = nullptr;
-            return;
-        }
-        s->allocs.push_back(*p.first);
+    void* all = nullptr;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b / 4 < need || hipMalloc(&all, need) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
     }
-    s->tiled = true;
+    s->allocs.push_back(all);
+    char* at = (char*)all;
+    for (const auto& p : want) *p.first = at, at += p.second;
+    t.on = true;
 }
-int hy_sync_tiles(BlockStack* s) {
-    if (!s->tiled || !s->tiles_dirty) return SLI_OK;
+static int hy_sync_tiles(BlockStack* s, bool head) {
+    hy_alloc_tiles(s, head);
+    HyTiles& t = head ? s->head_tiles : s->layer_tiles;
+    if (!t.on || !t.dirty) return SLI_OK;
     typedef HyIn<__half, float> In;
+    if (head) {
+        const int nh = (s->V + 1) / 2;
+        SLI_HIP(launch_bg_tile((const __half*)s->head, s->Dp, (nh + 7) / 8, BgPair<HyLogits>{{}, nh, 0}, s->head_t, s->stream));
+    }
     for (const HyLayer& l : s->layers) {
+        if (head) break;
         const int nt1 = (l.e_g + 7) / 8, nt2 = ((int)l.d.ff + 7) / 8, no = (s->D + 1) / 2;
         if (l.d.ff > 0)
             SLI_HIP(launch_bg_tile((const __half*)l.win, s->Dp, nt1 + nt2, BgPair2<In>{{}, l.e_g, (int)l.d.ff, l.u1p, nt1}, l.win_t, s->stream));
@@ -237,10 +245,22 @@ int hy_sync_tiles(BlockStack* s) {
             SLI_HIP(launch_bg_tile((const __half*)l.win, s->Dp, nt1, BgPair<In>{{}, l.e_g, 0}, l.win_t, s->stream));
         SLI_HIP(launch_bg_tile((const __half*)l.wout, l.Kp, (no + 7) / 8, BgPair<HyOut>{{}, no, 0}, l.wout_t, s->stream));
     }
-    const int nh = (s->V + 1) / 2;
-    SLI_HIP(launch_bg_tile((const __half*)s->head, s->Dp, (nh + 7) / 8, BgPair<HyLogits>{{}, nh, 0}, s->head_t, s->stream));
-    s->tiles_dirty = false;
+    t.dirty = false;
     return SLI_OK;
+}
+// The copies that a decode pass of `rows` rows (0: none) and a head over `heads` of them read, where they run the batched
+// projection (HyProj::path): one row does where a depth is past the GEMV's
+static int hy_tiles_for(BlockStack* s, int rows, int heads) {
+    int deep = s->Dp;
+    for (const HyLayer& l : s->layers) deep = std::max(deep, l.Kp);
+    const auto batched = [](int n, int K) { return n >= (K > kGemvMaxCols ? 1 : 2) && n <= kBgMaxBatch; };
+    if (batched(rows, deep)) HY_TRY(hy_sync_tiles(s, false));
+    if (batched(heads, s->Dp)) HY_TRY(hy_sync_tiles(s, true));
+    return SLI_OK;
+}
+int hy_prepare_step(BlockStack* s, int B) {
+    HY_TRY(hy_prepare(s));
+    return hy_tiles_for(s, B, B);
 }
 
 int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out) {
@@ -317,7 +337,6 @@ int hy_create(const sli_stack_config* cfg, hipStream_t stream, BlockStack** out)
     double w = 0.0, k = 0.0;
     hy_step_bytes(s, 1, 0.0, &w, &k);
     s->replays = w < kReplayBytes * (double)s->runs.size();
-    hy_alloc_tiles(s);
     return hy_allow_lds();
 }
 
@@ -538,7 +557,7 @@ int hy_prepare(BlockStack* s) {
     for (int d = 0; d < s->D; ++d) g[d] = (float)(g[d] * std::sqrt((double)s->D / Dp));
     SLI_HIP(hipMemcpy(s->fnorm_p, g.data(), sizeof(float) * Dp, hipMemcpyHostToDevice));
     s->dirty = false;
-    s->tiles_dirty = true;
+    s->head_tiles.dirty = s->layer_tiles.dirty = true;
     return SLI_OK;
 }
 
@@ -889,11 +908,7 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
         for (const SegRef& g : segs) kt += seq_key_tiles(s, g.pos0, g.n);
         SLI_CHECK(kt <= hy_key_tiles_max(s), SLI_ERR_SHAPE, "pass: too many expanded rows");
     }
-    // passes and heads that run the batched projection (HyProj::path): one row does where a depth is past the GEMV's
-    int deep = s->Dp;
-    for (const HyLayer& l : s->layers) deep = std::max(deep, l.Kp);
-    const auto batched = [](int k, int K) { return k >= (K > kGemvMaxCols ? 1 : 2) && k <= kBgMaxBatch; };
-    if ((one && batched(M, deep)) || batched((int)(want.size() % kHyLogitRows), s->Dp)) HY_TRY(hy_sync_tiles(s));
+    HY_TRY(hy_tiles_for(s, one ? M : 0, (int)(want.size() % kHyLogitRows)));
     long groups = 0;  // (one choice for the pass, so that a replayed one has two forms and not one per set of layers)
     for (const SegRef& g : segs) groups += (g.n + 15) / 16;
     s->by_16 = true;

@@ -38,7 +38,7 @@ struct HyLayer {
     int nsl = 0;  // retention: state slices per head
     int rot = -1;
     void *win = nullptr, *wout = nullptr;
-    void *win_t = nullptr, *wout_t = nullptr;  // the same in the batched projection's fragment layout (BlockStack::tiled)
+    void *win_t = nullptr, *wout_t = nullptr;  // the same in the batched projection's fragment layout (HyTiles)
     float *f1 = nullptr, *f2 = nullptr, *r1 = nullptr, *r2 = nullptr, *sink = nullptr, *decay = nullptr;
     // the output projection's input and the attention query rows, one buffer per shape: their padding columns are never
     // written, so they stay zero
@@ -98,6 +98,12 @@ struct HyRot {
     float *cs = nullptr, *sn = nullptr;
 };
 
+// Copies in the fragment layout (bgemm.h BgIn::tiled) that decode passes and heads of several rows stream: allocated by the first
+// that would, built before the first after weights were placed (hybrid.hip hy_sync_tiles)
+struct HyTiles {
+    bool asked = false, on = false, dirty = true;
+};
+
 struct BlockStack {
     sli_stack_config c{};
     hipStream_t stream = nullptr;
@@ -113,9 +119,7 @@ struct BlockStack {
     std::vector<float> fgain;  // one gain, or one per channel
     std::map<std::string, bool> want;  // tensor -> placed
     bool dirty = true;
-    // decode passes of several sequences stream copies in the fragment layout (bgemm.h BgIn::tiled), built before the first one
-    // after weights were placed (hy_sync_tiles)
-    bool tiled = false, tiles_dirty = true;
+    HyTiles layer_tiles, head_tiles;
     void* head_t = nullptr;
     // activations of a pass
     RowRef* rows = nullptr;

@@ -31,7 +31,7 @@ thread_local struct {
     void* s;
 } config;
 int wrong_device = 0, launches = 0, graph_launches = 0, mallocs = 0, fail_at = -1;
-size_t room = (size_t)-1, used = 0;
+size_t room = (size_t)-1, used = 0, free_bytes = (size_t)1 << 36;
 std::map<int, int> mallocs_on, attributes_on;
 std::map<void*, size_t> live;
 std::set<Stream*> streams;
@@ -71,6 +71,7 @@ int hh_mallocs_on(int d) { return mallocs_on[d]; }
 int hh_attributes_on(int d) { return attributes_on[d]; }
 int hh_live() { return (int)live.size(); }
 void hh_fail_at(int k) { fail_at = k < 0 ? -1 : mallocs + k; }  // the k-th allocation from now (0: the next) fails
+void hh_free(size_t n) { free_bytes = n ? n : (size_t)1 << 36; }  // what hipMemGetInfo tells (0: 64 GiB)
 void hh_room(size_t n) { room = n ? used + n : (size_t)-1; }    // bytes left to allocate (0: no limit)
 const char* hh_launched() {  // the kernels launched or recorded since the last call, one name a line
     names.clear();
@@ -120,7 +121,7 @@ int hipFree(void* p) {
     free(p);
     return kOk;
 }
-int hipMemGetInfo(size_t* f, size_t* t) { return *f = *t = (size_t)1 << 36, kOk; }
+int hipMemGetInfo(size_t* f, size_t* t) { return *f = free_bytes, *t = (size_t)1 << 36, kOk; }
 int hipMemcpy(void* d, const void* s, size_t n, int) { return memcpy(d, s, n), kOk; }
 int hipMemset(void* d, int v, size_t n) { return memset(d, v, n), kOk; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) {

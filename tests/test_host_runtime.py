@@ -9,6 +9,7 @@ import re
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -192,6 +193,51 @@ def batched_inputs_share_a_launch(H):
         m.close()
 
 
+def weight_copies_where_they_are_read(H):
+    """Stacks allocate the batched projections' copies of their weights (the blocks' and the head's, an allocation each) in the first
+    pass that reads them: not at creation, not for prompts, single rows and steps of more than 8 sequences, and not where they are
+    more than a quarter of the free memory or the allocation fails."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    b = BlockSpec("attention", 4, 64, 64, kv_heads=2, scale=0.1, ff=300, ff_limit=7.0)
+
+    def copies(m, call):
+        had = H.hh_mallocs()
+        H.hh_launched()
+        call()
+        return H.hh_mallocs() - had, len(re.findall("bg_tile_kernel", H.hh_launched().decode()))  # (each instance once)
+
+    def rows(m, n, pos, wanted=True):
+        return lambda: m.feed(range(n), [pos] * n, [[1]] * n, [[0]] * n if wanted else None)
+
+    def model(batch, width=256):
+        return StackModel(StackSpec(64, width, (b,) * 2, taps=4, max_length=64), batch=batch, seed=1).init()
+    m = model(3)
+    assert copies(m, lambda: m.feed([0, 1], [0, 0], [[1] * 20] * 2)) == (0, 0)
+    assert copies(m, rows(m, 1, 20)) == (0, 0)
+    assert copies(m, lambda: m.feed([0, 1], [0, 0], [[1] * 20] * 2, [[0, 5], [1]])) == (1, 1), "the head of three rows"
+    assert copies(m, rows(m, 2, 20)) == (1, 2), "the blocks' two matrices"
+    assert copies(m, rows(m, 3, 21)) == (0, 0)
+    m.set_tensor("l0.mix.o", np.zeros((256, 256), np.float32))
+    assert copies(m, rows(m, 2, 22)) == (0, 3)
+    m.close()
+    for batch, want in ((1, (0, 0)), (2, (2, 3)), (8, (2, 3)), (9, (0, 0))):
+        m = model(batch)
+        assert copies(m, m.step) == want, batch
+        m.close()
+    m = model(2)
+    H.hh_fail_at(0)
+    assert copies(m, rows(m, 2, 0)) == (2, 1), "the blocks' failed, the head's did not"
+    H.hh_fail_at(-1)
+    assert copies(m, rows(m, 2, 1)) == (0, 0)
+    m.close()
+    m = model(2)
+    H.hh_free(2 << 20)  # (more than the blocks' 1.7 MB, of which it is not four times as much)
+    assert copies(m, rows(m, 2, 0)) == (1, 1)
+    H.hh_free(0)
+    m.close()
+    assert H.hh_live() == 0
+
+
 def attention_forms_of_a_prompt_pass(H):
     """Prompt attention of a block stack: passes of few rows by 16 of them, others the flash form, wide where it fills the chip; one
     graph a form."""
@@ -360,7 +406,7 @@ def steps_of_the_batched_projection(H):
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
-         "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass",
+         "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass", "weight_copies_where_they_are_read",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
          "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
@@ -387,7 +433,7 @@ def test_host(host_hip, case):
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     H = ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)  # before libsli.so: its references to HIP end here
-    H.hh_room.argtypes = [ctypes.c_size_t]
+    H.hh_room.argtypes = H.hh_free.argtypes = [ctypes.c_size_t]
     H.hh_launched.restype = H.hh_kernels.restype = ctypes.c_char_p
     globals()[sys.argv[1]](H)
     print("ok", sys.argv[1])
