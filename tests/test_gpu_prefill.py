@@ -255,19 +255,23 @@ def test_prefill_rows_of_each_tiling(gpu, n):
                                             (64, 32, 32, 2050), (128, 16, 4, 2100)])
 def test_prefill_attention_groups(gpu, hd, heads, kvh, n):
     """The prompt attention's heads per workgroup (1, 2, 4 of a kv head, 8 as two workgroups), 16 and (the long prompts)
-    32 positions per wave, last tiles and position blocks of 1, 16 and 64 rows, against the engine's decode step. 1e-3 as
-    above."""
+    32 positions per wave, last tiles and position blocks of 1, 16 and 64 rows, against the engine's decode step. Two layers: the
+    first one's attention shows in the second's cache rows, and through them in the logits. 1e-3 as above; cache rows within one
+    fp16 rounding of the largest, in norm below 2^-12 (2^-11 / sqrt 3 would be every value rounded the other way)."""
     from simplellminference_amd.model import LlamaModel, LlamaModelConfig
     cfg = LlamaModelConfig(vocab_size=600, head_dim=hd, hidden_size=hd * heads, kv_hidden_size=hd * kvh,
-                           intermediate_size=512, max_length=n + 8, num_hidden_layers=1, num_attention_heads=heads,
+                           intermediate_size=512, max_length=n + 8, num_hidden_layers=2, num_attention_heads=heads,
                            num_key_value_heads=kvh, rms_norm_eps=1e-5, rope_theta=1e4)
     m = LlamaModel(config=cfg, w_dtype="f16", kv_dtype="f16", seed=2).init()
     prompt = _prompt(n, cfg.vocab_size)
     ref = m.predict(prompt, n + 2)
-    lref = m.logits()[0]
+    lref, kv = m.logits()[0], [m.kv(1, which, n - 1) for which in (0, 1)]
     m.reset()
     tok = m.predict_prefill(prompt, n + 2)
     log = m.logits()[0]
+    for a, b in zip([m.kv(1, which, n - 1) for which in (0, 1)], kv):
+        assert np.abs(a - b).max() <= 2.0 ** -10 * np.abs(b).max()
+        assert np.linalg.norm(a - b) <= 2.0 ** -12 * np.linalg.norm(b)
     m.close()
     assert np.array_equal(tok, ref)
     assert np.abs(log - lref).max() <= 1e-3
