@@ -1407,11 +1407,11 @@ hipError_t launch_pf_flash_rows(const PfAttnArgs<__half>& a, const PfPortions& x
 }
 
 // Where the portions take pf_attn_mfma_kernel instead: `groups` live groups of 16 rows in a pass, whose workgroups (heads of 128:
-// 2 a CU, of 64: 4) run side by side, each wave with a quarter of the keys, where a flash workgroup walks all of them. A layer, by
-// 16 rows | flash: 17 rows from position 15000 on, 8 query and 1 kv heads of 128, 233 | 384 us; 32 and 32 heads of 128, 256 rows
-// from 4000, 134 | 151; 32 and 8 heads of 64, 512 rows from 2000, 96 | 103. One more step of rows and flash leads: 512 rows of
-// the 32 of 128 227 | 211, 1024 of the 32 of 64 180 | 144. Over 1932 shapes (1 to 8 portions of 2 to 1024 rows, from position 0 to
-// 15000, 8 to 64 heads) no pass was slower by this rule than by 16 rows throughout.
+// 2 a CU, of 64: 4) run side by side, each wave with a quarter of the keys, where a flash workgroup walks all of them. A block of
+// a 256-wide stack without feed-forward, by 16 rows | flash: 17 rows from position 15000 on, 8 query and 1 kv heads of 128, 233 | 384
+// us; 32 and 32 heads of 128, 256 rows from 4000, 134 | 151; 32 and 8 heads of 64, 512 rows from 2000, 96 | 103. With twice the rows
+// flash leads: 512 of the 32 of 128 227 | 211, 1024 of the 32 of 64 180 | 144. Over 1932 shapes (1 to 8 portions of 2 to 1024 rows,
+// from position 0 to 15000, 8 to 64 heads) no pass was slower by this rule than by 16 rows throughout.
 inline bool pf_rows_by_16(long groups, int heads, int hd, int cus) { return groups * heads <= (hd > 64 ? 2L : 4L) * cus; }
 
 // The rows are packed portions (step_state.h RowRef; a 16-row group belongs to one portion, its valid rows first); one fp16
