@@ -1099,7 +1099,8 @@ __global__ void __launch_bounds__(256) pf_attn_kernel(PfAttnArgs<KT> a, PfState 
 
 // ---- 3b. block stacks' packed portions by 16 rows (PfRowsArgs): passes of few rows (pf_rows_by_16), and windowed attention over
 // expanded keys of the latent attention, on MFMA. A workgroup = 16 rows (queries) of one head; its 4 waves split the key range
-// into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o) through LDS at the end; per tile as pf_flash_kernel, with K and V in the wave's own images.
+// into 32-key tiles (wave w takes tiles w, w + 4, ...) and merge their (max, sum, o) through LDS at the end; per tile as
+// pf_flash_kernel, with K and V in the wave's own images.
 template <int HD>
 struct PaGeo {
     static constexpr int ROWB = HD * 2;          // bytes per image row
