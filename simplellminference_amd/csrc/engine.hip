@@ -18,9 +18,12 @@
 #include <unistd.h>
 
 #include <cmath>
+#include <condition_variable>
 #include <cstdlib>
 #include <type_traits>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "../../include/sli_synth.h"
@@ -144,7 +147,8 @@ struct sli_model {
         sli::sm_u2* g = nullptr;
         const void** w = nullptr;
         size_t granules = 0;
-        int nwg = 0;
+        int nwg = 0, one_nwg = 0;  // workgroups over all XCDs, on one (0: not there)
+        int turn = 0;              // of the tickets of the launches on one XCD
         float lost = 0.0f;  // small_lost_us
         unsigned tag = 4;  // the next launch's first tag
         unsigned spin = sli::kSmSpin;
@@ -626,6 +630,12 @@ static int tpl_launch(sli_model* m) {
 // 28.4 | 35.9, 512-wide 86 | 49 | 34.3 | 32.2. The graph's steps take 68.7 and 68.2. Models of 1024 take 77 as launches and 92 here
 // (a wave's rows of an op no longer fit its LDS), so they keep them.
 constexpr int kSmWgs = 64;
+// On one XCD an edge goes through its L2 (a granule handed on in 0.26 us, to another XCD 0.55; an edge that all read 0.4 and 1.1 to 2),
+// and all weights through that XCD's share of the memory. us a step over all XCDs | on one: the fp32 preset 25.3 | 17.0, as fp16 30.4 | 15.6, 128
+// wide 29.4 | 13.9, 384 wide in fp16 34.3 | 20.6, 512 wide and 2048 units (8 MB a layer) 31.7 | 27.5; fp32 with 2048 units, 7 MB a layer,
+// 24.5 | 26.6, and rows past 1 KiB (fp32 wider than 256) 34.5 | 68. So fp32 up to kSmOneLayer bytes a layer.
+constexpr int kSmOneWgs = 32;  // an XCD's CUs
+constexpr size_t kSmOneLayer = 5 << 20;
 // K of a head's context, which each of its workgroups reads: at 1000 positions of 64 (fp32) a step takes 6 us longer than at 36,
 // at 2048 about 24 and the launches are as fast soon after.
 constexpr size_t kSmMaxKey = 512 << 10;
@@ -638,11 +648,18 @@ constexpr float kSmSaves = 10.0f, kSmSavesLayer = 13.0f, kSmKeyLayer = 12.0f;
 static int small_alloc(sli_model* m) {
     const int wd = m->c.w_dtype;
     if (m->B != 1 || m->partial || m->group || m->bs || wd == SLI_DT_I8 || m->D > kSmMaxD || m->Il > kSmMaxI || m->D % 8 || m->Il % 8) return SLI_OK;
-    int J = 1;
-    while (m->hq * J * 2 <= kSmWgs) J *= 2;
-    const int nwg = m->hq * J, hd = m->hd;
-    if (nwg > kSmWgs || m->D < nwg || m->Il < nwg || nwg > device_cus()) return SLI_OK;
-    m->sm.granules = (size_t)(m->hq + 2 * m->hkv) * hd + (size_t)m->hq * m->D + m->Il + m->D + 2 * nwg;
+    auto groups = [&](int most) {  // workgroups: a power of two a head, at most `most`
+        int J = 1;
+        while (m->hq * J * 2 <= most) J *= 2;
+        const int n = m->hq * J;
+        return n > most || m->D < n || m->Il < n || n > device_cus() ? 0 : n;
+    };
+    const int nwg = groups(kSmWgs), hd = m->hd;
+    if (nwg == 0) return SLI_OK;
+    const size_t layer = m->wbytes * ((size_t)(m->hq + 2 * m->hkv) * hd * m->D + (size_t)m->D * m->hq * hd + 3 * (size_t)m->Il * m->D);
+    if (m->D * m->wbytes <= 1024 && (wd == SLI_DT_F16 || layer <= kSmOneLayer) && !std::getenv("SLI_DEBUG_SMALL_ALL") && small_xcds(kSmOneWgs))
+        m->sm.one_nwg = groups(kSmOneWgs);
+    m->sm.granules = (size_t)(m->hq + 2 * m->hkv) * hd + (size_t)m->hq * m->D + m->Il + m->D + 2 * nwg + 1;
     SLI_TRY(model_alloc(m, (void**)&m->sm.g, 8 * m->sm.granules));
     SLI_HIP(hipMemset(m->sm.g, 0, 8 * m->sm.granules));
     std::vector<const void*> w;
@@ -654,11 +671,56 @@ static int small_alloc(sli_model* m) {
     m->sm.w = wt;
     m->sm.nwg = nwg;
     m->sm.lost = small_lost_us(m->D, m->Il, m->L, m->V, (int)m->wbytes, nwg);
-    // tests: waits that give up at once, tags about to wrap
+    // tests: waits that give up at once, tags about to wrap (above: launches over all XCDs)
     if (const char* e = std::getenv("SLI_DEBUG_SMALL_SPIN")) m->sm.spin = (unsigned)std::strtoul(e, nullptr, 10);
     if (const char* e = std::getenv("SLI_DEBUG_SMALL_TAG")) m->sm.tag = (unsigned)std::strtoul(e, nullptr, 10);
     return SLI_OK;
 }
+
+// Where a launch runs: on an XCD of its own (xcd, of those in `mask`), or over all of them (-1). A launch's workgroups wait for each
+// other, so no two launches of the process may each hold a part of what both need: launches on XCDs of their own, or launches over
+// all of them (64 workgroups each beside the chip's 256 CUs), but never both kinds at once. Threads are served in the order they came;
+// the place is given back when the launch has ended.
+struct SmallPlace {
+    struct Chip {
+        std::mutex mu;
+        std::condition_variable cv;
+        unsigned one = 0;  // XCDs taken
+        int all = 0;       // launches over all XCDs
+        unsigned long long next = 0, serving = 0;
+    };
+    Chip& chip;
+    int xcd = -1;
+    SmallPlace(int device, unsigned mask) : chip(of(device)) {
+        std::unique_lock<std::mutex> lock(chip.mu);
+        const unsigned long long mine = chip.next++;
+        chip.cv.wait(lock, [&] { return mine == chip.serving && ((chip.all == 0 && (mask & ~chip.one)) || chip.one == 0); });
+        if (chip.all == 0 && (mask & ~chip.one)) {
+            xcd = __builtin_ctz(mask & ~chip.one);
+            chip.one |= 1u << xcd;
+        } else {
+            ++chip.all;
+        }
+        ++chip.serving;
+        chip.cv.notify_all();
+    }
+    ~SmallPlace() {
+        std::lock_guard<std::mutex> lock(chip.mu);
+        if (xcd >= 0)
+            chip.one &= ~(1u << xcd);
+        else
+            --chip.all;
+        chip.cv.notify_all();
+    }
+    SmallPlace(const SmallPlace&) = delete;
+    SmallPlace& operator=(const SmallPlace&) = delete;
+    static Chip& of(int device) {
+        static std::mutex mu;
+        static std::map<int, Chip> chips;
+        std::lock_guard<std::mutex> lock(mu);
+        return chips[device];
+    }
+};
 
 // Whether positions below `length` take that launch
 static bool small_takes(const sli_model* m, int length) {
@@ -668,7 +730,7 @@ static bool small_takes(const sli_model* m, int length) {
 }
 
 // n steps from the device's state on, as one launch
-static int small_steps(sli_model* m, int n) {
+static int small_steps(sli_model* m, int n, int xcd) {
     const unsigned need = 4u * (unsigned)n * (unsigned)(m->L + 1);
     if (m->sm.tag + need < m->sm.tag) {  // (the tags wrap: none of the old ones may be left)
         SLI_HIP(hipMemsetAsync(m->sm.g, 0, 8 * m->sm.granules, m->stream));
@@ -679,11 +741,13 @@ static int small_steps(sli_model* m, int n) {
     a.act_mode = m->c.act_mode, a.n = n, a.eps = m->c.eps, a.scale = 1.0f / sqrtf((float)m->hd);
     a.w = m->sm.w, a.emb = m->emb, a.norms = m->norms, a.kc = m->kc, a.vc = m->vc, a.sin_t = m->sin_t, a.cos_t = m->cos_t;
     a.st = m->st, a.prompt = m->prompt, a.hist = m->hist, a.logits = m->logits;
-    a.g_qkv = m->sm.g;
-    a.g_wo = a.g_qkv + (size_t)(m->hq + 2 * m->hkv) * m->hd;
-    a.g_act = a.g_wo + (size_t)m->hq * m->D;
+    a.g = m->sm.g;
+    a.g_wo = (m->hq + 2 * m->hkv) * m->hd;
+    a.g_act = a.g_wo + m->hq * m->D;
     a.g_x = a.g_act + m->Il;
     a.g_key = a.g_x + m->D;
+    a.xcd = xcd;
+    if (xcd >= 0) a.nwg = m->sm.one_nwg, a.ticket = reinterpret_cast<unsigned*>(m->sm.g + m->sm.granules - 1), a.turn = m->sm.turn ^= 1;
     a.tag0 = m->sm.tag;
     a.spin = m->sm.spin, a.look = m->sm.spin >= 1023 ? 1023 : 0;
     m->sm.tag += need;
@@ -2425,7 +2489,8 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     // launch's workgroups from running together: it took a second, so no later call tries again)
     bool loop = small_takes(m, max_length) && !logits_out && (n0 > 0 || !wants_chunks);
     if (loop) {
-        SLI_TRY(small_steps(m, max_length - n0));
+        const SmallPlace place(m->c.device, m->sm.one_nwg ? small_xcds(kSmOneWgs) : 0);
+        SLI_TRY(small_steps(m, max_length - n0, place.xcd));
         DevState d{};
         SLI_HIP(hipMemcpyAsync(&d, m->st, sizeof(d), hipMemcpyDeviceToHost, m->stream));
         SLI_HIP(hipMemcpyAsync(tokens_out, m->hist, sizeof(int32_t) * max_length, hipMemcpyDeviceToHost, m->stream));

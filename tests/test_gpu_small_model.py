@@ -89,3 +89,43 @@ def test_context_beyond_the_loop(gpu):
     assert np.array_equal(m.predict([3, 1, 4], 2048), want[:2048])
     assert np.array_equal(m.predict([3, 1, 4], 2049), want[:2049])
     m.close()
+
+
+@pytest.mark.parametrize("w", ["f32", "f16"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_loop_over_all_xcds(gpu, monkeypatch, shape, w):
+    """As test_loop_matches_steps, where that ran on one XCD."""
+    monkeypatch.setenv("SLI_DEBUG_SMALL_ALL", "1")
+    test_loop_matches_steps(gpu, shape, w, w)
+
+
+def test_loop_of_many_units(gpu, monkeypatch):
+    """An fp32 layer past what one XCD reads beside its edges."""
+    monkeypatch.setitem(SHAPES, "w2k", dict(intermediate_size=2048))
+    test_loop_matches_steps(gpu, "w2k", "f32", "f32")
+
+
+def test_loops_side_by_side(gpu):
+    """Models of both places (one XCD; all of them, fp32 wider than 256) called from threads at the same time: each gets its own
+    tokens, and no launch's workgroups keep another's from running (a wait that gave up would leave the model on its steps)."""
+    import threading
+    models, want = [], []
+    for i in range(8):
+        w = "f32" if i % 2 else "f16"
+        m = _model(w, w, max_length=100, **(SHAPES["h6"] if i in (1, 5) else {}))
+        models.append(m)
+        want.append(m.predict([i + 1, 7, 300 - i], 90))
+    got = [[] for _ in models]
+
+    def calls(i):
+        for _ in range(6):
+            got[i].append(models[i].predict([i + 1, 7, 300 - i], 90))
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(len(models))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for m, g, w in zip(models, got, want):
+        assert len(g) == 6 and all(np.array_equal(x, w) for x in g)
+        assert m.state()["error"] == 0
+        m.close()
