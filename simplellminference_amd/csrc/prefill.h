@@ -109,6 +109,12 @@ __global__ void __launch_bounds__(256) pf_embed_kernel(PfState ps, const int32_t
     for (int i = threadIdx.x; i < D; i += 256) x[(size_t)m * D + i] = to_f32(emb[(size_t)tok * D + i]) * s;
 }
 
+// y[b] = the residual row of sequence b's last valid position in the chunk
+static __global__ void __launch_bounds__(256) pf_last_rows_kernel(PfState ps, const float* __restrict__ x, float* __restrict__ y, int D) {
+    const float* r = x + ((size_t)blockIdx.x * ps.rps + ps.nv - 1) * D;
+    for (int i = threadIdx.x; i < D; i += 256) y[(size_t)blockIdx.x * D + i] = r[i];
+}
+
 // Partial sums of a GEMM that the next norm adds up (PgIn::defer): x += (part[0] + .. + part[n - 1]) * rscale, in x
 struct PfPart {
     const float* part = nullptr;  // [n][rows][D]

@@ -293,3 +293,27 @@ def test_predict_batch_prompt_chunks_match_steps(gpu, kv, name, batch, short, lo
     for a, b in zip(kv0, [m.kv(1, w, length, seq=b) for w in (0, 1) for b in range(batch)]):
         assert np.abs(a - b).max() <= 2 ** -7
     m.close()
+
+
+@pytest.mark.parametrize("w,batch,layers", [("f16", 3, 2), ("f16", 3, 1), ("f32", 1, 2), ("f32", 1, 1)])
+@pytest.mark.parametrize("short,length", [(9, 9), (12, 12), (33, 34), (499, 501)])
+def test_first_step_of_a_prompt_chunk(gpu, w, batch, layers, short, length):
+    """Calls whose first step (the last one too, where the shortest prompt is as long as the call) runs as a chunk's last position up to
+    its last layer: tokens, state, logits and K/V rows of the steps (bars of test_predict_batch_prompt_chunks_match_steps; fp32: sums in
+    another order). 1024 wide: no small model's launch; one layer: the step runs whole; 500 positions of 3 sequences: past one attention
+    block of rows."""
+    from simplellminference_amd.model import LlamaModel, preset
+    m = LlamaModel(config=preset("small-h128-gqa", num_hidden_layers=layers), w_dtype=w, kv_dtype=w, seed=6, batch=batch).init()
+    r = np.random.default_rng(short)
+    prompts = [r.integers(0, m.config.vocab_size, short + b).tolist() for b in range(batch)]
+    want, wl = m.predict_batch(prompts, length, want_logits=True)
+    states = [m.state(b) for b in range(batch)]
+    kv0 = [m.kv(layers - 1, which, length, seq=b) for which in (0, 1) for b in range(batch)]
+    m.reset()
+    for _ in range(2):
+        assert np.array_equal(m.predict_batch(prompts, length), want)
+        assert np.abs(m.logits()[0].reshape(batch, -1) - wl[:, -1]).max() <= (1e-3 if w == "f16" else 2e-5)
+        assert [m.state(b) for b in range(batch)] == states
+        for a, b in zip(kv0, [m.kv(layers - 1, which, length, seq=b) for which in (0, 1) for b in range(batch)]):
+            assert np.abs(a - b).max() <= (2 ** -7 if w == "f16" else 2e-5)
+    m.close()
