@@ -8,6 +8,7 @@
 // sees complete pairs under all three kernels' tilings.
 #pragma once
 #include "bgemm.h"
+#include "canon.h"
 #include "common.h"
 #include "gemv.h"
 #include "prefill.h"
@@ -48,7 +49,9 @@ __device__ __forceinline__ void store2(__half* p, const float* v) {
 // OT: element type of the feed-forward product in the output projection's input.
 template <typename KT, typename OT>
 struct HyIn {
-    static constexpr bool kRolled = true;  // (prefill.h; 34304 x 4096: 497 us for 1024 rows with the tiles indexed in scratch, 391 for 1152 so)
+    // (prefill.h. 34304 x 4096 at 1152 rows 363 -> 343 us and 22528 x 2048 136 -> 122 with the row lookups of a wave together and
+    // the feed-forward tiles unrolled, their products stored in 16 bytes a lane)
+    static constexpr bool kRolled = true;
     int retention;
     int H, G, dim, vdim, hpq, hpv;   // hpq / hpv: pairs per q,k / v,g head
     int e_q, e_k, e_v, e_g, u1p, ff;  // pair ranges
@@ -66,14 +69,47 @@ struct HyIn {
         const float gt = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
         return gt / (1.0f + expf(-1.702f * gt)) * (u + 1.0f);
     }
-    // pairs u and u + 1, u even: one row lookup and one head division, neighbouring results stored together
-    __device__ void pair2(int u, int m, const float* a, bool second) const {
+    struct Row {
+        int slot, pos;
+    };
+    __device__ Row row_of(int m) const { return Row{rows[m].slot, rows[m].pos}; }
+    // pairs u .. u + n - 1 are feed-forward pairs, whose products lie together, 16-byte pieces of 8 of them aligned
+    __device__ bool flat(int u, int n) const {
+        return std::is_same<OT, __half>::value && even && u >= u1p && u + n <= u1p + ff && act_ld % 8 == 0 && act_off % 8 == 0;
+    }
+    // N tiles of 8 pairs from pair u on, this lane pairs 2 kg and 2 kg + 1 of each in v[tile]. Four tiles are exchanged between
+    // the lane groups, so that each stores 16 bytes and a row's four 64 (of pairs alone 4 bytes a lane, 16 a row).
+    template <int N>
+    __device__ void flat_store(int u, int kg, int m, const pf_float4* v, Row r) const {
+        unsigned y[N];
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            const __half2 p = __halves2half2(__float2half_rn(glu(v[a][0], v[a][1])), __float2half_rn(glu(v[a][2], v[a][3])));
+            y[a] = *reinterpret_cast<const unsigned*>(&p);
+        }
+        OT* p = act + (size_t)m * act_ld + act_off + (u - u1p);
+        if constexpr (N % 4 == 0) {
+#pragma unroll
+            for (int a = 0; a < N; a += 4) {
+                const auto s02 = __builtin_amdgcn_permlane32_swap(y[a], y[a + 2], false, false);
+                const auto s13 = __builtin_amdgcn_permlane32_swap(y[a + 1], y[a + 3], false, false);
+                const auto lo = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+                const auto hi = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+                if (r.slot >= 0)
+                    *reinterpret_cast<u32x4*>(p + 8 * (a + kg)) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+            }
+        } else if (r.slot >= 0) {
+#pragma unroll
+            for (int a = 0; a < N; ++a) *reinterpret_cast<unsigned*>(p + 8 * a + 2 * kg) = y[a];
+        }
+    }
+    // pairs u and u + 1, u even: one head division, neighbouring results stored together
+    __device__ void pair2(int u, int m, const float* a, bool second, Row r) const {
         if (!even || !second || (u < u1p ? u + 1 >= e_g : u + 1 - u1p >= ff)) {
             pair(u, m, a[0], a[1]);
             if (second) pair(u + 1, m, a[2], a[3]);
             return;
         }
-        const RowRef r = rows[m];
         if (r.slot < 0) return;
         if (u >= u1p) {
             const float y[2] = {glu(a[0], a[1]), glu(a[2], a[3])};
@@ -85,7 +121,8 @@ struct HyIn {
         const int hp = qk ? hpq : hpv, h = uu / hp, j = uu - h * hp;
         if (qk && j < rh) {  // two rotation pairs {j, j + rh}, {j + 1, j + 1 + rh} (retention only)
             const size_t at = (size_t)r.pos * rh + j;
-            const float c0 = cs[at], s0 = sn[at], c1 = cs[at + 1], s1 = sn[at + 1], f = isq ? 1.0f : kscale;
+            const float2 cc = *reinterpret_cast<const float2*>(cs + at), ss = *reinterpret_cast<const float2*>(sn + at);
+            const float c0 = cc.x, s0 = ss.x, c1 = cc.y, s1 = ss.y, f = isq ? 1.0f : kscale;
             float* p = (isq ? q : k) + ((size_t)m * H + h) * dim + j;
             const float lo[2] = {(a[0] * c0 - a[1] * s0) * f, (a[2] * c1 - a[3] * s1) * f};
             const float hi[2] = {(a[1] * c0 + a[0] * s0) * f, (a[3] * c1 + a[2] * s1) * f};
@@ -98,8 +135,7 @@ struct HyIn {
                 *reinterpret_cast<float4*>(q + ((size_t)m * H + h) * hd + 2 * j) = make_float4(a[0], a[1], a[2], a[3]);
             } else {
                 KT* p = (qk ? kc : vc) + (((size_t)r.slot * G + h) * T + r.pos) * hd + 2 * j;
-                store2(p, a);
-                store2(p + 2, a + 2);
+                store4(p, make_float4(a[0], a[1], a[2], a[3]));
             }
             return;
         }
@@ -288,6 +324,18 @@ struct PgPair {  // prefill.h: plain 16-row tiles, 4 consecutive rows per store
     __device__ void store(int t, int i0, int m, const float* v, const PfState&) const {
         const int u = t * 8 + (i0 >> 1);
         if (u < n) e.pair2(u0 + u, m, v, u + 1 < n);
+    }
+    // (kRolled)
+    __device__ auto row_of(int m) const { return e.row_of(m); }
+    __device__ bool flat(int t, int tiles) const { return 8 * (t + tiles) <= n && e.flat(u0 + 8 * t, 8 * tiles); }
+    template <int N, class Row>
+    __device__ void flat_store(int t, int kg, int m, const pf_float4* v, const Row& r) const {
+        e.template flat_store<N>(u0 + 8 * t, kg, m, v, r);
+    }
+    template <class Row>
+    __device__ void store(int t, int i0, int m, const float* v, const Row& r) const {
+        const int u = t * 8 + (i0 >> 1);
+        if (u < n) e.pair2(u0 + u, m, v, u + 1 < n, r);
     }
 };
 

@@ -49,7 +49,12 @@ struct SeqIn {  // [q | latent | gate ; residual gate]
         put(2 * u, m, v0);
         put(2 * u + 1, m, v1);
     }
-    __device__ void pair2(int u, int m, const float* a, bool second) const {  // u even
+    struct Row {};
+    __device__ Row row_of(int) const { return {}; }
+    __device__ bool flat(int, int) const { return false; }
+    template <int N>
+    __device__ void flat_store(int, int, int, const pf_float4*, Row) const {}
+    __device__ void pair2(int u, int m, const float* a, bool second, Row) const {  // u even
         const int row = 2 * u;
         float* dst = nullptr;
         float4 y = make_float4(a[0], a[1], a[2], a[3]);

@@ -354,7 +354,9 @@ struct PgDefers : std::false_type {};
 template <class Epi>
 struct PgDefers<Epi, std::enable_if_t<Epi::kDefer>> : std::true_type {};
 
-// Epilogues with a member kRolled = true are looped over a wave's tiles instead of unrolled
+// Epilogues with a member kRolled = true are too large to be unrolled over a wave's tiles: they are looped over its weight tiles.
+// What a chunk row's stores need of it, row_of(m), is asked for once and for all of a wave's rows together; store(t, i0, m, v, r)
+// gets it. Waves whose weight tiles t0 .. t0 + n - 1 are all flat(t0, n) are not looped: flat_store<n>(t0, lane group, m, v[n], r).
 template <class Epi, class = void>
 struct PgRolled : std::false_type {};
 template <class Epi>
@@ -759,36 +761,55 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         }
     }
     if constexpr (PgRolled<Epi>::value) {
-        // an epilogue too large to be unrolled over the tiles: a loop over them, the sums indexed in the ring's LDS
-        // (indexed registers would live in scratch)
-        constexpr int NV = AT * Geo::WPT, H = NV * 16 * Geo::THREADS <= Geo::LDS ? NV : NV / 2;
-        static_assert(H * 16 * Geo::THREADS <= Geo::LDS && NV % H == 0, "sums in the ring");
+        // A loop over the weight tiles, their sums indexed in the ring's LDS (indexed registers would live in scratch), unrolled
+        // over the chunk rows: one tile at a time, each with its own look at its row, waited for memory and LDS in turn, 0.7 us
+        // a tile.
+        constexpr int NV = AT * Geo::WPT, H = NV * 16 * Geo::THREADS <= Geo::LDS ? AT : AT / 2;
+        static_assert(H * Geo::WPT * 16 * Geo::THREADS <= Geo::LDS && AT % H == 0, "sums in the ring");
+        const int t0 = rb * Geo::NA + wr * AT, m0 = pb * BM + wp * Geo::WPT * 16 + r16;
+        decltype(epi.row_of(0)) rr[Geo::WPT];
+#pragma unroll
+        for (int b = 0; b < Geo::WPT; ++b) rr[b] = epi.row_of(m0 + 16 * b);
         __syncthreads();  // every wave is done with its fragments
-        pf_float4* mine = reinterpret_cast<pf_float4*>(pg_smem) + threadIdx.x;
+        if (!live) return;
+        if (t0 + AT <= nt && epi.flat(t0, AT)) {
 #pragma unroll
-        for (int h = 0; h < NV; h += H) {
+            for (int b = 0; b < Geo::WPT; ++b) {
+                pf_float4 v[AT];
 #pragma unroll
-            for (int j = 0; j < H; ++j) mine[j * Geo::THREADS] = acc[(h + j) / Geo::WPT][(h + j) % Geo::WPT];
+                for (int a = 0; a < AT; ++a) v[a] = acc[a][b];
+                epi.template flat_store<AT>(t0, kg, m0 + 16 * b, v, rr[b]);
+            }
+            return;
+        }
+        pf_float4* mine = reinterpret_cast<pf_float4*>(pg_smem) + threadIdx.x;  // (each thread reads what it wrote)
+#pragma unroll
+        for (int h = 0; h < AT; h += H) {
+#pragma unroll
+            for (int j = 0; j < H * Geo::WPT; ++j) mine[j * Geo::THREADS] = acc[h + j / Geo::WPT][j % Geo::WPT];
 #pragma unroll 1
             for (int j = 0; j < H; ++j) {
-                const int t = rb * Geo::NA + wr * AT + (h + j) / Geo::WPT;
-                const pf_float4 o = mine[j * Geo::THREADS];
-                const float v[4] = {o[0], o[1], o[2], o[3]};
-                if (t < nt && live) epi.store(t, i0, pb * BM + (wp * Geo::WPT + (h + j) % Geo::WPT) * 16 + r16, v, ps);
+                if (t0 + h + j >= nt) break;
+                pg_for<Geo::WPT>([&](auto B) PG_INLINE {
+                    constexpr int b = decltype(B)::value;
+                    const pf_float4 o = mine[(j * Geo::WPT + b) * Geo::THREADS];
+                    const float v[4] = {o[0], o[1], o[2], o[3]};
+                    epi.store(t0 + h + j, i0, m0 + 16 * b, v, rr[b]);
+                });
             }
         }
-        return;
-    }
-    if (!live) return;
+    } else {
+        if (!live) return;
 #pragma unroll
-    for (int a = 0; a < AT; ++a) {
-        const int t = rb * Geo::NA + wr * AT + a;
-        if (t >= nt) continue;
+        for (int a = 0; a < AT; ++a) {
+            const int t = rb * Geo::NA + wr * AT + a;
+            if (t >= nt) continue;
 #pragma unroll
-        for (int b = 0; b < Geo::WPT; ++b) {
-            const int m = pb * BM + (wp * Geo::WPT + b) * 16 + r16;
-            const float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
-            epi.store(t, i0, m, v, ps);
+            for (int b = 0; b < Geo::WPT; ++b) {
+                const int m = pb * BM + (wp * Geo::WPT + b) * 16 + r16;
+                const float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
+                epi.store(t, i0, m, v, ps);
+            }
         }
     }
 }

@@ -586,6 +586,20 @@ def test_replays_of_both_attention_forms(gpu):
     plain.close()
 
 
+@pytest.mark.parametrize("n", [20, 50, 100, 200])
+@pytest.mark.parametrize("ff", [8, 31, 32, 64, 72, 129, 264])
+def test_feed_forward_products_at_tile_edges(gpu, ff, n):
+    """The feed-forward products of a prompt, whole tiles of 8 pairs stored in pieces exchanged between lanes and the rest pair
+    by pair, in every tile height, with padding rows; two portions, so that rows between them are padding too."""
+    c = stack(ret(heads=1, dim=16, vdim=16, ff=ff), att(heads=2, kv_heads=1, dim=16, vdim=16, ff=ff), width=64)
+    t = R.random_tensors(c, ff)
+    m = make(c, t, "bfloat16", batch=2)
+    a, b = tokens(n - 9, c["vocab"], n), tokens(9, c["vocab"], n + 1)
+    got = m.feed([1, 0], [0, 0], [b, a], [[8], list(range(n - 9))])
+    close(got, np.concatenate([R.forward(c, t, b)[0][8:], R.forward(c, t, a)[0]]), "bfloat16", (ff, n))
+    m.close()
+
+
 @pytest.mark.parametrize("n", [33, 65, 129, 257, 300, 700, 1025, 2048, 2049])
 def test_row_counts_of_a_pass(gpu, n):
     """Prompt passes of every tile height with padding rows, a launch's last tiles cut over the depth (narrow outputs: all of
