@@ -2487,11 +2487,13 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     if (m->pf.cap == 0) n0 = 0;
     // The first step too, up to its last layer, where no small model's launch begins with it: its tokens are the prompts', so its
     // layers run as one more row of each sequence, and only the last layer and the head are left of it. A step of 31 layers of 32:
-    // 75 tokens of Llama-2-7B in fp32 and 21 more 119.8 -> 116.8 ms, 8 x 121 of Llama-3-8B and 7 more 52.3 -> 49.2.
-    const bool first = n0 > 0 && m->L > 1 && !small_takes(m, max_length);
-    PfState last{};
-    if (n0 > 0)
-        for (const PfState& c : pf_batch_chunks(m, n0 + first)) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, last = c));
+    // 75 tokens of Llama-2-7B in fp32 and 21 more 119.8 -> 116.8 ms, 8 x 121 of Llama-3-8B and 7 more 52.3 -> 49.2. Prompts of
+    // several chunks keep the step: the row past a full chunk would be a chunk of its own, which reads all weights too.
+    std::vector<PfState> chunks;
+    if (n0 > 0) chunks = pf_batch_chunks(m, n0 + 1);
+    const bool first = chunks.size() == 1 && m->L > 1 && !small_takes(m, max_length);
+    if (n0 > 0 && !first) chunks = pf_batch_chunks(m, n0);
+    for (const PfState& c : chunks) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
     for (int b = 0; b < m->B; ++b) {
         const size_t row = (size_t)b * (m->T + 1);
         if (n0 > 0)
@@ -2515,7 +2517,7 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     }
     if (first) {
         SLI_TRY(bg_sync_tiles(m));
-        SLI_TRY(SLI_DISPATCH(m, record_last, m, last));
+        SLI_TRY(SLI_DISPATCH(m, record_last, m, chunks[0]));
     }
     for (int t = n0 + first; t < max_length; ++t) {  // model.cpp:157
         SLI_TRY(sli_model_step(m));
