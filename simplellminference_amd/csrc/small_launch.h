@@ -36,9 +36,10 @@ struct SmArgs {
 
 // us a step that the launch loses to rows which a wave cannot ask for ahead: it waits for each in turn, a head row of `each` KiB
 // 0.5 + 0.4 each, a gate/up pair 2.9. 256-wide fp32, two layers, us a step as launches | here: 512 tokens of vocabulary 69 | 26, 16384
-// 72 | 44, 32000 74 | 71, 128256 94 | 205; 512-wide 69 | 31, 75 | 67, 79 | 100, 109 | 371; 320-wide with 2048 units, 3 layers 92 | 96.
+// 72 | 44, 32000 74 | 71, 128256 94 | 205; 512-wide 69 | 31, 75 | 67, 79 | 100, 109 | 371; 320-wide with 2048 units, 3 layers 92 | 96
+// (the KiB of the norm weights off what is asked for ahead: the fit).
 inline float small_lost_us(int D, int I, int L, int V, int wbytes, int nwg) {
-    const int each = (D * wbytes + 1023) / 1024, ahead = kSmRowBytes / kSmWaves / 1024, waves = nwg * kSmWaves;
+    const int each = (D * wbytes + 1023) / 1024, ahead = kSmRowBytes / kSmWaves / 1024 - (D * 4 + 1023) / 1024, waves = nwg * kSmWaves;
     auto late = [&](int items, int rows) {
         const int n = (items + waves - 1) / waves - ahead / (rows * each);
         return (float)(n > 0 ? n : 0);
