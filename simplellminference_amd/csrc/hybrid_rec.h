@@ -77,16 +77,19 @@ struct HyProj {
     }
     // pairs [0, split) read X, pairs [split, npairs) X2 (split: a multiple of kHySection; X2 null: one input)
     template <class Epi>
-    int pgemm(const WT* w, const __half* X, const __half* X2, int split, int K, int npairs, int u0, const Epi& e, int spare = 0) const {
+    int pgemm(const WT* w, const __half* X, const __half* X2, int split, int K, int npairs, int u0, const Epi& e, int spare = 0,
+              int valid = 0x7fffffff) const {
         if constexpr (F16) {
             PgIn<__half> in{w, X, nullptr, pad_to(2 * npairs, 16), K, M};
+            in.valid = valid;
             if (X2) in.Bhi2 = X2, in.row_b2 = 2 * split;
             in.ws = s->pg_ws, in.cnt = s->pg_cnt;
             float best = INFINITY;
             int pick = 0;
             constexpr bool rolled = PgRolled<PgPair<Epi>>::value;
             // spare: rows there are. Tiles of 256 rows over more rows than there are to do may be faster than tiles of 128: 4096 x
-            // 15104 at 1152 rows 191 us, at 1280 rows 169.
+            // 15104 at 1152 rows 191 us, at 1280 rows 169; 22528 x 2048 137 and 124 (1025 tokens of the 1b stack 4.43 -> 4.10 ms).
+            // valid: waves whose rows are all padding past it multiply nothing (that 4096 x 15104 at 1025 rows 173 -> 169).
             for (int m : {M, pad_to(M, 256)}) {
                 int i = 0;
                 if (m > M && m > spare) break;

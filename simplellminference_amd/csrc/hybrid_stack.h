@@ -134,6 +134,7 @@ struct BlockStack {
     unsigned* bg_cnt = nullptr;
     size_t bg_ws_bytes = 0, bg_groups = 1;  // the most any projection needs (hy_bg_need)
     std::vector<void*> allocs;
+    int live = 0x7fffffff;  // rows of the prompt pass from here on are padding
     bool by_16 = false;  // the pass's prompt attention takes its portions by 16 rows (prefill.h pf_rows_by_16)
     // captured passes of `feed`: {0, rows} of a decode step, {1 + 2 grid of the expansion + by_16, rows} of a prompt pass
     // (null: launched once so far)

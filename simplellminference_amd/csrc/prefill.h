@@ -764,8 +764,8 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
         // A loop over the weight tiles, their sums indexed in the ring's LDS (indexed registers would live in scratch), unrolled
         // over the chunk rows: one tile at a time, each with its own look at its row, waited for memory and LDS in turn, 0.7 us
         // a tile.
-        constexpr int NV = AT * Geo::WPT, H = NV * 16 * Geo::THREADS <= Geo::LDS ? AT : AT / 2;
-        static_assert(H * Geo::WPT * 16 * Geo::THREADS <= Geo::LDS && AT % H == 0, "sums in the ring");
+        constexpr int W = AT * Geo::WPT * 16 * Geo::THREADS <= Geo::LDS ? Geo::WPT : Geo::WPT / 2;  // chunk row tiles at a time
+        static_assert(AT * W * 16 * Geo::THREADS <= Geo::LDS && Geo::WPT % W == 0, "sums in the ring");
         const int t0 = rb * Geo::NA + wr * AT, m0 = pb * BM + wp * Geo::WPT * 16 + r16;
         decltype(epi.row_of(0)) rr[Geo::WPT];
 #pragma unroll
@@ -783,21 +783,21 @@ __global__ void __launch_bounds__(128 * Cfg::WR) pgemm_kernel(PgIn<WT> in, Epi e
             return;
         }
         pf_float4* mine = reinterpret_cast<pf_float4*>(pg_smem) + threadIdx.x;  // (each thread reads what it wrote)
+        pg_for<Geo::WPT / W>([&](auto B0) PG_INLINE {
+            constexpr int b0 = decltype(B0)::value * W;
 #pragma unroll
-        for (int h = 0; h < AT; h += H) {
-#pragma unroll
-            for (int j = 0; j < H * Geo::WPT; ++j) mine[j * Geo::THREADS] = acc[h + j / Geo::WPT][j % Geo::WPT];
+            for (int j = 0; j < AT * W; ++j) mine[j * Geo::THREADS] = acc[j / W][b0 + j % W];
 #pragma unroll 1
-            for (int j = 0; j < H; ++j) {
-                if (t0 + h + j >= nt) break;
-                pg_for<Geo::WPT>([&](auto B) PG_INLINE {
+            for (int a = 0; a < AT; ++a) {
+                if (t0 + a >= nt) break;
+                pg_for<W>([&](auto B) PG_INLINE {
                     constexpr int b = decltype(B)::value;
-                    const pf_float4 o = mine[(j * Geo::WPT + b) * Geo::THREADS];
+                    const pf_float4 o = mine[(a * W + b) * Geo::THREADS];
                     const float v[4] = {o[0], o[1], o[2], o[3]};
-                    epi.store(t0 + h + j, i0, m0 + 16 * b, v, rr[b]);
+                    epi.store(t0 + a, i0, m0 + 16 * (b0 + b), v, rr[b0 + b]);
                 });
             }
-        }
+        });
     } else {
         if (!live) return;
 #pragma unroll
@@ -941,9 +941,9 @@ constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
 // plan that costs least is the fastest one, and are no times of their own (a large product's stages last longer: the clock
 // falls). Over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken lasts 1.1 % longer than the fastest, of
 // int8 0.4, of fp32 0.8, of block stacks 2 % (tools/pgemm_lab prints both).
-// rolled: a looped epilogue (kRolled) takes time by the tiles a wave loops over: a stack's 25600 x 3072 at 384 rows 100.6 us in
-// 128 x 256 tiles (16 a wave), 95.9 in 128 x 128 (8), with a plain epilogue 84 and 90. 0.7 us each, shared by the workgroups of
-// a CU, is what picks best.
+// rolled: a looped epilogue (kRolled) takes time by the tiles a wave holds: a stack's 22528 x 2048 at 1152 rows 137 us in 128 x
+// 256 tiles (16 a wave), over 1280 rows in 256 x 256 124. 0.35 us each, shared by the workgroups of a CU, is what picks best (0.7:
+// a prompt of 1280 rows of that stack 4.71 ms, so 4.56; 17 other row counts the same).
 template <class Cfg, typename WT>
 PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled = false) {
     using Geo = PgGeo<Cfg, WT>;
@@ -951,7 +951,7 @@ PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled =
     const int ns = (K + Geo::KS - 1) / Geo::KS;
     const int occ = (int)((160 * 1024) / Geo::LDS), cpx = std::max(1, cus / 8) * occ;
     constexpr float kTile = 16.0f * Geo::AT * Geo::WPT * Geo::THREADS / 131072.0f, kEdge = 2.0f + 6.0f * kTile;
-    const float epi = rolled ? 0.7f * Geo::AT * Geo::WPT / (float)occ : 0.0f;
+    const float epi = rolled ? 0.35f * Geo::AT * Geo::WPT / (float)occ : 0.0f;
     PgPlan best;
     best.slots = nx;
     best.us = (float)((nx + cpx - 1) / cpx) * ((float)ns * stage + kEdge + epi);

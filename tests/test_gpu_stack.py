@@ -685,6 +685,22 @@ def test_every_tiling_of_a_pass(gpu, n, model=wide_model):
     m.close()
 
 
+@pytest.mark.parametrize("n", [129, 513, 580, 641])
+def test_pass_after_a_longer_one(gpu, n):
+    """A pass whose GEMMs run over more rows than it has, those rows holding what a longer pass left: as on a new model, bit
+    for bit, also the cache that a step reads afterwards."""
+    m = wide_model()
+    ids = tokens(n, vocab=203, seed=n)
+
+    def once():
+        a = m.feed([0], [0], [ids], [list(range(n - 3, n))])
+        return np.concatenate([a, m.feed([0], [n], [[7]], [[0]])]).view(np.uint32)
+    new = once()
+    m.feed([0], [0], [tokens(790, vocab=203, seed=1)])
+    assert np.array_equal(once(), new)
+    m.close()
+
+
 def narrow_model(batch):
     """One block of width 2048 whose output projection has 10240 columns: five k-blocks a wave in a decode pass of 2 rows and
     more (test_host_runtime.py looks)."""
