@@ -774,12 +774,13 @@ struct HyRec : HyProj<WT> {
             SLI_HIP(hipGetLastError());
         }
         const auto ei = in_epi<OT>(l, r);
-        const int valid = one ? 0x7fffffff : s->live;
+        // (a decode pass sets no rows past its own)
+        const int valid = one ? 0x7fffffff : s->live, spare = one ? 0 : s->M;
         if constexpr (!std::is_same<OT, float>::value) {
             if (l.d.ff > 0)
-                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, (const __half*)s->c2, l.u1p, s->Dp, l.u1p + l.d.ff, 0, ei, s->M, valid));
+                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, (const __half*)s->c2, l.u1p, s->Dp, l.u1p + l.d.ff, 0, ei, spare, valid));
             else
-                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei, s->M, valid));
+                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei, spare, valid));
         } else {
             if (l.d.ff > 0 && path(M, s->Dp) == P::BG) {
                 HY_TRY(project2(l.win, s->c1, s->c2, s->Dp, l.e_g, l.u1p, l.d.ff, ei, l.win_t));

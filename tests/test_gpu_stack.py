@@ -701,6 +701,24 @@ def test_pass_after_a_longer_one(gpu, n):
     m.close()
 
 
+@pytest.mark.parametrize("batch", [9, 12, 33])
+def test_lockstep_after_a_longer_prompt(gpu, batch):
+    """Decode passes of more than 8 sequences set no rows past their own, and leave what a prompt pass put there alone: the
+    longer prompt's sequence goes on as if there had been none."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    b = BlockSpec("attention", 4, 64, 64, kv_heads=2, scale=0.125, ff=8192, ff_limit=7.0)
+    m = StackModel(StackSpec(203, 4096, (b,), taps=4, residual_mult=0.4, max_length=320), batch=batch, seed=4).init()
+    ids = tokens(290, vocab=203, seed=1)
+    m.feed([0], [0], [ids])
+    want = m.feed([0], [290], [[5]], [[0]])
+    m.feed([0], [0], [ids])
+    others = list(range(1, batch))
+    for t in range(2):
+        m.feed(others, [t] * len(others), [[t + 1]] * len(others))
+    assert np.array_equal(m.feed([0], [290], [[5]], [[0]]).view(np.uint32), want.view(np.uint32))
+    m.close()
+
+
 def narrow_model(batch):
     """One block of width 2048 whose output projection has 10240 columns: five k-blocks a wave in a decode pass of 2 rows and
     more (test_host_runtime.py looks)."""
