@@ -774,13 +774,12 @@ struct HyRec : HyProj<WT> {
             SLI_HIP(hipGetLastError());
         }
         const auto ei = in_epi<OT>(l, r);
-        // (a decode pass sets no rows past its own)
-        const int valid = one ? 0x7fffffff : s->live, spare = one ? 0 : s->M;
+        const int valid = one ? 0x7fffffff : s->live;
         if constexpr (!std::is_same<OT, float>::value) {
             if (l.d.ff > 0)
-                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, (const __half*)s->c2, l.u1p, s->Dp, l.u1p + l.d.ff, 0, ei, spare, valid));
+                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, (const __half*)s->c2, l.u1p, s->Dp, l.u1p + l.d.ff, 0, ei, 0, valid));
             else
-                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei, spare, valid));
+                HY_TRY(pgemm((const WT*)l.win, (const __half*)s->c1, nullptr, 0, s->Dp, l.e_g, 0, ei, 0, valid));
         } else {
             if (l.d.ff > 0 && path(M, s->Dp) == P::BG) {
                 HY_TRY(project2(l.win, s->c1, s->c2, s->Dp, l.e_g, l.u1p, l.d.ff, ei, l.win_t));
@@ -917,10 +916,10 @@ int hy_pass(BlockStack* s, const std::vector<RowRef>& rows_in, const std::vector
     for (const HyLayer& l : s->layers)
         if (l.d.mixer == SLI_MIX_ATTENTION && l.hd <= 128) s->by_16 = s->by_16 && pf_rows_by_16(groups, l.d.heads, l.hd, device_cus());
     std::vector<RowRef> rows(rows_in);
-    rows.resize(one ? M : std::min(pad_to(M, 256), s->M), RowRef{-1, 0, 0, 0});  // (a GEMM may run over the next multiple of 256)
+    rows.resize(M, RowRef{-1, 0, 0, 0});
     s->live = s->replays ? 0x7fffffff : n;  // (a graph's passes are of other row counts)
     const int32_t ns = (int32_t)segs.size();
-    SLI_HIP(hipMemcpyAsync(s->rows, rows.data(), sizeof(RowRef) * rows.size(), hipMemcpyHostToDevice, s->stream));
+    SLI_HIP(hipMemcpyAsync(s->rows, rows.data(), sizeof(RowRef) * M, hipMemcpyHostToDevice, s->stream));
     SLI_HIP(hipMemcpyAsync(s->segs, segs.data(), sizeof(SegRef) * ns, hipMemcpyHostToDevice, s->stream));
     SLI_HIP(hipMemcpyAsync(s->nsegs, &ns, sizeof(ns), hipMemcpyHostToDevice, s->stream));
     const int msegs = one ? M : s->replays ? std::min(s->B, M / kHyTile) : ns;  // (a replayed pass has other portions)

@@ -88,7 +88,7 @@ struct HyProj {
             int pick = 0;
             constexpr bool rolled = PgRolled<PgPair<Epi>>::value;
             // spare: rows there are. Tiles of 256 rows over more rows than there are to do may be faster than tiles of 128: 4096 x
-            // 15104 at 1152 rows 191 us, at 1280 rows 169; 22528 x 2048 137 and 124 (1025 tokens of the 1b stack 4.43 -> 4.10 ms).
+            // 15104 at 1152 rows 191 us, at 1280 rows 169.
             // valid: waves whose rows are all padding past it multiply nothing (that 4096 x 15104 at 1025 rows 173 -> 169).
             for (int m : {M, pad_to(M, 256)}) {
                 int i = 0;

@@ -941,9 +941,11 @@ constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
 // plan that costs least is the fastest one, and are no times of their own (a large product's stages last longer: the clock
 // falls). Over 600 sizes of fp16 (1024 to 28672 outputs, 9 to 4096 rows) the plan taken lasts 1.1 % longer than the fastest, of
 // int8 0.4, of fp32 0.8, of block stacks 2 % (tools/pgemm_lab prints both).
-// rolled: a looped epilogue (kRolled) takes time by the tiles a wave holds: a stack's 22528 x 2048 at 1152 rows 137 us in 128 x
-// 256 tiles (16 a wave), over 1280 rows in 256 x 256 124. 0.35 us each, shared by the workgroups of a CU, is what picks best (0.7:
-// a prompt of 1280 rows of that stack 4.71 ms, so 4.56; 17 other row counts the same).
+// rolled: a looped epilogue (kRolled) is priced by the tiles a wave loops over: 0.7 us each, shared by the workgroups of a CU. That was
+// fitted to a stack's 25600 x 3072 at 384 rows, 100.6 us in 128 x 256 tiles (16 a wave) and 95.9 in 128 x 128 (8); a plain epilogue 84
+// and 90. It takes about half of that by now, and the price stays all the same: it sets where the depth is cut, so the order of a prompt's
+// sums. (0.35, and rows to spare as the output GEMM has, cut elsewhere at 15 of 36 row counts of a 2048-wide stack's two inputs and would
+// take 4.43 ms for 4.61 at 1280 rows, 4.03 for 4.09 at 1025.)
 template <class Cfg, typename WT>
 PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled = false) {
     using Geo = PgGeo<Cfg, WT>;
@@ -951,7 +953,7 @@ PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled =
     const int ns = (K + Geo::KS - 1) / Geo::KS;
     const int occ = (int)((160 * 1024) / Geo::LDS), cpx = std::max(1, cus / 8) * occ;
     constexpr float kTile = 16.0f * Geo::AT * Geo::WPT * Geo::THREADS / 131072.0f, kEdge = 2.0f + 6.0f * kTile;
-    const float epi = rolled ? 0.35f * Geo::AT * Geo::WPT / (float)occ : 0.0f;
+    const float epi = rolled ? 0.7f * Geo::AT * Geo::WPT / (float)occ : 0.0f;
     PgPlan best;
     best.slots = nx;
     best.us = (float)((nx + cpx - 1) / cpx) * ((float)ns * stage + kEdge + epi);

@@ -322,6 +322,29 @@ def stack_prompts_take_the_fast_tilings(H):
         m.close()
 
 
+# Input GEMMs of 2048-wide blocks with 8192 units: (block, prompt) -> (BM, WR, AT). A tiling and its cuts set the order of the sums,
+# so they are part of what a prompt's rows are; each of these would be another one at half the price of the looped epilogue, or with
+# rows to spare.
+STACK_IN_TILES = {("attention", 20): (32, 2, 2), ("attention", 120): (128, 4, 2), ("attention", 500): (128, 4, 2),
+                  ("attention", 620): (128, 4, 2), ("retention", 380): (128, 4, 2), ("retention", 1100): (128, 4, 4)}
+
+
+def stack_inputs_keep_their_sums(H):
+    """The input GEMM of a stack's prompt runs the tiling, and so the order of sums, that its price gives."""
+    from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
+    blocks = dict(attention=BlockSpec("attention", 32, 64, 64, kv_heads=8, scale=0.125, ff=8192, ff_limit=7.0),
+                  retention=BlockSpec("retention", 8, 128, 256, decay=(0.9,) * 8, rot_dims=128, rot_base=1e4, ff=8192, ff_limit=7.0))
+    for kind, b in blocks.items():
+        m = StackModel(StackSpec(64, 2048, (b,), taps=4, max_length=1200), batch=1, seed=1).init()
+        for (k, n), tiling in STACK_IN_TILES.items():
+            if k == kind:
+                H.hh_launched()
+                m.feed([0], [0], [[1] * n])
+                ran = {(c[0], c[1], c[3]) for _, c in _tilings(H.hh_launched(), "HyIn")}
+                assert ran == {tiling}, (kind, n, ran)
+        m.close()
+
+
 # Prompts of Llama-2-7B: (weights, positions through the chunk, epilogue) -> (BM, WR, AT) of the tilings, each within 4 % of the
 # fastest at its best split. us of that tiling | of the one that stale stage times took: fp16 512 rows wo 39 | 43, down 79 | 103;
 # 64 rows down 28 | 33; int8 96 rows gate/up 45 | 54; fp32 512 rows gate/up 1024 | 1350, 96 rows gate/up 238 | 294
@@ -407,7 +430,7 @@ def steps_of_the_batched_projection(H):
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
          "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
          "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass", "weight_copies_where_they_are_read",
-         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "prompts_take_the_fast_tilings",
+         "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "stack_inputs_keep_their_sums", "prompts_take_the_fast_tilings",
          "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
 
