@@ -1228,23 +1228,41 @@ struct StepRecorder {
     // attention, wo, gate/up and down of one layer in 32: 512 tokens of Llama-2-7B 17.01 -> 16.57 ms). A model of one layer,
     // which only serves to look at that layer's launches, runs it whole.
     // one GEMM over a chunk's rows: the tiling (prefill.h pg_tilings) whose plan costs least over the rows padded to its BM
+    struct PgPick {
+        int tiling = 0, M = 0;
+        PgPlan plan;
+    };
+    static int pg_valid(const PfState& st) { return st.nseq == 1 ? st.nv : st.nseq * st.rps; }
+    static PgPick pg_pick(int N, int K, const PfState& st) {
+        PgPick best;
+        best.plan.us = INFINITY;
+        const int valid = pg_valid(st);
+        int i = 0;
+        pg_tilings<WT>([&](auto cfg, float us) {
+            using Geo = PgGeo<decltype(cfg), WT>;
+            const int M = (valid + Geo::BM - 1) / Geo::BM * Geo::BM;
+            // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
+            // in 16 ranges and more
+            if (Geo::FOLD == 0 && (st.nseq > 1 || !pg_one_chain(N, K, valid))) us = INFINITY;
+            const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true, us);
+            if (p.us < best.plan.us) best = PgPick{i, M, p};
+            ++i;
+        });
+        return best;
+    }
+    // us of the GEMMs of a layer over a chunk, by their plans
+    static float pg_price(const sli_model* m, const PfState& st) {
+        const int QD = m->hq * m->hd;
+        return pg_pick(QD + 2 * m->hkv * m->hd, m->D, st).plan.us + pg_pick(m->D, QD, st).plan.us + pg_pick(2 * m->Il, m->D, st).plan.us +
+               pg_pick(m->D, m->Il, st).plan.us;
+    }
     template <class Epi>
     static int pg(sli_model* m, const void* W, int N, int K, const __half* hi, const __half* lo, const Epi& e,
                   const PfState& st, PfPart* part = nullptr) {
         PgIn<WT> in{(const WT*)W, hi, lo, N, K, 0};
-        in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = st.nseq == 1 ? st.nv : st.nseq * st.rps;
-        float best = INFINITY;
-        int pick = 0, i = 0;
-        pg_tilings<WT>([&](auto cfg, float us) {
-            using Geo = PgGeo<decltype(cfg), WT>;
-            const int M = (in.valid + Geo::BM - 1) / Geo::BM * Geo::BM;
-            // rows of several sequences take the tilings with short chains, as the batched projections (bgemm.h) sum
-            // in 16 ranges and more
-            if (Geo::FOLD == 0 && (st.nseq > 1 || !pg_one_chain(N, K, in.valid))) us = INFINITY;
-            const PgPlan p = pg_plan<decltype(cfg), WT>(N, K, M, device_cus(), true, us);
-            if (p.us < best) best = p.us, pick = i, in.full = p.full, in.splits = p.splits, in.M = M;
-            ++i;
-        });
+        in.ws = m->pf.ws, in.cnt = m->pf.cnt, in.valid = pg_valid(st);
+        const PgPick best = pg_pick(N, K, st);
+        in.full = best.plan.full, in.splits = best.plan.splits, in.M = best.M;
         // part: the launch may leave its sums to the next norm, where they are few (a merge in the GEMM is its last workgroups'
         // store, arrival and load; in the norm it is a load): 45 rows of Llama-2-7B, wo and down with their norms 51.3 -> 46.6
         // us, int8 46.4 -> 43.5, 100 rows 64.8 -> 61.5; at 511 rows nothing is left of it
@@ -1253,9 +1271,9 @@ struct StepRecorder {
             *part = PfPart{in.ws, in.splits, (size_t)in.M * N, e.rscale};
         }
         hipError_t err = hipSuccess;
-        i = 0;
+        int i = 0;
         pg_tilings<WT>([&](auto cfg, float) {
-            if (i++ == pick) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
+            if (i++ == best.tiling) err = launch_pgemm<Epi, decltype(cfg), WT>(in, e, st, m->stream);
         });
         SLI_HIP(err);
         return SLI_OK;
@@ -1337,6 +1355,17 @@ struct StepRecorder {
             else if (m->partial)  // debug no-comm mode: keep the local partial as the residual stream
                 SLI_HIP(hipMemcpyAsync(m->pf.x, m->pf.xpart, sizeof(float) * n, hipMemcpyDeviceToDevice, m->stream));
         }
+        return SLI_OK;
+    }
+    // Whether a chunk takes one position more instead of leaving it to a step: where the position opens no new tile, or one that
+    // costs less than the weights the step would read, at 6.5 TB/s. Actual times, not plans, against the step: Llama-2-7B in fp32, 64 -> 65
+    // positions 6.9 ms, 128 -> 129 8.7, 192 -> 193 8.2, 256 -> 257 12.1, a step 4.4; but 32 -> 33 3.7, 96 -> 97 2.3 and none within a
+    // tile. Eight sequences of Llama-3-8B: 32 -> 33 3.1, 80 -> 81 3.9, 128 -> 129 4.4, a step 2.9; 16 -> 17 2.6, 48 -> 49 2.5, 96 -> 97 1.8.
+    // By plan these are 6.3, 8.0, 5.5, 9.7 (step 3.9) 3.0, 0.7; 2.2, 2.2, 2.9 (step 2.1) 1.5, 1.4, 1.7.
+    static int first_step_pays(sli_model* m, const PfState& with, const PfState& without, bool* pays) {
+        const int QD = m->hq * m->hd, KD = m->hkv * m->hd;
+        const double bytes = (double)sizeof(WT) * ((double)m->D * (QD + 2 * KD) + (double)m->D * QD + 3.0 * m->D * m->Il);
+        *pays = pg_price(m, with) - pg_price(m, without) < bytes / 6.5e6;
         return SLI_OK;
     }
     // The rest of the step at the last position of a chunk that held it (record_prefill left its row as the last layer reads it): that
@@ -2487,12 +2516,17 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     if (m->pf.cap == 0) n0 = 0;
     // The first step too, up to its last layer, where no small model's launch begins with it: its tokens are the prompts', so its
     // layers run as one more row of each sequence, and only the last layer and the head are left of it. A step of 31 layers of 32:
-    // 75 tokens of Llama-2-7B in fp32 and 21 more 119.8 -> 116.8 ms, 8 x 121 of Llama-3-8B and 7 more 52.3 -> 49.2. Prompts of
-    // several chunks keep the step: the row past a full chunk would be a chunk of its own, which reads all weights too.
+    // 75 tokens of Llama-2-7B in fp32 and 21 more 119.8 -> 116.8 ms, 8 x 121 of Llama-3-8B and 7 more 52.3 -> 49.2. Where the row opens
+    // new tiles that cost more (first_step_pays), and in prompts of several chunks (the row past a full chunk would be a chunk of its own,
+    // which reads all weights too), the step stays.
     std::vector<PfState> chunks;
-    if (n0 > 0) chunks = pf_batch_chunks(m, n0 + 1);
-    const bool first = chunks.size() == 1 && m->L > 1 && !small_takes(m, max_length);
-    if (n0 > 0 && !first) chunks = pf_batch_chunks(m, n0);
+    if (n0 > 0) chunks = pf_batch_chunks(m, n0);
+    bool first = false;
+    if (chunks.size() == 1 && m->L > 1 && !small_takes(m, max_length)) {
+        const std::vector<PfState> with = pf_batch_chunks(m, n0 + 1);
+        if (with.size() == 1) SLI_TRY(SLI_DISPATCH(m, first_step_pays, m, with[0], chunks[0], &first));
+        if (first) chunks = with;
+    }
     for (const PfState& c : chunks) SLI_TRY(SLI_DISPATCH(m, record_prefill, m, c));
     for (int b = 0; b < m->B; ++b) {
         const size_t row = (size_t)b * (m->T + 1);

@@ -367,6 +367,31 @@ def prompts_take_the_fast_tilings(H):
         m.close()
 
 
+# Prompts -> whether predict runs their first step as one more row of the chunk: (preset, weights, cache, batch) -> (taken, left). ms of a
+# call with the row | with the step: fp32 65 tokens 29.2 | 26.7, 129 40.5 | 36.3, 193 50.4 | 46.8, 257 62.6 | 55.3, 33 22.1 | 22.7, 64 22.3 |
+# 26.7; eight of 8B 33 tokens 18.5 | 18.3, 81 28.2 | 27.7, 129 37.2 | 35.6, 49 21.0 | 21.7, 121 32.7 | 35.6; with a fp32 cache 65 tokens
+# 34.2 | 25.4, 129 49.3 | 38.0, 66 34.2 | 37.8; three of 8B 33 tokens 14.1 | 15.1, 129 20.0 | 21.1
+FIRST_STEPS = {("llama2-7b", "f32", "f32", 1): ((9, 32, 33, 64, 66, 75, 97, 128, 130), (65, 129, 193, 257, 385)),
+               ("llama3-8b", "f16", "f16", 8): ((16, 17, 32, 34, 49, 64, 97, 121, 128), (33, 81, 129, 257)),
+               ("llama3-8b", "f16", "f32", 8): ((33, 64, 66, 128), (65, 129, 257)),
+               ("llama3-8b", "f16", "f16", 3): ((16, 33, 65, 129), ())}
+
+
+def first_steps_join_the_chunk_where_they_pay(H):
+    """predict runs its first step in the prompt's chunk, but not where the row opens a tile that costs more than the step."""
+    from simplellminference_amd.model import LlamaModel, preset
+    for (name, w, kv, batch), (taken, left) in FIRST_STEPS.items():
+        m = LlamaModel(config=preset(name, num_hidden_layers=2, vocab_size=500, max_length=400), w_dtype=w, kv_dtype=kv, seed=1,
+                       batch=batch).init()
+        for n in taken + left:
+            H.hh_launched()
+            had = H.hh_graph_launches()
+            m.predict_batch(_prompts(m, n), n + 2)
+            joined = b"pf_last_rows_kernel" in H.hh_launched()
+            assert joined == (n in taken) and H.hh_graph_launches() - had == 3 - joined, (name, w, kv, batch, n, joined)
+        m.close()
+
+
 def short_prompts_sum_in_short_chains(H):
     """GEMMs that sum in one chain over the depth: none up to 769 tokens, gate/up alone up to 1537, then down too."""
     from simplellminference_amd.model import LlamaModel, preset
@@ -431,7 +456,7 @@ CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_c
          "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
          "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass", "weight_copies_where_they_are_read",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "stack_inputs_keep_their_sums", "prompts_take_the_fast_tilings",
-         "short_prompts_sum_in_short_chains",
+         "first_steps_join_the_chunk_where_they_pay", "short_prompts_sum_in_short_chains",
          "fp32_output_projection_steps", "steps_of_the_batched_projection"]
 
 
