@@ -209,6 +209,9 @@ int sli_model_prefill(sli_model* m, const int32_t* ids, int32_t n);
 /* Which path sli_model_prefill takes for this model: 1 = chunked MFMA GEMMs (prefill.h), 0 = the decode step,
  * teacher-forced (fp32 weights, batch > 1, unsupported shapes, or a TP rank without an RCCL communicator). */
 int sli_model_prefill_path(const sli_model* m);
+/* Which way the last sli_model_predict[_batch] of this model went from its prompt's chunks on: 0 = step by step, 1 / 2 = a small model's
+ * greedy loop as one launch (small_model.h) over all XCDs / on one. */
+int sli_model_predict_path(const sli_model* m);
 /* 1: the batch-1 decode step runs each layer's q/k/v projection and attention as ONE launch (qkv_attn.h: the
  * attention's K/V rows below the position stream while the projection runs; q and this step's K/V row are
  * handed over inside the launch); 0: separate launches (model.cpp:70-84's matmul / rope / mha sequence either

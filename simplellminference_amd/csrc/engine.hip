@@ -149,10 +149,12 @@ struct sli_model {
         size_t granules = 0;
         int nwg = 0, one_nwg = 0;  // workgroups over all XCDs, on one (0: not there)
         int turn = 0;              // of the tickets of the launches on one XCD
+        bool stale = false;        // such a launch may have left its tickets as they were
+        int path = 0;              // sli_model_predict_path
         float lost = 0.0f;  // small_lost_us
         unsigned tag = 4;  // the next launch's first tag
         unsigned spin = sli::kSmSpin;
-        bool gave_up = false;  // a launch did: this model takes the steps from then on
+        bool gave_up = false;  // a launch over all XCDs did: this model takes the steps from then on
     } sm;
 };
 
@@ -747,7 +749,12 @@ static int small_steps(sli_model* m, int n, int xcd) {
     a.g_x = a.g_act + m->Il;
     a.g_key = a.g_x + m->D;
     a.xcd = xcd;
-    if (xcd >= 0) a.nwg = m->sm.one_nwg, a.ticket = reinterpret_cast<unsigned*>(m->sm.g + m->sm.granules - 1), a.turn = m->sm.turn ^= 1;
+    if (xcd >= 0) {
+        a.nwg = m->sm.one_nwg, a.ticket = reinterpret_cast<unsigned*>(m->sm.g + m->sm.granules - 1);
+        if (m->sm.stale) SLI_HIP(hipMemsetAsync(a.ticket, 0, 8, m->stream));
+        m->sm.stale = true;  // (until the call has seen that it ran)
+        a.turn = m->sm.turn ^ 1;
+    }
     a.tag0 = m->sm.tag;
     a.spin = m->sm.spin, a.look = m->sm.spin >= 1023 ? 1023 : 0;
     m->sm.tag += need;
@@ -2229,6 +2236,8 @@ static std::vector<PfState> pf_chunks(int n, int cap) {
     return cs;
 }
 
+extern "C" int sli_model_predict_path(const sli_model* m) { return m ? m->sm.path : 0; }
+
 extern "C" int sli_model_prefill_path(const sli_model* m) { return m && m->bs ? 1 : m && m->B == 1 && m->c.w_dtype != SLI_DT_F32 && pf_supported(m) ? 1 : 0; }
 
 extern "C" int sli_model_fused_qkv_attn(sli_model* m) {
@@ -2535,18 +2544,29 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
         SLI_TRY(set_state(m, b, prompts[(size_t)b * ld + n0], n0, 1));
     }
     const size_t per_step = (size_t)m->B * m->v_n;
-    // (scratch that did not fit leaves the steps; so does a wait that gave up, which happens where other work keeps the
-    // launch's workgroups from running together: it took a second, so no later call tries again)
-    bool loop = small_takes(m, max_length) && !logits_out && (n0 > 0 || !wants_chunks);
-    if (loop) {
-        const SmallPlace place(m->c.device, m->sm.one_nwg ? small_xcds(kSmOneWgs) : 0);
+    // (scratch that did not fit leaves the steps)
+    const bool loop = small_takes(m, max_length) && !logits_out && (n0 > 0 || !wants_chunks);
+    m->sm.path = 0;
+    while (loop && !m->sm.gave_up) {
+        // (a launch on one XCD counts if the position moved: one of which no workgroup came to its XCD does nothing)
+        const SmallPlace place(m->c.device, m->sm.one_nwg > 0 && n0 + 1 < m->T ? small_xcds(kSmOneWgs) : 0);
+        const bool one = place.xcd >= 0;
         SLI_TRY(small_steps(m, max_length - n0, place.xcd));
         DevState d{};
         SLI_HIP(hipMemcpyAsync(&d, m->st, sizeof(d), hipMemcpyDeviceToHost, m->stream));
         SLI_HIP(hipMemcpyAsync(tokens_out, m->hist, sizeof(int32_t) * max_length, hipMemcpyDeviceToHost, m->stream));
         SLI_TRY(wait_stream(m));
-        if (!(d.error & kSmErrWait)) return d.error ? check_device_errors(m) : SLI_OK;
-        m->sm.gave_up = true;
+        if (!(d.error & kSmErrWait) && (!one || d.pos == std::min(max_length, m->T - 1))) {
+            if (one) m->sm.stale = false, m->sm.turn ^= 1;
+            m->sm.path = one ? 2 : 1;
+            return d.error ? check_device_errors(m) : SLI_OK;
+        }
+        // A wait that gave up: other work, another process's too, kept the launch's workgroups from running together. It took a second,
+        // so no later call tries that place again: from one XCD to all of them, and from there to the steps.
+        if (one)
+            m->sm.one_nwg = 0;
+        else
+            m->sm.gave_up = true;
         SLI_TRY(set_state(m, 0, prompts[n0], n0, 1));
     }
     if (first) {

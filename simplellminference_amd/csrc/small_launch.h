@@ -51,7 +51,7 @@ inline float small_lost_us(int D, int I, int L, int V, int wbytes, int nwg) {
 hipError_t small_allow(int wd, int kd, int hd);
 hipError_t small_launch(const SmArgs& a, int wd, int kd, int hd, hipStream_t s);
 // The current device's XCDs that take every eighth workgroup of a launch, `per` of 8 per workgroups each (their XCC_IDs as a mask; 0:
-// it is not so). Asked of the device once.
+// it is not so). Asked of the device once for each `per`.
 unsigned small_xcds(int per);
 
 }  // namespace sli

@@ -26,7 +26,8 @@
 // A wave asks for its weight rows of the next op (LDS-DMA, its share of 64 KiB) when that of the op at hand has its input. K and V rows
 // of earlier steps are read with sc1 loads: other CUs wrote them.
 // Every wait is bounded: one that gives up sets DevState::error kSmErrWait, the workgroup skips every later wait, the others'
-// waits give up too and the grid drains; the host then runs the steps as launches, and every later call of the model's.
+// waits give up too and the grid drains; the host then launches the loop over all XCDs, or runs the steps, and so every later call of
+// the model's.
 #pragma once
 #include "common.h"
 #include "prefill.h"

@@ -50,23 +50,25 @@ static __global__ void xcd_kernel(unsigned* count) {  // workgroups by XCC_ID
 }
 unsigned small_xcds(int per) {
     static std::mutex mu;
-    static std::map<int, unsigned> known;  // by device
+    static std::map<std::pair<int, int>, unsigned> known;  // by device and per
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     std::lock_guard<std::mutex> lock(mu);
-    const auto it = known.find(dev);
+    const auto it = known.find({dev, per});
     if (it != known.end()) return it->second;
     unsigned *n = nullptr, h[16] = {}, mask = 0;
+    bool asked = false;
     if (hipMalloc(&n, sizeof(h)) == hipSuccess && hipMemset(n, 0, sizeof(h)) == hipSuccess) {
         hipLaunchKernelGGL(xcd_kernel, dim3(8 * per), dim3(64), 0, nullptr, n);
-        if (hipMemcpy(h, n, sizeof(h), hipMemcpyDeviceToHost) == hipSuccess)
-            for (int i = 0; i < 16; ++i) mask |= h[i] == (unsigned)per ? 1u << i : 0u;
+        asked = hipGetLastError() == hipSuccess && hipMemcpy(h, n, sizeof(h), hipMemcpyDeviceToHost) == hipSuccess;
+        for (int i = 0; asked && i < 16; ++i) mask |= h[i] == (unsigned)per ? 1u << i : 0u;
         for (int i = 0; i < 16; ++i)
             if (h[i] && h[i] != (unsigned)per) mask = 0;
     }
     if (n) (void)hipFree(n);
     (void)hipGetLastError();
-    return known[dev] = mask;
+    if (asked) known[{dev, per}] = mask;  // (memory that was not there may be there for the next model)
+    return mask;
 }
 
 }  // namespace sli

@@ -271,6 +271,11 @@ class LlamaModel:
         """'mfma' (chunked MFMA GEMMs) or 'decode' (teacher-forced decode steps): sli_model_prefill_path."""
         return "mfma" if _lib.load().sli_model_prefill_path(self._h) == 1 else "decode"
 
+    def predict_path(self) -> str:
+        """How the last predict ran after its prompt's chunks: 'steps', or a small model's greedy loop as one launch over all XCDs ('all')
+        or on one ('one'): sli_model_predict_path."""
+        return ("steps", "all", "one")[_lib.load().sli_model_predict_path(self._h)]
+
     def fused_qkv_attn(self) -> int:
         """1 when the decode step runs q/k/v + attention as one launch per layer, 0 otherwise:
         sli_model_fused_qkv_attn."""

@@ -30,7 +30,9 @@ thread_local struct {
     size_t sh;
     void* s;
 } config;
-int wrong_device = 0, launches = 0, graph_launches = 0, mallocs = 0, fail_at = -1;
+int wrong_device = 0, launches = 0, graph_launches = 0, mallocs = 0, memsets = 0, fail_at = -1;
+bool xcds = false;
+std::string fail_launch;
 size_t room = (size_t)-1, used = 0, free_bytes = (size_t)1 << 36;
 std::map<int, int> mallocs_on, attributes_on;
 std::map<void*, size_t> live;
@@ -73,6 +75,9 @@ int hh_live() { return (int)live.size(); }
 void hh_fail_at(int k) { fail_at = k < 0 ? -1 : mallocs + k; }  // the k-th allocation from now (0: the next) fails
 void hh_free(size_t n) { free_bytes = n ? n : (size_t)1 << 36; }  // what hipMemGetInfo tells (0: 64 GiB)
 void hh_room(size_t n) { room = n ? used + n : (size_t)-1; }    // bytes left to allocate (0: no limit)
+int hh_memsets() { return memsets; }                           // of streams
+void hh_xcds(int on) { xcds = on; }                            // workgroups go to eight XCDs in turn (what xcd_kernel counts)
+void hh_fail_launch(const char* name) { fail_launch = name; }  // the next launch of such a kernel fails
 const char* hh_launched() {  // the kernels launched or recorded since the last call, one name a line
     names.clear();
     for (auto& n : launched) names += n + "\n";
@@ -133,6 +138,7 @@ int hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, siz
     });
 }
 int hipMemsetAsync(void* d, int v, size_t n, void* st) {
+    ++memsets;
     return queue(st, false, [=] { memset(d, v, n); });
 }
 int hipStreamCreateWithFlags(void** s, unsigned) {
@@ -161,7 +167,10 @@ int hipGraphDestroy(void* g) { return free(g), kOk; }
 int hipGraphExecDestroy(void* e) { return free(e), kOk; }
 int hipGraphLaunch(void*, void*) { return ++graph_launches, kOk; }
 int hipFuncSetAttribute(const void*, int, int) { return ++attributes_on[current], kOk; }
-int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void* st) {
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3, void** args, size_t, void* st) {
+    if (!fail_launch.empty() && kernels[f].find(fail_launch) != std::string::npos) return fail_launch.clear(), done(kInvalid);
+    if (xcds && kernels[f].find("xcd_kernel") != std::string::npos)
+        for (int i = 0; i < 8; ++i) (*(uint32_t**)args[0])[i] = grid.x / 8;
     Stream* s = (Stream*)st;
     if (s && s->device != current) ++wrong_device;
     if (!s || !s->capturing) ++launches;

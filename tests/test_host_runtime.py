@@ -180,6 +180,37 @@ def small_models_predict_in_one_launch(H):
         m.close()
 
 
+def small_models_on_one_xcd(H):
+    """A loop's launch on one XCD that did nothing (all of these, as kernels do nothing here) is not taken for its result but goes over
+    all XCDs, and one that failed leaves no tickets to the next."""
+    from simplellminference_amd import _lib
+    H.hh_xcds(1)
+    loops = lambda: set(re.findall(r"small_predict_kernelI\w+?Li(?:64|128)ELi(\d+)ELb([01])E", H.hh_launched().decode()))
+    one, over_all = ("16", "1"), ("8", "0")
+    m = _llama(w_dtype="f32", kv_dtype="f32")
+    H.hh_launched()
+    for again in range(2):
+        steps = H.hh_graph_launches()
+        m.predict([1, 2, 3], 30)
+        # (a launch over all XCDs is not asked whether it ran)
+        assert loops() == ({over_all} if again else {one, over_all}), again
+        assert m.predict_path() == "all" and H.hh_graph_launches() == steps, again
+    m.close()
+    m = _llama(w_dtype="f32", kv_dtype="f32")
+    had = H.hh_memsets()
+    H.hh_fail_launch(b"small_predict_kernel")
+    try:
+        m.predict([1, 2, 3], 30)
+        assert False, "the launch's error"
+    except _lib.SliError:
+        pass
+    assert H.hh_memsets() == had
+    m.predict([1, 2, 3], 30)
+    assert H.hh_memsets() == had + 1, "the tickets"
+    m.close()
+    assert H.hh_live() == 0
+
+
 def batched_inputs_share_a_launch(H):
     """A decode pass of a block with a feed-forward projects both of its inputs in one launch; without one there is one input."""
     from simplellminference_amd.stack import BlockSpec, StackModel, StackSpec
@@ -453,7 +484,7 @@ def steps_of_the_batched_projection(H):
 
 # ---------------------------------------------------------------- the tests
 CASES = ["device_of_predict", "scratch_that_does_not_fit", "scratch_of_smaller_chunks",
-         "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch",
+         "callers_arrays_are_read", "small_stacks_replay_their_prompts", "small_models_predict_in_one_launch", "small_models_on_one_xcd",
          "batched_inputs_share_a_launch", "attention_forms_of_a_prompt_pass", "weight_copies_where_they_are_read",
          "every_tiling_is_tested", "stack_prompts_take_the_fast_tilings", "stack_inputs_keep_their_sums", "prompts_take_the_fast_tilings",
          "first_steps_join_the_chunk_where_they_pay", "short_prompts_sum_in_short_chains",
