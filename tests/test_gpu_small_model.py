@@ -23,9 +23,14 @@ SHAPES = {"tiny": {}, "h128": dict(head_dim=128, hidden_size=512, kv_hidden_size
                      num_hidden_layers=1, vocab_size=50)}
 
 
+def _place(shape, w):
+    """Where the loop runs: over all XCDs with fp32 rows past 1 KiB or layers past 5 MB."""
+    return "all" if w == "f32" and shape in ("h128", "h8", "h6", "w2k") else "one"
+
+
 @pytest.mark.parametrize("w,kv", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("f32", "f16")])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_loop_matches_steps(gpu, shape, w, kv):
+def test_loop_matches_steps(gpu, shape, w, kv, place=None):
     m = _model(w, kv, max_length=150, **SHAPES[shape])
     V = m.config.vocab_size
     # one step; a prompt alone; past the keys of one pass (16 to 64) and of several; up to the last position
@@ -36,6 +41,7 @@ def test_loop_matches_steps(gpu, shape, w, kv):
         m.reset()
         for _ in range(2):
             assert np.array_equal(m.predict(ids, length), want), (n, length)
+            assert m.predict_path() == (place or _place(shape, w)), (n, length)
             log = m.logits()[0]
             # fp32 sums in another order (1e-6 of the norm); an fp16 cache rounds K and V either way (2^-11 of a value)
             assert np.linalg.norm(log - wl[-1]) <= (5e-6 if kv == "f32" else 5e-4) * np.linalg.norm(wl[-1]), (n, length)
@@ -60,7 +66,7 @@ def test_wait_that_gives_up(gpu, monkeypatch, shape, w):
     monkeypatch.setenv("SLI_DEBUG_SMALL_SPIN", "0")
     m = _model(w, w, max_length=150, **SHAPES[shape])
     for (ids, length), (tok, log, kv) in zip(calls, want):
-        assert np.array_equal(m.predict(ids, length), tok), length
+        assert np.array_equal(m.predict(ids, length), tok) and m.predict_path() == "steps", length
         # fp32: prompts of 9 and more run as chunks, their sums in another order
         assert np.linalg.norm(m.logits()[0] - log) <= (5e-6 if w == "f32" else 0) * np.linalg.norm(log), length
         for which in (0, 1):
@@ -96,7 +102,7 @@ def test_context_beyond_the_loop(gpu):
 def test_loop_over_all_xcds(gpu, monkeypatch, shape, w):
     """As test_loop_matches_steps, where that ran on one XCD."""
     monkeypatch.setenv("SLI_DEBUG_SMALL_ALL", "1")
-    test_loop_matches_steps(gpu, shape, w, w)
+    test_loop_matches_steps(gpu, shape, w, w, "all")
 
 
 def test_loop_of_many_units(gpu, monkeypatch):
@@ -119,13 +125,14 @@ def test_loops_side_by_side(gpu):
 
     def calls(i):
         for _ in range(6):
-            got[i].append(models[i].predict([i + 1, 7, 300 - i], 90))
+            got[i].append((models[i].predict([i + 1, 7, 300 - i], 90), models[i].predict_path()))
     threads = [threading.Thread(target=calls, args=(i,)) for i in range(len(models))]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
-    for m, g, w in zip(models, got, want):
-        assert len(g) == 6 and all(np.array_equal(x, w) for x in g)
+    for i, (m, g, w) in enumerate(zip(models, got, want)):
+        assert len(g) == 6 and all(np.array_equal(x, w) for x, _ in g)
+        assert "steps" not in {p for _, p in g}, i
         assert m.state()["error"] == 0
         m.close()
