@@ -18,7 +18,6 @@
 #include <unistd.h>
 
 #include <cmath>
-#include <condition_variable>
 #include <cstdlib>
 #include <type_traits>
 #include <cstring>
@@ -39,6 +38,7 @@
 #include "qkv_attn.h"
 #include "rope_table.h"
 #include "small_launch.h"
+#include "small_place.h"
 #include "step_state.h"
 #include "tp_layers.h"
 
@@ -633,11 +633,16 @@ static int tpl_launch(sli_model* m) {
 // (a wave's rows of an op no longer fit its LDS), so they keep them.
 constexpr int kSmWgs = 64;
 // On one XCD an edge goes through its L2 (a granule handed on in 0.26 us, to another XCD 0.55; an edge that all read 0.4 and 1.1 to 2),
-// and all weights through that XCD's share of the memory. us a step over all XCDs | on one: the fp32 preset 25.3 | 17.0, as fp16 30.4 | 15.6, 128
-// wide 29.4 | 13.9, 384 wide in fp16 34.3 | 20.6, 512 wide and 2048 units (8 MB a layer) 31.7 | 27.5; fp32 with 2048 units, 7 MB a layer,
-// 24.5 | 26.6, and rows past 1 KiB (fp32 wider than 256) 34.5 | 68. So fp32 up to kSmOneLayer bytes a layer.
-constexpr int kSmOneWgs = 32;  // an XCD's CUs
-constexpr size_t kSmOneLayer = 5 << 20;
+// and all weights through that XCD's share of the memory. Half of its CUs: all 32 of them take 17.5 us a step of the fp32 preset where
+// 16 take 19.4, but nothing else runs on that XCD for the whole loop then, and every other launch has a share there: a 7B step
+// beside such calls 20.7 ms, with half of the CUs 3.8 (beside loops over all XCDs 3.8, alone 2.6), a call of 0.6 ms beside a long one 141
+// ms and 0.7.
+constexpr int kSmOneWgs = 16;
+// Whether one XCD is the faster place: it saves 6 us a layer, less 0.9 for each MB of the layer's weights, and loses 1.2 us for 1000 rows of
+// the vocabulary. us a step over all XCDs | on one, 36 positions: fp32 256 wide, 2 layers, 512 tokens 24.6 | 19.4, 4096 26.5 | 25.9, 20000 35.7 |
+// 51.8, 12 layers 128 | 95, 125 | 101, 135 | 126; fp16 128 wide 29.8 | 15.1, 30.6 | 21.0, 39.6 | 50.9; fp16 384 wide 34.7 | 27.1, 37.4 |
+// 36.2, 12 layers and 20000 tokens 206 | 186; fp16 512 wide 31.9 | 30.6, 34.3 | 37.1. Rows past 1 KiB (fp32 wider than 256) 34.5 | 68.
+static bool small_on_one(int L, int V, size_t layer_bytes) { return (float)L * (6.0f - 0.9e-6f * (float)layer_bytes) > 1.2e-3f * (float)V; }
 // K of a head's context, which each of its workgroups reads: at 1000 positions of 64 (fp32) a step takes 6 us longer than at 36,
 // at 2048 about 24 and the launches are as fast soon after.
 constexpr size_t kSmMaxKey = 512 << 10;
@@ -659,7 +664,8 @@ static int small_alloc(sli_model* m) {
     const int nwg = groups(kSmWgs), hd = m->hd;
     if (nwg == 0) return SLI_OK;
     const size_t layer = m->wbytes * ((size_t)(m->hq + 2 * m->hkv) * hd * m->D + (size_t)m->D * m->hq * hd + 3 * (size_t)m->Il * m->D);
-    if (m->D * m->wbytes <= 1024 && (wd == SLI_DT_F16 || layer <= kSmOneLayer) && !std::getenv("SLI_DEBUG_SMALL_ALL") && small_xcds(kSmOneWgs))
+    if (m->D * m->wbytes <= 1024 && small_on_one(m->L, m->V, layer) && !std::getenv("SLI_DEBUG_SMALL_ALL") && kSmOneWgs <= device_cus() / 16 &&
+        small_xcds(kSmOneWgs))
         m->sm.one_nwg = groups(kSmOneWgs);
     m->sm.granules = (size_t)(m->hq + 2 * m->hkv) * hd + (size_t)m->hq * m->D + m->Il + m->D + 2 * nwg + 1;
     SLI_TRY(model_alloc(m, (void**)&m->sm.g, 8 * m->sm.granules));
@@ -679,50 +685,12 @@ static int small_alloc(sli_model* m) {
     return SLI_OK;
 }
 
-// Where a launch runs: on an XCD of its own (xcd, of those in `mask`), or over all of them (-1). A launch's workgroups wait for each
-// other, so no two launches of the process may each hold a part of what both need: launches on XCDs of their own, or launches over
-// all of them (64 workgroups each beside the chip's 256 CUs), but never both kinds at once. Threads are served in the order they came;
-// the place is given back when the launch has ended.
-struct SmallPlace {
-    struct Chip {
-        std::mutex mu;
-        std::condition_variable cv;
-        unsigned one = 0;  // XCDs taken
-        int all = 0;       // launches over all XCDs
-        unsigned long long next = 0, serving = 0;
-    };
-    Chip& chip;
-    int xcd = -1;
-    SmallPlace(int device, unsigned mask) : chip(of(device)) {
-        std::unique_lock<std::mutex> lock(chip.mu);
-        const unsigned long long mine = chip.next++;
-        chip.cv.wait(lock, [&] { return mine == chip.serving && ((chip.all == 0 && (mask & ~chip.one)) || chip.one == 0); });
-        if (chip.all == 0 && (mask & ~chip.one)) {
-            xcd = __builtin_ctz(mask & ~chip.one);
-            chip.one |= 1u << xcd;
-        } else {
-            ++chip.all;
-        }
-        ++chip.serving;
-        chip.cv.notify_all();
-    }
-    ~SmallPlace() {
-        std::lock_guard<std::mutex> lock(chip.mu);
-        if (xcd >= 0)
-            chip.one &= ~(1u << xcd);
-        else
-            --chip.all;
-        chip.cv.notify_all();
-    }
-    SmallPlace(const SmallPlace&) = delete;
-    SmallPlace& operator=(const SmallPlace&) = delete;
-    static Chip& of(int device) {
-        static std::mutex mu;
-        static std::map<int, Chip> chips;
-        std::lock_guard<std::mutex> lock(mu);
-        return chips[device];
-    }
-};
+static SmallPlace::Chip& small_chip(int device) {
+    static std::mutex mu;
+    static std::map<int, SmallPlace::Chip> chips;
+    std::lock_guard<std::mutex> lock(mu);
+    return chips[device];
+}
 
 // Whether positions below `length` take that launch
 static bool small_takes(const sli_model* m, int length) {
@@ -2549,8 +2517,9 @@ int sli_model_predict_batch(sli_model* m, const int32_t* prompts, const int32_t*
     m->sm.path = 0;
     while (loop && !m->sm.gave_up) {
         // (a launch on one XCD counts if the position moved: one of which no workgroup came to its XCD does nothing)
-        const SmallPlace place(m->c.device, m->sm.one_nwg > 0 && n0 + 1 < m->T ? small_xcds(kSmOneWgs) : 0);
-        const bool one = place.xcd >= 0;
+        const bool one = m->sm.one_nwg > 0 && n0 + 1 < m->T;
+        const SmallPlace place(small_chip(m->c.device), device_cus() / 8, one ? small_xcds(kSmOneWgs) : 0, one ? kSmOneWgs : 0, kSmWgs / 8,
+                               (int)getpid() % 8);
         SLI_TRY(small_steps(m, max_length - n0, place.xcd));
         DevState d{};
         SLI_HIP(hipMemcpyAsync(&d, m->st, sizeof(d), hipMemcpyDeviceToHost, m->stream));

@@ -3,17 +3,16 @@
 // the next token, with every dependency inside the launch.
 //
 // Why: a step of the 256-wide two-layer preset reads 7 MB (1 us), and its 13 graph launches of 2 to 8 us take 69. Here a step
-// has four all-to-all edges a layer and one for the token, each a store and a load and what a workgroup does between them: 17 us a step
-// on one XCD, 25 over all eight, 36 greedy tokens in 0.61 and 0.91 ms instead of 2.5. The edges bound it (and, with large
+// has four all-to-all edges a layer and one for the token, each a store and a load and what a workgroup does between them: 19.4 us a step
+// on half of one XCD, 25 over all eight, 36 greedy tokens in 0.70 and 0.90 ms instead of 2.5. The edges bound it (and, with large
 // vocabularies, the head's rows: small_launch.h small_lost_us), and within an edge the instructions: on one XCD a granule is handed on
 // in 0.3 of an edge's 1.8 us, the rest is some 200 instructions of 4 waves a SIMD. So sums end in one lane (sm_sum63), the norm's
 // factor is applied to finished sums, beside which its squares are added up, LDS is read by LDS loads only, and each wave asks for its
 // rows by 5 instructions a KiB (as 64-bit addresses and flat loads, each of them waited for, the same step took 28 us over all XCDs and 26
 // on one).
 //
-// Structure: hq J workgroups, all resident (ONE: of 16 waves on one XCD, where small_launch says; else of 8 waves over all of them);
-// every workgroup holds the whole residual row and runs every op on its
-// share of the rows. An edge is 8-byte {value, tag} granules as in tp_layers.h: one store each, no flag, no drain;
+// Structure: hq J workgroups, all resident (ONE: of 16 waves on half of one XCD's CUs; else of 8 waves, twice the workgroups, over all
+// XCDs: engine.hip small_on_one); every workgroup holds the whole residual row and runs every op on its share of the rows. An edge is 8-byte {value, tag} granules as in tp_layers.h: one store each, no flag, no drain;
 // readers sweep them with sc1 loads until the tags are this edge's. Between XCDs the stores are sc1 too; on one they end in its L2,
 // where sc1 loads look. Tags count (launch, step, layer, edge), so one array an
 // edge serves every layer: before a workgroup writes an edge's granules again it has read a later edge to which every

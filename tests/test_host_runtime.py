@@ -181,21 +181,26 @@ def small_models_predict_in_one_launch(H):
 
 
 def small_models_on_one_xcd(H):
-    """A loop's launch on one XCD that did nothing (all of these, as kernels do nothing here) is not taken for its result but goes over
-    all XCDs, and one that failed leaves no tickets to the next."""
+    """The loop's place by the model's sizes; a launch that did nothing (all of these, as kernels do nothing here) is not taken for its
+    result but goes over all XCDs, and one that failed leaves no tickets to the next."""
     from simplellminference_amd import _lib
     H.hh_xcds(1)
     loops = lambda: set(re.findall(r"small_predict_kernelI\w+?Li(?:64|128)ELi(\d+)ELb([01])E", H.hh_launched().decode()))
     one, over_all = ("16", "1"), ("8", "0")
-    m = _llama(w_dtype="f32", kv_dtype="f32")
-    H.hh_launched()
-    for again in range(2):
-        steps = H.hh_graph_launches()
-        m.predict([1, 2, 3], 30)
-        # (a launch over all XCDs is not asked whether it ran)
-        assert loops() == ({over_all} if again else {one, over_all}), again
-        assert m.predict_path() == "all" and H.hh_graph_launches() == steps, again
-    m.close()
+    wide = dict(hidden_size=512, num_attention_heads=8, num_key_value_heads=4, kv_hidden_size=256, intermediate_size=1536)
+    for w, over, place in (("f32", {}, one), ("f16", {}, one), ("f32", dict(vocab_size=4096), one), ("f32", dict(vocab_size=20000), over_all),
+                           ("f16", dict(vocab_size=20000), over_all), ("f32", dict(vocab_size=20000, num_hidden_layers=12), one),
+                           ("f32", dict(intermediate_size=2048), over_all), ("f32", wide, over_all), ("f16", wide, one),
+                           ("f16", dict(wide, vocab_size=4096), over_all)):
+        m = _llama(w_dtype=w, kv_dtype=w, over=over)
+        H.hh_launched()
+        for again in range(2):
+            steps = H.hh_graph_launches()
+            m.predict([1, 2, 3], 30)
+            # (a launch over all XCDs is not asked whether it ran)
+            assert loops() == ({one, over_all} if place == one and not again else {over_all}), (w, over, again)
+            assert m.predict_path() == "all" and H.hh_graph_launches() == steps, (w, over, again)
+        m.close()
     m = _llama(w_dtype="f32", kv_dtype="f32")
     had = H.hh_memsets()
     H.hh_fail_launch(b"small_predict_kernel")
