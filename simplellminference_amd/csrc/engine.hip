@@ -1196,12 +1196,14 @@ struct StepRecorder {
     // ---- prompt prefill (model.cpp:157-165 runs the prompt one token per forward; prefill.h): a chunk of
     // M prompt positions runs through every layer together, each projection one MFMA GEMM over the chunk
     // (weights read once per BM positions), attention block-causal over the cache rows the chunk's own qkv
-    // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); the last prompt
-    // position runs as an ordinary decode step. Phases as record_phase: 2l = qkv, attention, wo; 2l+1 =
-    // gate/up, down; under tensor parallelism each ends with the all-reduce of the chunk's residual rows.
+    // GEMM just wrote. No LM head: the prompt's logits are not used (teacher forcing); after a prefill the last prompt
+    // position runs as an ordinary decode step, in predict it may be a row of the chunk up to its last layer (record_last).
+    // Phases as record_phase: 2l = qkv, attention, wo; 2l+1 = gate/up, down; under tensor parallelism each ends with the all-reduce of
+    // the chunk's residual rows.
     // kv_only: the last layer. Nothing reads its residual rows, so it ends with the K and V rows that the cache keeps (no
     // attention, wo, gate/up and down of one layer in 32: 512 tokens of Llama-2-7B 17.01 -> 16.57 ms). A model of one layer,
     // which only serves to look at that layer's launches, runs it whole.
+    //
     // one GEMM over a chunk's rows: the tiling (prefill.h pg_tilings) whose plan costs least over the rows padded to its BM
     struct PgPick {
         int tiling = 0, M = 0;
