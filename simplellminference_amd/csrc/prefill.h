@@ -944,7 +944,7 @@ constexpr int kPgWsTiles = 4096;          // tiles cut at most (counters)
 // rolled: a looped epilogue (kRolled) is priced by the tiles a wave loops over: 0.7 us each, shared by the workgroups of a CU. That was
 // fitted to a stack's 25600 x 3072 at 384 rows, 100.6 us in 128 x 256 tiles (16 a wave) and 95.9 in 128 x 128 (8); a plain epilogue 84
 // and 90. It takes about half of that by now, and the price stays all the same: it sets where the depth is cut, so the order of a prompt's
-// sums. (0.35, and rows to spare as the output GEMM has, cut elsewhere at 15 of 36 row counts of a 2048-wide stack's two inputs and would
+// sums. (0.35, and rows to spare as the output GEMM has, pick other tiles or cuts at 10 of 36 row counts of a 2048-wide stack's two inputs and would
 // take 4.43 ms for 4.61 at 1280 rows, 4.03 for 4.09 at 1025.)
 template <class Cfg, typename WT>
 PgPlan pg_plan(int N, int K, int M, int cus, bool ws, float stage, bool rolled = false) {
